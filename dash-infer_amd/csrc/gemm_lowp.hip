@@ -485,13 +485,16 @@ static PanelPlan make_panel_plan(int wbits, int M, int N, int K, int group_size,
   return p;
 }
 
-// ---- batched decode, FRAG32 activations, register-resident K-slices (gemm_kslice_kernel.hpp) ---------------------
-// Context-phase GEMM, tail split (gemm_prefill_kernel.hpp, PrefillArgs::tail_cb): when the grid of 128 x 256 tiles ends in a
+// Context-phase GEMM, split in K (gemm_prefill_kernel.hpp, PrefillArgs::tail_cb): when the grid of 128 x 256 tiles ends in a
 // round that fills at most half the chip, the column blocks of that round are split in K instead -- `ksplit` workgroups per
 // tile, whole quantisation groups each, all of them within one round -- and a reduction launch adds the parts.  Qwen2-7B at
-// 2048 rows: qkv 288 tiles -> 256 + 32 x 7 parts (176 -> ~115 us), gate / up 2368 -> 2304 + 64 x 4.  DIHIP_PREFILL_TAIL_SPLIT=0: off.
+// 2048 rows: qkv 288 tiles -> 256 + 32 x 7 parts (176 -> ~115 us), gate / up 2368 -> 2304 + 64 x 4.  A grid that fills at most
+// half the chip altogether (a short prompt against a narrow matrix: 217 x 18944 -> 3584 is 28 tiles) is that round: all of its
+// tiles are split, and a part walks at least 512 of K: below, its prologue and its share of the slab cost what the split gains
+// (two prompts of 217 and 109 rows through four int8 layers of that width: 5.72 -> 2.39 ms).
+// DIHIP_PREFILL_TAIL_SPLIT=0: off.
 struct PrefillTail {
-  int col_blocks, mblocks, tail_cb, ksplit;
+  int col_blocks, mblocks, tail_cb, ksplit, kunit;
   size_t slab_bytes;
 };
 static PrefillTail prefill_tail_plan(int wbits, int M, int N, int K, int group_size, bool dual) {
@@ -502,18 +505,19 @@ static PrefillTail prefill_tail_plan(int wbits, int M, int N, int K, int group_s
   t.mblocks = (M + PF_BM - 1) / PF_BM;
   t.tail_cb = t.col_blocks;
   t.ksplit = 1;
+  t.kunit = d.group ? std::max(d.group / d.KTILE, 1) : 1;  // K parts hold whole groups (per-channel: whole k-tiles)
   static const bool on = !env_off("DIHIP_PREFILL_TAIL_SPLIT");
   int ncu = cached_num_cus();
   if (ncu <= 0) ncu = 256;
   const int blocks = t.col_blocks * t.mblocks, rem = blocks % ncu;
-  if (!on || M < 64 || (wbits != 4 && wbits != 8) || blocks <= ncu || rem == 0 || rem > ncu / 2) return t;
+  if (!on || M < 64 || (wbits != 4 && wbits != 8) || rem == 0 || rem > ncu / 2) return t;
   const int tcb = (rem + t.mblocks - 1) / t.mblocks, tiles = tcb * t.mblocks;
-  if (tiles > ncu / 2 || tcb >= t.col_blocks) return t;
-  const int ktpg = d.group ? d.group / d.KTILE : d.KT;
-  const int units = d.group ? d.KT / std::max(ktpg, 1) : d.KT;  // K parts hold whole groups (per-channel: whole k-tiles)
+  if (tiles > ncu / 2 || tcb > t.col_blocks) return t;
+  const bool all = tcb == t.col_blocks;
+  const int units = d.KT / t.kunit, at_least = all ? std::max(1, 512 / (d.KTILE * t.kunit)) : 1;
   int best = 1;
-  for (int ks = 2; ks <= 8; ++ks)
-    if (units % ks == 0 && tiles * ks <= ncu) best = ks;
+  for (int ks = 2; ks <= (all ? 16 : 8) && tiles * ks <= ncu && units / ks >= at_least; ++ks)
+    if ((units + ks - 1) / ks < (units + best - 1) / best) best = ks;  // the longest part decides; the fewest parts that reach it
   if (best == 1) return t;
   t.tail_cb = t.col_blocks - tcb;
   t.ksplit = best;
@@ -521,6 +525,7 @@ static PrefillTail prefill_tail_plan(int wbits, int M, int N, int K, int group_s
   return t;
 }
 
+// ---- batched decode, FRAG32 activations, register-resident K-slices (gemm_kslice_kernel.hpp) ---------------------
 struct KslicePlan {
   bool ok;
   int groups, nslices, waves, nunits;
@@ -915,12 +920,13 @@ static int run_gemm(hipStream_t stream, const GemmCall& c) {
     const int tiles_per_block = dual ? PF_WN * PF_CW / 2 : PF_WN * PF_CW;
     g.col_blocks = (d.NTILES + tiles_per_block - 1) / tiles_per_block;
     g.tail_cb = g.col_blocks;
-    g.ksplit = 1;
+    g.ksplit = g.kunit = 1;
     int blocks = g.col_blocks * ((c.M + PF_BM - 1) / PF_BM);
     const PrefillTail pt = prefill_tail_plan(c.wbits, c.M, c.N, c.K, c.group_size, dual);
     if (pt.ksplit > 1 && c.ws && c.ws_bytes >= pt.slab_bytes && reinterpret_cast<uintptr_t>(c.ws) % 16 == 0) {
       g.tail_cb = pt.tail_cb;
       g.ksplit = pt.ksplit;
+      g.kunit = pt.kunit;
       g.slab = reinterpret_cast<float*>(c.ws);
       blocks = pt.tail_cb * pt.mblocks + (pt.col_blocks - pt.tail_cb) * pt.mblocks * pt.ksplit;
     }
@@ -1239,10 +1245,12 @@ static int norm_to_ws(hipStream_t s, const float* h, const void* gamma, float ep
     slab = std::max(slab, make_panel_plan(wbits, M, N, K, group_size, dual).slab_bytes);
     slab = std::max(slab, make_kslice_plan(wbits, M, N, K, group_size, dual, true).slab_bytes);
   }
-  const size_t off = (slab + 255) & ~(size_t)255;
+  size_t off = (slab + 255) & ~(size_t)255;
   const bool frag = force_frag || batch_kernel_shape(wbits, M, N, K, group_size, dual);  // (bf16 and f16: both instantiated since round 5)
   const int mt = M > 16 ? 2 : 1;
   const size_t xbytes = frag ? (size_t)mt * 16 * K * 2 : (size_t)M * K * 2;
+  // (a workspace sized for another row count may lack the slab of this one's K split: the GEMM then runs unsplit)
+  if (wbits != 16 && M >= 64 && ws_bytes < off + xbytes) off = (p.slab_bytes + 255) & ~(size_t)255;
   DIHIP_REQUIRE(ws && ws_bytes >= off + xbytes, DIHIP_MEMORY_ERROR, "fused gemm: workspace too small");
   *xnorm = reinterpret_cast<char*>(ws) + off;
   *ws_left = off;

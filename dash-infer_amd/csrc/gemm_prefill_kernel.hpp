@@ -88,12 +88,14 @@ struct PrefillArgs {
   int Gp;      // (scale, zero) groups stored per tile
   int ktpg;    // k-tiles per quantisation group (per-channel: >= KT)
   int col_blocks;
-  // Tail split (round 5): column blocks [tail_cb, col_blocks) -- the workgroups that would otherwise run as a last, mostly empty
-  // round on the chip (qkv of Qwen2-7B at 2048 rows: 288 tiles on 256 CUs) -- are walked by `ksplit` workgroups each, one
-  // K range apiece (whole quantisation groups), which leave their f32 tile in `slab`; gemm_prefill_tail_reduce_kernel adds the
-  // parts in order and applies the epilogue.  tail_cb == col_blocks: no split.
+  // Split in K: column blocks [tail_cb, col_blocks) -- the workgroups that would otherwise run as a last, mostly empty
+  // round on the chip (qkv of Qwen2-7B at 2048 rows: 288 tiles on 256 CUs), or all of them where the whole grid fills at most half
+  // of it (short prompts) -- are walked by `ksplit` workgroups each, one K range apiece (whole quantisation groups; the ranges
+  // differ by at most one), which leave their f32 tile in `slab`; gemm_prefill_tail_reduce_kernel adds the parts in order and
+  // applies the epilogue.  tail_cb == col_blocks: no split.
   int tail_cb;
   int ksplit;
+  int kunit;    // k-tiles that a K range must not cut (grouped weights: a group; per-channel: 1)
   float* slab;  // [tail tile][ksplit][PF_BM][256] f32
   unsigned long long* trace;  // per-wave cycle stamps (library built with -DDIHIP_PF_TRACE, tools/prefill_trace.py)
 };
@@ -131,9 +133,9 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
     split_part = t % a.ksplit;
     const int cbt = t / a.ksplit;
     cb = a.tail_cb + cbt;
-    const int per = a.KT / a.ksplit;
-    kt0 = split_part * per;
-    kt1 = kt0 + per;
+    const int ku = GPT ? 1 : a.kunit, units = a.KT / ku;
+    kt0 = split_part * units / a.ksplit * ku;
+    kt1 = split_part + 1 == a.ksplit ? a.KT : (split_part + 1) * units / a.ksplit * ku;
     split_tile = cbt * mblocks + mb;
   }
   const int m0 = mb * PF_BM;
@@ -297,11 +299,12 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
   }
 #undef DIHIP_PF_STAMP
 
-  // ---- tail split: this part's f32 tile to the slab (rows / columns of the workgroup tile; SwiGLU: gate columns, then up) ----
+  // ---- split in K: this part's f32 tile to the slab (rows / columns of the workgroup tile; SwiGLU: gate columns, then up) ----
   if (split_part >= 0) {  // (uniform)
     float* st = a.slab + ((size_t)split_tile * a.ksplit + split_part) * (PF_BM * 256);
 #pragma unroll
-    for (int rt = 0; rt < PF_RT; ++rt)
+    for (int rt = 0; rt < PF_RT; ++rt) {
+      if (m0 + (wm * PF_RT + rt) * 16 >= a.M) break;  // (uniform) rows past M are never read
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = (wm * PF_RT + rt) * 16 + kb * 4 + r;
@@ -311,6 +314,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
           st[(size_t)row * 256 + col] = tot[rt][c][r];
         }
       }
+    }
     return;
   }
   // ---- epilogue: lane (kb, ni) holds rows rt * 16 + kb * 4 + r of column tile c, column ni --------------------
@@ -351,7 +355,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
   }
 }
 
-// tail split: the K parts of every split tile added in order + the epilogue of gemm_prefill_kernel
+// split in K: the K parts of every split tile added in order + the epilogue of gemm_prefill_kernel
 template <int FT, int EPI>
 __global__ __launch_bounds__(256) void gemm_prefill_tail_reduce_kernel(const PrefillArgs a) {
   constexpr bool DUAL = EPI == EPI_SWIGLU;

@@ -672,3 +672,40 @@ def test_prefill_gemm_tail_split(ops, wbits, G, M, N, K):
     u = gemm_ref.gemm_a16wx(x, qu, su, zu, G, wbits, round_out=False).astype(np.float64)
     assert_close(act.float().cpu().numpy(), bf16_round(((g / (1 + np.exp(-g))) * u).astype(np.float32)), "bf16", what=f"tail split SwiGLU ({parts2} parts)")
     print(f"\n[prefill tail split] W{wbits} g{G} M{M} N{N} K{K}: {parts} parts per tail tile; SwiGLU pair N{Ns}: {parts2}")
+
+
+# The same split over a whole grid that leaves most of the chip idle (short prompts): K ranges of unequal length, a last row block of one row,
+# and a workspace sized without the slab (another row count's), which must run unsplit with the same result.
+@pytest.mark.gpu
+@pytest.mark.parametrize("wbits,G,M,N,K", [(4, 128, 64, 272, 1664),     # 13 groups in 3 parts: 4, 4, 5
+                                           (4, 256, 129, 520, 2816),    # 11 groups of two k-tiles; one row in the second row block
+                                           (8, -1, 217, 3584, 4736),    # per channel: 74 k-tiles in 9 parts
+                                           (8, 128, 100, 256, 8192)])   # the most parts
+def test_prefill_gemm_whole_grid_split(ops, wbits, G, M, N, K):
+    from dash_infer_amd.capi import lib
+    rng = np.random.default_rng(M + N + K + wbits)
+    x, q, s, z = make_case(rng, M, N, K, G, wbits, "bf16", style="iq")
+    pw = ops.pack_lowp(to_dev(q), to_dev(s, "bf16"), to_dev(z, "bf16"), G, wbits)
+    xd = to_dev(x, "bf16")
+    need = ops.lowp_workspace_bytes(wbits, M, N, K, G)
+    sc = ops.Scratch(need)
+    parts = int(lib().dihip_gemm_prefill_tail_parts(wbits, M, N, K, G, 0))
+    assert parts > 1 and K // parts >= 512
+    bias = bf16_round(rng.normal(0, 0.3, N).astype(np.float32))
+    y = ops.gemm_lowp(xd, pw, bias=to_dev(bias, "bf16"), act="silu", alpha=0.5, scratch=sc)
+    ref = gemm_ref.gemm_a16wx(x, q, s, z, G, wbits, alpha=0.5, bias=bias, act="silu", ft="bf16")
+    assert_close(y.float().cpu().numpy(), ref, "bf16", what=f"grid split STD ({parts} parts)", pre=ref)
+    h = rng.normal(0, 1.5, (M, N)).astype(np.float32)
+    h2 = ops.fused_gemm_addto(xd, pw, to_dev(h), sc, M=M)
+    ref = h + gemm_ref.gemm_a16wx(x, q, s, z, G, wbits, round_out=False)
+    np.testing.assert_allclose(h2.cpu().numpy(), ref, rtol=2e-5, atol=3e-5 * np.abs(ref).max())
+    if (M, K) != (217, 4736):
+        return
+    # norm + GEMM from a workspace that is 256 bytes short of the slab and the normalised rows (in the narrow shapes the general kernel's slab is
+    # the larger one, and has always been asked for)
+    slab = parts * -(-M // 128) * -(-N // 256) * 128 * 256 * 4
+    small = ops.Scratch(slab + M * K * 2 - 256)
+    gamma = to_dev(bf16_round(rng.normal(1, 0.1, K).astype(np.float32)), "bf16")
+    rows = to_dev(rng.normal(0, 1, (M, K)).astype(np.float32))
+    a, b = ops.fused_norm_gemm(rows, gamma, 1e-6, pw, None, sc).float(), ops.fused_norm_gemm(rows, gamma, 1e-6, pw, None, small).float()
+    assert float((a - b).abs().max()) <= 2 ** -7 * float(b.abs().max())     # f32 sums in another order, rounded to bf16
