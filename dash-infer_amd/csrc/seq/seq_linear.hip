@@ -1,9 +1,12 @@
 // seq_linear.hip -- dihip_linear: y = epilogue(x . W^T + bias) for row-major [N, K] weights as checkpoints store them,
-// grouped (block-diagonal / per-head) forms included.  Three kernels:
+// grouped (block-diagonal / per-head) forms included.  The kernels:
 //   linear_tile_kernel   every product and sum in f32, k ascending (DIHIP_MATH_F32; also any operand type / odd shape)
 //   linear_mfma_kernel   bf16 operands on the 16x16x32 matrix-core tiles, 128 x 128 x 32 block tiles, f32 accumulation
-//   linear_skinny_kernel up to 4 rows at a time against a streamed weight (decode): one wave per 4 weight rows
-// An output element is computed by one thread (or one MFMA column) over k in a fixed order: it does not depend on T.
+//   linear_stream_kernel bf16 operands, 2 .. 64 rows: weights straight from memory into the matrix cores, K split over a workgroup's waves
+//   linear_skinny_kernel one row against a streamed weight (decode), one wave per 2 weight rows; up to 4 rows at a time in f32 products
+//   linear_fewcols_kernel a router's logits
+// Within a kernel an output element is summed over k in a fixed order: it does not depend on T.
+#include <type_traits>
 #include "seq_common.h"
 
 namespace dihip {
@@ -191,6 +194,133 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(LinArgs a) {
         if (t < t_hi && n < a.N) lin_epilogue(a, g, t, n, acc[i][j][r], DIHIP_BF16);
       }
     }
+}
+
+// ------------------------------------------------------------------------------------------ weight-streaming kernel, matrix cores
+// Up to 64 rows against weights that are read once (decoding steps of a batch, short portions).  Bound by the weights' bytes and by what the
+// workgroups pull of the activations, so everything serves the loads in flight:
+//   * a workgroup owns ROWS weight rows and its WV waves split K among them (block b of 128 elements belongs to wave b % WV): a narrow
+//     matrix still gives every wave a stream of its own, and at any time the workgroup reads adjacent blocks of the same rows;
+//   * weights and activations go straight from memory into MFMA operands (the weight rows are the A operand: a lane ends with 4
+//     neighbouring columns of one output row); a wave issues all loads of a block before the first product, and with PRE the weights of
+//     its next block as well.  Nothing is staged, no barrier before the end: the activations (T x K bf16) live in the L2s;
+//   * the waves' partial sums meet in LDS and are added in the order of the waves: an element's sum does not depend on the rows beside it.
+// 24 rows: 8192 -> 2048 180 -> 24 us, 2048 -> 8192 57 -> 16, 4096 -> 14336 100 -> 41, 4096 -> 32000 104 -> 69 (before: 128 x 128 tiles); 13 rows
+// (before: four passes of the kernel below) 77 -> 18, 41 -> 12, 121 -> 35, 230 -> 69.  What is left is the activations: each workgroup
+// pulls T x K of them from its L2 for ROWS x K weights (one row alone: 15, 11, 28, 54 us).
+// K % 8 == 0 and 16-byte aligned rows (host-checked).
+template <int XT>
+__device__ __forceinline__ u32x4_t stream_x(const char* p, bool ok) {
+  u32x4_t r = {0u, 0u, 0u, 0u};
+  if (ok) {
+    if constexpr (XT == DIHIP_F32) {
+      const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(p), hi = *reinterpret_cast<const f32x4_t*>(p + 16);
+      r = u32x4_t{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]), pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
+    } else {
+      r = *reinterpret_cast<const u32x4_t*>(p);
+    }
+  }
+  return r;
+}
+
+constexpr int STREAM_MAX_ROWS = 64;
+constexpr int STREAM_SPLIT_K = 256;   // shorter walks are not split
+
+template <int XT, int ROWS, int TF, int WV, bool PRE>
+__global__ __launch_bounds__(64 * WV, (ROWS * TF > 64 || XT == DIHIP_F32) ? 2 : 4) void linear_stream_kernel(LinArgs a) {
+  constexpr int RF = ROWS / 16, U = 4, BK = U * 32;
+  constexpr int XE = XT == DIHIP_F32 ? 4 : 2;
+  __shared__ __attribute__((aligned(16))) f32x4_t red[WV][RF * TF][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int i16 = lane & 15, q = lane >> 4;
+  const int g = blockIdx.y, n0 = blockIdx.x * ROWS;
+  int lo, hi;
+  lin_rows(a, g, lo, hi);
+  if (lo >= hi) return;
+  const int count = min(hi - lo, 16 * TF);
+  const uint16_t* wp[RF];   // rows past N re-read the last one, rows past the group's the last of those: never stored
+#pragma unroll
+  for (int r = 0; r < RF; ++r) wp[r] = (const uint16_t*)a.w + ((size_t)g * a.N + min(n0 + r * 16 + i16, a.N - 1)) * a.K + q * 8;
+  const char* xp[TF];
+#pragma unroll
+  for (int t = 0; t < TF; ++t)
+    xp[t] = (const char*)a.x + (lin_xrow(a, lo + min(t * 16 + i16, count - 1)) * a.ldx + (size_t)(g % a.xgroups) * a.xg + q * 8) * XE;
+  const f32x4_t z4 = {0.f, 0.f, 0.f, 0.f};
+  f32x4_t acc[RF][TF];
+#pragma unroll
+  for (int r = 0; r < RF; ++r)
+#pragma unroll
+    for (int t = 0; t < TF; ++t) acc[r][t] = z4;
+  auto walk = [&](auto whole) {   // WHOLE: K is a multiple of the block; else lanes past K read nothing and multiply zeros
+    constexpr bool WHOLE = decltype(whole)::value;
+    auto load_w = [&](u32x4_t (&w)[U][RF], int k) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int r = 0; r < RF; ++r) {
+          if constexpr (!WHOLE) w[u][r] = u32x4_t{0u, 0u, 0u, 0u};
+          if (WHOLE || k + u * 32 + q * 8 < a.K) w[u][r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(wp[r] + k + u * 32));
+        }
+    };
+    u32x4_t w[U][RF], wn[U][RF];
+    // a short K is one wave's: the sum of the tile kernel, bit for bit
+    const int first = a.K >= STREAM_SPLIT_K ? wave * BK : (wave == 0 ? 0 : a.K), step = a.K >= STREAM_SPLIT_K ? WV * BK : BK;
+    if (PRE && first < a.K) load_w(w, first);
+    for (int k = first; k < a.K; k += step) {
+      u32x4_t x[U][TF];
+      if constexpr (!PRE) load_w(w, k);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int t = 0; t < TF; ++t) x[u][t] = stream_x<XT>(xp[t] + (size_t)(k + u * 32) * XE, WHOLE || k + u * 32 + q * 8 < a.K);
+      if (PRE && k + step < a.K) load_w(wn, k + step);   // (uniform)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int r = 0; r < RF; ++r) {
+#pragma unroll
+          for (int t = 0; t < TF; ++t) acc[r][t] = mfma_bf16(w[u][r], x[u][t], acc[r][t]);
+          if constexpr (PRE) w[u][r] = wn[u][r];
+        }
+    }
+  };
+  if (a.K % BK == 0) walk(std::true_type{});
+  else walk(std::false_type{});
+#pragma unroll
+  for (int r = 0; r < RF; ++r)
+#pragma unroll
+    for (int t = 0; t < TF; ++t) red[wave][r * TF + t][lane] = acc[r][t];
+  __syncthreads();
+  for (int e = tid; e < RF * TF * 64; e += 64 * WV) {   // 4 neighbouring columns of one row
+    const int f = e >> 6, l = e & 63, t = (f % TF) * 16 + (l & 15), n = n0 + (f / TF) * 16 + (l >> 4) * 4;
+    if (t >= count) continue;
+    f32x4_t v = red[0][f][l];
+#pragma unroll
+    for (int i = 1; i < WV; ++i) v += red[i][f][l];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (n + r < a.N) lin_epilogue(a, g, lo + t, n + r, v[r], DIHIP_BF16);
+  }
+}
+
+template <int XT, int ROWS, int WV, bool PRE>
+void launch_stream(const LinArgs& a, int Tg, int groups, hipStream_t s) {
+  const dim3 grid((a.N + ROWS - 1) / ROWS, groups), threads(64 * WV);
+  const int tf = (Tg + 15) / 16;
+  if (tf <= 1) hipLaunchKernelGGL((linear_stream_kernel<XT, ROWS, 1, WV, PRE>), grid, threads, 0, s, a);
+  else if (tf == 2) hipLaunchKernelGGL((linear_stream_kernel<XT, ROWS, 2, WV, PRE>), grid, threads, 0, s, a);
+  else if (tf == 3) hipLaunchKernelGGL((linear_stream_kernel<XT, ROWS, 3, WV, PRE>), grid, threads, 0, s, a);
+  else hipLaunchKernelGGL((linear_stream_kernel<XT, ROWS, 4, WV, PRE>), grid, threads, 0, s, a);
+}
+// weight rows per workgroup: more of them re-read the activations less often, but the workgroups have to fill 256 CUs.  16 / 32 / 64 at
+// 24 rows: 4096 -> 4096 15.1 / 18.8 / 28, 4096 -> 6144 25.0 / 22.4 / 24, 4096 -> 14336 43.1 / 40.9 / 36.9, 4096 -> 32000 106 / 84 / 69 us; at
+// 4 rows the activations are cheap and 16 is never behind.
+template <int XT>
+void launch_stream_rows(const LinArgs& a, int Tg, int groups, hipStream_t s) {
+  const long n = (long)a.N * groups;
+  if (Tg > 16 && n >= 16384) launch_stream<XT, 64, 4, false>(a, Tg, groups, s);
+  else if (Tg > 8 && n >= 6144) launch_stream<XT, 32, 4, true>(a, Tg, groups, s);
+  else launch_stream<XT, 16, 8, true>(a, Tg, groups, s);
 }
 
 // ------------------------------------------------------------------------------------------ weight-streaming kernel
@@ -390,14 +520,15 @@ static int linear_impl(void* stream, const void* x, int x_dtype, long ldx, long 
     math = DIHIP_MATH_F32;
   }
   if (math == DIHIP_MATH_BF16 && w_dtype == DIHIP_BF16) {
-    const int tmax = K <= 8192 ? 4 : (K <= 16384 ? 2 : 1);  // rows whose bf16 copy fits 64 KB of LDS
-    if (Tg <= 4 * tmax && vec && !no_skinny && K <= 32768) {
-      for (int t0 = 0; t0 < Tg; t0 += tmax) {
-        const int tc = Tg - t0 < tmax ? Tg - t0 : tmax;
-        const dim3 grid((N + 7) / 8, groups);
-        if (x_dtype == DIHIP_F32) hipLaunchKernelGGL((linear_skinny_kernel<DIHIP_F32, false>), grid, dim3(256), (size_t)tc * K * 2, s, a, t0, tc);
-        else hipLaunchKernelGGL((linear_skinny_kernel<DIHIP_BF16, false>), grid, dim3(256), (size_t)tc * K * 2, s, a, t0, tc);
-      }
+    if (Tg == 1 && vec && !no_skinny && K <= 32768) {   // the row's bf16 copy fits 64 KB of LDS
+      const dim3 grid((N + 7) / 8, groups);
+      if (x_dtype == DIHIP_F32) hipLaunchKernelGGL((linear_skinny_kernel<DIHIP_F32, false>), grid, dim3(256), (size_t)K * 2, s, a, 0, 1);
+      else hipLaunchKernelGGL((linear_skinny_kernel<DIHIP_BF16, false>), grid, dim3(256), (size_t)K * 2, s, a, 0, 1);
+      return launch_status();
+    }
+    if (Tg <= STREAM_MAX_ROWS && vec) {
+      if (x_dtype == DIHIP_F32) launch_stream_rows<DIHIP_F32>(a, Tg, groups, s);
+      else launch_stream_rows<DIHIP_BF16>(a, Tg, groups, s);
       return launch_status();
     }
     const dim3 grid((N + 127) / 128, (Tg + 127) / 128, groups);

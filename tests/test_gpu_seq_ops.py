@@ -49,6 +49,43 @@ def test_linear_f32_and_bf16(so, T, N, K, groups, wdt):
     assert rel_err(y16.cpu().numpy(), ref(xr, w)) < 2e-5      # same rounded operands, f32 accumulation
 
 
+@pytest.mark.parametrize("T,N,K,groups", [(2, 33, 256, 1), (16, 16, 264, 1), (17, 6160, 392, 1), (9, 6145, 1032, 1), (33, 40, 1024, 2), (48, 100, 2056, 1),
+                                          (64, 16385, 256, 1), (18, 16400, 520, 1), (65, 32, 512, 1), (5, 17, 4096, 3), (24, 1024, 64, 1), (30, 70, 8, 4), (20, 6200, 248, 1)])
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float32])
+def test_linear_streams_few_rows(so, T, N, K, groups, xdt):
+    """Row counts at the edges of the 16-row operands, outputs at the edges of 16 / 32 / 64 weight rows, K that is no whole block (or shorter than
+    the waves' blocks together), strided rows, every part of the epilogue: products of the same rounded operands in 64 bits."""
+    rng = np.random.default_rng(T * 100 + N + K)
+    wide = dev(rng.normal(0, 1, (T, groups * K + 16)), xdt)
+    x = wide[:, 8:8 + groups * K]
+    w, b = dev(rng.normal(0, K ** -0.5, (groups, N, K)), torch.bfloat16), dev(rng.normal(0, 0.3, (groups, N)), torch.bfloat16)
+    mul = dev(rng.normal(0, 1, (T, groups * N)))
+    lo, hi = N // 3, groups * N - 2
+    xr = x.to(torch.bfloat16).double()
+    want = torch.cat([xr[:, g * K:(g + 1) * K] @ w[g].double().t() + b[g].double() for g in range(groups)], 1)
+    plain = want.clone()
+    want[:, lo:hi] = torch.nn.functional.gelu(want[:, lo:hi], approximate="tanh")
+    wt, bt = (w[0], b[0]) if groups == 1 else (w, b)
+    y = so.linear(x, wt, bt, act="gelu_tanh", act_cols=(lo, hi), mul=mul, math=so.MATH_BF16, groups=groups)
+    assert rel_err(y.cpu().numpy(), (want * mul.double()).cpu().numpy()) < 2e-5
+    out = torch.zeros(T, groups * N + 7, dtype=torch.bfloat16, device="cuda")
+    so.linear(x, wt, bt, math=so.MATH_BF16, groups=groups, out=out[:, 3:3 + groups * N])
+    assert rel_err(out[:, 3:3 + groups * N].float().cpu().numpy(), plain.cpu().numpy()) < 2.0 ** -8      # one rounding of the result
+    assert float(out[:, :3].abs().max()) == 0 and float(out[:, -4:].abs().max()) == 0
+
+
+def test_linear_segmented_streams_few_rows(so):
+    rng = np.random.default_rng(77)
+    counts = [0, 1, 16, 5, 40, 0]
+    seg = np.cumsum([0] + counts)
+    R, N, K = int(seg[-1]), 50, 328
+    x, w = dev(rng.normal(0, 1, (30, K)), torch.bfloat16), dev(rng.normal(0, K ** -0.5, (len(counts), N, K)), torch.bfloat16)
+    rows = rng.integers(0, 30, R)
+    y = so.linear_segmented(x, w, torch.tensor(seg, dtype=torch.int32).cuda(), torch.tensor(rows, dtype=torch.int32).cuda(), max(counts), R, math=so.MATH_BF16)
+    want = torch.cat([x[torch.tensor(rows[seg[g]:seg[g + 1]]).cuda()].double() @ w[g].double().t() for g in range(len(counts))])
+    assert rel_err(y.cpu().numpy(), want.cpu().numpy()) < 2e-5
+
+
 def test_linear_rows_do_not_depend_on_the_batch(so):
     rng = np.random.default_rng(5)
     K, N = 192, 100
