@@ -1,42 +1,18 @@
 // seq_linear.hip -- dihip_linear: y = epilogue(x . W^T + bias) for row-major [N, K] weights as checkpoints store them,
 // grouped (block-diagonal / per-head) forms included.  The kernels:
 //   linear_tile_kernel   every product and sum in f32, k ascending (DIHIP_MATH_F32; also any operand type / odd shape)
-//   linear_mfma_kernel   bf16 operands on the 16x16x32 matrix-core tiles, 128 x 128 x 32 block tiles, f32 accumulation
+//   linear_pipe_kernel   bf16 operands on the matrix cores, pipelined tiles of 256 x 256 or 128 x 128, K split where tiles are few (seq_linear_tile.hip)
+//   linear_mfma_kernel   the same for f32 rows (rounded to bf16), K % 64 != 0 or unaligned operands: 128 x 128 x 32 tiles through registers
 //   linear_stream_kernel bf16 operands, 2 .. 64 rows: weights straight from memory into the matrix cores, K split over a workgroup's waves
 //   linear_skinny_kernel one row against a streamed weight (decode), one wave per 2 weight rows; up to 4 rows at a time in f32 products
 //   linear_fewcols_kernel a router's logits
 // Within a kernel an output element is summed over k in a fixed order: it does not depend on T.
+#include <algorithm>
 #include <type_traits>
-#include "seq_common.h"
+#include "seq_linear.h"
 
 namespace dihip {
 namespace {
-
-struct LinArgs {
-  const void* x; long ldx, xg; int xgroups;
-  const void* w; const void* bias;
-  void* y; long ldy, yg;
-  const float* mul; long ldm;
-  int T, N, K, act, act_lo, act_hi, ydt, round_ops;
-  int mul_group; float act_param;               // mul holds one number per group; the parameter of an activation that has one
-  const int32_t* seg; const int32_t* row_map;   // segmented form: group g owns the output rows seg[g] .. seg[g + 1], row r reads x row row_map[r]
-};
-
-// the rows of group g: [lo, hi)
-__device__ __forceinline__ void lin_rows(const LinArgs& a, int g, int& lo, int& hi) {
-  lo = 0; hi = a.T;
-  if (a.seg) { lo = a.seg[g]; hi = a.seg[g + 1]; }
-}
-__device__ __forceinline__ size_t lin_xrow(const LinArgs& a, int r) { return (size_t)(a.row_map ? a.row_map[r] : r); }
-
-__device__ __forceinline__ void lin_epilogue(const LinArgs& a, int g, int t, int n, float v, int wdt) {
-  if (a.bias) v += ld_any(a.bias, (size_t)g * a.N + n, wdt);
-  const int col = g * a.N + n;
-  if (col >= a.act_lo && col < a.act_hi) v = a.act == DIHIP_SEQ_ACT_SOFTCAP ? a.act_param * tanhf(v / a.act_param) : apply_act(v, a.act);
-  const size_t o = (size_t)t * a.ldy + (size_t)g * a.yg + n;
-  if (a.mul) v *= a.mul[(size_t)t * a.ldm + (a.mul_group ? (size_t)g : (size_t)g * a.yg + n)];
-  st_any(a.y, o, a.ydt, v);
-}
 
 // ------------------------------------------------------------------------------------------ exact f32 tile kernel
 template <int XT, int WT>
@@ -94,10 +70,6 @@ __global__ __launch_bounds__(256) void linear_tile_kernel(LinArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------ bf16 matrix-core kernel
-__device__ __forceinline__ f32x4_t mfma_bf16(const u32x4_t& a, const u32x4_t& b, const f32x4_t& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
-
 // 8 consecutive k of one row as packed bf16; VEC: the 8 are in range and 16-byte aligned (host-checked), else guarded
 template <int XT, bool VEC>
 __device__ __forceinline__ u32x4_t load8_bf16(const void* p, size_t i, int kleft, bool row_ok) {
@@ -122,7 +94,7 @@ __device__ __forceinline__ u32x4_t load8_bf16(const void* p, size_t i, int kleft
 }
 
 template <int XT, bool VEC>
-__global__ __launch_bounds__(256) void linear_mfma_kernel(LinArgs a) {
+__global__ __launch_bounds__(256) void linear_mfma_kernel(LinArgs a, bool vec4) {
   constexpr int BK = 32, UPR = BK / 8, UN = 128 * UPR / 256;   // k per step (64 measured slower: fewer workgroups per CU), 16-byte units per tile row, units per thread
   constexpr int LD = BK + 8;  // bf16 elements per LDS row: 8 of padding (80 bytes: 16-byte aligned fragments)
   __shared__ __attribute__((aligned(16))) uint16_t As[128 * LD];
@@ -178,22 +150,20 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(LinArgs a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = mfma_bf16(af[i], bf[j], acc[i][j]);
+        for (int j = 0; j < 4; ++j) acc[i][j] = mfma_bf16(bf[j], af[i], acc[i][j]);
     }
     __syncthreads();
   }
-  asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");  // the matrix pipe's write-back before the results are read
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int j = 0; j < 4; ++j) {   // a lane holds 4 neighbouring columns
+    const int n = n0 + wn * 64 + j * 16 + (lane >> 4) * 4;
+    const f32x4_t b = lin_bias4(a, g, n, vec4);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + wn * 64 + j * 16 + (lane & 15);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = m0 + wm * 64 + i * 16 + (lane >> 4) * 4 + r;
-        if (t < t_hi && n < a.N) lin_epilogue(a, g, t, n, acc[i][j][r], DIHIP_BF16);
-      }
+    for (int i = 0; i < 4; ++i) {
+      const int t = m0 + wm * 64 + i * 16 + (lane & 15);
+      if (t < t_hi) lin_epilogue4(a, g, t, n, acc[i][j], b, vec4);
     }
+  }
 }
 
 // ------------------------------------------------------------------------------------------ weight-streaming kernel, matrix cores
@@ -227,7 +197,7 @@ constexpr int STREAM_MAX_ROWS = 64;
 constexpr int STREAM_SPLIT_K = 256;   // shorter walks are not split
 
 template <int XT, int ROWS, int TF, int WV, bool PRE>
-__global__ __launch_bounds__(64 * WV, (ROWS * TF > 64 || XT == DIHIP_F32) ? 2 : 4) void linear_stream_kernel(LinArgs a) {
+__global__ __launch_bounds__(64 * WV, (ROWS * TF > 64 || XT == DIHIP_F32) ? 2 : 4) void linear_stream_kernel(LinArgs a, bool vec4) {
   constexpr int RF = ROWS / 16, U = 4, BK = U * 32;
   constexpr int XE = XT == DIHIP_F32 ? 4 : 2;
   __shared__ __attribute__((aligned(16))) f32x4_t red[WV][RF * TF][64];
@@ -297,9 +267,7 @@ __global__ __launch_bounds__(64 * WV, (ROWS * TF > 64 || XT == DIHIP_F32) ? 2 : 
     f32x4_t v = red[0][f][l];
 #pragma unroll
     for (int i = 1; i < WV; ++i) v += red[i][f][l];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (n + r < a.N) lin_epilogue(a, g, lo + t, n + r, v[r], DIHIP_BF16);
+    lin_epilogue4(a, g, lo + t, n, v, lin_bias4(a, g, n, vec4), vec4);
   }
 }
 
@@ -307,10 +275,11 @@ template <int XT, int ROWS, int WV, bool PRE>
 void launch_stream(const LinArgs& a, int Tg, int groups, hipStream_t s) {
   const dim3 grid((a.N + ROWS - 1) / ROWS, groups), threads(64 * WV);
   const int tf = (Tg + 15) / 16;
-  if (tf <= 1) hipLaunchKernelGGL((linear_stream_kernel<XT, ROWS, 1, WV, PRE>), grid, threads, 0, s, a);
-  else if (tf == 2) hipLaunchKernelGGL((linear_stream_kernel<XT, ROWS, 2, WV, PRE>), grid, threads, 0, s, a);
-  else if (tf == 3) hipLaunchKernelGGL((linear_stream_kernel<XT, ROWS, 3, WV, PRE>), grid, threads, 0, s, a);
-  else hipLaunchKernelGGL((linear_stream_kernel<XT, ROWS, 4, WV, PRE>), grid, threads, 0, s, a);
+  const bool vec4 = lin_vec4(a);
+  if (tf <= 1) hipLaunchKernelGGL((linear_stream_kernel<XT, ROWS, 1, WV, PRE>), grid, threads, 0, s, a, vec4);
+  else if (tf == 2) hipLaunchKernelGGL((linear_stream_kernel<XT, ROWS, 2, WV, PRE>), grid, threads, 0, s, a, vec4);
+  else if (tf == 3) hipLaunchKernelGGL((linear_stream_kernel<XT, ROWS, 3, WV, PRE>), grid, threads, 0, s, a, vec4);
+  else hipLaunchKernelGGL((linear_stream_kernel<XT, ROWS, 4, WV, PRE>), grid, threads, 0, s, a, vec4);
 }
 // weight rows per workgroup: more of them re-read the activations less often, but the workgroups have to fill 256 CUs.  16 / 32 / 64 at
 // 24 rows: 4096 -> 4096 15.1 / 18.8 / 28, 4096 -> 6144 25.0 / 22.4 / 24, 4096 -> 14336 43.1 / 40.9 / 36.9, 4096 -> 32000 106 / 84 / 69 us; at
@@ -483,7 +452,7 @@ using namespace dihip;
 static int linear_impl(void* stream, const void* x, int x_dtype, long ldx, long x_gstride, int x_groups, const void* w,
                        int w_dtype, const void* bias, void* y, int y_dtype, long ldy, long y_gstride, const float* mul,
                        long ldm, int mul_group, int T, int N, int K, int groups, int act, int act_lo, int act_hi, float act_param, int math,
-                       const int32_t* seg, const int32_t* row_map, int seg_max_rows) {
+                       const int32_t* seg, const int32_t* row_map, int seg_max_rows, void* ws, size_t ws_bytes) {
   DIHIP_REQUIRE(T >= 0 && N > 0 && K > 0 && groups > 0 && x_groups > 0, DIHIP_PARAM_ERROR, "linear: bad shape T %d N %d K %d groups %d", T, N, K, groups);
   DIHIP_REQUIRE(seq_dtype_ok(x_dtype) && seq_dtype_ok(w_dtype) && seq_dtype_ok(y_dtype), DIHIP_PARAM_ERROR, "linear: f32 / bf16 only");
   DIHIP_REQUIRE(x && w && y, DIHIP_PARAM_ERROR, "linear: null pointer");
@@ -531,14 +500,22 @@ static int linear_impl(void* stream, const void* x, int x_dtype, long ldx, long 
       else launch_stream_rows<DIHIP_BF16>(a, Tg, groups, s);
       return launch_status();
     }
+    if (vec && x_dtype == DIHIP_BF16) {
+      // (segments: planned for twice the average, the bound is often all rows)
+      const int rows = seg ? (int)std::min<long>(Tg, 1 + 2L * T / groups) : Tg;
+      LinTilePlan p = plan_linear_tile(rows, N, K, groups, ldx, !seg && ws);
+      if (p.ok && p.slab > ws_bytes) p = plan_linear_tile(rows, N, K, groups, ldx, false);
+      if (p.ok) return launch_linear_tile(a, p, Tg, groups, (float*)ws, s);
+    }
     const dim3 grid((N + 127) / 128, (Tg + 127) / 128, groups);
     DIHIP_REQUIRE(grid.y <= 65535, DIHIP_PARAM_ERROR, "linear: too many rows for one launch");
+    const bool vec4 = lin_vec4(a);
     if (x_dtype == DIHIP_F32) {
-      if (vec) hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_F32, true>), grid, dim3(256), 0, s, a);
-      else hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_F32, false>), grid, dim3(256), 0, s, a);
+      if (vec) hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_F32, true>), grid, dim3(256), 0, s, a, vec4);
+      else hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_F32, false>), grid, dim3(256), 0, s, a, vec4);
     } else {
-      if (vec) hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_BF16, true>), grid, dim3(256), 0, s, a);
-      else hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_BF16, false>), grid, dim3(256), 0, s, a);
+      if (vec) hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_BF16, true>), grid, dim3(256), 0, s, a, vec4);
+      else hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_BF16, false>), grid, dim3(256), 0, s, a, vec4);
     }
     return launch_status();
   }
@@ -557,7 +534,21 @@ extern "C" int dihip_linear(void* stream, const void* x, int x_dtype, long ldx, 
                             long ldm, int mul_group, int T, int N, int K, int groups, int act, int act_lo, int act_hi,
                             float act_param, int math) {
   return linear_impl(stream, x, x_dtype, ldx, x_gstride, x_groups, w, w_dtype, bias, y, y_dtype, ldy, y_gstride, mul, ldm, mul_group, T, N, K, groups,
-                     act, act_lo, act_hi, act_param, math, nullptr, nullptr, 0);
+                     act, act_lo, act_hi, act_param, math, nullptr, nullptr, 0, nullptr, 0);
+}
+
+extern "C" size_t dihip_linear_workspace_bytes(int T, int N, int K, int groups, long ldx) {
+  if (T <= STREAM_MAX_ROWS || N <= 0 || K <= 0 || groups <= 0) return 0;
+  return plan_linear_tile(T, N, K, groups, ldx, true).slab;
+}
+
+extern "C" int dihip_linear_ws(void* stream, const void* x, int x_dtype, long ldx, long x_gstride, int x_groups, const void* w,
+                               int w_dtype, const void* bias, void* y, int y_dtype, long ldy, long y_gstride, const float* mul,
+                               long ldm, int mul_group, int T, int N, int K, int groups, int act, int act_lo, int act_hi,
+                               float act_param, int math, void* ws, size_t ws_bytes) {
+  DIHIP_REQUIRE(!ws || aligned16(ws), DIHIP_PARAM_ERROR, "linear: a workspace starts on 16 bytes");
+  return linear_impl(stream, x, x_dtype, ldx, x_gstride, x_groups, w, w_dtype, bias, y, y_dtype, ldy, y_gstride, mul, ldm, mul_group, T, N, K, groups,
+                     act, act_lo, act_hi, act_param, math, nullptr, nullptr, 0, ws, ws_bytes);
 }
 
 extern "C" int dihip_linear_segmented(void* stream, const void* x, int x_dtype, long ldx, const void* w, int w_dtype, const void* bias,
@@ -566,5 +557,5 @@ extern "C" int dihip_linear_segmented(void* stream, const void* x, int x_dtype, 
   DIHIP_REQUIRE(seg && seg_max_rows >= 0, DIHIP_PARAM_ERROR, "linear_segmented: no segment table");
   if (seg_max_rows == 0) return DIHIP_SUCCESS;
   return linear_impl(stream, x, x_dtype, ldx, 0, 1, w, w_dtype, bias, y, y_dtype, ldy, 0, nullptr, 0, 0, R, N, K, groups, act, 0,
-                     act ? groups * N : 0, 0.f, math, seg, row_map, seg_max_rows);
+                     act ? groups * N : 0, 0.f, math, seg, row_map, seg_max_rows, nullptr, 0);
 }

@@ -21,6 +21,9 @@ _SIGS = {
     "dihip_seq_version": (C.c_char_p, []),
     "dihip_seq_last_error": (C.c_char_p, []),
     "dihip_linear": (i32, [vp, vp, i32, lng, lng, i32, vp, i32, vp, vp, i32, lng, lng, vp, lng, i32, i32, i32, i32, i32, i32, i32, i32, f32, i32]),
+    "dihip_linear_workspace_bytes": (sz, [i32, i32, i32, i32, lng]),
+    "dihip_linear_ws": (i32, [vp, vp, i32, lng, lng, i32, vp, i32, vp, vp, i32, lng, lng, vp, lng, i32, i32, i32, i32, i32, i32, i32, i32, f32, i32, vp,
+                              sz]),
     "dihip_embed_sum": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32]),
     "dihip_embed_rows": (i32, [vp, vp, i32, lng, vp, vp, i32, lng, lng, f32, i32, i32]),
     "dihip_rmsnorm_strided": (i32, [vp, vp, i32, lng, vp, lng, vp, vp, i32, f32, f32, f32, i32, i32]),

@@ -32,6 +32,9 @@ def _rows(t):
     return t.stride(0)
 
 
+LINEAR_FEW_ROWS = 64     # up to here a product never takes a workspace
+
+
 def linear(x, w, bias=None, out=None, act=None, act_cols=None, mul=None, math=MATH_F32, groups=1, x_groups=None, mul_group=False,
            act_param=0.0):
     """y = epilogue(x . w^T + bias).  w: [N, K] (groups == 1) or [groups, N, K]; x: [T, x_groups * K] (group g reads the K
@@ -52,9 +55,13 @@ def linear(x, w, bias=None, out=None, act=None, act_cols=None, mul=None, math=MA
     lo, hi = (0, groups * N) if act_cols is None else act_cols
     if act is None:
         lo = hi = 0
-    check(lib().dihip_linear(stream(), ptr(x), dt(x), _rows(x), K, xg, ptr(w), dt(w), ptr(bias), ptr(y), dt(y), _rows(y), N,
-                             ptr(mul), _rows(mul) if mul is not None else 0, 1 if mul_group else 0, T, N, K, groups, ACT[act], lo, hi, float(act_param), math),
-          "dihip_linear")
+    ws, need = None, 0
+    if T > LINEAR_FEW_ROWS and math == MATH_BF16 and x.dtype == w.dtype == torch.bfloat16:     # tiles that do not fill the chip split K
+        need = int(lib().dihip_linear_workspace_bytes(T, N, K, groups, _rows(x)))
+        ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+    check(lib().dihip_linear_ws(stream(), ptr(x), dt(x), _rows(x), K, xg, ptr(w), dt(w), ptr(bias), ptr(y), dt(y), _rows(y), N, ptr(mul),
+                                _rows(mul) if mul is not None else 0, 1 if mul_group else 0, T, N, K, groups, ACT[act], lo, hi, float(act_param), math,
+                                ptr(ws), need), "dihip_linear_ws")
     return y
 
 

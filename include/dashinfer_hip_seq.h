@@ -26,7 +26,7 @@ const char* dihip_seq_version(void);
 const char* dihip_seq_last_error(void);
 
 /* math of dihip_linear: EXACT = every product and sum in f32, k ascending; BF16 = operands rounded to bf16, f32
- * accumulation on the matrix cores (T > DIHIP_LINEAR_SKINNY_ROWS) or in a weight-streaming dot-product kernel */
+ * accumulation on the matrix cores (one row: in a weight-streaming dot-product kernel) */
 enum { DIHIP_MATH_F32 = 0, DIHIP_MATH_BF16 = 1, DIHIP_MATH_F32_STREAM = 2 };
 /* F32_STREAM = F32 products of the unrounded operands, but few rows (decoding) stream the weight through the dot-product
  * kernel, whose sums run in the lanes' order: for the f32 parts of a bf16 engine (gates of a recurrence) */
@@ -42,6 +42,15 @@ int dihip_linear(void* stream, const void* x, int x_dtype, long ldx, long x_gstr
                  const void* w, int w_dtype, const void* bias, void* y, int y_dtype, long ldy, long y_gstride,
                  const float* mul, long ldm, int mul_group, int T, int N, int K, int groups, int act, int act_lo, int act_hi,
                  float act_param, int math);
+
+/* The same with a workspace (16-byte aligned; contents irrelevant): bf16 rows whose tiles would leave most of the chip idle are then
+ * computed in parts of K that meet in it.  dihip_linear_workspace_bytes: what the call can use (0: nothing); with less, or NULL, K is
+ * not split. */
+size_t dihip_linear_workspace_bytes(int T, int N, int K, int groups, long ldx);
+int dihip_linear_ws(void* stream, const void* x, int x_dtype, long ldx, long x_gstride, int x_groups,
+                    const void* w, int w_dtype, const void* bias, void* y, int y_dtype, long ldy, long y_gstride,
+                    const float* mul, long ldm, int mul_group, int T, int N, int K, int groups, int act, int act_lo, int act_hi,
+                    float act_param, int math, void* ws, size_t ws_bytes);
 
 /* The same product for rows that are grouped by owner (mixture of experts): group g owns the output rows seg[g] .. seg[g + 1]
  * (seg: [groups + 1] on the device, ascending, seg[groups] <= R), output row r reads the x row row_map[r] (NULL: r itself) and

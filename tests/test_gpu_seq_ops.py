@@ -74,6 +74,50 @@ def test_linear_streams_few_rows(so, T, N, K, groups, xdt):
     assert float(out[:, :3].abs().max()) == 0 and float(out[:, -4:].abs().max()) == 0
 
 
+@pytest.mark.parametrize("T,N,K,groups", [(65, 64, 64, 1), (128, 128, 128, 1), (129, 130, 192, 1), (257, 255, 1024, 1), (513, 2048, 576, 1), (300, 36, 2048, 3),
+                                          (100, 512, 8192, 1), (2049, 1028, 64, 1), (700, 16, 4096, 1), (1030, 4100, 320, 2)])
+@pytest.mark.parametrize("ws", [True, False])
+def test_linear_tiles_many_rows(so, T, N, K, groups, ws):
+    """bf16 rows in pipelined tiles: rows and columns at the edges of 128 and 256, the shortest walks (one and two steps), K in parts and -- without a
+    workspace -- whole; strided rows, every part of the epilogue in both store forms.  Products of the same operands in 64 bits."""
+    rng = np.random.default_rng(T + N + K)
+    wide = torch.randn(T, groups * K + 16, generator=torch.Generator("cuda").manual_seed(T), device="cuda").to(torch.bfloat16)
+    x = wide[:, 8:8 + groups * K]
+    w, b = dev(rng.normal(0, K ** -0.5, (groups, N, K)), torch.bfloat16), dev(rng.normal(0, 0.3, (groups, N)), torch.bfloat16)
+    mul = dev(rng.normal(0, 1, (T, groups * N)))
+    lo, hi = N // 3, groups * N - 2
+    want = torch.cat([x[:, g * K:(g + 1) * K].double() @ w[g].double().t() + b[g].double() for g in range(groups)], 1)
+    plain = want.clone()
+    want[:, lo:hi] = torch.nn.functional.gelu(want[:, lo:hi], approximate="tanh")
+    wt, bt = (w[0], b[0]) if groups == 1 else (w, b)
+    few, so.LINEAR_FEW_ROWS = so.LINEAR_FEW_ROWS, (so.LINEAR_FEW_ROWS if ws else 1 << 30)
+    try:
+        y = so.linear(x, wt, bt, act="gelu_tanh", act_cols=(lo, hi), mul=mul, math=so.MATH_BF16, groups=groups)
+        out = torch.zeros(T, groups * N + 8, dtype=torch.bfloat16, device="cuda")
+        so.linear(x, wt, bt, math=so.MATH_BF16, groups=groups, out=out[:, 4:4 + groups * N])
+        odd = torch.zeros(T, groups * N + 7, device="cuda")
+        so.linear(x, wt, bt, math=so.MATH_BF16, groups=groups, out=odd[:, 3:3 + groups * N])
+    finally:
+        so.LINEAR_FEW_ROWS = few
+    assert rel_err(y.cpu().numpy(), (want * mul.double()).cpu().numpy()) < 2e-5
+    assert rel_err(out[:, 4:4 + groups * N].float().cpu().numpy(), plain.cpu().numpy()) < 2.0 ** -8      # one rounding of the result
+    assert float(out[:, :4].abs().max()) == 0 and float(out[:, -4:].abs().max()) == 0
+    assert rel_err(odd[:, 3:3 + groups * N].cpu().numpy(), plain.cpu().numpy()) < 2e-5 and float(odd[:, -4:].abs().max()) == 0
+
+
+def test_linear_segmented_tiles(so):
+    rng = np.random.default_rng(78)
+    counts = [0, 1, 300, 129, 64, 0]
+    seg = np.cumsum([0] + counts)
+    R, N, K = int(seg[-1]), 140, 192
+    x, w = dev(rng.normal(0, 1, (90, K)), torch.bfloat16), dev(rng.normal(0, K ** -0.5, (len(counts), N, K)), torch.bfloat16)
+    rows = rng.integers(0, 90, R)
+    for bound in (300, 10 ** 6):
+        y = so.linear_segmented(x, w, torch.tensor(seg, dtype=torch.int32).cuda(), torch.tensor(rows, dtype=torch.int32).cuda(), bound, R, math=so.MATH_BF16)
+        want = torch.cat([x[torch.tensor(rows[seg[g]:seg[g + 1]]).cuda()].double() @ w[g].double().t() for g in range(len(counts))])
+        assert rel_err(y.cpu().numpy(), want.cpu().numpy()) < 2e-5
+
+
 def test_linear_segmented_streams_few_rows(so):
     rng = np.random.default_rng(77)
     counts = [0, 1, 16, 5, 40, 0]
