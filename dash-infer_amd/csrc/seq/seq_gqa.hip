@@ -615,6 +615,234 @@ __global__ __launch_bounds__(256) void gqa_attn_mc_kernel(GqaArgs a) {
   }
 }
 
+// The same for head sizes of exactly 64 or 128 and pages of whole 64-key tiles (D / DV compile-time: no guard inside the walk).
+//   * a workgroup owns 64 * MT (row, query head) pairs, 16 * MT per wave: with MT = 2 every key and value operand read from LDS serves two products;
+//   * 64-key tiles go straight into LDS (global_load_lds, two copies): the loads of the next tile are issued behind the one barrier of a tile and
+//     have that tile's time to land.  The 16-byte chunks of a row change places on the memory side (keys: chunk ^ key; values: pairs
+//     of chunks ^ key), so that neither the operand reads nor the transposing reads meet in a bank;
+//   * the mask is looked at only in tiles where some pair of the wave does not see every key; exp2 with the scale folded in;
+//   * row tiles are dealt so that the two workgroups a CU holds have together the same walk (up to 512 of them), else longest first.
+// A portion of 2048 rows, 32 heads of 128 over 8 key heads: 300 -> 77 us (115 -> 447 TFLOP/s; with capped scores 89); 500 rows beside 13 decoded ones, 16
+// heads over 4: 139 -> 27; 24 decoded rows at 160 .. 700 keys, five splits: 21 -> 11.  The kernel above, which tests the head sizes inside the walk,
+// waited for every tile's loads.  What bounds this one is the instruction stream between the products (softmax: ~180 vector
+// instructions per 64 products).
+template <int D, int DV, int MT, bool CAP>
+__global__ __launch_bounds__(256, 2) void gqa_attn_tile_kernel(GqaArgs a, int gx) {
+  constexpr int KS = D / 32, DT = DV / 16, NT = 4, TABLE = 128;
+  constexpr int KROW = D * 2, VROW = DV * 2, KBYTES = 64 * KROW, VBYTES = 64 * VROW, COPY = KBYTES + VBYTES;
+  constexpr int KPP = 1024 / KROW, VPP = 1024 / VROW;                 // keys per 1 KiB piece
+  constexpr int KPW = 64 / KPP / 4, VPW = 64 / VPP / 4;               // pieces per wave and tile: piece wave + 4 j
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ const char* ktabs[TABLE];
+  __shared__ const char* vtabs[TABLE];
+  const int G = a.G, H = a.H, hpg = H / G, M = a.maps, GK = G * M, gy = gridDim.x / gx;
+  // linear index -> (row tile, portion and key head)
+  int tile_x, ey;
+  {
+    const int lin = blockIdx.x, total = gridDim.x;
+    const int order = total <= 512 && lin >= total / 2 ? lin - total / 2 : total - 1 - lin;
+    tile_x = order / gy;
+    ey = order - tile_x * gy;
+  }
+  const int e = ey / GK, gk = ey - e * GK, g = gk / M, mp = gk - g * M, split = blockIdx.z, nsplit = gridDim.z;
+  const int cnt = a.ent_count[e], row0 = a.ent_row0[e];
+  const int nrows = cnt * hpg, r0 = tile_x * (64 * MT);
+  if (r0 >= nrows) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ni = lane & 15, kb = lane >> 4;
+  const int pos0 = a.tok_pos[row0], end = pos0 + cnt - 1;             // the sequence's last position
+  const int p_lo = pos0 + r0 / hpg, p_hi = pos0 + min(r0 + 64 * MT - 1, nrows - 1) / hpg;
+  const int win_t0 = (a.window > 0 ? max(0, p_lo - a.window + 1) : 0) >> 6;
+  const int n_first = min(win_t0, (min(a.keep_first, p_hi + 1) + 63) >> 6);
+  const int n_tiles = n_first + (p_hi >> 6) - win_t0 + 1;
+  const int per = (n_tiles + nsplit - 1) / nsplit;
+  const int my_lo = split * per, my_hi = min(n_tiles - 1, my_lo + per - 1);
+  auto tile_of = [&](int i) { return i < n_first ? i : win_t0 + (i - n_first); };
+  // this wave's pairs
+  const int w0 = r0 + wave * 16 * MT;
+  const int wp_lo = pos0 + min(w0, nrows - 1) / hpg, wp_hi = pos0 + min(w0 + 16 * MT - 1, nrows - 1) / hpg;   // positions of its first and last pair
+  const bool wave_on = w0 < nrows;
+  int hq[MT], tq[MT], h[MT];
+  bool ok[MT];
+  u32x4_t qf[MT][KS];
+  f32x4_t oacc[MT][DT];
+  float m[MT], l[MT];
+  constexpr float LOG2E = 1.44269504088896341f;
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int r = w0 + i * 16 + ni, rr = min(r, nrows - 1);
+    ok[i] = r < nrows;
+    tq[i] = rr / hpg;
+    h[i] = g * hpg + (rr - tq[i] * hpg);
+    hq[i] = h[i] * M + mp;
+    const float* qrow = a.q + (size_t)(row0 + tq[i]) * a.ldq + (size_t)hq[i] * D + kb * 8;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(qrow + ks * 32), hi = *reinterpret_cast<const f32x4_t*>(qrow + ks * 32 + 4);
+      qf[i][ks] = u32x4_t{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]), pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
+    }
+    const bool with_sink = a.sink_mode != 0 && split == 0;
+    m[i] = with_sink ? (a.sink_mode == 1 ? ld_any(a.sink, h[i], a.wdt) * LOG2E : 0.f) : -1e30f;      // scores and maxima: times log2 e
+    l[i] = with_sink && kb == 0 ? 1.f : 0.f;                            // (a lane's own keys: summed over kb at the end)
+#pragma unroll
+    for (int t = 0; t < DT; ++t) oacc[i][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  void* const* gkp = a.kspans + (size_t)a.ent_slot[e] * a.span_stride;
+  void* const* gv = a.vspans + (size_t)a.ent_slot[e] * a.span_stride;
+  // span pointers of the walk, TABLE at a time
+  auto fill = [&](int first) {
+    for (int i = tid; i < TABLE; i += 256) {
+      const bool in = (long)(first + i) * a.span_len <= p_hi;
+      ktabs[i] = in ? (const char*)gload<void*>(gkp + first + i) : nullptr;
+      vtabs[i] = in ? (const char*)gload<void*>(gv + first + i) : nullptr;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __syncthreads();
+  };
+  int table0 = my_lo <= my_hi ? tile_of(my_lo) * 64 / a.span_len : 0;
+  fill(table0);
+  // where this lane's 16 bytes of a piece come from
+  const int kk = lane / (KROW / 16), kc = lane % (KROW / 16), vk = lane / (VROW / 16), vc = lane % (VROW / 16);
+  const int kkey = wave * KPP + kk, vkey = wave * VPP + vk;            // key of piece `wave`; piece wave + 4 j: 4 j KPP further
+  const uint32_t koff = (uint32_t)(kkey * GK + gk) * KROW + (uint32_t)((kc ^ (D == 128 ? kkey & 15 : kkey & 7)) * 16);
+  const uint32_t voff = (uint32_t)(vkey * G + g) * VROW + (uint32_t)((vc ^ (DV == 128 ? (vkey & 7) * 2 : ((vkey >> 1) & 3) * 2)) * 16);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem + wave * 1024;
+  auto fetch = [&](int i, int copy) {
+    const int key0 = tile_of(i) * 64, sp = key0 / a.span_len, in = key0 - sp * a.span_len;
+    if (sp - table0 >= TABLE || sp < table0) {    // (uniform)
+      __syncthreads();
+      table0 = sp;
+      fill(table0);
+    }
+    const uint64_t ka = (uint64_t)ktabs[sp - table0], va = (uint64_t)vtabs[sp - table0];
+    const uint64_t ku = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)ka) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(ka >> 32)) << 32;
+    const uint64_t vu = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)va) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(va >> 32)) << 32;
+    const char* kp = (const char*)ku + (size_t)in * GK * KROW;
+    const char* vp = (const char*)vu + (size_t)in * G * VROW;
+#pragma unroll
+    for (int j = 0; j < KPW; ++j)
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds0 + copy * COPY + j * 4096), "v"(koff),
+                   "s"(kp + (size_t)j * 4 * KPP * GK * KROW) : "memory");
+#pragma unroll
+    for (int j = 0; j < VPW; ++j)
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds0 + copy * COPY + KBYTES + j * 4096), "v"(voff),
+                   "s"(vp + (size_t)j * 4 * VPP * G * VROW) : "memory");
+  };
+  // operand addresses: keys nt * 16 + ni, chunks ks * 4 + kb; values rows kb * 4 + ni / 4 (+ 16, + 32 ..), chunks 2 t + ni % 4 / 2
+  int kfo[KS], vfo[DT];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) kfo[ks] = ni * KROW + (((ks * 4 + kb) ^ (D == 128 ? ni : ni & 7)) * 16);
+  {
+    const int vr = kb * 4 + (ni >> 2), f = DV == 128 ? (vr & 7) * 2 : ((vr >> 1) & 3) * 2;
+#pragma unroll
+    for (int t = 0; t < DT; ++t) vfo[t] = KBYTES + vr * VROW + (((2 * t) ^ f) + ((ni & 3) >> 1)) * 16 + (ni & 1) * 8;
+  }
+  const float sl2 = a.scale * LOG2E, cap = a.softcap, cap_in = CAP ? 2.f * a.scale * LOG2E / cap : 0.f, cap2 = cap * LOG2E;
+  if (my_lo <= my_hi) fetch(my_lo, 0);
+  for (int ti = my_lo; ti <= my_hi; ++ti) {
+    const int copy = (ti - my_lo) & 1, key0 = tile_of(ti) * 64;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();     // the tile has landed; the other copy has been read
+    asm volatile("" ::: "memory");
+    if (ti + 1 <= my_hi) fetch(ti + 1, copy ^ 1);
+    const unsigned char* base = smem + copy * COPY;
+    if (key0 + 63 > end) {            // (uniform) rows that no token has written: an infinity there would reach the sums through a weight of 0
+      for (int i = tid; i < (key0 + 63 - end) * (VROW / 16); i += 256)
+        *reinterpret_cast<u32x4_t*>(const_cast<unsigned char*>(base) + KBYTES + (size_t)(end + 1 - key0) * VROW + i * 16) = u32x4_t{0u, 0u, 0u, 0u};
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+    if (!wave_on || key0 > wp_hi) continue;
+    if (a.window > 0 && key0 + 63 <= wp_lo - a.window && key0 >= a.keep_first) continue;   // before every window of the wave
+    f32x4_t sacc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) sacc[i][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      u32x4_t kf[NT];
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) kf[nt] = *reinterpret_cast<const u32x4_t*>(base + kfo[ks] + nt * 16 * KROW);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) sacc[i][nt] = mfma_bf16g(kf[nt], qf[i][ks], sacc[i][nt]);
+    }
+    const bool whole = key0 + 63 <= wp_lo && (a.window <= 0 || wp_hi - key0 < a.window || key0 + 63 < a.keep_first);   // (uniform)
+    u32x4_t pf[MT][2];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int p = pos0 + tq[i];
+      float mx = -INFINITY;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float s;
+          if constexpr (CAP) s = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(sacc[i][nt][r] * cap_in));   // cap * tanh(s / cap)
+          else s = sacc[i][nt][r] * sl2;
+          if (!whole) {
+            const int key = key0 + nt * 16 + kb * 4 + r;
+            if (!(key <= p && (a.window <= 0 || p - key < a.window || key < a.keep_first))) s = -INFINITY;
+          }
+          sacc[i][nt][r] = s;
+          mx = fmaxf(mx, s);
+        }
+      mx = fmaxf(m[i], rows_max(mx));
+      const float corr = __builtin_amdgcn_exp2f(m[i] - mx);
+      m[i] = mx;
+      float ps = 0.f;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          sacc[i][nt][r] = __builtin_amdgcn_exp2f(sacc[i][nt][r] - mx);
+          ps += sacc[i][nt][r];
+        }
+      l[i] = l[i] * corr + ps;
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh)
+        pf[i][hh] = u32x4_t{pack_bf16x2(sacc[i][2 * hh][0], sacc[i][2 * hh][1]), pack_bf16x2(sacc[i][2 * hh][2], sacc[i][2 * hh][3]),
+                            pack_bf16x2(sacc[i][2 * hh + 1][0], sacc[i][2 * hh + 1][1]), pack_bf16x2(sacc[i][2 * hh + 1][2], sacc[i][2 * hh + 1][3])};
+      if (__builtin_amdgcn_ballot_w64(corr != 1.f) != 0ull) {
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) oacc[i][t][r] *= corr;
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        const u32x2_t lo2 = lds_read_tr16(base + vfo[t] + hh * 32 * VROW), hi2 = lds_read_tr16(base + vfo[t] + hh * 32 * VROW + 16 * VROW);
+        const u32x4_t vf = {lo2[0], lo2[1], hi2[0], hi2[1]};
+#pragma unroll
+        for (int i = 0; i < MT; ++i) oacc[i][t] = mfma_bf16g(vf, pf[i][hh], oacc[i][t]);
+      }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // nothing may be on its way into LDS when the workgroup leaves
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const float den = rows_sum(l[i]);
+    if (!ok[i]) continue;
+    if (nsplit == 1) {
+      const float inv = (a.gate ? a.gate[(size_t)(row0 + tq[i]) * a.ldg + h[i]] : 1.f) / den;
+      const size_t o = (size_t)(row0 + tq[i]) * a.ldo + (size_t)hq[i] * DV + kb * 4;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+        store4(a.out, o + t * 16, a.odt, f32x4_t{oacc[i][t][0] * inv, oacc[i][t][1] * inv, oacc[i][t][2] * inv, oacc[i][t][3] * inv});
+    } else {   // [split][row, query vector][DV sums, maximum, denominator, ..]
+      const int gi = (row0 + tq[i]) * H * M + hq[i];
+      float* o = a.ws + ((size_t)split * a.rows_total + gi) * (DV + 4);
+#pragma unroll
+      for (int t = 0; t < DT; ++t) *reinterpret_cast<f32x4_t*>(o + t * 16 + kb * 4) = oacc[i][t];
+      if (kb == 0) { o[DV] = m[i] * 0.69314718055994531f; o[DV + 1] = den; }
+    }
+  }
+}
+
 // The splits' (maximum, denominator, sums) records of one (row, query vector) -> column threadIdx.x of its softmax-weighted sum
 // (0 for threads past DV; DV <= 256).  wgt / red: LDS scratch of the workgroup; the call synchronises it.
 __device__ __forceinline__ float merge_splits(const float* __restrict__ base, size_t stride, int nsplit, int Vp, int DV, float* wgt, float* red) {
@@ -827,7 +1055,34 @@ int dihip_gqa_attn_mc(void* stream, void* out, int out_dtype, long ldo, const fl
     if (DV <= 64) go(dm, std::integral_constant<int, 64>{});
     else go(dm, std::integral_constant<int, 128>{});
   };
-  if (D <= 64) by_v(std::integral_constant<int, 64>{});
+  // head sizes of exactly 64 / 128, whole 64-key tiles per page
+  const bool tiles = (D == 64 || D == 128) && (DV == 64 || DV == 128) && span_len % 64 == 0;
+  auto go_tile = [&](auto d, auto v, auto mt, auto cap) {
+    constexpr int D_ = decltype(d)::value, V_ = decltype(v)::value, MT = decltype(mt)::value;
+    constexpr bool CAP = decltype(cap)::value;
+    const int gx = (int)(((long)max_count * hpg + 64 * MT - 1) / (64 * MT));
+    const size_t bytes = (size_t)2 * 64 * (D_ + V_) * 2;
+    auto kern = gqa_attn_tile_kernel<D_, V_, MT, CAP>;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return;   // (reported below)
+    hipLaunchKernelGGL(kern, dim3((unsigned)gx * E * G * maps, 1, nsplit), dim3(256), bytes, s, a, gx);
+  };
+  auto by_cap = [&](auto d, auto v, auto mt) {
+    if (softcap > 0.f) go_tile(d, v, mt, std::true_type{});
+    else go_tile(d, v, mt, std::false_type{});
+  };
+  auto by_mt = [&](auto d, auto v) {
+    // two 16-pair operands per wave unless that leaves CUs without a workgroup, or 64 pairs are all there are (decoding)
+    if ((long)max_count * hpg > 64 && ((long)max_count * hpg + 127) / 128 * E * G * maps * nsplit >= 256) by_cap(d, v, std::integral_constant<int, 2>{});
+    else by_cap(d, v, std::integral_constant<int, 1>{});
+  };
+  constexpr std::integral_constant<int, 64> c64{};
+  constexpr std::integral_constant<int, 128> c128{};
+  if (tiles) {
+    if (D == 64 && DV == 64) by_mt(c64, c64);
+    else if (D == 64) by_mt(c64, c128);
+    else if (DV == 64) by_mt(c128, c64);
+    else by_mt(c128, c128);
+  } else if (D <= 64) by_v(std::integral_constant<int, 64>{});
   else if (D <= 128) by_v(std::integral_constant<int, 128>{});
   else by_v(std::integral_constant<int, 256>{});
   if (nsplit > 1 && diff_out)      // the merge of both maps, their difference and its norm in one launch

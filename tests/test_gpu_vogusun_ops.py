@@ -305,3 +305,76 @@ def test_router_logits_many_rows_few_columns(so, T, N, K):
     x16 = dev(x, torch.bfloat16)
     got16 = so.linear(x16, dev(w, torch.bfloat16), dev(b, torch.bfloat16), math=so.MATH_F32_STREAM)
     assert rel_err(got16.cpu().numpy(), x16.double().cpu().numpy() @ w.astype(np.float64).T + b) < 2e-6
+
+
+# ---- the 64-key tile form (head sizes of exactly 64 / 128) -------------------------------------------------------------------------
+def attention_f64(q, k, v, pos, scale, sink=None, softcap=0.0, gate=None, window=0, keep_first=0):
+    """q [n, H, maps, D] at positions pos, k [m, G, maps, D], v [m, G, V], all float64 on the device -> [n, H, maps, V]"""
+    n, H, M, _ = q.shape
+    hpg = H // k.shape[1]
+    kk, vv = k.repeat_interleave(hpg, 1), v.repeat_interleave(hpg, 1)
+    s = torch.einsum("nhmd,khmd->nhmk", q, kk) * scale
+    if softcap:
+        s = softcap * torch.tanh(s / softcap)
+    key = torch.arange(k.shape[0], device=q.device)
+    p = pos[:, None]
+    seen = (key <= p) & ((p - key < window) | (key < keep_first) if window else True)
+    s = s.masked_fill(~seen[:, None, None], -torch.inf)
+    if sink is not None:
+        s = torch.cat([s, sink.double()[None, :, None, None].expand(n, H, M, 1)], -1)
+    w = torch.softmax(s, -1)[..., :k.shape[0]]
+    o = torch.einsum("nhmk,khv->nhmv", w, vv)
+    return o * gate.double()[:, :, None, None] if gate is not None else o
+
+
+@pytest.mark.parametrize("H,G,D,V,maps,span,kw", [
+    (8, 2, 128, 128, 1, 64, dict()),
+    (8, 2, 128, 128, 1, 128, dict(sink=True, gate=True)),
+    (6, 6, 64, 64, 1, 64, dict(softcap=8.0)),
+    (3, 1, 64, 128, 1, 64, dict(window=70, keep_first=5)),
+    (4, 2, 128, 64, 2, 64, dict(window=64, sink=True)),
+    (64, 8, 128, 128, 1, 64, dict(softcap=30.0, window=130, gate=True)),
+])
+@pytest.mark.parametrize("nsplit", [1, 4])
+def test_attention_in_64_key_tiles(so, H, G, D, V, maps, span, kw, nsplit):
+    """Portions that end at, before and behind the borders of 64 keys, of 64 and 128 (row, head) pairs and of pages, from the start and from the
+    middle of a sequence, one row alone; pages whose unwritten rows hold infinities (what another request may have left)."""
+    from dash_infer_amd.seq_state import SequenceStateManager
+    torch.manual_seed(H * 1000 + D + V + span)
+    past, counts = [0, 0, 63, 128, 300, 191, 700], [1, 130, 65, 64, 33, 1, 1]
+    st = SequenceStateManager(8192, len(past), span, "cuda")
+    kt, vt = st.add_span_cache("k", G * maps * D, torch.bfloat16), st.add_span_cache("v", G * V, torch.bfloat16)
+    for t in (kt, vt):
+        t.pool.pool.view(torch.bfloat16).fill_(float("inf"))
+    want, qs, poss, slots, row0 = [], [], [], [], []
+    T = sum(counts)
+    sink = torch.randn(H, device="cuda") if kw.get("sink") else None
+    gate = torch.rand(T, H, device="cuda") if kw.get("gate") else None
+    scale, at = D ** -0.5, 0
+    for r, (p0, n) in enumerate(zip(past, counts)):
+        st.admit(r)
+        st.reserve(r, p0 + n)
+        st.upload()
+        slot = st.live[r].index
+        m = p0 + n
+        rows = torch.randn(m, (H + G) * maps * D + G * V, device="cuda")
+        nq, nk = H * maps * D, G * maps * D
+        rows[:, :nq] *= 2.0
+        so.qkv_prep_append(rows, 0, nq, nq + nk, H, G, D, V, None, None, 1e-5, None, 0, 0, 1.0, 0.0, None, None, kt, vt, i32([slot] * m), i32(list(range(m))),
+                           maps=maps)
+        q = rows[p0:, :nq].contiguous()
+        r16 = rows.to(torch.bfloat16).double()
+        want.append(attention_f64(r16[p0:, :nq].view(n, H, maps, D), r16[:, nq:nq + nk].view(m, G, maps, D), r16[:, nq + nk:].view(m, G, V),
+                                  torch.arange(p0, m, device="cuda"), scale, sink, kw.get("softcap", 0.0), gate[at:at + n] if gate is not None else None,
+                                  kw.get("window", 0), kw.get("keep_first", 0)).reshape(n, -1))
+        qs.append(q)
+        poss += list(range(p0, m))
+        slots.append(slot)
+        row0.append(at)
+        at += n
+    got = so.gqa_attn_mc(torch.cat(qs), kt, vt, i32(poss), i32(slots), i32(row0), i32(counts), max(counts), max(poss), H, G, D, V, scale, sink,
+                         so.SINK_PER_HEAD if sink is not None else so.SINK_NONE, kw.get("softcap", 0.0), gate, nsplit=nsplit, maps=maps,
+                         window=kw.get("window", 0), keep_first=kw.get("keep_first", 0))
+    for r in range(len(past)):       # weights rounded to bf16 (2^-9 each, independent) against sums of as many
+        g, w = got[row0[r]:row0[r] + counts[r]].cpu().numpy(), want[r].cpu().numpy()
+        assert rel_err(g, w) < 2.0 ** -8, (r, nsplit)
