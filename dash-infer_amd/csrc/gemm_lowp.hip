@@ -14,6 +14,10 @@
 
 namespace dihip {
 
+// dense_stream.hip: f32 logits of 5 .. 32 rows (FRAG32) against a wide 16-bit matrix
+bool dense_stream_takes(int M, int N, int K);
+int launch_dense_stream(hipStream_t s, const void* w, const void* x_frag, float* out, int M, int N, int K, int dtype);
+
 // ------------------------------------------------------------------------------------------
 // "dihip tile-major" weight layout
 //   W4: Kp = roundup(K,128), Np = roundup(N,16); 16-byte chunk index ((nt*KT + kt)*64 + lane),
@@ -1618,7 +1622,7 @@ int dihip_dense_pack(void* stream, const void* w_kn, int N, int K, int dtype, vo
 size_t dihip_dense_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const GemmPlan p = make_plan(16, M, N, K, -1, false);
-  return p.slab_bytes + GEMM_SYNC_BYTES + (size_t)M * K * 2 + 512;
+  return p.slab_bytes + GEMM_SYNC_BYTES + (size_t)((M + 15) / 16 * 16) * K * 2 + 512;  // (norm rows: FRAG32 where the streaming kernel takes them)
 }
 
 int dihip_gemm_a16w16(void* stream, const void* x, const void* w_packed, const void* bias, const void* residual,
@@ -1676,6 +1680,13 @@ int dihip_lm_head(void* stream, float* logits, const float* h, const void* gamma
     c.ws_bytes = ws_bytes;
   } else {
     DIHIP_REQUIRE(gamma != nullptr, DIHIP_PARAM_ERROR, "lm_head: needs gamma");
+    // a decoding batch against a wide matrix: the rows in FRAG32 at the start of the workspace, the weights streamed past them
+    const int mt = M > 16 ? 2 : 1;
+    if (dense_stream_takes(M, N, K) && ws && ws_bytes >= (size_t)mt * 16 * K * 2 && reinterpret_cast<uintptr_t>(ws) % 16 == 0 &&
+        (N % 4 != 0 || reinterpret_cast<uintptr_t>(logits) % 16 == 0)) {
+      const int st = launch_rmsnorm_rows(s, h, gamma, eps, M, K, ws, mt, dtype);
+      return st ? st : launch_dense_stream(s, w_packed, ws, logits, M, N, K, dtype);
+    }
     void* xn;
     size_t left;
     int st = norm_to_ws(s, h, gamma, eps, M, K, dtype, ws, ws_bytes, 16, N, -1, false, &xn, &left, &c.x_layout);

@@ -307,6 +307,27 @@ def test_lm_head_and_argmax(ops):
     assert ops.argmax(t).tolist() == [7, 999]
 
 
+@pytest.mark.parametrize("M,K,V,ft", [(5, 512, 16385, "bf16"), (16, 3584, 16400, "bf16"), (17, 512, 41000, "bf16"), (32, 3584, 20003, "bf16"),
+                                      (32, 4608, 16384, "f16"), (7, 5120, 50001, "f16"), (9, 544, 16400, "bf16")])
+def test_lm_head_of_a_batch_against_a_wide_matrix(ops, M, K, V, ft):
+    """5 .. 32 rows: at the edges of 16 rows and 16 columns, K of one pair of batches, of one and of several ranges, more tiles than one round
+    of workgroups holds, K that the streaming kernel does not take; against float64 of the same rounded operands."""
+    dt = torch.bfloat16 if ft == "bf16" else torch.float16
+    gen = torch.Generator("cuda").manual_seed(M + K + V)
+    W = (torch.randn(K, V, generator=gen, device="cuda") * K ** -0.5).to(dt)
+    h = torch.randn(M, K, generator=gen, device="cuda")
+    gamma = (1 + 0.1 * torch.randn(K, generator=gen, device="cuda")).to(dt)
+    pw = ops.pack_dense(W)
+    xn = torch.from_numpy(glue.rmsnorm(h.cpu().numpy(), gamma.float().cpu().numpy(), 1e-6)).cuda().to(dt)
+    ref = (xn.double() @ W.double()).cpu().numpy()
+    full = int(ops.lib().dihip_dense_workspace_bytes(M, V, K))
+    logits = ops.lm_head(h, gamma, 1e-6, pw, ops.Scratch(full)).cpu().numpy()
+    # the rows' own rounding can fall either way where the f32 norms differ in the last bit: half an ulp of single elements
+    err = float(np.linalg.norm(logits - ref) / np.linalg.norm(ref))
+    assert err < (2e-4 if ft == "bf16" else 5e-5), err
+    assert np.abs(logits - ref).max() < (2 ** -9 if ft == "bf16" else 2 ** -12) * np.abs(ref).max()
+
+
 # ------------------------------------------------------------------ batched decode shapes ----
 CFG4_RANK = {"qkv": (8192, 1280), "o": (1024, 8192), "gate": (8192, 3712), "down": (3712, 8192)}  # Qwen2-72B, TP = 8 (SURVEY 8 a3)
 
