@@ -675,6 +675,8 @@ class DecodeSession:
             self.pool.pool.view(-1, per)[:, g * S * hb: g * S * hb + g * S * 8] = allp.view(torch.uint8).view(-1, g * S * 8)
 
     # -- context (prefill) phase ----------------------------------------------------------------
+    PREFILL_ROWS = 4096   # rows of several prompts that the products take together: past it a row costs the same in any company
+
     def prefill(self, seqs, return_logits=True):
         """Context phase of every request through the product's op-boundary entry points, in the order of the reference
         graph (qwen_v15.py:210-388; SpanAttnOp::runContext, span_attn_op_cuda.cpp:205-330): embedding -> per layer
@@ -685,36 +687,49 @@ class DecodeSession:
         m, cfg = self.model, self.model.cfg
         assert m.nranks == 1 and len(seqs) == self.B
         n, g, H, dev = self.n_loc, self.g_loc, self.H, self.h.device
-        Lmax = max(len(s) for s in seqs)
+        lens = [len(s) for s in seqs]
+        assert all(0 < L <= self.max_len for L in lens)
+        # the products take the rows of several prompts together (the weights are read once), up to PREFILL_ROWS of them
+        groups = []
+        for b, L in enumerate(lens):
+            if groups and sum(lens[i] for i in groups[-1]) + L <= self.PREFILL_ROWS:
+                groups[-1].append(b)
+            else:
+                groups.append([b])
         l0, wb, gsz = m.layers[0], m.quant.wbits, m.quant.group
-        # per prompt length: a shorter prompt can take a split-K plan with a larger slab than the longest one
-        need = max(ops.lowp_workspace_bytes(wb, L, p.N, p.K, gsz) for L in {len(s) for s in seqs} for p in (l0.qkv, l0.o, l0.gate, l0.down))
-        need = max(need, int(lib().dihip_dense_workspace_bytes(1, m.lm_head.N, m.lm_head.K)))
+        # per row count: fewer rows can take a split-K plan with a larger slab than more of them
+        need = max(ops.lowp_workspace_bytes(wb, T, p.N, p.K, gsz) for T in {sum(lens[b] for b in grp) for grp in groups} for p in (l0.qkv, l0.o, l0.gate, l0.down))
+        need = max(need, int(lib().dihip_dense_workspace_bytes(self.B, m.lm_head.N, m.lm_head.K)))
         sc = ops.Scratch(need, dev)
-        logits = torch.empty(self.B, m.vocab_local, dtype=torch.float32, device=dev) if return_logits else None
-        for b, seq in enumerate(seqs):
-            L = len(seq)
-            assert 0 < L <= self.max_len
-            ids = torch.as_tensor(seq, dtype=torch.int64, device=dev)
-            pos = torch.arange(L, dtype=torch.int32, device=dev)
+        last = torch.empty(self.B, cfg.hidden, dtype=torch.float32, device=dev)
+        for grp in groups:
+            T, cut = sum(lens[b] for b in grp), [0]
+            for b in grp:
+                cut.append(cut[-1] + lens[b])
+            ids = torch.as_tensor([t for b in grp for t in seqs[b]], dtype=torch.int64, device=dev)
+            pos = torch.cat([torch.arange(lens[b], dtype=torch.int32, device=dev) for b in grp])
             h = ops.embedding(ids, m.embed)
             for li, lw in enumerate(m.layers):
                 qkv = ops.fused_norm_gemm(h, lw.ln1, cfg.eps, lw.qkv, lw.qkv_bias, sc)
                 ops.rope_qk_(qkv, pos, self.inv_freq, n, g, H)
                 kv = self.kv[li]
                 stride = (n + 2 * g) * H
-                ops.kv_context_copy(kv.k_ptrs[b], qkv[:, n * H:], stride, L, 0, g, H, self.pool.S, self.kv_mode)
-                ops.kv_context_copy(kv.v_ptrs[b], qkv[:, (n + g) * H:], stride, L, 0, g, H, self.pool.S, self.kv_mode)
-                attn = ops.prefill_attn(qkv[:, : n * H], qkv[:, n * H:(n + g) * H], qkv[:, (n + g) * H:], n, g, H, self.scale)
-                h = ops.fused_gemm_addto(attn, lw.o, h, sc, M=L)
+                attn = torch.empty(T, n * H, dtype=qkv.dtype, device=dev)
+                for b, lo, hi in zip(grp, cut, cut[1:]):
+                    rows = qkv[lo:hi]
+                    q, k, v = rows[:, : n * H], rows[:, n * H:(n + g) * H], rows[:, (n + g) * H:]
+                    ops.kv_context_copy(kv.k_ptrs[b], k, stride, hi - lo, 0, g, H, self.pool.S, self.kv_mode)
+                    ops.kv_context_copy(kv.v_ptrs[b], v, stride, hi - lo, 0, g, H, self.pool.S, self.kv_mode)
+                    ops.prefill_attn(q, k, v, n, g, H, self.scale, out=attn[lo:hi])
+                h = ops.fused_gemm_addto(attn, lw.o, h, sc, M=T)
                 if cfg.moe is not None:
                     h = self._moe_rows(h, lw, sc)
                     continue
                 act = ops.fused_norm_swiglu(h, lw.ln2, cfg.eps, lw.gate, lw.up, sc)
-                h = ops.fused_gemm_addto(act, lw.down, h, sc, M=L)
-            if return_logits:
-                ops.lm_head(h[L - 1:L].contiguous(), m.final_norm, cfg.eps, m.lm_head, sc, out=logits[b:b + 1])
-        lens = [len(s) for s in seqs]
+                h = ops.fused_gemm_addto(act, lw.down, h, sc, M=T)
+            for b, hi in zip(grp, cut[1:]):
+                last[b].copy_(h[hi - 1])
+        logits = ops.lm_head(last, m.final_norm, cfg.eps, m.lm_head, sc) if return_logits else None
         if return_logits:
             nxt = torch.argmax(logits, dim=-1).cpu()
             self.set_state(nxt, lens)
