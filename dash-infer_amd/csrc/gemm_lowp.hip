@@ -934,7 +934,6 @@ static int run_gemm(hipStream_t stream, const GemmCall& c) {
       g.slab = reinterpret_cast<float*>(c.ws);
       blocks = pt.tail_cb * pt.mblocks + (pt.col_blocks - pt.tail_cb) * pt.mblocks * pt.ksplit;
     }
-    g.trace = debug_trace_buffer((size_t)blocks * PF_WAVES * 4 * 8 * sizeof(unsigned long long));
     const bool gpt = g.ktpg == 1;
     hipError_t e = hipErrorInvalidValue;
 #define PREFILL_GO(W_, EPI_, G_) \

@@ -8,64 +8,49 @@
 //
 //   * workgroup tile 128 rows x 256 columns (8 waves side by side in N, each 128 x 32 = 8 row tiles x 2 column tiles of
 //     v_mfma_f32_16x16x32: 16 accumulators), K walked in packed k-tiles (W4: 128 k, W8: 64 k);
-//   * A (activations, FT row-major) goes global -> registers -> LDS once per workgroup and k-tile, stored as the MFMA A
-//     fragments (one fragment = one contiguous 1 KiB: conflict-free ds_write_b128 / ds_read_b128), double-buffered: the loads of
-//     k-tile t + 1 are in flight while t is multiplied, ONE barrier per k-tile; every wave reads all 8 row tiles;
+//   * A (activations, FT row-major) goes straight from memory into LDS (global_load_lds: no registers, no instructions for staging),
+//     double-buffered: the loads of k-tile t + 1 are in flight while t is multiplied, ONE barrier per k-tile; every wave reads all
+//     8 row tiles;
 //   * B (weights) never touches LDS: "dihip tile-major" packing makes a lane's 16-byte load the B fragment of its own column
 //     tile (x KSTEPS), and no two waves share a column tile;
 //   * the same exact-integer arithmetic as the decode kernels: q expands to 128 + q in FT with the magic-number trick, the MFMA
 //     sums exact products, and per quantisation group  y += s * (acc - (z + 128) * sum_k x)  on the f32 accumulator, with
-//     sum_k x per (row, k-tile) taken while A is staged -- four MFMAs against a fragment of ones per wave and k-tile (the VALU
-//     form cost 72 instructions per wave and k-tile: +3 % tokens/s);
+//     sum_k x per (row, k-tile) taken under the multiply -- an MFMA against a fragment of ones per wave and k-step;
+//   * the fix-up of a closed group runs under the first products of the next one, row tile by row tile (vector instructions
+//     while the matrix unit works), and so do the expansions of the next k-step's weights;
 //   * epilogues as everywhere: STD (alpha, bias, UnaryType activation, FT residual), SwiGLU over a gate / up pair (a wave's two
 //     column tiles are then the SAME 16 columns of the two matrices: 128 output columns per workgroup), f32 hidden-stream update.
 //
 // Host contract (gemm_lowp.hip: run_gemm): bf16 / f16 activations row-major with ldx % 8 == 0, 16-byte aligned; K a multiple of
 // the k-tile; group_size a multiple of the k-tile or per-channel.  Rows >= M are clamped on load and masked on store.
 //
-// Where the time goes (round 3, SQ counters of the SwiGLU launch, profiles/r03_prefill_gemm_sq_counters.txt): 244 registers mean
-// one workgroup = two waves per SIMD; per wave and k-tile 68 MFMAs (16 cycles of the matrix pipe each) + 193 other VALU + 45 LDS +
-// 32 scalar instructions.  MFMA and VALU share the SIMD's one VALU-class issue slot per 4 cycles, so the two waves need
-// 2 x 261 x 4 = 2088 issue cycles next to 2176 cycles of matrix pipe: the loop only runs at the MFMA rate if every gap of every
-// MFMA carries exactly its three VALU instructions.  Measured: matrix pipe busy 39 % of the kernel (790-870 TFLOP/s), waves
-// issuing 31 %, issue-stalled 44 %, parked at waitcnt / barrier 25 %.  Tried and measured, none better than +-3 %: the loop
-// without per-k-step scheduling fences (kept, +3 % with s_setprio around the multiply), an explicit sched_group_barrier
-// interleave with software-pipelined expansion, a 2 x 4 wave grid (half the LDS reads, twice the expansions: -10 %), a ping-pong
-// schedule (two groups of four waves half a k-tile period apart so that each SIMD always has one multiplying wave: -7 %, or
-// -2 % with scalar instead of SLP-packed FMAs), scalar FMAs alone (-2 %).  The instruction mix is the limit: the fix-up
-// (2 FMA per accumulator element and group) and the 4-bit expansion (7 VALU per 8 weights) are inherent to multiplying the
-// integer weights in place.
-// Where the rest goes (per-wave cycle stamps + tools/gemm_skeleton_bench, same profile): the multiply phase itself runs at the
-// rate of the bare skeleton -- LDS fragment reads + MFMAs + barrier with nothing else reach 70 % of the matrix peak in this
-// tile shape, 82 % with the reads of k-step s + 1 issued ahead of the MFMAs of s (2 657 / 2 454 cycles per k-tile; the kernel's
-// two waves multiply for 2 620-3 312) -- and then ~1 600 cycles per k-tile pass with the pipe idle: fix-up 564, staging 408,
-// barrier 628.  Next: stage A with direct global -> LDS loads (no staging phase, 16 registers back; the row-sum MFMAs move to
-// the multiply, which reads those fragments anyway), spend the registers on pipelined fragment reads, and slide the fix-up under
-// the first k-step of the next tile.  (A one-wave-per-SIMD 128 x 128 wave tile measured WORSE as a bare skeleton: 54 %.)
+// What bounds it (gate / up pair of 2048 rows, K = 3584, 2 x 18944 columns, W4 in groups of 128; counters): 240 registers mean one
+// workgroup = two waves per SIMD.  Per wave and k-tile 68 MFMAs of 16 cycles, about 190 other vector and 45 LDS instructions; the LDS
+// reads (256 KiB per k-tile) alone take the products' time once.  The matrix units are busy 44 % of the time at 2.05 GHz; timing copies
+// of the kernel with one part left out: - 16 % without the fix-up, - 13 % without the row sums, - 14 % without the loads, - 5 % without the
+// expansions, - 10 % without the LDS reads of all but the first k-step, - 44 % without all of them (1 600 TFLOP/s).  The parts add up:
+// what is left is instruction issue and power, not one wait.
+// Measured (A through registers, fix-up between the tiles before): 2048 rows of four W4 layers 5.29 -> 5.09 ms, 434 rows of four W8 layers
+// 1.76 -> 1.62 ms.
+// A 2 x 4 grid of waves with 64 x 64 tiles (half the LDS reads, twice the expansions and twice the weight loads) is 10-14 % slower.
 #pragma once
 #include <atomic>
+#include <type_traits>
 #include "gemm_lowp_kernel.hpp"
 #include "gemv_stream_kernel.hpp"  // ExpandV: the 128 + q expansion of the decode kernels
 
 namespace dihip {
 
-// what-if timing builds (tools/build_ksl_variant.sh NAME -DDIHIP_PF_X=.. gemm_prefill_inst; results WRONG with any bit set):
-//   1 no scale / zero-point fix-up   2 no A staging (LDS keeps what the prologue wrote)   4 no barrier   8 no nibble expansion
-// Round 4, the SwiGLU GEMM of a 2048-token prompt (profiles/r04af_*): 676 us as built (822 TFLOP/s); 645 without (1), 597 without (2),
-// 649 without (4), 654 without (8); 459 without all four (1 212 TFLOP/s = 48 % of the dense peak): the bare LDS-read + MFMA loop
-// of this tile shape is the ceiling, and the A staging (registers -> ds_write + the row-sum MFMAs) is the largest single extra.
-#ifndef DIHIP_PF_X
-#define DIHIP_PF_X 0
-#endif
 constexpr int PF_WAVES = 8;
 constexpr int PF_THREADS = PF_WAVES * 64;
 constexpr int PF_BM = 128;           // rows per workgroup (8 row tiles)
-constexpr int PF_WM = 1;             // waves along M (a 2 x 4 grid with 4 x 4 tiles per wave measured 10 % slower: twice the expansions)
+constexpr int PF_WM = 1;             // waves along M
 constexpr int PF_WN = PF_WAVES / PF_WM;
 constexpr int PF_TR = PF_BM / 16;    // row tiles of the workgroup (= waves: wave w stages row tile w)
 constexpr int PF_RT = PF_TR / PF_WM; // row tiles per wave
 constexpr int PF_CW = 2 * PF_WM;     // column tiles per wave (the workgroup covers 256 columns either way)
 static_assert(PF_TR == PF_WAVES, "one staged row tile per wave");
+static_assert(PF_CW == 2, "the two column tiles of a wave are named one by one where the sums change hands");
 
 struct PrefillArgs {
   const u32x4_t* w0;
@@ -97,12 +82,11 @@ struct PrefillArgs {
   int ksplit;
   int kunit;    // k-tiles that a K range must not cut (grouped weights: a group; per-channel: 1)
   float* slab;  // [tail tile][ksplit][PF_BM][256] f32
-  unsigned long long* trace;  // per-wave cycle stamps (library built with -DDIHIP_PF_TRACE, tools/prefill_trace.py)
 };
 
 template <int WBITS>
 constexpr size_t prefill_lds_bytes() {
-  // 2 x A tile (PF_TR x KSTEPS fragments of 1 KiB) + 2 x 128 row sums
+  // 2 x A tile (128 rows x KSTEPS x 64 bytes) + 2 x 128 row sums
   return (size_t)2 * PF_TR * WTraits<WBITS>::KSTEPS * 1024 + 2 * PF_BM * sizeof(float);
 }
 
@@ -145,54 +129,47 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
   constexpr int HCW = PF_CW / 2;
   int tile[PF_CW];
   bool tile_ok[PF_CW];
-  const u32x4_t* wp[PF_CW];
-  const uint32_t* szp[PF_CW];
+  // (buffer loads: bases in scalar registers, one lane offset for all)
+  __amdgpu_buffer_rsrc_t wp[PF_CW], szp[PF_CW];
 #pragma unroll
   for (int c = 0; c < PF_CW; ++c) {
     const int t = DUAL ? (cb * PF_WN + wn) * HCW + (c % HCW) : (cb * PF_WN + wn) * PF_CW + c;
     tile_ok[c] = t < a.NTILES;
     tile[c] = min(t, a.NTILES - 1);
     const bool second = DUAL && c >= HCW;
-    wp[c] = (second ? a.w1 : a.w0) + (size_t)tile[c] * a.KT * 64 + lane;
-    szp[c] = (second ? a.sz1 : a.sz0) + (size_t)tile[c] * a.Gp * 16 + ni;
+    wp[c] = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4_t*>((second ? a.w1 : a.w0) + (size_t)tile[c] * a.KT * 64), 0, a.KT * 1024, 0x00020000);
+    szp[c] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>((second ? a.sz1 : a.sz0) + (size_t)tile[c] * a.Gp * 16), 0, a.Gp * 64, 0x00020000);
   }
 
-  // ---- A staging: wave w stages row tile w (all KSTEPS fragments of the k-tile): lane (kb, r) <- 16 bytes of row m0 + 16 w + r
-  const int arow = min(m0 + wave * 16 + ni, a.M - 1);  // rows past M re-read the last row (masked on store)
-  const char* xrow = reinterpret_cast<const char*>(a.x) + ((size_t)arow * a.ldx + kb * 8) * 2;
-  u32x4_t areg[KSTEPS];
-  u32x4_t wreg[PF_CW];
-  uint32_t szreg[PF_CW] = {};
-  auto load_a = [&](int kt) {
+  // ---- A: wave w brings row tile w straight into LDS (global_load_lds: no registers, no instructions for staging), pieces of 8 rows x 128
+  // bytes; the 16-byte chunks of a row change places on the memory side (chunk ^ row % 8): 8 consecutive lanes of an operand read then
+  // touch every bank once.  Rows past M re-read the last row (masked on store)
+  constexpr int HALVES = KTILE / 64;                       // 64 k of 128 rows: 16 KiB
+  const int prow = lane >> 3, pchunk = (lane & 7) ^ prow;
+  const char* abase = reinterpret_cast<const char*>(a.x) + (size_t)m0 * a.ldx * 2;
+  uint32_t aoff[2];
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) areg[ks] = *reinterpret_cast<const u32x4_t*>(xrow + ((size_t)kt * KTILE + ks * 32) * 2);
+  for (int p = 0; p < 2; ++p) aoff[p] = (uint32_t)((size_t)min(wave * 16 + p * 8 + prow, a.M - 1 - m0) * a.ldx * 2 + pchunk * 16);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem + wave * 2048;
+  auto load_a = [&](int kt, int buf) {
+    const char* src = abase + (size_t)kt * KTILE * 2;
+#pragma unroll
+    for (int hh = 0; hh < HALVES; ++hh)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds0 + (uint32_t)(buf * ABYTES) + hh * 16384 + p * 1024),
+                     "v"(aoff[p]), "s"(src + hh * 128) : "memory");
   };
+  u32x4_t wreg[PF_CW];
+  uint32_t szreg[PF_CW] = {}, sznew[PF_CW] = {};
   auto load_b = [&](int kt) {
 #pragma unroll
-    for (int c = 0; c < PF_CW; ++c) wreg[c] = __builtin_nontemporal_load(wp[c] + (size_t)kt * 64);
+    for (int c = 0; c < PF_CW; ++c) wreg[c] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(wp[c], lane * 16, kt * 1024, 2));   // (2: nontemporal)
   };
-  // stages the loaded k-tile into A buffer `buf`; its row sums go into (or are added to) the row-sum table of its quantisation
-  // group, `gbuf` = group parity (the lane with kb == 0 of a row's 4 k-block lanes owns that row's entry: no race)
-  auto stage_a = [&](int buf, int gbuf, bool group_start) {
-    unsigned char* dst = smem + buf * ABYTES + ((size_t)wave * KSTEPS * 64 + lane) * 16;
-    // A = the staged fragment, B = ones: every column of the result tile is the row sum (lane (kb, ni): rows kb * 4 + r)
-    const u32x4_t ones = FT == DIHIP_BF16 ? u32x4_t{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u}
-                                    : u32x4_t{0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
-    f32x4_t sx = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-      *reinterpret_cast<u32x4_t*>(dst + ks * 1024) = areg[ks];
-      sx = mfma16<FT>(areg[ks], ones, sx);
-    }
-    if (ni == 0) {
-      f32x4_t* p = reinterpret_cast<f32x4_t*>(xsum + gbuf * PF_BM + wave * 16 + kb * 4);
-      if (group_start) {
-        *p = sx;
-      } else {
-        const f32x4_t o = *p;
-        *p = f32x4_t{o[0] + sx[0], o[1] + sx[1], o[2] + sx[2], o[3] + sx[3]};
-      }
-    }
+  // operand (row ni of a row tile, 16 bytes kb of k-step ks)
+  const int f0 = ni * 128 + ((kb ^ (ni & 7)) * 16), f1 = f0 ^ 64;
+  auto aread = [&](const unsigned char* tile, int rt, int ks) {
+    return *reinterpret_cast<const u32x4_t*>(tile + (ks >> 1) * 16384 + rt * 2048 + ((ks & 1) ? f1 : f0));
   };
 
   // acc: exact integer products of the running quantisation group (MFMA); tot: the scaled result
@@ -204,100 +181,132 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
     for (int c = 0; c < PF_CW; ++c) acc[rt][c] = tot[rt][c] = zero4;
   uint32_t ex_mask = 0x000F000Fu, ex_magic = FT == DIHIP_BF16 ? 0x43004300u : 0x64006400u;
   asm volatile("" : "+v"(ex_mask), "+v"(ex_magic));
+  // scale / zero-point of a closed group on the accumulators of one row tile, with the group's row sums
+  float s_[PF_CW], nz_[PF_CW];
+  const float* xs = nullptr;
+  auto open_fix = [&](int group) {
+    xs = xsum + (group & 1) * PF_BM + kb * 4;
+#pragma unroll
+    for (int c = 0; c < PF_CW; ++c) {
+      s_[c] = ft_bits_to_f32<FT>(szreg[c] & 0xFFFFu);
+      nz_[c] = -(ft_bits_to_f32<FT>(szreg[c] >> 16) + EX::OFFSET);
+    }
+  };
+  auto fix = [&](int rt, const f32x4_t& xv) {
+#pragma unroll
+    for (int c = 0; c < PF_CW; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) tot[rt][c][r] = fmaf(s_[c], fmaf(nz_[c], xv[r], acc[rt][c][r]), tot[rt][c][r]);
+  };
 
-  // ---- prologue: the first k-tile into buffer 0 ----------------------------------------------------------------
+  // One barrier per k-tile.  Behind it: this tile (its loads are a k-tile old) is in LDS, the other buffer has been read, the row sums of the tile
+  // before are there.  The next tile's loads go out, then the products: the first k-step's carry the fix-up of the group that the tile before
+  // closed (one k-tile per group; longer groups are fixed up in one go, once per group), every row operand is re-read for the next k-step
+  // right behind its last product, and the row sums of this tile (sum_k x: the staged row tile times a fragment of ones) are taken on the way.
   int gl = 0;                                                   // k-tiles of the running group done
   int grp = GPT ? kt0 : (a.ktpg < a.KT ? kt0 / a.ktpg : 0);     // running group (a K part starts on a group boundary)
-  load_a(kt0);
+  load_a(kt0, 0);
   load_b(kt0);
 #pragma unroll
-  for (int c = 0; c < PF_CW; ++c) szreg[c] = szp[c][(size_t)min(grp, a.Gp - 1) * 16];
-  stage_a(0, grp & 1, true);
-  __syncthreads();
-
-#ifdef DIHIP_PF_TRACE
-  // k-tiles 8..11 of every workgroup: 8 stamps per k-tile (loop top, after each k-step, after the fix-up, after staging, after the barrier)
-#define DIHIP_PF_STAMP(I)                                                                                                \
-  do {                                                                                                                   \
-    if (a.trace && lane == 0 && kt >= 8 && kt < 12)                                                                       \
-      a.trace[(((size_t)blockIdx.x * PF_WAVES + wave) * 4 + (kt - 8)) * 8 + (I)] = __builtin_readcyclecounter();         \
-  } while (0)
-#else
-#define DIHIP_PF_STAMP(I) do { } while (0)
-#endif
+  for (int c = 0; c < PF_CW; ++c) sznew[c] = __builtin_amdgcn_raw_buffer_load_b32(szp[c], ni * 4, min(grp, a.Gp - 1) * 64, 0);
+  const u32x4_t ones = FT == DIHIP_BF16 ? u32x4_t{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u}
+                                  : u32x4_t{0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
+  if constexpr (GPT) {   // the first tile closes a group of nothing: sums, scales and products 0
+    if (tid < 2 * PF_BM) xsum[tid] = 0.f;
+  }
+  __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): scalar loads still in flight would make every wait for an LDS read this one
   for (int kt = kt0; kt < kt1; ++kt) {
     const int buf = (kt - kt0) & 1;
-    DIHIP_PF_STAMP(0);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     u32x4_t wcur[PF_CW];
 #pragma unroll
-    for (int c = 0; c < PF_CW; ++c) wcur[c] = wreg[c];
-    const bool more = kt + 1 < kt1;
-    if (more) {  // (uniform) the loads of the next k-tile fly while this one is multiplied
-      load_a(kt + 1);
-      load_b(kt + 1);
+    for (int c = 0; c < PF_CW; ++c) {
+      asm volatile("" : "+v"(wreg[c]), "+v"(sznew[c]));   // here they are: nothing further down waits for loads again
+      wcur[c] = wreg[c];
     }
-    // ---- multiply: every wave reads all row tiles of the A tile
-    const unsigned char* abase = smem + buf * ABYTES + (size_t)lane * 16;
-    __builtin_amdgcn_s_setprio(1);  // the multiplying wave wins the issue arbitration against its SIMD neighbour's VALU phase
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-      u32x4_t bf[PF_CW];
-#pragma unroll
-      for (int c = 0; c < PF_CW; ++c) {
-        if constexpr ((DIHIP_PF_X & 8) != 0) bf[c] = wcur[c];
-        else bf[c] = EX::frag(wcur[c], ks, ex_mask, ex_magic);
-      }
+    if constexpr (GPT) {
+      open_fix(grp - 1);
+    } else if (kt > kt0 && gl == 0) {                         // (uniform) the tile before closed its group
+      open_fix(grp - 1);
 #pragma unroll
       for (int rt = 0; rt < PF_RT; ++rt) {
-        const u32x4_t af = *reinterpret_cast<const u32x4_t*>(abase + ((size_t)(wm * PF_RT + rt) * KSTEPS + ks) * 1024);
+        fix(rt, *reinterpret_cast<const f32x4_t*>(xs + (wm * PF_RT + rt) * 16));
 #pragma unroll
-        for (int c = 0; c < PF_CW; ++c) acc[rt][c] = mfma16<FT>(af, bf[c], acc[rt][c]);
+        for (int c = 0; c < PF_CW; ++c) acc[rt][c] = zero4;
       }
-#ifdef DIHIP_PF_TRACE
-      if (ks == 0) DIHIP_PF_STAMP(1);
-      if (ks == 1) DIHIP_PF_STAMP(2);
-      if (ks == 2) DIHIP_PF_STAMP(3);
-      if (ks == 3) DIHIP_PF_STAMP(4);
-#endif
     }
-    __builtin_amdgcn_s_setprio(0);
-    // ---- at the group's end: scale / zero-point on the f32 accumulators, with the group's row sums
-    ++gl;
-    const bool gend = (GPT || gl == a.ktpg || !more) && (!(DIHIP_PF_X & 1) || !more);
-    if (gend) {  // (uniform)
-      const float* xs = xsum + (grp & 1) * PF_BM + wm * PF_RT * 16 + kb * 4;
-      float s_[PF_CW], nz_[PF_CW];
+    if (GPT || gl == 0) {
 #pragma unroll
-      for (int c = 0; c < PF_CW; ++c) {
-        s_[c] = ft_bits_to_f32<FT>(szreg[c] & 0xFFFFu);
-        nz_[c] = -(ft_bits_to_f32<FT>(szreg[c] >> 16) + EX::OFFSET);
-      }
+      for (int c = 0; c < PF_CW; ++c) szreg[c] = sznew[c];      // the running group's
+    }
+    const int nkt = min(kt + 1, kt1 - 1);                       // past the end: once more the last, read by nobody
+    load_a(nkt, buf ^ 1);
+    load_b(nkt);
+#pragma unroll
+    for (int c = 0; c < PF_CW; ++c) sznew[c] = __builtin_amdgcn_raw_buffer_load_b32(szp[c], ni * 4, min(grp + 1, a.Gp - 1) * 64, 0);
+    const unsigned char* tile = smem + buf * ABYTES;
+    u32x4_t af[PF_RT], bf[PF_CW], own;
+    f32x4_t xv = zero4;
+    if constexpr (GPT) xv = *reinterpret_cast<const f32x4_t*>(xs + wm * PF_RT * 16);
+#pragma unroll
+    for (int rt = 0; rt < PF_RT; ++rt) af[rt] = aread(tile, wm * PF_RT + rt, 0);
+    own = aread(tile, wave, 0);
+#pragma unroll
+    for (int c = 0; c < PF_CW; ++c) bf[c] = EX::frag(wcur[c], 0, ex_mask, ex_magic);
+    f32x4_t sx = zero4;
+    __builtin_amdgcn_sched_barrier(0);
+    auto kstep = [&](int ks, auto first) {
+      constexpr bool FIRST = decltype(first)::value;            // closes the group before
+      u32x4_t bn[PF_CW];
 #pragma unroll
       for (int rt = 0; rt < PF_RT; ++rt) {
-        const f32x4_t xv = *reinterpret_cast<const f32x4_t*>(xs + rt * 16);
-#pragma unroll
-        for (int c = 0; c < PF_CW; ++c) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) tot[rt][c][r] = fmaf(s_[c], fmaf(nz_[c], xv[r], acc[rt][c][r]), tot[rt][c][r]);
-          acc[rt][c] = zero4;
+        if constexpr (FIRST) {
+          fix(rt, xv);
+          // (the products that start the next sums wait for the old sums to be used: one set of registers)
+          asm volatile("" : "+v"(tot[rt][0]), "+v"(tot[rt][1]), "+v"(af[rt]));
+          if (rt + 1 < PF_RT) xv = *reinterpret_cast<const f32x4_t*>(xs + (wm * PF_RT + rt + 1) * 16);
         }
+#pragma unroll
+        for (int c = 0; c < PF_CW; ++c) acc[rt][c] = mfma16<FT>(af[rt], bf[c], FIRST ? zero4 : acc[rt][c]);
+        if (ks + 1 < KSTEPS) af[rt] = aread(tile, wm * PF_RT + rt, ks + 1);
+        if (rt == 2) {
+          sx = mfma16<FT>(own, ones, sx);
+          if (ks + 1 < KSTEPS) own = aread(tile, wave, ks + 1);
+        }
+        if (ks + 1 < KSTEPS && rt >= PF_RT - 1 - PF_CW && rt < PF_RT - 1) bn[rt - (PF_RT - 1 - PF_CW)] = EX::frag(wcur[rt - (PF_RT - 1 - PF_CW)], ks + 1, ex_mask, ex_magic);
+        __builtin_amdgcn_sched_barrier(0);
       }
+      if (ks + 1 < KSTEPS) {
+#pragma unroll
+        for (int c = 0; c < PF_CW; ++c) bf[c] = bn[c];
+      }
+    };
+    kstep(0, std::integral_constant<bool, GPT != 0>{});
+#pragma unroll
+    for (int ks = 1; ks < KSTEPS; ++ks) kstep(ks, std::false_type{});
+    if (ni == 0) {   // the lane with ni == 0 of a row's lanes owns its entry: no race
+      f32x4_t* p = reinterpret_cast<f32x4_t*>(xsum + (grp & 1) * PF_BM + wave * 16 + kb * 4);
+      if (GPT || gl == 0) {
+        *p = sx;
+      } else {
+        const f32x4_t o = *p;
+        *p = f32x4_t{o[0] + sx[0], o[1] + sx[1], o[2] + sx[2], o[3] + sx[3]};
+      }
+    }
+    ++gl;
+    if (GPT || gl == a.ktpg || kt + 1 == kt1) {
       gl = 0;
       ++grp;
-      if (more) {
-#pragma unroll
-        for (int c = 0; c < PF_CW; ++c) szreg[c] = szp[c][(size_t)min(grp, a.Gp - 1) * 16];
-      }
     }
-    // ---- the next A tile into the other buffer (its last readers passed the previous barrier); its row sums belong to
-    // group `grp` (already advanced when this k-tile closed one): that group's table was last read two groups ago
-    DIHIP_PF_STAMP(5);
-    if (more && !(DIHIP_PF_X & 2)) stage_a(buf ^ 1, grp & 1, gl == 0);
-    DIHIP_PF_STAMP(6);
-    if constexpr (!(DIHIP_PF_X & 4)) __syncthreads();
-    DIHIP_PF_STAMP(7);
   }
-#undef DIHIP_PF_STAMP
+  // the last group; and nothing may be on its way into LDS when the workgroup leaves
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __syncthreads();
+  open_fix(grp - 1);
+#pragma unroll
+  for (int rt = 0; rt < PF_RT; ++rt) fix(rt, *reinterpret_cast<const f32x4_t*>(xs + (wm * PF_RT + rt) * 16));
 
   // ---- split in K: this part's f32 tile to the slab (rows / columns of the workgroup tile; SwiGLU: gate columns, then up) ----
   if (split_part >= 0) {  // (uniform)
