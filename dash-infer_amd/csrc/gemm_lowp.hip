@@ -899,7 +899,8 @@ static int run_gemm(hipStream_t stream, const GemmCall& c) {
   // (gemm_prefill_kernel.hpp).  DIHIP_GEMM_PREFILL=0 keeps the general kernel (A/B, diagnostics).
   static const bool prefill_on = !env_off("DIHIP_GEMM_PREFILL");
   if (prefill_on && (c.dtype == DIHIP_BF16 || f16_act) && c.pro == PRO_PLAIN && c.M >= 64 && (c.wbits == 4 || c.wbits == 8) && gemv_aligned &&
-      (d.group == 0 || d.group % d.KTILE == 0) && (c.epi != EPI_SWIGLU || (c.w1 && c.sz1))) {
+      (d.group == 0 || d.group % d.KTILE == 0) && (c.epi != EPI_SWIGLU || (c.w1 && c.sz1)) &&
+      c.N <= (1 << 21) && c.ldx <= (1 << 22)) {  // (a workgroup's 128 rows are addressed with 31-bit byte offsets)
     PrefillArgs g{};
     g.w0 = reinterpret_cast<const u32x4_t*>(c.w0);
     g.w1 = reinterpret_cast<const u32x4_t*>(c.w1);
@@ -934,6 +935,8 @@ static int run_gemm(hipStream_t stream, const GemmCall& c) {
       g.slab = reinterpret_cast<float*>(c.ws);
       blocks = pt.tail_cb * pt.mblocks + (pt.col_blocks - pt.tail_cb) * pt.mblocks * pt.ksplit;
     }
+    const auto aligned = [](const void* p, uintptr_t b) { return reinterpret_cast<uintptr_t>(p) % b == 0; };  // (null: yes)
+    g.wide_out = c.N % 4 == 0 && (c.epi == EPI_ADDTO ? aligned(c.h_res, 16) && aligned(c.h_out, 16) : aligned(c.y, 8) && aligned(c.residual, 8));
     const bool gpt = g.ktpg == 1;
     hipError_t e = hipErrorInvalidValue;
 #define PREFILL_GO(W_, EPI_, G_) \

@@ -30,8 +30,8 @@
 // of the kernel with one part left out: - 16 % without the fix-up, - 13 % without the row sums, - 14 % without the loads, - 5 % without the
 // expansions, - 10 % without the LDS reads of all but the first k-step, - 44 % without all of them (1 600 TFLOP/s).  The parts add up:
 // what is left is instruction issue and power, not one wait.
-// Measured (A through registers, fix-up between the tiles before): 2048 rows of four W4 layers 5.29 -> 5.09 ms, 434 rows of four W8 layers
-// 1.76 -> 1.62 ms.
+// Measured: 2048 rows of four W4 layers 5.29 ms with A through registers and the fix-up between the tiles, 5.05 as above, 4.86 with four
+// neighbouring columns per lane and an epilogue without branches; 434 rows of four W8 layers 1.76 -> 1.63 ms.
 // A 2 x 4 grid of waves with 64 x 64 tiles (half the LDS reads, twice the expansions and twice the weight loads) is 10-14 % slower.
 #pragma once
 #include <atomic>
@@ -81,6 +81,7 @@ struct PrefillArgs {
   int tail_cb;
   int ksplit;
   int kunit;    // k-tiles that a K range must not cut (grouped weights: a group; per-channel: 1)
+  int wide_out; // four neighbouring columns of an output (and residual) row make one aligned access
   float* slab;  // [tail tile][ksplit][PF_BM][256] f32
 };
 
@@ -98,6 +99,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
   constexpr int KSTEPS = WT::KSTEPS;
   constexpr int KTILE = WT::KTILE;
   constexpr bool DUAL = EPI == EPI_SWIGLU;
+  constexpr bool LACE = GPT && WBITS == 4;  // fix-up under the first k-step's products (8 bits: two k-steps, no registers left for it)
   constexpr size_t ABYTES = (size_t)PF_TR * KSTEPS * 1024;  // one A tile
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   float* xsum = reinterpret_cast<float*>(smem + 2 * ABYTES);  // [2][PF_BM]
@@ -161,7 +163,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
                      "v"(aoff[p]), "s"(src + hh * 128) : "memory");
   };
   u32x4_t wreg[PF_CW];
-  uint32_t szreg[PF_CW] = {}, sznew[PF_CW] = {};
+  u32x4_t szreg[PF_CW] = {};   // the running group's, of this lane's four columns of each tile
   auto load_b = [&](int kt) {
 #pragma unroll
     for (int c = 0; c < PF_CW; ++c) wreg[c] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(wp[c], lane * 16, kt * 1024, 2));   // (2: nontemporal)
@@ -172,7 +174,8 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
     return *reinterpret_cast<const u32x4_t*>(tile + (ks >> 1) * 16384 + rt * 2048 + ((ks & 1) ? f1 : f0));
   };
 
-  // acc: exact integer products of the running quantisation group (MFMA); tot: the scaled result
+  // acc: exact integer products of the running quantisation group (MFMA); tot: the scaled result.  The weights are the first operand: lane
+  // (kb, ni) holds columns kb * 4 .. + 3 of a column tile, row ni of a row tile -- four neighbours of one row, stored together
   f32x4_t acc[PF_RT][PF_CW], tot[PF_RT][PF_CW];
   const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -182,21 +185,25 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
   uint32_t ex_mask = 0x000F000Fu, ex_magic = FT == DIHIP_BF16 ? 0x43004300u : 0x64006400u;
   asm volatile("" : "+v"(ex_mask), "+v"(ex_magic));
   // scale / zero-point of a closed group on the accumulators of one row tile, with the group's row sums
-  float s_[PF_CW], nz_[PF_CW];
+  f32x4_t s_[PF_CW], nz_[PF_CW];
   const float* xs = nullptr;
   auto open_fix = [&](int group) {
-    xs = xsum + (group & 1) * PF_BM + kb * 4;
-#pragma unroll
-    for (int c = 0; c < PF_CW; ++c) {
-      s_[c] = ft_bits_to_f32<FT>(szreg[c] & 0xFFFFu);
-      nz_[c] = -(ft_bits_to_f32<FT>(szreg[c] >> 16) + EX::OFFSET);
-    }
-  };
-  auto fix = [&](int rt, const f32x4_t& xv) {
+    xs = xsum + (group & 1) * PF_BM + wm * PF_RT * 16 + ni;
 #pragma unroll
     for (int c = 0; c < PF_CW; ++c)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) tot[rt][c][r] = fmaf(s_[c], fmaf(nz_[c], xv[r], acc[rt][c][r]), tot[rt][c][r]);
+      for (int r = 0; r < 4; ++r) {
+        s_[c][r] = ft_bits_to_f32<FT>(szreg[c][r] & 0xFFFFu);
+        nz_[c][r] = -(ft_bits_to_f32<FT>(szreg[c][r] >> 16) + EX::OFFSET);
+      }
+  };
+  auto fix = [&](int rt, int c, float xv) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) tot[rt][c][r] = fmaf(s_[c][r], fmaf(nz_[c][r], xv, acc[rt][c][r]), tot[rt][c][r]);
+  };
+  auto load_sz = [&](int group) {
+#pragma unroll
+    for (int c = 0; c < PF_CW; ++c) szreg[c] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(szp[c], kb * 16, min(group, a.Gp - 1) * 64, 0));
   };
 
   // One barrier per k-tile.  Behind it: this tile (its loads are a k-tile old) is in LDS, the other buffer has been read, the row sums of the tile
@@ -207,11 +214,9 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
   int grp = GPT ? kt0 : (a.ktpg < a.KT ? kt0 / a.ktpg : 0);     // running group (a K part starts on a group boundary)
   load_a(kt0, 0);
   load_b(kt0);
-#pragma unroll
-  for (int c = 0; c < PF_CW; ++c) sznew[c] = __builtin_amdgcn_raw_buffer_load_b32(szp[c], ni * 4, min(grp, a.Gp - 1) * 64, 0);
   const u32x4_t ones = FT == DIHIP_BF16 ? u32x4_t{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u}
                                   : u32x4_t{0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
-  if constexpr (GPT) {   // the first tile closes a group of nothing: sums, scales and products 0
+  if constexpr (LACE) {   // the first tile closes a group of nothing: sums, scales and products 0
     if (tid < 2 * PF_BM) xsum[tid] = 0.f;
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): scalar loads still in flight would make every wait for an LDS read this one
@@ -223,33 +228,31 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
     u32x4_t wcur[PF_CW];
 #pragma unroll
     for (int c = 0; c < PF_CW; ++c) {
-      asm volatile("" : "+v"(wreg[c]), "+v"(sznew[c]));   // here they are: nothing further down waits for loads again
+      asm volatile("" : "+v"(wreg[c]), "+v"(szreg[c]));   // here they are: nothing further down waits for loads again
       wcur[c] = wreg[c];
     }
-    if constexpr (GPT) {
+    if constexpr (LACE) {
       open_fix(grp - 1);
-    } else if (kt > kt0 && gl == 0) {                         // (uniform) the tile before closed its group
+    } else if (kt > kt0 && (GPT || gl == 0)) {                         // (uniform) the tile before closed its group
       open_fix(grp - 1);
 #pragma unroll
       for (int rt = 0; rt < PF_RT; ++rt) {
-        fix(rt, *reinterpret_cast<const f32x4_t*>(xs + (wm * PF_RT + rt) * 16));
+        const float xv = xs[rt * 16];
 #pragma unroll
-        for (int c = 0; c < PF_CW; ++c) acc[rt][c] = zero4;
+        for (int c = 0; c < PF_CW; ++c) {
+          fix(rt, c, xv);
+          acc[rt][c] = zero4;
+        }
       }
-    }
-    if (GPT || gl == 0) {
-#pragma unroll
-      for (int c = 0; c < PF_CW; ++c) szreg[c] = sznew[c];      // the running group's
     }
     const int nkt = min(kt + 1, kt1 - 1);                       // past the end: once more the last, read by nobody
     load_a(nkt, buf ^ 1);
     load_b(nkt);
-#pragma unroll
-    for (int c = 0; c < PF_CW; ++c) sznew[c] = __builtin_amdgcn_raw_buffer_load_b32(szp[c], ni * 4, min(grp + 1, a.Gp - 1) * 64, 0);
+    load_sz(grp);
     const unsigned char* tile = smem + buf * ABYTES;
     u32x4_t af[PF_RT], bf[PF_CW], own;
-    f32x4_t xv = zero4;
-    if constexpr (GPT) xv = *reinterpret_cast<const f32x4_t*>(xs + wm * PF_RT * 16);
+    float xv = 0.f;
+    if constexpr (LACE) xv = xs[0];
 #pragma unroll
     for (int rt = 0; rt < PF_RT; ++rt) af[rt] = aread(tile, wm * PF_RT + rt, 0);
     own = aread(tile, wave, 0);
@@ -263,16 +266,17 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
 #pragma unroll
       for (int rt = 0; rt < PF_RT; ++rt) {
         if constexpr (FIRST) {
-          fix(rt, xv);
+          fix(rt, 0, xv);
+          fix(rt, 1, xv);
+          if (rt + 1 < PF_RT) xv = xs[(rt + 1) * 16];
           // (the products that start the next sums wait for the old sums to be used: one set of registers)
           asm volatile("" : "+v"(tot[rt][0]), "+v"(tot[rt][1]), "+v"(af[rt]));
-          if (rt + 1 < PF_RT) xv = *reinterpret_cast<const f32x4_t*>(xs + (wm * PF_RT + rt + 1) * 16);
         }
 #pragma unroll
-        for (int c = 0; c < PF_CW; ++c) acc[rt][c] = mfma16<FT>(af[rt], bf[c], FIRST ? zero4 : acc[rt][c]);
+        for (int c = 0; c < PF_CW; ++c) acc[rt][c] = mfma16<FT>(bf[c], af[rt], FIRST ? zero4 : acc[rt][c]);
         if (ks + 1 < KSTEPS) af[rt] = aread(tile, wm * PF_RT + rt, ks + 1);
         if (rt == 2) {
-          sx = mfma16<FT>(own, ones, sx);
+          sx = mfma16<FT>(ones, own, sx);
           if (ks + 1 < KSTEPS) own = aread(tile, wave, ks + 1);
         }
         if (ks + 1 < KSTEPS && rt >= PF_RT - 1 - PF_CW && rt < PF_RT - 1) bn[rt - (PF_RT - 1 - PF_CW)] = EX::frag(wcur[rt - (PF_RT - 1 - PF_CW)], ks + 1, ex_mask, ex_magic);
@@ -283,17 +287,12 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
         for (int c = 0; c < PF_CW; ++c) bf[c] = bn[c];
       }
     };
-    kstep(0, std::integral_constant<bool, GPT != 0>{});
+    kstep(0, std::integral_constant<bool, LACE>{});
 #pragma unroll
     for (int ks = 1; ks < KSTEPS; ++ks) kstep(ks, std::false_type{});
-    if (ni == 0) {   // the lane with ni == 0 of a row's lanes owns its entry: no race
-      f32x4_t* p = reinterpret_cast<f32x4_t*>(xsum + (grp & 1) * PF_BM + wave * 16 + kb * 4);
-      if (GPT || gl == 0) {
-        *p = sx;
-      } else {
-        const f32x4_t o = *p;
-        *p = f32x4_t{o[0] + sx[0], o[1] + sx[1], o[2] + sx[2], o[3] + sx[3]};
-      }
+    if (kb == 0) {   // the lane with kb == 0 of a row's lanes owns its entry: no race
+      float* p = xsum + (grp & 1) * PF_BM + wave * 16 + ni;
+      *p = GPT || gl == 0 ? sx[0] : *p + sx[0];
     }
     ++gl;
     if (GPT || gl == a.ktpg || kt + 1 == kt1) {
@@ -306,58 +305,106 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
   __syncthreads();
   open_fix(grp - 1);
 #pragma unroll
-  for (int rt = 0; rt < PF_RT; ++rt) fix(rt, *reinterpret_cast<const f32x4_t*>(xs + (wm * PF_RT + rt) * 16));
+  for (int rt = 0; rt < PF_RT; ++rt) {
+    const float xv = xs[rt * 16];
+#pragma unroll
+    for (int c = 0; c < PF_CW; ++c) fix(rt, c, xv);
+  }
 
   // ---- split in K: this part's f32 tile to the slab (rows / columns of the workgroup tile; SwiGLU: gate columns, then up) ----
   if (split_part >= 0) {  // (uniform)
-    float* st = a.slab + ((size_t)split_tile * a.ksplit + split_part) * (PF_BM * 256);
+    float* st = a.slab + ((size_t)split_tile * a.ksplit + split_part) * (PF_BM * 256) + (size_t)(wm * PF_RT * 16 + ni) * 256;
 #pragma unroll
     for (int rt = 0; rt < PF_RT; ++rt) {
       if (m0 + (wm * PF_RT + rt) * 16 >= a.M) break;  // (uniform) rows past M are never read
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = (wm * PF_RT + rt) * 16 + kb * 4 + r;
-#pragma unroll
-        for (int c = 0; c < PF_CW; ++c) {
-          const int col = DUAL ? (c < HCW ? 0 : 128) + (wn * HCW + (c % HCW)) * 16 + ni : (wn * PF_CW + c) * 16 + ni;
-          st[(size_t)row * 256 + col] = tot[rt][c][r];
-        }
+      for (int c = 0; c < PF_CW; ++c) {
+        const int col = DUAL ? (c < HCW ? 0 : 128) + (wn * HCW + (c % HCW)) * 16 : (wn * PF_CW + c) * 16;
+        *reinterpret_cast<f32x4_t*>(st + (size_t)rt * 16 * 256 + col + kb * 4) = tot[rt][c];
       }
     }
     return;
   }
-  // ---- epilogue: lane (kb, ni) holds rows rt * 16 + kb * 4 + r of column tile c, column ni --------------------
+  // ---- epilogue: lane (kb, ni) holds row rt * 16 + ni, columns kb * 4 .. + 3 of column tile c.  Through buffer accesses whose bounds drop what
+  // lies past M and N: no branch per element, the exponentials and divisions of neighbours overlap (with a branch around every
+  // element they ran one after the other: the epilogue was 15 % of the gate / up pair's time) ----
+  const int rows = min(PF_BM, a.M - m0);
+  const bool wide = a.wide_out != 0;   // (uniform) four columns of a row are one aligned access
+  constexpr int OB = EPI == EPI_ADDTO ? 4 : 2;
+  const int ldo = EPI == EPI_ADDTO ? a.N : a.ldy;
+  const auto view = [&](const void* p) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(static_cast<const char*>(p) + (size_t)m0 * ldo * OB), 0, p ? ((rows - 1) * ldo + a.N) * OB : 0, 0x00020000);
+  };
+  const auto out = view(EPI == EPI_ADDTO ? a.h_out : a.y);
+  const auto res = view(EPI == EPI_ADDTO ? static_cast<const void*>(a.h_res) : EPI == EPI_STD ? a.residual : nullptr);
 #pragma unroll
-  for (int rt = 0; rt < PF_RT; ++rt) {
+  for (int c = 0; c < (DUAL ? HCW : PF_CW); ++c) {
+    const int n = tile[c] * 16 + kb * 4;
+    float bias[4] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (EPI == EPI_STD) {
+      if (a.bias) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m0 + (wm * PF_RT + rt) * 16 + kb * 4 + r;
-      if (m >= a.M) continue;
+        for (int r = 0; r < 4; ++r) bias[r] = load_ft<FT>(a.bias, min(n + r, a.N - 1));
+      }
+    }
+    // byte offset of an element; what may not be touched lies outside every view
+    const auto at = [&](int rt, int r) {
+      const int row = (wm * PF_RT + rt) * 16 + ni;
+      return tile_ok[c] && n + r < a.N && row < rows ? (row * ldo + n + r) * OB : 0x7FFFFFF0;
+    };
+#pragma unroll
+    for (int rt = 0; rt < PF_RT; ++rt) {
+      f32x4_t v = tot[rt][c];
       if constexpr (DUAL) {
 #pragma unroll
-        for (int c = 0; c < HCW; ++c) {
-          const int n = tile[c] * 16 + ni;
-          if (tile_ok[c] && n < a.N) {
-            const float g = tot[rt][c][r], u = tot[rt][HCW + c][r];
-            store_ft<FT>(a.y, (size_t)m * a.ldy + n, (g / (1.f + expf(-g))) * u);
+        for (int r = 0; r < 4; ++r) v[r] = (v[r] / (1.f + expf(-v[r]))) * tot[rt][HCW + c][r];
+      } else if constexpr (EPI == EPI_STD) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          v[r] = a.alpha * v[r];
+          if (a.bias) v[r] += bias[r];
+          v[r] = apply_act(v[r], a.act);
+        }
+        if (a.residual) {
+          u32x2_t q;
+          if (wide) {
+            q = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(res, at(rt, 0), 0, 0));
+          } else {
+            uint32_t e[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) e[r] = __builtin_amdgcn_raw_buffer_load_b16(res, at(rt, r), 0, 0);
+            q = u32x2_t{e[0] | e[1] << 16, e[2] | e[3] << 16};
           }
+          const u32x2_t w = {pack_ft2<FT>(v[0], v[1]), pack_ft2<FT>(v[2], v[3])};
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            v[r] = ft_bits_to_f32<FT>((w[r >> 1] >> (r & 1) * 16) & 0xFFFFu) + ft_bits_to_f32<FT>((q[r >> 1] >> (r & 1) * 16) & 0xFFFFu);
         }
       } else {
+        f32x4_t base;   // (no h_res: an empty view, zeros)
+        if (wide) {
+          base = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(res, at(rt, 0), 0, 0));
+        } else {
 #pragma unroll
-        for (int c = 0; c < PF_CW; ++c) {
-          const int n = tile[c] * 16 + ni;
-          if (!tile_ok[c] || n >= a.N) continue;
-          float v = tot[rt][c][r];
-          if constexpr (EPI == EPI_STD) {
-            v = a.alpha * v;
-            if (a.bias) v += load_ft<FT>(a.bias, n);
-            v = apply_act(v, a.act);
-            if (a.residual) v = ft_round<FT>(v) + load_ft<FT>(a.residual, (size_t)m * a.ldy + n);
-            store_ft<FT>(a.y, (size_t)m * a.ldy + n, v);
-          } else {
-            const float base = a.h_res ? a.h_res[(size_t)m * a.N + n] : 0.f;
-            a.h_out[(size_t)m * a.N + n] = base + a.alpha * v;
-          }
+          for (int r = 0; r < 4; ++r) base[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(res, at(rt, r), 0, 0));
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = base[r] + a.alpha * v[r];
+      }
+      if constexpr (EPI == EPI_ADDTO) {
+        if (wide) {
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), out, at(rt, 0), 0, 0);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v[r]), out, at(rt, r), 0, 0);
+        }
+      } else {
+        const u32x2_t q = {pack_ft2<FT>(v[0], v[1]), pack_ft2<FT>(v[2], v[3])};
+        if (wide) {
+          __builtin_amdgcn_raw_buffer_store_b64(q, out, at(rt, 0), 0, 0);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(q[r >> 1] >> (r & 1) * 16), out, at(rt, r), 0, 0);
         }
       }
     }

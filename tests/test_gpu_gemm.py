@@ -730,3 +730,29 @@ def test_prefill_gemm_whole_grid_split(ops, wbits, G, M, N, K):
     rows = to_dev(rng.normal(0, 1, (M, K)).astype(np.float32))
     a, b = ops.fused_norm_gemm(rows, gamma, 1e-6, pw, None, sc).float(), ops.fused_norm_gemm(rows, gamma, 1e-6, pw, None, small).float()
     assert float((a - b).abs().max()) <= 2 ** -7 * float(b.abs().max())     # f32 sums in another order, rounded to bf16
+
+
+# The unsplit epilogue of the context-phase GEMM writes four columns of a row at once where output and residual allow it: rows past M in the last
+# block, an output and a residual that start one element off (the element path), and nothing written outside the output.
+@pytest.mark.gpu
+@pytest.mark.parametrize("wbits,G,M,N,K", [(4, 128, 130, 264, 512), (8, -1, 64, 20, 512), (4, 128, 255, 516, 384)])
+def test_prefill_gemm_output_alignment(ops, wbits, G, M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    x, q, s, z = make_case(rng, M, N, K, G, wbits, "bf16", style="iq")
+    pw = ops.pack_lowp(to_dev(q), to_dev(s, "bf16"), to_dev(z, "bf16"), G, wbits)
+    xd = to_dev(x, "bf16")
+    sc = ops.Scratch(ops.lowp_workspace_bytes(wbits, M, N, K, G))
+    res = to_dev(bf16_round(rng.normal(0, 1, (M, N)).astype(np.float32)), "bf16")
+    pre = gemm_ref.gemm_a16wx(x, q, s, z, G, wbits, ft="bf16")
+    want = bf16_round(pre + res.float().cpu().numpy())
+    outs = []
+    for off in (4, 1):
+        buf = torch.full((M * N + 8,), 77.0, dtype=torch.bfloat16, device="cuda")
+        rbuf = torch.zeros(M * N + 8, dtype=torch.bfloat16, device="cuda")
+        y, r = buf[off:off + M * N].view(M, N), rbuf[off:off + M * N].view(M, N)
+        r.copy_(res)
+        ops.gemm_lowp(xd, pw, residual=r, scratch=sc, out=y)
+        assert_close(y.float().cpu().numpy(), want, "bf16", what=f"offset {off}", pre=pre)
+        assert bool((buf[:off] == 77).all()) and bool((buf[off + M * N:] == 77).all())
+        outs.append(y.clone())
+    assert torch.equal(outs[0], outs[1])
