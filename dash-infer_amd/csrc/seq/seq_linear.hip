@@ -4,7 +4,8 @@
 //   linear_pipe_kernel   bf16 operands on the matrix cores, pipelined tiles of 256 x 256 or 128 x 128, K split where tiles are few (seq_linear_tile.hip)
 //   linear_mfma_kernel   the same for f32 rows (rounded to bf16), K % 64 != 0 or unaligned operands: 128 x 128 x 32 tiles through registers
 //   linear_stream_kernel bf16 operands, 2 .. 64 rows: weights straight from memory into the matrix cores, K split over a workgroup's waves
-//   linear_skinny_kernel one row against a streamed weight (decode), one wave per 2 weight rows; up to 4 rows at a time in f32 products
+//   linear_row_kernel    one row (decode), bf16 operands: two workgroups per CU walk the weight rows past x in registers
+//   linear_skinny_kernel one short row, one row per group, up to 4 rows at a time in f32 products: a streamed weight, one wave per 2 weight rows
 //   linear_fewcols_kernel a router's logits
 // Within a kernel an output element is summed over k in a fixed order: it does not depend on T.
 #include <algorithm>
@@ -302,6 +303,123 @@ __device__ __forceinline__ float dot8_bf16(const u32x4_t& w, const u32x4_t& x, f
   return acc;
 }
 
+// One row of x (decoding one sequence) against bf16 weights.  Bound by the weights' bytes, in launches too short for workgroups that come and go: two
+// workgroups per CU live for the whole launch, each owns a run of neighbouring weight rows, its 4 waves hold a quarter of x each -- C pieces of
+// 512 elements, in registers as f32 -- and walk the same weight rows, so that the loop is weight loads and multiply-adds and nothing else.  Two batches of
+// about 8 KiB per wave in turn, the next in flight while one is multiplied (copying one into the other would wait for it).
+// The sums of the waves meet in LDS once, at the end; a lane's k ascend, lanes and waves are added in a fixed order.
+// One wave per two weight rows (linear_skinny_kernel) -> this, us: 4096 -> 4096 11.5 -> 8.0, 14336 -> 4096 29.4 -> 21.7, 4096 -> 14336 26.9 -> 21.8,
+// 4096 -> 32000 52.7 -> 44.5 (5.9 TB/s).
+// MASK: K does not fill the pieces: x is zero there and the loads stay inside the row.
+constexpr int ROW_WAVES = 4, ROW_WGS = 512, ROW_MAXC = 8, ROW_MAX_ROWS = 1024;   // weight rows of a workgroup: 16 KB of sums
+template <int XT, int C, bool MASK>
+__global__ __launch_bounds__(64 * ROW_WAVES, 2) void linear_row_kernel(LinArgs a) {
+  constexpr int R = C >= 5 ? 1 : 8 / C;        // weight rows per batch
+  extern __shared__ __attribute__((aligned(16))) float part[];   // [row][wave]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lo = (int)((long)a.N * blockIdx.x / gridDim.x), hi = (int)((long)a.N * (blockIdx.x + 1) / gridDim.x);
+  const uint16_t* w = (const uint16_t*)a.w + (size_t)lo * a.K;
+  int k[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) k[c] = ((wave * C + c) * 64 + lane) * 8;
+  const int rows = hi - lo;
+  auto load = [&](u32x4_t (&d)[R][C], int r0) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const uint16_t* row = w + (size_t)min(r0 + r, rows - 1) * a.K;   // (uniform) past the end: the last row once more
+#pragma unroll
+      for (int c = 0; c < C; ++c) d[r][c] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(row + (MASK ? min(k[c], a.K - 8) : k[c])));
+    }
+  };
+  u32x4_t wa[R][C], wb[R][C], q[C], q2[C];   // (q2: f32 rows)
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const size_t src = lin_xrow(a, 0) * a.ldx + (MASK ? min(k[c], a.K - 8) : k[c]);
+    q[c] = *reinterpret_cast<const u32x4_t*>((const unsigned char*)a.x + src * (XT == DIHIP_F32 ? 4 : 2));
+    if constexpr (XT == DIHIP_F32) q2[c] = *reinterpret_cast<const u32x4_t*>((const float*)a.x + src + 4);
+  }
+  load(wa, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  float x[C][8];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    if constexpr (XT == DIHIP_F32) {
+      const f32x4_t l4 = __builtin_bit_cast(f32x4_t, q[c]), h4 = __builtin_bit_cast(f32x4_t, q2[c]);
+      q[c] = u32x4_t{pack_bf16x2(l4[0], l4[1]), pack_bf16x2(l4[2], l4[3]), pack_bf16x2(h4[0], h4[1]), pack_bf16x2(h4[2], h4[3])};
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      x[c][2 * i] = __uint_as_float(q[c][i] << 16);
+      x[c][2 * i + 1] = __uint_as_float(q[c][i] & 0xffff0000u);
+    }
+  }
+  auto mul = [&](u32x4_t (&d)[R][C], int r0) {
+    float v[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      v[r] = 0.f;
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        if (MASK && k[c] >= a.K) d[r][c] = u32x4_t{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          v[r] = __builtin_fmaf(__uint_as_float(d[r][c][i] << 16), x[c][2 * i], v[r]);
+          v[r] = __builtin_fmaf(__uint_as_float(d[r][c][i] & 0xffff0000u), x[c][2 * i + 1], v[r]);
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = wave_sum(v[r]);
+    if (lane == 0) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (r0 + r < rows) part[(r0 + r) * ROW_WAVES + wave] = v[r];
+    }
+  };
+  for (int r0 = 0; r0 < rows; r0 += 2 * R) {
+    load(wb, r0 + R);
+    __builtin_amdgcn_sched_barrier(0);
+    mul(wa, r0);
+    __builtin_amdgcn_sched_barrier(0);
+    load(wa, r0 + 2 * R);
+    __builtin_amdgcn_sched_barrier(0);
+    mul(wb, r0 + R);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __syncthreads();
+  for (int r = tid; r < rows; r += 64 * ROW_WAVES) {
+    const f32x4_t p = *reinterpret_cast<const f32x4_t*>(part + r * ROW_WAVES);
+    lin_epilogue(a, 0, 0, lo + r, (p[0] + p[1]) + (p[2] + p[3]), DIHIP_BF16);
+  }
+}
+template <int XT, int C>
+void launch_row_c(const LinArgs& a, hipStream_t s) {
+  const int wgs = a.N < ROW_WGS ? a.N : ROW_WGS;
+  const size_t lds = (size_t)((a.N + wgs - 1) / wgs) * ROW_WAVES * sizeof(float);
+  if (a.K == C * 512 * ROW_WAVES) hipLaunchKernelGGL((linear_row_kernel<XT, C, false>), dim3(wgs), dim3(64 * ROW_WAVES), lds, s, a);
+  else hipLaunchKernelGGL((linear_row_kernel<XT, C, true>), dim3(wgs), dim3(64 * ROW_WAVES), lds, s, a);
+}
+inline int row_pieces(int K) { return (K + 512 * ROW_WAVES - 1) / (512 * ROW_WAVES); }
+// where it is the faster one: long rows always, rows of 1024 .. 2048 from 12 MB of weights on.  linear_skinny_kernel / this, us: 64 x 4096 5.4 / 3.6,
+// 1000 x 2560 5.5 / 5.1, 4096 x 1536 6.2 / 6.0, 8192 x 1024 7.1 / 5.9; but 2048 x 2048 5.3 / 5.6, 4096 x 1024 4.9 / 5.4, 100000 x 256 25.2 / 29.2
+// (waves without a piece)
+inline bool row_kernel(int N, int K) {
+  return row_pieces(K) <= ROW_MAXC && (N + ROW_WGS - 1) / ROW_WGS <= ROW_MAX_ROWS && (K > 2048 || (K >= 1024 && (long)N * K >= 6000000));
+}
+template <int XT>
+void launch_row(const LinArgs& a, hipStream_t s) {
+  switch (row_pieces(a.K)) {
+    case 1: return launch_row_c<XT, 1>(a, s);
+    case 2: return launch_row_c<XT, 2>(a, s);
+    case 3: return launch_row_c<XT, 3>(a, s);
+    case 4: return launch_row_c<XT, 4>(a, s);
+    case 5: return launch_row_c<XT, 5>(a, s);
+    case 6: return launch_row_c<XT, 6>(a, s);
+    case 7: return launch_row_c<XT, 7>(a, s);
+    default: return launch_row_c<XT, 8>(a, s);
+  }
+}
+
 // rows t0 .. t0 + tc (tc <= 4) of x staged in LDS -- as bf16, or as they are (EXACT: f32 products of the unrounded row) --;
 // wave w of block b owns weight rows (b * 4 + w) * 2 .. + 2 and keeps two 1 KiB slices of each in flight.
 // K % 8 == 0 and 16-byte aligned weight rows (host-checked).
@@ -489,6 +607,11 @@ static int linear_impl(void* stream, const void* x, int x_dtype, long ldx, long 
     math = DIHIP_MATH_F32;
   }
   if (math == DIHIP_MATH_BF16 && w_dtype == DIHIP_BF16) {
+    if (Tg == 1 && groups == 1 && !seg && vec && !no_skinny && row_kernel(N, K)) {
+      if (x_dtype == DIHIP_F32) launch_row<DIHIP_F32>(a, s);
+      else launch_row<DIHIP_BF16>(a, s);
+      return launch_status();
+    }
     if (Tg == 1 && vec && !no_skinny && K <= 32768) {   // the row's bf16 copy fits 64 KB of LDS
       const dim3 grid((N + 7) / 8, groups);
       if (x_dtype == DIHIP_F32) hipLaunchKernelGGL((linear_skinny_kernel<DIHIP_F32, false>), grid, dim3(256), (size_t)K * 2, s, a, 0, 1);

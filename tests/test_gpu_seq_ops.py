@@ -74,6 +74,34 @@ def test_linear_streams_few_rows(so, T, N, K, groups, xdt):
     assert float(out[:, :3].abs().max()) == 0 and float(out[:, -4:].abs().max()) == 0
 
 
+@pytest.mark.parametrize("N,K", [(1, 2056), (511, 2048 + 512), (513, 4096), (1030, 4104), (300, 6144), (600, 8192), (514, 10248), (33, 12000), (700, 14336), (40, 16384),
+                                 (5900, 1024), (4100, 2048), (64, 16392)])
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float32])
+def test_linear_one_row(so, N, K, xdt):
+    """One row: every number of pieces per wave, K that fills the waves, ends inside a piece or leaves waves without one (the last: beyond the registers), fewer
+    weight rows than workgroups; every part of the epilogue.  Products of the same rounded operands in 64 bits, f32 sums of at most K / 256 + 12 steps."""
+    rng = np.random.default_rng(N + K)
+    x = dev(rng.normal(0, 1, (1, K + 16)), xdt)[:, 8:8 + K]
+    w, b = dev(rng.normal(0, K ** -0.5, (N, K)), torch.bfloat16), dev(rng.normal(0, 0.3, N), torch.bfloat16)
+    mul = dev(rng.normal(0, 1, (1, N)))
+    xr = x.to(torch.bfloat16).double()
+    plain = xr @ w.double().t() + b.double()
+    size = xr.abs() @ w.double().abs().t() + b.double().abs()
+    y = so.linear(x, w, b, math=so.MATH_BF16)
+    assert bool(((y.double() - plain).abs() <= (K / 256 + 12) * 2.0 ** -24 * size).all())
+    lo, hi = N // 3, N - 1
+    want = plain.clone()
+    want[:, lo:hi] = torch.nn.functional.gelu(want[:, lo:hi], approximate="tanh")
+    y = so.linear(x, w, b, act="gelu_tanh", act_cols=(lo, hi), mul=mul, math=so.MATH_BF16)
+    assert rel_err(y.cpu().numpy(), (want * mul.double()).cpu().numpy()) < 2e-5
+    w[0, K - 8:] = float("inf")            # what the loads past K re-read must not reach another row, nor a zero of x
+    y = so.linear(x, w, b, math=so.MATH_BF16)
+    assert not bool(torch.isfinite(y[0, 0])) and bool(torch.isfinite(y[0, 1:]).all())
+    w[0, K - 8:] = 0
+    w[0, K - 8] = float("inf")
+    assert float(so.linear(x, w, b, math=so.MATH_BF16)[0, 0]) == float(torch.sign(xr[0, K - 8]) * float("inf"))
+
+
 @pytest.mark.parametrize("T,N,K,groups", [(65, 64, 64, 1), (128, 128, 128, 1), (129, 130, 192, 1), (257, 255, 1024, 1), (513, 2048, 576, 1), (300, 36, 2048, 3),
                                           (100, 512, 8192, 1), (2049, 1028, 64, 1), (700, 16, 4096, 1), (1030, 4100, 320, 2)])
 @pytest.mark.parametrize("ws", [True, False])
