@@ -74,7 +74,8 @@ __device__ __forceinline__ f32x4_t mfma_bf16(const u32x4_t& a, const u32x4_t& b,
 // seq_linear_tile.hip: bf16 rows times bf16 weights in pipelined tiles.  ok: the shape is taken (K % 64 == 0; the caller checks types and 16-byte
 // alignment); slab: bytes of workspace for the K parts (0: not split)
 struct LinTilePlan {
-  bool ok, big;        // big: tiles of 256 x 256, else 128 x 128
+  bool ok;
+  int shape;           // of the tiles (seq_linear_tile.hip)
   int parts;
   size_t slab;
 };

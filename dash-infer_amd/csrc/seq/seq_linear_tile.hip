@@ -1,6 +1,6 @@
 // seq_linear_tile.hip -- linear_pipe_kernel: products of many bf16 rows (prompts, portions) with bf16 weights, on the matrix cores.
 //
-// A tile of 256 x 256 (8 waves, 128 x 64 each) walks K in steps of 64 through two LDS slots:
+// A tile of 256 x 256 (8 waves, 128 x 64 each; smaller ones below) walks K in steps of 64 through two LDS slots:
 //   * rows and weights go straight into LDS (global_load_lds, 16 bytes a lane): no registers and no instructions for staging.  A 1 KiB piece is 8
 //     rows x 128 bytes in the order of the lanes (whole cache lines: with 64-byte pieces the L2s had twice the requests, 236 against
 //     226 us), so the 16-byte chunks of a row change places on the memory side (chunk ^ row % 8) and the operand reads of 8
@@ -190,9 +190,18 @@ int go(const LinArgs& a, const LinTilePlan& p, int Tg, int groups, float* slab, 
 }  // namespace
 
 // Which tile, and into how many parts K is split: the shortest of (rounds over the CUs) x (steps of a part) x (time of a step) + the slab's way
-// through memory.  A step, with every CU busy: 256 x 256 1.8 us; 128 x 128 0.9 us for one workgroup per CU, 1.25 for two.  A launch with its
-// prologue 5 us, the launch that adds parts 4 us and the slab's bytes, out and in, at 6 TB/s.  Over 65 .. 2048 rows and 512 .. 32000 columns
-// the choice is within 8 % of the best of 1 .. 12 parts of either tile; unsplit, 513 rows 8192 -> 2048 take 107 us instead of 40.
+// through memory.  192 x 256 is there for row counts that the others cut badly: 513 rows 14336 -> 4096 take 100.7 us in 128 x 128, 102.7 in 256 x 256
+// and 91.3 in 192 x 256; 300 rows 4096 -> 14336 82 / 85 / 74.5; 1500 rows 226 / 208 / 193.  (256 x 224 and 256 x 192, which fill the last round better at
+// some widths, gave 2 % at 2048 rows: the clock falls as the chip fills.)  A launch with its prologue 5 us, the launch that adds parts 4 us and the slab's
+// bytes, out and in, at 4.5 TB/s.  Over 300 .. 2048 rows and 2048 .. 32000 columns the choice is on average within 1 % of the best tile, at worst 11 %
+// behind it; unsplit, 513 rows 8192 -> 2048 take 107 us instead of 39.
+struct TileShape {
+  int bm, bn;
+  double step_us;   // of 64 of K, on every CU at once.  128 x 128: for one workgroup per CU (two at a time: TWO_SMALL_US)
+};
+constexpr TileShape SHAPES[] = {{256, 256, 1.70}, {192, 256, 1.47}, {128, 128, 0.9}};
+constexpr int SMALL = 2;
+constexpr double TWO_SMALL_US = 1.2;
 LinTilePlan plan_linear_tile(int Tg, int N, int K, int groups, long ldx, bool split) {
   LinTilePlan best{};
   if (K % LT_BK || K <= 0 || (size_t)256 * (size_t)K * 2 >= (1ull << 31) || (size_t)Tg * (size_t)ldx * 2 >= (1ull << 30)) return best;
@@ -200,18 +209,17 @@ LinTilePlan plan_linear_tile(int Tg, int N, int K, int groups, long ldx, bool sp
   constexpr int ncu = 256;
   const int all = K / LT_BK;
   double best_us = 0;
-  for (int big = 1; big >= 0; --big) {
-    const int b = big ? 256 : 128;
-    const long tiles = (long)((Tg + b - 1) / b) * ((N + b - 1) / b) * groups;
+  for (int sh = 0; sh <= SMALL; ++sh) {
+    const long tiles = (long)((Tg + SHAPES[sh].bm - 1) / SHAPES[sh].bm) * ((N + SHAPES[sh].bn - 1) / SHAPES[sh].bn) * groups;
     for (int p = 1; p <= (split ? 16 : 1); ++p) {
       if (p > 1 && (all / p < 4 || tiles * p > 2 * ncu)) break;
       const size_t slab = p > 1 ? (size_t)p * Tg * groups * ((N + 3) & ~3) * sizeof(float) : 0;
       if (slab > MOST) break;
       const long wgs = tiles * p;
-      const double round_us = big ? 1.8 * ((wgs + ncu - 1) / ncu) : wgs <= ncu ? 0.9 : 1.25 * ((wgs + 2 * ncu - 1) / (2 * ncu));
-      const double us = round_us * ((all + p - 1) / p) + 5 + (p > 1 ? 4 + 2.0 * slab / 6e6 : 0);
+      const double round_us = sh == SMALL && wgs > ncu ? TWO_SMALL_US * ((wgs + 2 * ncu - 1) / (2 * ncu)) : SHAPES[sh].step_us * ((wgs + ncu - 1) / ncu);
+      const double us = round_us * ((all + p - 1) / p) + 5 + (p > 1 ? 4 + 2.0 * slab / 4.5e6 : 0);
       if (!best.ok || us < best_us) {
-        best = LinTilePlan{true, big != 0, p, slab};
+        best = LinTilePlan{true, sh, p, slab};
         best_us = us;
       }
     }
@@ -221,7 +229,11 @@ LinTilePlan plan_linear_tile(int Tg, int N, int K, int groups, long ldx, bool sp
 
 int launch_linear_tile(const LinArgs& a, const LinTilePlan& p, int Tg, int groups, float* slab, hipStream_t s) {
   DIHIP_REQUIRE(groups <= 65535, DIHIP_PARAM_ERROR, "linear: more than 65535 groups");
-  return p.big ? go<8, 4, 2, 4>(a, p, Tg, groups, slab, s) : go<4, 4, 2, 2>(a, p, Tg, groups, slab, s);
+  switch (p.shape) {
+    case 0: return go<8, 4, 2, 4>(a, p, Tg, groups, slab, s);
+    case 1: return go<6, 4, 2, 4>(a, p, Tg, groups, slab, s);
+    default: return go<4, 4, 2, 2>(a, p, Tg, groups, slab, s);
+  }
 }
 
 }  // namespace dihip

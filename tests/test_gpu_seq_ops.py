@@ -133,6 +133,12 @@ def test_linear_tiles_many_rows(so, T, N, K, groups, ws):
     assert rel_err(odd[:, 3:3 + groups * N].cpu().numpy(), plain.cpu().numpy()) < 2e-5 and float(odd[:, -4:].abs().max()) == 0
 
 
+# 256 x 256 tiles whole and in K parts, 192 x 256 whole and in parts (the plan's choice on 256 CUs; on any other count the same products run in other tiles)
+@pytest.mark.parametrize("T,N,K", [(2040, 16380, 64), (1800, 4096, 8192), (1500, 14337, 64), (190, 14340, 192), (513, 4096, 14336)])
+def test_linear_tile_shapes(so, T, N, K):
+    test_linear_tiles_many_rows(so, T, N, K, 1, True)
+
+
 def test_linear_segmented_tiles(so):
     rng = np.random.default_rng(78)
     counts = [0, 1, 300, 129, 64, 0]
