@@ -61,6 +61,7 @@ _SIGS = {
     "dihip_span_bytes": (sz, [i32, i32, i32, i32, i32]),
     "dihip_kv_append": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32, i32]),
     "dihip_rope_kv_append": (i32, [vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32, i32]),
+    "dihip_rope_kv_context": (i32, [vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32, i32]),
     "dihip_kv_context_copy": (i32, [vp, vp, vp, i32, i32, i32, i32, i32, i32, i32, i32]),
     "dihip_kv_prefix_gather": (i32, [vp, vp, vp, i32, i32, i32, i32, i32, i32]),
     "dihip_span_gather": (i32, [vp, vp, vp, i32, sz]),

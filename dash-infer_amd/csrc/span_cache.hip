@@ -115,6 +115,58 @@ __global__ __launch_bounds__(64) void kv_context_copy_kernel(void* const* spans,
   store_token_head<FT, MODE, EPL>(spans[tok / S], x, head, tok % S, g, S, H, lane);
 }
 
+// ---- Rotary + ContextSpanCopy of K and V over the rows of several prompts, one launch -------------------------------------------
+// Same results as dihip_rope_qk on the rows followed by dihip_kv_context_copy of their K and V parts.  Bound by the rows' bytes, in and out (2048 x 4608
+// bf16: 36 MB with the cache).  A workgroup takes a row, a wave every ROPE_WAVESth head of it: the sines of the row are computed once per wave
+// instead of once per head (range reduction in f64: 18 us for those rows, and two copies of 4.8), and eight heads are in flight at once.
+constexpr int ROPE_WAVES = 4, ROPE_HEADS = 8;
+template <int FT, int MODE, int EPL>
+__global__ __launch_bounds__(64 * ROPE_WAVES) void rope_kv_context_kernel(void* const* k_spans, void* const* v_spans, void* qkv, const uint32_t* __restrict__ positions,
+                                                                          const int32_t* __restrict__ request, const float* __restrict__ inv_freq, int n, int g, int S,
+                                                                          int span_stride) {
+  constexpr int H = 64 * EPL;
+  const int t = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int heads = n + 2 * g;
+  const size_t row = (size_t)t * heads * H;
+  const uint32_t pos = positions[t], span = pos / S, slot = pos - span * S;
+  const bool held = span < (uint32_t)span_stride;   // past the request's span table: not stored
+  const size_t entry = (size_t)request[t] * span_stride + (held ? span : 0);
+  void* const ks = k_spans[entry];
+  void* const vs = v_spans[entry];
+  // lane holds d = lane * EPL ..; the rotate-half partner (d +- H / 2) lives in lane ^ 32
+  float cs[EPL], sn[EPL];
+#pragma unroll
+  for (int i = 0; i < EPL; ++i) rope_sincos(pos, inv_freq[(lane * EPL + i) & (H / 2 - 1)], &sn[i], &cs[i]);
+  for (int h0 = wave; h0 < heads; h0 += ROPE_WAVES * ROPE_HEADS) {
+    float x[ROPE_HEADS][EPL];
+#pragma unroll
+    for (int j = 0; j < ROPE_HEADS; ++j) {
+      const int head = min(h0 + j * ROPE_WAVES, heads - 1);
+#pragma unroll
+      for (int i = 0; i < EPL; ++i) x[j][i] = load_ft<FT>(qkv, row + (size_t)head * H + lane * EPL + i);
+    }
+#pragma unroll
+    for (int j = 0; j < ROPE_HEADS; ++j) {
+      const int head = h0 + j * ROPE_WAVES;
+      if (head >= heads) break;   // (uniform)
+      if (head < n + g) {
+#pragma unroll
+        for (int i = 0; i < EPL; ++i) {
+          const float partner = __shfl_xor(x[j][i], 32, 64);
+          const float r = lane < 32 ? x[j][i] * cs[i] - partner * sn[i] : x[j][i] * cs[i] + partner * sn[i];
+          x[j][i] = FT == DIHIP_F32 ? r : ft_round<FT == DIHIP_F32 ? DIHIP_BF16 : FT>(r);
+        }
+#pragma unroll
+        for (int i = 0; i < EPL; ++i) store_ft<FT>(qkv, row + (size_t)head * H + lane * EPL + i, x[j][i]);
+      }
+      if (head >= n && held) {
+        const bool isk = head < n + g;
+        store_token_head<FT, MODE, EPL>(isk ? ks : vs, x[j], head - (isk ? n : n + g), slot, g, S, H, lane);
+      }
+    }
+  }
+}
+
 // ---- PrefixCacheCopy (prefix_cache_copy.cuh:37-106): spans -> contiguous, dequantised ----------
 template <int FT, int MODE, int EPL>
 __global__ __launch_bounds__(64) void kv_prefix_gather_kernel(void* dst, void* const* spans, int g, int S) {
@@ -241,6 +293,23 @@ int dihip_kv_context_copy(void* stream, void* const* spans, const void* src, int
     constexpr int FT = decltype(ftc)::value, MODE = decltype(mc)::value, EPL = decltype(ec)::value;
     hipLaunchKernelGGL((kv_context_copy_kernel<FT, MODE, EPL>), dim3(seq_len, num_groups), dim3(64), 0, s, spans, src,
                        src_stride, start_pos, num_groups, span_len);
+  });
+  if (!ok) return DIHIP_PARAM_ERROR;
+  return launch_status();
+}
+
+int dihip_rope_kv_context(void* stream, void* const* k_spans, void* const* v_spans, void* qkv, const uint32_t* positions,
+                          const int32_t* request, const float* inv_freq, int rows, int num_heads, int num_groups, int head_size,
+                          int span_len, int span_stride, int kv_mode, int dtype) {
+  DIHIP_REQUIRE(rows >= 0 && num_heads > 0 && num_groups > 0 && span_stride > 0, DIHIP_PARAM_ERROR, "rope_kv_context: bad shape");
+  DIHIP_REQUIRE(span_len_ok(span_len), DIHIP_PARAM_ERROR, "rope_kv_context: span size %d", span_len);
+  DIHIP_REQUIRE(k_spans && v_spans && qkv && positions && request && inv_freq, DIHIP_PARAM_ERROR, "rope_kv_context: null pointer");
+  if (rows == 0) return DIHIP_SUCCESS;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const bool ok = kv_dispatch(dtype, kv_mode, head_size, [&](auto ftc, auto mc, auto ec) {
+    constexpr int FT = decltype(ftc)::value, MODE = decltype(mc)::value, EPL = decltype(ec)::value;
+    hipLaunchKernelGGL((rope_kv_context_kernel<FT, MODE, EPL>), dim3(rows), dim3(64 * ROPE_WAVES), 0, s, k_spans, v_spans, qkv, positions, request,
+                       inv_freq, num_heads, num_groups, span_len, span_stride);
   });
   if (!ok) return DIHIP_PARAM_ERROR;
   return launch_status();

@@ -707,19 +707,19 @@ class DecodeSession:
             for b in grp:
                 cut.append(cut[-1] + lens[b])
             ids = torch.as_tensor([t for b in grp for t in seqs[b]], dtype=torch.int64, device=dev)
-            pos = torch.cat([torch.arange(lens[b], dtype=torch.int32, device=dev) for b in grp])
+            rows_of = torch.empty(2, T, dtype=torch.int32)     # position and request of every row
+            for b, lo, hi in zip(grp, cut, cut[1:]):
+                torch.arange(hi - lo, dtype=torch.int32, out=rows_of[0, lo:hi])
+                rows_of[1, lo:hi] = b
+            pos, req = rows_of.to(dev)
             h = ops.embedding(ids, m.embed)
             for li, lw in enumerate(m.layers):
                 qkv = ops.fused_norm_gemm(h, lw.ln1, cfg.eps, lw.qkv, lw.qkv_bias, sc)
-                ops.rope_qk_(qkv, pos, self.inv_freq, n, g, H)
-                kv = self.kv[li]
-                stride = (n + 2 * g) * H
+                ops.rope_kv_context(self.kv[li], qkv, pos, req, self.inv_freq, n, g, H)
                 attn = torch.empty(T, n * H, dtype=qkv.dtype, device=dev)
-                for b, lo, hi in zip(grp, cut, cut[1:]):
+                for lo, hi in zip(cut, cut[1:]):
                     rows = qkv[lo:hi]
                     q, k, v = rows[:, : n * H], rows[:, n * H:(n + g) * H], rows[:, (n + g) * H:]
-                    ops.kv_context_copy(kv.k_ptrs[b], k, stride, hi - lo, 0, g, H, self.pool.S, self.kv_mode)
-                    ops.kv_context_copy(kv.v_ptrs[b], v, stride, hi - lo, 0, g, H, self.pool.S, self.kv_mode)
                     ops.prefill_attn(q, k, v, n, g, H, self.scale, out=attn[lo:hi])
                 h = ops.fused_gemm_addto(attn, lw.o, h, sc, M=T)
                 if cfg.moe is not None:

@@ -425,6 +425,13 @@ def rope_kv_append(kv, q_out, qkv, old_lens, inv_freq, n, g, H):
           "dihip_rope_kv_append")
 
 
+def rope_kv_context(kv, qkv, positions, request, inv_freq, n, g, H):
+    """Rotary in place on the fused rows of prompts, and their K and V into the spans of kv: row r is token positions[r] of request[r]."""
+    pool = kv.pool
+    check(lib().dihip_rope_kv_context(cur_stream(), ptr(kv.k_ptrs), ptr(kv.v_ptrs), ptr(qkv), ptr(positions), ptr(request), ptr(inv_freq),
+                                      qkv.shape[0], n, g, H, pool.S, kv.max_spans, capi.KV[pool.mode], dt_code(qkv)), "dihip_rope_kv_context")
+
+
 def kv_context_copy(span_ptrs_row, src, src_stride, seq_len, start_pos, g, H, S, mode):
     check(lib().dihip_kv_context_copy(cur_stream(), ptr(span_ptrs_row), ptr(src), src_stride, seq_len, start_pos, g, H,
                                       S, capi.KV[mode], dt_code(src)), "dihip_kv_context_copy")

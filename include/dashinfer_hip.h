@@ -283,6 +283,13 @@ int dihip_kv_context_copy(void* stream, void* const* spans, const void* src, int
                           int seq_len, int start_pos, int num_groups, int head_size, int span_len,
                           int kv_mode, int dtype);
 
+/* Rotary + ContextSpanCopy of K and V in one launch, over fused qkv rows [rows, (n+2g)*H] of one or several prompts: the same results
+ * as dihip_rope_qk (q and k rotated in place, at positions[row]) followed by dihip_kv_context_copy of the rows' K and V parts to token
+ * positions[row] of request request[row].  k_spans / v_spans: device arrays [requests][span_stride] of span pointers.            */
+int dihip_rope_kv_context(void* stream, void* const* k_spans, void* const* v_spans, void* qkv, const uint32_t* positions,
+                          const int32_t* request, const float* inv_freq, int rows, int num_heads, int num_groups,
+                          int head_size, int span_len, int span_stride, int kv_mode, int dtype);
+
 /* PrefixCacheCopyLauncher: spans -> contiguous dst [prefix_len, g, H] FT with dequantisation.  */
 int dihip_kv_prefix_gather(void* stream, void* dst, void* const* spans, int prefix_len,
                            int num_groups, int head_size, int span_len, int kv_mode, int dtype);

@@ -92,6 +92,47 @@ def test_kv_append_byte_exact(ops, mode, ft):
             np.testing.assert_array_equal(pool.span_view(kv.v_idx[b][i]).cpu().numpy(), sp, err_msg=f"V b{b} span{i}")
 
 
+@pytest.mark.parametrize("mode,ft,H,n,g,S", [("none", "bf16", 128, 28, 4, 32), ("i8", "bf16", 128, 7, 1, 16), ("u4", "f16", 128, 3, 3, 64), ("none", "f16", 64, 33, 2, 32),
+                                             ("u4", "bf16", 128, 64, 8, 128)])
+def test_rope_kv_context_is_rotary_and_two_copies(ops, mode, ft, H, n, g, S):
+    """Rows of several prompts in one launch: the rotated rows and the spans hold the bytes of Rotary followed by a copy of K and one of V per prompt -- fewer and
+    more heads than the waves hold at once, a prompt of one row, ends inside and at the end of a span; a row past the span table is rotated and not stored."""
+    rng = np.random.default_rng(n + g)
+    lens, cap = [1, 2 * S, 77], -(-max(2 * S, 77) // S)
+    T = sum(lens)
+    rows = dev(RND[ft](rng.normal(0, 2, (T, (n + 2 * g) * H)).astype(np.float32)), ft)
+    inv = torch.from_numpy((1e4 ** (-np.arange(0, H, 2) / H)).astype(np.float32)).cuda()
+    pos = torch.cat([torch.arange(L, dtype=torch.int32) for L in lens]).cuda()
+    req = torch.as_tensor([b for b, L in enumerate(lens) for _ in range(L)], dtype=torch.int32, device="cuda")
+    got = []
+    for fused in (True, False):
+        pool = ops.SpanPool(64, g, S, H, mode, TD[ft])
+        pool.pool.zero_()
+        kv = ops.KVCacheSet(pool, len(lens), cap)
+        for b, L in enumerate(lens):
+            kv.ensure(b, L)
+        kv.sync()
+        q = rows.clone()
+        if fused:
+            ops.rope_kv_context(kv, q, pos, req, inv, n, g, H)
+        else:
+            ops.rope_qk_(q, pos, inv, n, g, H)
+            lo = 0
+            for b, L in enumerate(lens):
+                part = q[lo:lo + L]
+                ops.kv_context_copy(kv.k_ptrs[b], part[:, n * H:], (n + 2 * g) * H, L, 0, g, H, S, mode)
+                ops.kv_context_copy(kv.v_ptrs[b], part[:, (n + g) * H:], (n + 2 * g) * H, L, 0, g, H, S, mode)
+                lo += L
+        got.append((q, pool.pool.clone()))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    before = pool.pool.clone()
+    far = torch.full((1,), cap * S, dtype=torch.int32, device="cuda")
+    one, two = rows[:1].clone(), rows[:1].clone()
+    ops.rope_kv_context(kv, one, far, req[:1], inv, n, g, H)
+    ops.rope_qk_(two, far, inv, n, g, H)
+    assert torch.equal(one, two) and torch.equal(before, pool.pool)
+
+
 @pytest.mark.parametrize("mode", ["none", "i8", "u4"])
 def test_context_copy_prefix_gather_roundtrip(ops, mode):
     """ContextSpanCopy writes the prefill K into spans byte-exactly; PrefixCacheCopy reads them
