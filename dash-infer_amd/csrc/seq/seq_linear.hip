@@ -3,7 +3,8 @@
 //   linear_tile_kernel   every product and sum in f32, k ascending (DIHIP_MATH_F32; also any operand type / odd shape)
 //   linear_pipe_kernel   bf16 operands on the matrix cores, pipelined tiles of 256 x 256 or 128 x 128, K split where tiles are few (seq_linear_tile.hip)
 //   linear_mfma_kernel   the same for f32 rows (rounded to bf16), K % 64 != 0 or unaligned operands: 128 x 128 x 32 tiles through registers
-//   linear_stream_kernel bf16 operands, 2 .. 64 rows: weights straight from memory into the matrix cores, K split over a workgroup's waves
+//   linear_stream_lds_kernel  bf16 operands, 2 .. 64 rows, K % 64 == 0 and 1024 or more: both streamed through LDS, K split over a workgroup's waves
+//   linear_stream_kernel the same for f32 rows, other K, gathered rows: weights straight from memory into the matrix cores
 //   linear_row_kernel    one row (decode), bf16 operands: two workgroups per CU walk the weight rows past x in registers
 //   linear_skinny_kernel one short row, one row per group, up to 4 rows at a time in f32 products: a streamed weight, one wave per 2 weight rows
 //   linear_fewcols_kernel a router's logits
@@ -176,9 +177,8 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(LinArgs a, bool vec4) 
 //     neighbouring columns of one output row); a wave issues all loads of a block before the first product, and with PRE the weights of
 //     its next block as well.  Nothing is staged, no barrier before the end: the activations (T x K bf16) live in the L2s;
 //   * the waves' partial sums meet in LDS and are added in the order of the waves: an element's sum does not depend on the rows beside it.
-// 24 rows: 8192 -> 2048 180 -> 24 us, 2048 -> 8192 57 -> 16, 4096 -> 14336 100 -> 41, 4096 -> 32000 104 -> 69 (before: 128 x 128 tiles); 13 rows
-// (before: four passes of the kernel below) 77 -> 18, 41 -> 12, 121 -> 35, 230 -> 69.  What is left is the activations: each workgroup
-// pulls T x K of them from its L2 for ROWS x K weights (one row alone: 15, 11, 28, 54 us).
+// 24 rows: 8192 -> 2048 180 -> 23 us, 2048 -> 8192 57 -> 13, 4096 -> 14336 100 -> 39, 4096 -> 32000 104 -> 70 (before: 128 x 128 tiles).  What is left is the activations:
+// each workgroup pulls T x K of them from its L2 for ROWS x K weights.
 // K % 8 == 0 and 16-byte aligned rows (host-checked).
 template <int XT>
 __device__ __forceinline__ u32x4_t stream_x(const char* p, bool ok) {
@@ -270,6 +270,132 @@ __global__ __launch_bounds__(64 * WV, (ROWS * TF > 64 || XT == DIHIP_F32) ? 2 : 
     for (int i = 1; i < WV; ++i) v += red[i][f][l];
     lin_epilogue4(a, g, lo + t, n, v, lin_bias4(a, g, n, vec4), vec4);
   }
+}
+
+// The same walk for bf16 rows with K % 64 == 0, by LDS: what binds the form above is the number of pieces that its loads touch (an operand is 16 rows x
+// 64 bytes), not the bytes.  Here a wave brings its blocks of 64 elements -- pieces of 8 rows x 128 bytes, whole cache lines -- straight into LDS of its own (D blocks
+// deep, no barrier: only the wave itself waits for its loads) and reads the operands from there.  Piece and swizzle as in linear_pipe_kernel.
+// 24 rows, the form above -> this, us: 8192 -> 2048 23.0 -> 15.4, 2048 -> 8192 13.4 -> 10.6, 4096 -> 14336 38.6 -> 25.7, 4096 -> 32000 69.6 -> 58; 64 rows 45.7 -> 22.2,
+// 17.8 -> 13.1, 56.3 -> 29.9, 90 -> 63.  (The form above with its blocks asked for one ahead of the other was slower: it does not wait for latency.)
+constexpr int STREAM_LDS_WAVES = 4;
+template <int ROWS, int TF, int WV, int D>
+__global__ __launch_bounds__(64 * WV, 2) void linear_stream_lds_kernel(LinArgs a, bool vec4) {
+  constexpr int RF = ROWS / 16, PER = 2 * (RF + TF), SLOT = PER * 1024;
+  static_assert((D - 1) * PER < 64, "what is in flight is counted");
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = blockIdx.y, n0 = blockIdx.x * ROWS;
+  int lo, hi;
+  lin_rows(a, g, lo, hi);
+  if (lo >= hi) return;
+  const int count = min(hi - lo, 16 * TF);
+  const int prow = lane >> 3, pchunk = (lane & 7) ^ prow;
+  const char* wbase = (const char*)((const uint16_t*)a.w + ((size_t)g * a.N + n0) * a.K);
+  const char* xbase = (const char*)((const uint16_t*)a.x + (size_t)(g % a.xgroups) * a.xg);
+  uint32_t off[PER];   // (the host checks that they fit); rows past N re-read the last one, rows past the group's the last of those: never stored
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    const int r = (p < 2 * RF ? p : p - 2 * RF) * 8 + prow;
+    off[p] = p < 2 * RF ? (uint32_t)min(r, a.N - 1 - n0) * (uint32_t)a.K * 2 + pchunk * 16
+                        : (uint32_t)(lin_xrow(a, lo + min(r, count - 1)) * a.ldx * 2) + pchunk * 16;
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds + wave * D * SLOT;
+  const unsigned char* mine = lds + wave * D * SLOT;
+  const int blocks = a.K / 64, steps = (blocks - wave + WV - 1) / WV;   // blocks wave, wave + WV, ..
+  auto fetch = [&](int i, int slot) {
+    const char* wk = wbase + (size_t)(wave + i * WV) * 128;
+    const char* xk = xbase + (size_t)(wave + i * WV) * 128;
+#pragma unroll
+    for (int p = 0; p < PER; ++p)
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds0 + slot * SLOT + p * 1024), "v"(off[p]), "s"(p < 2 * RF ? wk : xk) : "memory");
+  };
+  const f32x4_t z4 = {0.f, 0.f, 0.f, 0.f};
+  f32x4_t acc[RF][TF];
+#pragma unroll
+  for (int r = 0; r < RF; ++r)
+#pragma unroll
+    for (int t = 0; t < TF; ++t) acc[r][t] = z4;
+  const int f0 = (lane & 15) * 128 + (((lane >> 4) ^ (lane & 7)) * 16);
+  auto mul = [&](int slot) {
+    const unsigned char* b = mine + slot * SLOT;
+    u32x4_t w[2][RF], x[2][TF];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int r = 0; r < RF; ++r) w[h][r] = *reinterpret_cast<const u32x4_t*>(b + r * 2048 + (h ? f0 ^ 64 : f0));
+#pragma unroll
+      for (int t = 0; t < TF; ++t) x[h][t] = *reinterpret_cast<const u32x4_t*>(b + (RF + t) * 2048 + (h ? f0 ^ 64 : f0));
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < RF; ++r)
+#pragma unroll
+        for (int t = 0; t < TF; ++t) acc[r][t] = mfma_bf16(w[h][r], x[h][t], acc[r][t]);
+  };
+  if (steps >= D) {
+#pragma unroll
+    for (int i = 0; i < D; ++i) fetch(i, i);
+    int slot = 0;
+    for (int i = 0; i + D < steps; ++i) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * PER) : "memory");
+      mul(slot);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the slot has been read
+      fetch(i + D, slot);
+      slot = slot + 1 == D ? 0 : slot + 1;
+    }
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1 - j) * PER) : "memory");
+      mul(slot);
+      slot = slot + 1 == D ? 0 : slot + 1;
+    }
+  } else {
+    for (int i = 0; i < steps; ++i) fetch(i, i);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    for (int i = 0; i < steps; ++i) mul(i);
+  }
+  __syncthreads();   // every wave is done with the ring: the sums meet in its place
+  f32x4_t* red = reinterpret_cast<f32x4_t*>(lds);
+#pragma unroll
+  for (int r = 0; r < RF; ++r)
+#pragma unroll
+    for (int t = 0; t < TF; ++t) red[(wave * RF * TF + r * TF + t) * 64 + lane] = acc[r][t];
+  __syncthreads();
+  for (int e = tid; e < RF * TF * 64; e += 64 * WV) {   // 4 neighbouring columns of one row
+    const int f = e >> 6, l = e & 63, t = (f % TF) * 16 + (l & 15), n = n0 + (f / TF) * 16 + (l >> 4) * 4;
+    if (t >= count) continue;
+    f32x4_t v = red[f * 64 + l];
+#pragma unroll
+    for (int i = 1; i < WV; ++i) v += red[(i * RF * TF + f) * 64 + l];
+    lin_epilogue4(a, g, lo + t, n, v, lin_bias4(a, g, n, vec4), vec4);
+  }
+}
+template <int ROWS, int TF>
+int launch_stream_lds_tf(const LinArgs& a, int groups, hipStream_t s) {
+  // two workgroups per CU where two blocks per wave fit half of its LDS, else one
+  constexpr int WV = STREAM_LDS_WAVES, PER = 2 * (ROWS / 16 + TF), LDS_KB = ROWS < 64 && WV * 2 * PER <= 80 ? 80 : 160;
+  constexpr int BY_LDS = LDS_KB / (WV * PER), BY_COUNT = 63 / PER + 1, D = BY_LDS < BY_COUNT ? BY_LDS : BY_COUNT, LDS = WV * D * PER * 1024;
+  static_assert(D >= 2 && LDS >= WV * (ROWS / 16) * TF * 1024, "two blocks, and room for the sums");
+  auto kern = linear_stream_lds_kernel<ROWS, TF, WV, D>;
+  if (LDS > 64 * 1024)
+    DIHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS), DIHIP_RUNTIME_ERROR);
+  hipLaunchKernelGGL(kern, dim3((a.N + ROWS - 1) / ROWS, groups), dim3(64 * WV), LDS, s, a, lin_vec4(a));
+  return launch_status();
+}
+template <int ROWS>
+int launch_stream_lds(const LinArgs& a, int Tg, int groups, hipStream_t s) {
+  const int tf = (Tg + 15) / 16;
+  return tf <= 1 ? launch_stream_lds_tf<ROWS, 1>(a, groups, s) : tf == 2 ? launch_stream_lds_tf<ROWS, 2>(a, groups, s)
+         : tf == 3 ? launch_stream_lds_tf<ROWS, 3>(a, groups, s) : launch_stream_lds_tf<ROWS, 4>(a, groups, s);
+}
+// weight rows per workgroup: more of them bring the activations less often, but the workgroups have to fill 256 CUs.  16 / 32 / 64, us: 24 rows 4096 -> 4096
+// 11.1 / 13.6 / 17.1, 2048 -> 8192 11.4 / 10.6 / 13.0, 4096 -> 14336 30.5 / 29.3 / 25.7, 4096 -> 32000 61 / 58 / 58 (64 rows of x: 88 / 74 / 63); 2 rows, whose
+// activations are cheap, 9.1 / 9.8 / 11.0, 23.7 / 27.4 / 24.8 and 47 / 56 / 55.  Four waves in each form: an element's sum is the same in all of them.
+inline int launch_stream_lds_rows(const LinArgs& a, int Tg, int groups, hipStream_t s) {
+  const long n = (long)a.N * groups;
+  if (n < 6144 || Tg <= 8) return launch_stream_lds<16>(a, Tg, groups, s);
+  return n < 13312 ? launch_stream_lds<32>(a, Tg, groups, s) : launch_stream_lds<64>(a, Tg, groups, s);
 }
 
 template <int XT, int ROWS, int WV, bool PRE>
@@ -618,6 +744,9 @@ static int linear_impl(void* stream, const void* x, int x_dtype, long ldx, long 
       else hipLaunchKernelGGL((linear_skinny_kernel<DIHIP_BF16, false>), grid, dim3(256), (size_t)K * 2, s, a, 0, 1);
       return launch_status();
     }
+    if (Tg <= STREAM_MAX_ROWS && vec && x_dtype == DIHIP_BF16 && K % 64 == 0 && K >= 1024 && !row_map && (size_t)64 * K * 2 < (1ull << 31) &&
+        (size_t)T * ldx * 2 < (1ull << 31))   // (32-bit offsets; a row map's targets are not known here)
+      return launch_stream_lds_rows(a, Tg, groups, s);
     if (Tg <= STREAM_MAX_ROWS && vec) {
       if (x_dtype == DIHIP_F32) launch_stream_rows<DIHIP_F32>(a, Tg, groups, s);
       else launch_stream_rows<DIHIP_BF16>(a, Tg, groups, s);

@@ -74,6 +74,32 @@ def test_linear_streams_few_rows(so, T, N, K, groups, xdt):
     assert float(out[:, :3].abs().max()) == 0 and float(out[:, -4:].abs().max()) == 0
 
 
+@pytest.mark.parametrize("T,N,K,groups", [(2, 15, 1024, 1), (16, 17, 1088, 1), (17, 2050, 1024, 3), (33, 100, 4160, 1), (64, 2049, 1152, 1), (9, 6150, 1024, 1), (31, 6145, 2048, 1),
+                                          (48, 6200, 1216, 1), (64, 12300, 1024, 1), (12, 13313, 1024, 1), (30, 4440, 1024, 3), (40, 13330, 1088, 1), (57, 14336, 2112, 1)])
+def test_linear_streams_through_lds(so, T, N, K, groups):
+    """Every form (16 / 32 / 64 weight rows, one to four 16-row operands): waves with fewer blocks than the ring holds, more, and one more than others; edges of
+    rows and columns; strided rows, every part of the epilogue.  Products of the same operands in 64 bits; a row's bits do not depend on the rows beside it."""
+    rng = np.random.default_rng(T * 100 + N + K)
+    wide = dev(rng.normal(0, 1, (64, groups * K + 16)), torch.bfloat16)
+    rows = wide[:, 8:8 + groups * K]
+    x = rows[:T]
+    w, b = dev(rng.normal(0, K ** -0.5, (groups, N, K)), torch.bfloat16), dev(rng.normal(0, 0.3, (groups, N)), torch.bfloat16)
+    mul = dev(rng.normal(0, 1, (T, groups * N)))
+    lo, hi = N // 3, groups * N - 2
+    want = torch.cat([x[:, g * K:(g + 1) * K].double() @ w[g].double().t() + b[g].double() for g in range(groups)], 1)
+    plain = want.clone()
+    want[:, lo:hi] = torch.nn.functional.gelu(want[:, lo:hi], approximate="tanh")
+    wt, bt = (w[0], b[0]) if groups == 1 else (w, b)
+    y = so.linear(x, wt, bt, act="gelu_tanh", act_cols=(lo, hi), mul=mul, math=so.MATH_BF16, groups=groups)
+    assert rel_err(y.cpu().numpy(), (want * mul.double()).cpu().numpy()) < 2e-5
+    out = torch.zeros(T, groups * N + 7, dtype=torch.bfloat16, device="cuda")
+    so.linear(x, wt, bt, math=so.MATH_BF16, groups=groups, out=out[:, 3:3 + groups * N])
+    assert rel_err(out[:, 3:3 + groups * N].float().cpu().numpy(), plain.cpu().numpy()) < 2.0 ** -8      # one rounding of the result
+    assert float(out[:, :3].abs().max()) == 0 and float(out[:, -4:].abs().max()) == 0
+    few, many = so.linear(rows[:2], wt, bt, math=so.MATH_BF16, groups=groups), so.linear(rows, wt, bt, math=so.MATH_BF16, groups=groups)
+    assert torch.equal(few, many[:2])
+
+
 @pytest.mark.parametrize("N,K", [(1, 2056), (511, 2048 + 512), (513, 4096), (1030, 4104), (300, 6144), (600, 8192), (514, 10248), (33, 12000), (700, 14336), (40, 16384),
                                  (5900, 1024), (4100, 2048), (64, 16392)])
 @pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float32])
