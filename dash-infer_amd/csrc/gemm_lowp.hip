@@ -1157,7 +1157,15 @@ size_t dihip_gemm_lowp_sync_bytes(void) { return GEMM_SYNC_BYTES; }
 // K parts per tail tile the context-phase GEMM of this shape is launched with on this GPU (1: no tail split; diagnostics / tests)
 int dihip_gemm_prefill_tail_parts(int wbits, int M, int N, int K, int group_size, int dual) {
   if (M < 64 || N <= 0 || K <= 0) return 1;
-  return prefill_tail_plan(wbits, M, N, K, group_size, dual != 0).ksplit;
+  const PrefillTail t = prefill_tail_plan(wbits, M, N, K, group_size, dual != 0);
+  return t.tail_cb > 0 ? t.ksplit : 1;
+}
+
+// ... and per tile where the whole grid is split (1: it is not)
+int dihip_gemm_prefill_grid_parts(int wbits, int M, int N, int K, int group_size, int dual) {
+  if (M < 64 || N <= 0 || K <= 0) return 1;
+  const PrefillTail t = prefill_tail_plan(wbits, M, N, K, group_size, dual != 0);
+  return t.tail_cb > 0 ? 1 : t.ksplit;
 }
 
 size_t dihip_gemm_lowp_workspace_bytes(int wbits, int M, int N, int K, int group_size) {

@@ -710,7 +710,7 @@ def test_prefill_gemm_whole_grid_split(ops, wbits, G, M, N, K):
     xd = to_dev(x, "bf16")
     need = ops.lowp_workspace_bytes(wbits, M, N, K, G)
     sc = ops.Scratch(need)
-    parts = int(lib().dihip_gemm_prefill_tail_parts(wbits, M, N, K, G, 0))
+    parts = int(lib().dihip_gemm_prefill_grid_parts(wbits, M, N, K, G, 0))
     assert parts > 1 and K // parts >= 512
     bias = bf16_round(rng.normal(0, 0.3, N).astype(np.float32))
     y = ops.gemm_lowp(xd, pw, bias=to_dev(bias, "bf16"), act="silu", alpha=0.5, scratch=sc)
