@@ -689,19 +689,20 @@ class DecodeSession:
         n, g, H, dev = self.n_loc, self.g_loc, self.H, self.h.device
         lens = [len(s) for s in seqs]
         assert all(0 < L <= self.max_len for L in lens)
-        # the products take the rows of several prompts together (the weights are read once), up to PREFILL_ROWS of them
+        # the products take the rows of several prompts together (the weights are read once), up to PREFILL_ROWS of them, where each alone
+        # has the rows of the context-phase GEMM; shorter ones run alone, bit for bit the runner's requests one after the other
         groups = []
         for b, L in enumerate(lens):
-            if groups and sum(lens[i] for i in groups[-1]) + L <= self.PREFILL_ROWS:
+            if L >= 64 and groups and lens[groups[-1][0]] >= 64 and sum(lens[i] for i in groups[-1]) + L <= self.PREFILL_ROWS:
                 groups[-1].append(b)
             else:
                 groups.append([b])
         l0, wb, gsz = m.layers[0], m.quant.wbits, m.quant.group
         # per row count: fewer rows can take a split-K plan with a larger slab than more of them
         need = max(ops.lowp_workspace_bytes(wb, T, p.N, p.K, gsz) for T in {sum(lens[b] for b in grp) for grp in groups} for p in (l0.qkv, l0.o, l0.gate, l0.down))
-        need = max(need, int(lib().dihip_dense_workspace_bytes(self.B, m.lm_head.N, m.lm_head.K)))
+        need = max([need] + [int(lib().dihip_dense_workspace_bytes(len(grp), m.lm_head.N, m.lm_head.K)) for grp in groups])
         sc = ops.Scratch(need, dev)
-        last = torch.empty(self.B, cfg.hidden, dtype=torch.float32, device=dev)
+        logits = torch.empty(self.B, m.vocab_local, dtype=torch.float32, device=dev) if return_logits else None
         for grp in groups:
             T, cut = sum(lens[b] for b in grp), [0]
             for b in grp:
@@ -727,9 +728,9 @@ class DecodeSession:
                     continue
                 act = ops.fused_norm_swiglu(h, lw.ln2, cfg.eps, lw.gate, lw.up, sc)
                 h = ops.fused_gemm_addto(act, lw.down, h, sc, M=T)
-            for b, hi in zip(grp, cut[1:]):
-                last[b].copy_(h[hi - 1])
-        logits = ops.lm_head(last, m.final_norm, cfg.eps, m.lm_head, sc) if return_logits else None
+            if return_logits:
+                last = h[-1:] if len(grp) == 1 else torch.stack([h[hi - 1] for hi in cut[1:]])
+                ops.lm_head(last, m.final_norm, cfg.eps, m.lm_head, sc, out=logits[grp[0]:grp[-1] + 1])
         if return_logits:
             nxt = torch.argmax(logits, dim=-1).cpu()
             self.set_state(nxt, lens)
