@@ -433,3 +433,32 @@ def test_f16_greedy_decode_matches_oracle(pkg, shape, wbits, group, kv_mode, bat
             lo = ref.step(gpu_ids[t])
     assert decided >= (steps + 1) * batch // 2
     print(f"f16 int{wbits} kv {kv_mode} batch {batch}: worst logit error {worst:.2e}; {decided}/{(steps + 1) * batch} decisive greedy choices")
+
+
+@pytest.mark.parametrize("lens", [[70, 64, 3, 130, 200], [63, 90, 64]])
+@pytest.mark.parametrize("wbits,group,kv_mode", [(4, 128, "none"), (8, -1, "u4")])
+def test_prompts_that_share_products_equal_prompts_alone(pkg, wbits, group, kv_mode, lens):
+    """Prompts of 64 rows and more share the products (f32 sums in another order: logits within the tolerance of this file, at the same tokens wherever the margin
+    exceeds it); one below runs alone, to the bit."""
+    from dash_infer_amd import decoder
+    cfg = decoder.ModelConfig("prompts-test", **SMALL)
+    model = decoder.build_random_model(cfg, decoder.QuantSpec(wbits, group), seed=77, keep_fp=True)
+    rng = np.random.default_rng(len(lens))
+    prompts = [[int(t) for t in rng.integers(0, cfg.vocab, n)] for n in lens]
+    both = decoder.DecodeSession(model, len(lens), max_len=256, span_len=16, kv_mode=kv_mode)
+    got, ids = both.prefill(prompts).clone(), both.ids.cpu().tolist()
+    both.step()
+    torch.cuda.synchronize()
+    for b, p in enumerate(prompts):
+        one = decoder.DecodeSession(model, 1, max_len=256, span_len=16, kv_mode=kv_mode)
+        want = one.prefill([p])[0].clone()
+        if len(p) < 64:
+            assert torch.equal(got[b], want)
+        tol = LOGIT_TOL[kv_mode] * max(1.0, float(want.abs().max()))
+        assert float((got[b] - want).abs().max()) <= tol
+        top = torch.topk(want, 2).values
+        if float(top[0] - top[1]) > 2 * tol:
+            assert ids[b] == int(want.argmax())
+            one.step()                             # reads what the prompt left in the spans
+            torch.cuda.synchronize()
+            assert float((both.logits[b] - one.logits[0]).abs().max()) <= 2 * tol
