@@ -12,6 +12,7 @@ struct LinArgs {
   int T, N, K, act, act_lo, act_hi, ydt, round_ops;
   int mul_group; float act_param;               // mul holds one number per group; the parameter of an activation that has one
   const int32_t* seg; const int32_t* row_map;   // segmented form: group g owns the output rows seg[g] .. seg[g + 1], row r reads x row row_map[r]
+  const void* w2;                               // gated form: y = act(x . w^T) * (x . w2^T); w2 is shaped as w.  No groups, bias or mul
 };
 
 // the rows of group g: [lo, hi)
@@ -67,6 +68,24 @@ __device__ __forceinline__ void lin_epilogue4(const LinArgs& a, int g, int t, in
                                                                   f32_to_bf16_bits(v[2]) | (f32_to_bf16_bits(v[3]) << 16)};
 }
 
+// the gated form's: g and u are the sums of columns n .. n + 3 with w and with w2
+__device__ __forceinline__ void lin_gated4(const LinArgs& a, int t, int n, f32x4_t g, const f32x4_t& u, bool vec4) {
+  if (n >= a.N) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) g[r] = apply_act(g[r], a.act) * u[r];
+  const size_t o = (size_t)t * a.ldy + n;
+  if (!vec4) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (n + r < a.N) st_any(a.y, o + r, a.ydt, g[r]);
+  } else if (a.ydt == DIHIP_F32) {
+    *reinterpret_cast<f32x4_t*>((float*)a.y + o) = g;
+  } else {
+    *reinterpret_cast<u32x2_t*>((uint16_t*)a.y + o) = u32x2_t{f32_to_bf16_bits(g[0]) | (f32_to_bf16_bits(g[1]) << 16),
+                                                              f32_to_bf16_bits(g[2]) | (f32_to_bf16_bits(g[3]) << 16)};
+  }
+}
+
 __device__ __forceinline__ f32x4_t mfma_bf16(const u32x4_t& a, const u32x4_t& b, const f32x4_t& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
@@ -79,7 +98,7 @@ struct LinTilePlan {
   int parts;
   size_t slab;
 };
-LinTilePlan plan_linear_tile(int Tg, int N, int K, int groups, long ldx, bool split);
+LinTilePlan plan_linear_tile(int Tg, int N, int K, int groups, long ldx, bool split);   // (gated form: N is the columns of both matrices)
 int launch_linear_tile(const LinArgs& a, const LinTilePlan& p, int Tg, int groups, float* slab, hipStream_t s);
 
 }  // namespace dihip

@@ -10,6 +10,7 @@
 //   linear_skinny_kernel one short row, one row per group, a few rows where that is faster (skinny_rows) or the products are f32: a streamed weight, one wave
 //                        per 2 weight rows, 4 rows at a time
 //   linear_fewcols_kernel a router's logits
+// dihip_linear_gated (act(x . w^T) * (x . w2^T)) runs in forms of linear_pipe, linear_stream_lds and linear_row_kernel that walk both matrices in one launch.
 // f32 products: an output element is one chain over k, ascending, whatever T is.  bf16 products: the order of its f32 sum follows the kernel, which T chooses (one
 // row; 2 .. 64; more), and in linear_pipe_kernel the number of K parts, which T chooses too: results of other row counts are equal within f32 rounding,
 // not to the bit.  Within 2 .. 64 rows of one kernel, and above 64 where K is in one part (segments: always), T does not matter.
@@ -285,19 +286,21 @@ __global__ __launch_bounds__(64 * WV, (ROWS * TF > 64 || XT == DIHIP_F32) ? 2 : 
 // than the bound that TF was chosen for (copies of its last row would be half of what is brought).  Gathered [gate | up] products of 64 experts, 6 per token, 2048 -> 2816, the form
 // above -> this: 2 / 8 / 17 / 64 tokens 32.4 / 87 / 164 / 193 -> 26.2 / 79 / 114 / 139.
 constexpr int STREAM_LDS_WAVES = 4;
-template <int ROWS, int TF, int WV, int D, bool SEG>
+// GATED (linear_gated): the first half of the workgroup's weight rows are w's, the second the same ones of w2.
+template <int ROWS, int TF, int WV, int D, bool SEG, bool GATED>
 __global__ __launch_bounds__(64 * WV, 2) void linear_stream_lds_kernel(LinArgs a, bool vec4) {
-  constexpr int RF = ROWS / 16, PER = 2 * (RF + TF), SLOT = PER * 1024;
+  constexpr int RF = ROWS / 16, PER = 2 * (RF + TF), SLOT = PER * 1024, COLS = GATED ? ROWS / 2 : ROWS;   // (of y)
   static_assert((D - 1) * PER < 64, "what is in flight is counted");
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = blockIdx.y, n0 = blockIdx.x * ROWS;
+  const int g = blockIdx.y, n0 = blockIdx.x * COLS;
   int lo, hi;
   lin_rows(a, g, lo, hi);
   if (lo >= hi) return;
   const int count = min(hi - lo, 16 * TF);
   const int prow = lane >> 3, pchunk = (lane & 7) ^ prow;
   const char* wbase = (const char*)((const uint16_t*)a.w + ((size_t)g * a.N + n0) * a.K);
+  const char* w2base = GATED ? (const char*)((const uint16_t*)a.w2 + (size_t)n0 * a.K) : nullptr;
   const char* xbase = (const char*)((const uint16_t*)a.x + (size_t)(g % a.xgroups) * a.xg);
   uint32_t off[PER];   // (the host checks that they fit); rows past N re-read the last one, rows past the group's the last of those: never stored
   const char* xaddr[2 * TF];   // (SEG: of the next block)
@@ -305,7 +308,7 @@ __global__ __launch_bounds__(64 * WV, 2) void linear_stream_lds_kernel(LinArgs a
   for (int p = 0; p < PER; ++p) {
     const int r = (p < 2 * RF ? p : p - 2 * RF) * 8 + prow;
     if (p < 2 * RF) {
-      off[p] = (uint32_t)min(r, a.N - 1 - n0) * (uint32_t)a.K * 2 + pchunk * 16;
+      off[p] = (uint32_t)min(r % COLS, a.N - 1 - n0) * (uint32_t)a.K * 2 + pchunk * 16;
     } else {
       const size_t from = lin_xrow(a, lo + min(r, count - 1)) * a.ldx * 2 + pchunk * 16;
       if constexpr (SEG) xaddr[p - 2 * RF] = xbase + from + wave * 128;
@@ -326,6 +329,7 @@ __global__ __launch_bounds__(64 * WV, 2) void linear_stream_lds_kernel(LinArgs a
     constexpr int TN = decltype(used)::value, USED = 2 * (RF + TN);
     auto fetch = [&](int i, int slot) {   // (called for i = 0, 1, 2, ..)
       const char* wk = wbase + (size_t)(wave + i * WV) * 128;
+      const char* w2k = GATED ? w2base + (size_t)(wave + i * WV) * 128 : wk;
       const char* xk = xbase + (size_t)(wave + i * WV) * 128;
 #pragma unroll
       for (int p = 0; p < USED; ++p) {
@@ -336,7 +340,7 @@ __global__ __launch_bounds__(64 * WV, 2) void linear_stream_lds_kernel(LinArgs a
           xaddr[p - 2 * RF] += WV * 128;
         } else {
           const uint32_t o = off[p];
-          asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(o), "s"(p < 2 * RF ? wk : xk) : "memory");
+          asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(o), "s"(p < (GATED ? RF : 2 * RF) ? wk : p < 2 * RF ? w2k : xk) : "memory");
         }
       }
     };
@@ -390,32 +394,41 @@ __global__ __launch_bounds__(64 * WV, 2) void linear_stream_lds_kernel(LinArgs a
 #pragma unroll
     for (int t = 0; t < TF; ++t) red[(wave * RF * TF + r * TF + t) * 64 + lane] = acc[r][t];
   __syncthreads();
-  for (int e = tid; e < RF * TF * 64; e += 64 * WV) {   // 4 neighbouring columns of one row
-    const int f = e >> 6, l = e & 63, t = (f % TF) * 16 + (l & 15), n = n0 + (f / TF) * 16 + (l >> 4) * 4;
+  for (int e = tid; e < (GATED ? RF * TF * 32 : RF * TF * 64); e += 64 * WV) {   // 4 neighbouring columns of one row
+    int f = e >> 6, l = e & 63, f2 = 0, l2 = 0;
+    if constexpr (GATED) {   // ROWS 16: both halves in one operand, 32 lanes apart
+      if constexpr (RF == 1) { f = e >> 5; l = e & 31; f2 = f; l2 = l + 32; }
+      else { f2 = f + RF / 2 * TF; l2 = l; }
+    }
+    const int t = (f % TF) * 16 + (l & 15), n = n0 + (f / TF) * 16 + (l >> 4) * 4;
     if (t >= count) continue;
-    f32x4_t v = red[f * 64 + l];
+    auto sum = [&](int ff, int ll) {
+      f32x4_t v = red[ff * 64 + ll];
 #pragma unroll
-    for (int i = 1; i < WV; ++i) v += red[(i * RF * TF + f) * 64 + l];
-    lin_epilogue4(a, g, lo + t, n, v, lin_bias4(a, g, n, vec4), vec4);
+      for (int i = 1; i < WV; ++i) v += red[(i * RF * TF + ff) * 64 + ll];
+      return v;
+    };
+    if constexpr (GATED) lin_gated4(a, lo + t, n, sum(f, l), sum(f2, l2), vec4);
+    else lin_epilogue4(a, g, lo + t, n, sum(f, l), lin_bias4(a, g, n, vec4), vec4);
   }
 }
-template <int ROWS, int TF, bool SEG>
+template <int ROWS, int TF, bool SEG, bool GATED>
 int launch_stream_lds_tf(const LinArgs& a, int groups, hipStream_t s) {
   // two workgroups per CU where two blocks per wave fit half of its LDS, else one
   constexpr int WV = STREAM_LDS_WAVES, PER = 2 * (ROWS / 16 + TF), LDS_KB = ROWS < 64 && WV * 2 * PER <= 80 ? 80 : 160;
   constexpr int BY_LDS = LDS_KB / (WV * PER), BY_COUNT = 63 / PER + 1, D = BY_LDS < BY_COUNT ? BY_LDS : BY_COUNT, LDS = WV * D * PER * 1024;
   static_assert(D >= 2 && LDS >= WV * (ROWS / 16) * TF * 1024, "two blocks, and room for the sums");
-  auto kern = linear_stream_lds_kernel<ROWS, TF, WV, D, SEG>;
+  auto kern = linear_stream_lds_kernel<ROWS, TF, WV, D, SEG, GATED>;
   if (LDS > 64 * 1024)
     DIHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS), DIHIP_RUNTIME_ERROR);
-  hipLaunchKernelGGL(kern, dim3((a.N + ROWS - 1) / ROWS, groups), dim3(64 * WV), LDS, s, a, lin_vec4(a));
+  hipLaunchKernelGGL(kern, dim3(GATED ? (a.N + ROWS / 2 - 1) / (ROWS / 2) : (a.N + ROWS - 1) / ROWS, groups), dim3(64 * WV), LDS, s, a, lin_vec4(a));
   return launch_status();
 }
-template <int ROWS, bool SEG>
+template <int ROWS, bool SEG, bool GATED = false>
 int launch_stream_lds(const LinArgs& a, int Tg, int groups, hipStream_t s) {
   const int tf = (Tg + 15) / 16;
-  return tf <= 1 ? launch_stream_lds_tf<ROWS, 1, SEG>(a, groups, s) : tf == 2 ? launch_stream_lds_tf<ROWS, 2, SEG>(a, groups, s)
-         : tf == 3 ? launch_stream_lds_tf<ROWS, 3, SEG>(a, groups, s) : launch_stream_lds_tf<ROWS, 4, SEG>(a, groups, s);
+  return tf <= 1 ? launch_stream_lds_tf<ROWS, 1, SEG, GATED>(a, groups, s) : tf == 2 ? launch_stream_lds_tf<ROWS, 2, SEG, GATED>(a, groups, s)
+         : tf == 3 ? launch_stream_lds_tf<ROWS, 3, SEG, GATED>(a, groups, s) : launch_stream_lds_tf<ROWS, 4, SEG, GATED>(a, groups, s);
 }
 // weight rows per workgroup: more of them bring the activations less often, but the workgroups have to fill 256 CUs.  16 / 32 / 64, us: 24 rows 4096 -> 4096
 // 11.1 / 13.6 / 17.1, 2048 -> 8192 11.4 / 10.6 / 13.0, 4096 -> 14336 30.5 / 29.3 / 25.7, 4096 -> 32000 61 / 58 / 58 (64 rows of x: 88 / 74 / 63); 2 rows, whose
@@ -428,6 +441,14 @@ inline int launch_stream_lds_rows(const LinArgs& a, int Tg, int groups, hipStrea
   if (a.seg) return a.K < 4096 && Tg <= 48 ? launch_stream_lds<32, true>(a, Tg, groups, s) : launch_stream_lds<16, true>(a, Tg, groups, s);
   if (n < 6144 || Tg <= 8) return launch_stream_lds<16, false>(a, Tg, groups, s);
   return n < 13312 ? launch_stream_lds<32, false>(a, Tg, groups, s) : launch_stream_lds<64, false>(a, Tg, groups, s);
+}
+
+// The gated form has twice the weight rows of one product, so its lines lie elsewhere.  Two products / 16 / 32 / 64, us (weights from memory): 2048 -> 1408 24 rows 10.7 / 5.7 /
+// 6.5 / 7.8; 1024 -> 3072 24 rows 9.3 / 6.3 / 5.7 / 6.3; 2048 -> 8192 13 rows 21.0 / 16.2 / 15.0 / 17.0, 24 rows 21.4 / 18.3 / 15.5 / 17.4, 64 rows 26.6 / 25.9 / 21.4 / 19.2; 4096 -> 6144
+// 8 rows 27.8 / 20.6 / 23.3 / 23.9; 4096 -> 14336 13 rows 49.8 / 44.1 / 46.1 / 48.0, 24 rows 52.2 / 52.4 / 48.7 / 49.1, 64 rows 61.3 / 75.9 / 65.4 / 56.3.
+inline int launch_stream_lds_gated(const LinArgs& a, hipStream_t s) {
+  if (a.N < 3072 || (a.T <= 16 && a.K >= 4096)) return launch_stream_lds<16, false, true>(a, a.T, 1, s);
+  return a.T <= 48 || a.N < 4096 ? launch_stream_lds<32, false, true>(a, a.T, 1, s) : launch_stream_lds<64, false, true>(a, a.T, 1, s);
 }
 
 template <int XT, int ROWS, int WV, bool PRE>
@@ -472,21 +493,24 @@ __device__ __forceinline__ float dot8_bf16(const u32x4_t& w, const u32x4_t& x, f
 // 4096 -> 32000 52.7 -> 44.5 (5.9 TB/s).
 // MASK: K does not fill the pieces: the loads stay inside the row, and both x and the weights are zero past K (either may hold an infinity where it is re-read).
 constexpr int ROW_WAVES = 4, ROW_WGS = 512, ROW_MAXC = 8, ROW_MAX_ROWS = 1024;   // weight rows of a workgroup: 16 KB of sums
-template <int XT, int C, bool MASK>
+// GATED: the rows of w that a workgroup owns, then the same ones of w2.  4096 -> 14336 twice 39.9 -> 35.1 us.
+template <int XT, int C, bool MASK, bool GATED>
 __global__ __launch_bounds__(64 * ROW_WAVES, 2) void linear_row_kernel(LinArgs a) {
   constexpr int R = C >= 5 ? 1 : 8 / C;        // weight rows per batch
   extern __shared__ __attribute__((aligned(16))) float part[];   // [row][wave]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lo = (int)((long)a.N * blockIdx.x / gridDim.x), hi = (int)((long)a.N * (blockIdx.x + 1) / gridDim.x);
   const uint16_t* w = (const uint16_t*)a.w + (size_t)lo * a.K;
+  const uint16_t* w2 = GATED ? (const uint16_t*)a.w2 + (size_t)lo * a.K : nullptr;
   int k[C];
 #pragma unroll
   for (int c = 0; c < C; ++c) k[c] = ((wave * C + c) * 64 + lane) * 8;
-  const int rows = hi - lo;
+  const int own = hi - lo, rows = GATED ? 2 * own : own;
   auto load = [&](u32x4_t (&d)[R][C], int r0) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const uint16_t* row = w + (size_t)min(r0 + r, rows - 1) * a.K;   // (uniform) past the end: the last row once more
+      const int i = min(r0 + r, rows - 1);   // (uniform) past the end: the last row once more
+      const uint16_t* row = GATED && i >= own ? w2 + (size_t)(i - own) * a.K : w + (size_t)i * a.K;
 #pragma unroll
       for (int c = 0; c < C; ++c) d[r][c] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(row + (MASK ? min(k[c], a.K - 8) : k[c])));
     }
@@ -548,17 +572,23 @@ __global__ __launch_bounds__(64 * ROW_WAVES, 2) void linear_row_kernel(LinArgs a
     __builtin_amdgcn_sched_barrier(0);
   }
   __syncthreads();
-  for (int r = tid; r < rows; r += 64 * ROW_WAVES) {
+  for (int r = tid; r < own; r += 64 * ROW_WAVES) {
     const f32x4_t p = *reinterpret_cast<const f32x4_t*>(part + r * ROW_WAVES);
-    lin_epilogue(a, 0, 0, lo + r, (p[0] + p[1]) + (p[2] + p[3]), DIHIP_BF16);
+    const float v = (p[0] + p[1]) + (p[2] + p[3]);
+    if constexpr (GATED) {
+      const f32x4_t u = *reinterpret_cast<const f32x4_t*>(part + (own + r) * ROW_WAVES);
+      st_any(a.y, (size_t)(lo + r), a.ydt, apply_act(v, a.act) * ((u[0] + u[1]) + (u[2] + u[3])));
+    } else {
+      lin_epilogue(a, 0, 0, lo + r, v, DIHIP_BF16);
+    }
   }
 }
-template <int XT, int C>
+template <int XT, int C, bool GATED>
 void launch_row_c(const LinArgs& a, hipStream_t s) {
   const int wgs = a.N < ROW_WGS ? a.N : ROW_WGS;
-  const size_t lds = (size_t)((a.N + wgs - 1) / wgs) * ROW_WAVES * sizeof(float);
-  if (a.K == C * 512 * ROW_WAVES) hipLaunchKernelGGL((linear_row_kernel<XT, C, false>), dim3(wgs), dim3(64 * ROW_WAVES), lds, s, a);
-  else hipLaunchKernelGGL((linear_row_kernel<XT, C, true>), dim3(wgs), dim3(64 * ROW_WAVES), lds, s, a);
+  const size_t lds = (size_t)((a.N + wgs - 1) / wgs) * ROW_WAVES * sizeof(float) * (GATED ? 2 : 1);
+  if (a.K == C * 512 * ROW_WAVES) hipLaunchKernelGGL((linear_row_kernel<XT, C, false, GATED>), dim3(wgs), dim3(64 * ROW_WAVES), lds, s, a);
+  else hipLaunchKernelGGL((linear_row_kernel<XT, C, true, GATED>), dim3(wgs), dim3(64 * ROW_WAVES), lds, s, a);
 }
 inline int row_pieces(int K) { return (K + 512 * ROW_WAVES - 1) / (512 * ROW_WAVES); }
 // where it is the faster one: long rows always, rows of 1024 .. 2048 from 12 MB of weights on.  linear_skinny_kernel / this, us: 64 x 4096 5.4 / 3.6,
@@ -567,17 +597,17 @@ inline int row_pieces(int K) { return (K + 512 * ROW_WAVES - 1) / (512 * ROW_WAV
 inline bool row_kernel(int N, int K) {
   return row_pieces(K) <= ROW_MAXC && (N + ROW_WGS - 1) / ROW_WGS <= ROW_MAX_ROWS && (K > 2048 || (K >= 1024 && (long)N * K >= 6000000));
 }
-template <int XT>
+template <int XT, bool GATED = false>
 void launch_row(const LinArgs& a, hipStream_t s) {
   switch (row_pieces(a.K)) {
-    case 1: return launch_row_c<XT, 1>(a, s);
-    case 2: return launch_row_c<XT, 2>(a, s);
-    case 3: return launch_row_c<XT, 3>(a, s);
-    case 4: return launch_row_c<XT, 4>(a, s);
-    case 5: return launch_row_c<XT, 5>(a, s);
-    case 6: return launch_row_c<XT, 6>(a, s);
-    case 7: return launch_row_c<XT, 7>(a, s);
-    default: return launch_row_c<XT, 8>(a, s);
+    case 1: return launch_row_c<XT, 1, GATED>(a, s);
+    case 2: return launch_row_c<XT, 2, GATED>(a, s);
+    case 3: return launch_row_c<XT, 3, GATED>(a, s);
+    case 4: return launch_row_c<XT, 4, GATED>(a, s);
+    case 5: return launch_row_c<XT, 5, GATED>(a, s);
+    case 6: return launch_row_c<XT, 6, GATED>(a, s);
+    case 7: return launch_row_c<XT, 7, GATED>(a, s);
+    default: return launch_row_c<XT, 8, GATED>(a, s);
   }
 }
 
@@ -853,6 +883,43 @@ extern "C" int dihip_linear(void* stream, const void* x, int x_dtype, long ldx, 
                             float act_param, int math) {
   return linear_impl(stream, x, x_dtype, ldx, x_gstride, x_groups, w, w_dtype, bias, y, y_dtype, ldy, y_gstride, mul, ldm, mul_group, T, N, K, groups,
                      act, act_lo, act_hi, act_param, math, nullptr, nullptr, 0, nullptr, 0);
+}
+
+// Where the gated form runs as one launch: where each of its two products would take a kernel that has one
+static bool gated_as_one(int T, int N, int K, long ldx) {
+  static const bool no_skinny = env_off("DIHIP_LINEAR_SKINNY");
+  if (T < 1 || N < 1 || K < 1 || K % 8 != 0 || ldx < K || ldx % 8 != 0) return false;
+  if (T == 1) return !no_skinny && row_kernel(2 * N, K);
+  if (T <= STREAM_MAX_ROWS) return K % 64 == 0 && K >= 1024 && (size_t)64 * K * 2 < (1ull << 31) && (size_t)T * ldx * 2 < (1ull << 31);
+  return plan_linear_tile(T, 2 * N, K, 1, ldx, false).ok;
+}
+
+extern "C" int dihip_linear_gated_query(int T, int N, int K, long ldx, size_t* ws_bytes) {
+  if (N > INT32_MAX / 2 || !gated_as_one(T, N, K, ldx)) return 0;
+  *ws_bytes = T > STREAM_MAX_ROWS ? plan_linear_tile(T, 2 * N, K, 1, ldx, true).slab : 0;
+  return 1;
+}
+
+extern "C" int dihip_linear_gated(void* stream, const void* x, long ldx, const void* w_gate, const void* w_up, void* y, int y_dtype, long ldy, int T, int N, int K,
+                                  int act, void* ws, size_t ws_bytes) {
+  DIHIP_REQUIRE(T >= 0 && N > 0 && N <= INT32_MAX / 2 && K > 0, DIHIP_PARAM_ERROR, "linear_gated: bad shape T %d N %d K %d", T, N, K);
+  DIHIP_REQUIRE(x && w_gate && w_up && y && seq_dtype_ok(y_dtype) && ldy >= N && ldx >= K, DIHIP_PARAM_ERROR, "linear_gated: bad argument");
+  DIHIP_REQUIRE(act >= 0 && act != DIHIP_SEQ_ACT_SOFTCAP, DIHIP_PARAM_ERROR, "linear_gated: no activation with a parameter");
+  if (T == 0) return DIHIP_SUCCESS;
+  DIHIP_REQUIRE(aligned16(x) && aligned16(w_gate) && aligned16(w_up) && (!ws || aligned16(ws)) && gated_as_one(T, N, K, ldx), DIHIP_EXCEED_LIMIT_ERROR,
+                "linear_gated: T %d N %d K %d does not run as one launch", T, N, K);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  LinArgs a{};
+  a.x = x; a.ldx = ldx; a.xgroups = 1; a.w = w_gate; a.w2 = w_up; a.y = y; a.ydt = y_dtype; a.ldy = ldy;
+  a.T = T; a.N = N; a.K = K; a.act = act; a.act_hi = N;
+  if (T == 1) {
+    launch_row<DIHIP_BF16, true>(a, s);
+    return launch_status();
+  }
+  if (T <= STREAM_MAX_ROWS) return launch_stream_lds_gated(a, s);
+  LinTilePlan p = plan_linear_tile(T, 2 * N, K, 1, ldx, ws != nullptr);
+  if (p.slab > ws_bytes) p = plan_linear_tile(T, 2 * N, K, 1, ldx, false);
+  return launch_linear_tile(a, p, T, 1, (float*)ws, s);
 }
 
 extern "C" size_t dihip_linear_workspace_bytes(int T, int N, int K, int groups, long ldx) {

@@ -69,7 +69,10 @@ __device__ __forceinline__ bool seg_tile(const int32_t* __restrict__ seg, int gr
 
 // MF / NF: 16-row operands of a wave along the rows (x) and the output columns (weight rows); WM x WN waves
 // MAP: the rows of x are named by a map and may lie anywhere: 64-bit addresses per lane.  Else a tile's rows are neighbours: 32-bit offsets from its first
-template <int MF, int NF, int WM, int WN, bool MAP>
+// GATED: half of a tile's columns are w's, half the same ones of w2 -- of every wave, so that both sums of an element meet in its piece of LDS.  What two launches
+// cost beside the products: f32 sums out and in again, and the last round of tiles twice.  2048 rows 4096 -> 14336 twice 491 -> 444 us, 1500 rows 423 -> 334; 2048 -> 8192
+// twice, 513 rows 92.7 -> 58.2, 128 rows 44.8 -> 28.7.
+template <int MF, int NF, int WM, int WN, bool MAP, bool GATED>
 __global__ __launch_bounds__(64 * WM * WN, (WM * WN) / 4) void linear_pipe_kernel(LinArgs a, int mtiles, int ntiles, int groups, bool vec4, int parts, float* slab) {
   constexpr int WAVES = WM * WN, BM = 16 * MF * WM, BN = 16 * NF * WN;
   constexpr int PIECES = (BM + BN) / 8, PER = PIECES / WAVES;     // 1 KiB pieces (8 rows x 128 bytes) of a K step, per wave
@@ -88,7 +91,8 @@ __global__ __launch_bounds__(64 * WM * WN, (WM * WN) / 4) void linear_pipe_kerne
   }
   int t_lo, t_hi;
   lin_rows(a, g, t_lo, t_hi);
-  const int m0 = t_lo + mt * BM, n0 = nt * BN;
+  constexpr int HALVES = GATED ? 2 : 1, WCOLS = 16 * NF / HALVES;   // columns of y of a wave
+  const int m0 = t_lo + mt * BM, n0 = nt * (BN / HALVES);
   if (m0 >= t_hi) return;
   const size_t xoff = (size_t)(g % a.xgroups) * a.xg;
   // pieces: first the rows of x, then those of w; lane l of a piece brings row l / 8, 16 bytes (l % 8) ^ (row % 8) of its 128
@@ -96,6 +100,7 @@ __global__ __launch_bounds__(64 * WM * WN, (WM * WN) / 4) void linear_pipe_kerne
   const int all = a.K / LT_BK, part = blockIdx.z, k0 = (int)((long)all * part / parts), steps = (int)((long)all * (part + 1) / parts) - k0;
   const char* xbase = (const char*)((const uint16_t*)a.x + (MAP ? 0 : (size_t)m0 * a.ldx) + xoff + k0 * LT_BK);
   const char* wbase = (const char*)((const uint16_t*)a.w + ((size_t)g * a.N + n0) * a.K + k0 * LT_BK);
+  const char* w2base = GATED ? (const char*)((const uint16_t*)a.w2 + (size_t)n0 * a.K + k0 * LT_BK) : nullptr;
   const char* base[PER];
   uint32_t off[PER];   // (the host checks that 256 rows lie within 2 GB)
   const char* addr[PER];   // (MAP, instead of both)
@@ -103,8 +108,13 @@ __global__ __launch_bounds__(64 * WM * WN, (WM * WN) / 4) void linear_pipe_kerne
   for (int p = 0; p < PER; ++p) {
     const int piece = wave * PER + p;
     const bool isx = piece < BM / 8;   // (uniform)
+    int wrow = (piece - BM / 8) * 8;
     base[p] = isx ? xbase : wbase;
-    const int r = isx ? min(m0 + piece * 8 + prow, t_hi - 1) : min((piece - BM / 8) * 8 + prow, a.N - 1 - n0);
+    if constexpr (GATED) {
+      if (!isx && wrow % (2 * WCOLS) >= WCOLS) base[p] = w2base;
+      wrow = wrow / (2 * WCOLS) * WCOLS + wrow % WCOLS;
+    }
+    const int r = isx ? min(m0 + piece * 8 + prow, t_hi - 1) : min(wrow + prow, a.N - 1 - n0);
     const size_t row = isx ? (MAP ? a.row_map[r] : r - m0) : r, from = (row * (size_t)(isx ? a.ldx : (long)a.K) + pchunk * 8) * 2;
     if constexpr (MAP) addr[p] = base[p] + from;
     else off[p] = (uint32_t)from;
@@ -177,7 +187,7 @@ __global__ __launch_bounds__(64 * WM * WN, (WM * WN) / 4) void linear_pipe_kerne
   // 4 * NF lanes a whole run of them
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();                               // every wave has read its last operands, and no load is on its way into LDS
-  constexpr int EI = MF / 2, LDT = 16 * NF + 4, RPP = 64 / (4 * NF);
+  constexpr int EI = MF / 2, LDT = 16 * NF + 4, LPR = 4 * NF / HALVES, RPP = 64 / LPR;   // (lanes per row, rows per pass)
   float* tile_lds = reinterpret_cast<float*>(lds) + wave * (EI * 16 * LDT);
 #pragma unroll
   for (int i0 = 0; i0 < MF; i0 += EI) {
@@ -188,17 +198,28 @@ __global__ __launch_bounds__(64 * WM * WN, (WM * WN) / 4) void linear_pipe_kerne
       for (int j = 0; j < NF; ++j)
         *reinterpret_cast<f32x4_t*>(tile_lds + (i * 16 + (lane & 15)) * LDT + j * 16 + (lane >> 4) * 4) = acc[j][i0 + i];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    const int n = n0 + wn * NF * 16 + (lane % (4 * NF)) * 4;
-    const f32x4_t b = lin_bias4(a, g, n, vec4);
+    const int n = n0 + wn * WCOLS + (lane % LPR) * 4;
+    f32x4_t b;
+    if constexpr (!GATED) b = lin_bias4(a, g, n, vec4);
 #pragma unroll 1
     for (int r0 = 0; r0 < EI * 16; r0 += RPP) {
-      const int row = r0 + lane / (4 * NF), t = m0 + (wm * MF + i0) * 16 + row;
+      const int row = r0 + lane / LPR, t = m0 + (wm * MF + i0) * 16 + row;
       if (t >= t_hi || n >= a.N) continue;
-      const f32x4_t v = *reinterpret_cast<const f32x4_t*>(tile_lds + row * LDT + (lane % (4 * NF)) * 4);
-      if (parts == 1) {
+      const f32x4_t v = *reinterpret_cast<const f32x4_t*>(tile_lds + row * LDT + (lane % LPR) * 4);
+      // parts: [part][row][group][column], padded to whole 4 columns (GATED: the sums with w and w2 as two groups)
+      const int n4 = (a.N + 3) & ~3;
+      if constexpr (GATED) {
+        const f32x4_t u = *reinterpret_cast<const f32x4_t*>(tile_lds + row * LDT + WCOLS + (lane % LPR) * 4);
+        if (parts == 1) {
+          lin_gated4(a, t, n, v, u, vec4);
+        } else {
+          float* to = slab + ((size_t)part * a.T + t) * 2 * n4 + n;
+          *reinterpret_cast<f32x4_t*>(to) = v;
+          *reinterpret_cast<f32x4_t*>(to + n4) = u;
+        }
+      } else if (parts == 1) {
         lin_epilogue4(a, g, t, n, v, b, vec4);
-      } else {   // [part][row][group][column], padded to whole 4 columns
-        const int n4 = (a.N + 3) & ~3;
+      } else {
         *reinterpret_cast<f32x4_t*>(slab + (((size_t)part * a.T + t) * gridDim.y + g) * n4 + n) = v;
       }
     }
@@ -219,22 +240,40 @@ __global__ __launch_bounds__(256) void linear_parts_kernel(LinArgs a, int groups
   }
 }
 
-template <int MF, int NF, int WM, int WN, bool MAP>
+// the same for the gated form
+__global__ __launch_bounds__(256) void linear_gated_parts_kernel(LinArgs a, int parts, const float* slab, bool vec4) {
+  const int n4 = (a.N + 3) & ~3, quads = n4 / 4;
+  const size_t total = (size_t)a.T * quads, step = (size_t)a.T * 2 * n4;
+  for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < total; e += (size_t)gridDim.x * 256) {
+    const int n = (int)(e % quads) * 4, t = (int)(e / quads);
+    const float* from = slab + (size_t)t * 2 * n4 + n;
+    f32x4_t v = *reinterpret_cast<const f32x4_t*>(from), u = *reinterpret_cast<const f32x4_t*>(from + n4);
+    for (int p = 1; p < parts; ++p) {
+      v += *reinterpret_cast<const f32x4_t*>(from + p * step);
+      u += *reinterpret_cast<const f32x4_t*>(from + p * step + n4);
+    }
+    lin_gated4(a, t, n, v, u, vec4);
+  }
+}
+
+template <int MF, int NF, int WM, int WN, bool MAP, bool GATED = false>
 int go(const LinArgs& a, const LinTilePlan& p, int Tg, int groups, float* slab, hipStream_t s) {
   constexpr int BM = 16 * MF * WM, BN = 16 * NF * WN, RING = LT_SLOTS * (BM + BN) * LT_BK * 2;
   constexpr int EPI = WM * WN * (MF / 2) * 16 * (16 * NF + 4) * 4, LDS = RING > EPI ? RING : EPI;
-  auto kern = linear_pipe_kernel<MF, NF, WM, WN, MAP>;
+  auto kern = linear_pipe_kernel<MF, NF, WM, WN, MAP, GATED>;
   // the grant is per device: asked for at every launch (a lookup in the runtime)
   if (LDS > 64 * 1024)
     DIHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS), DIHIP_RUNTIME_ERROR);
-  const int mt = (Tg + BM - 1) / BM, nt = (a.N + BN - 1) / BN;
+  const int mt = (Tg + BM - 1) / BM, nt = GATED ? (a.N + BN / 2 - 1) / (BN / 2) : (a.N + BN - 1) / BN;
   const bool vec4 = lin_vec4(a);
   // (segments: as many row tiles as T rows in `groups` segments of at most Tg can need)
   const dim3 grid(a.seg ? (unsigned)nt * (unsigned)(mt * (long)groups < a.T / BM + groups ? mt * groups : a.T / BM + groups) : mt * nt, a.seg ? 1 : groups, p.parts);
   hipLaunchKernelGGL(kern, grid, dim3(64 * WM * WN), LDS, s, a, mt, nt, groups, vec4, p.parts, slab);
   if (p.parts > 1) {
     const size_t quads = (size_t)a.T * groups * ((a.N + 3) / 4);
-    hipLaunchKernelGGL(linear_parts_kernel, dim3((unsigned)((quads + 255) / 256 < 4096 ? (quads + 255) / 256 : 4096)), dim3(256), 0, s, a, groups, p.parts, slab, vec4);
+    const dim3 pgrid((unsigned)((quads + 255) / 256 < 4096 ? (quads + 255) / 256 : 4096));
+    if constexpr (GATED) hipLaunchKernelGGL(linear_gated_parts_kernel, pgrid, dim3(256), 0, s, a, p.parts, slab, vec4);
+    else hipLaunchKernelGGL(linear_parts_kernel, pgrid, dim3(256), 0, s, a, groups, p.parts, slab, vec4);
   }
   return launch_status();
 }
@@ -282,6 +321,13 @@ LinTilePlan plan_linear_tile(int Tg, int N, int K, int groups, long ldx, bool sp
 
 int launch_linear_tile(const LinArgs& a, const LinTilePlan& p, int Tg, int groups, float* slab, hipStream_t s) {
   DIHIP_REQUIRE(groups <= 65535, DIHIP_PARAM_ERROR, "linear: more than 65535 groups");
+  if (a.w2) {
+    switch (p.shape) {
+      case 0: return go<8, 4, 2, 4, false, true>(a, p, Tg, 1, slab, s);
+      case 1: return go<6, 4, 2, 4, false, true>(a, p, Tg, 1, slab, s);
+      default: return go<4, 4, 2, 2, false, true>(a, p, Tg, 1, slab, s);
+    }
+  }
   if (a.row_map) {
     switch (p.shape) {
       case 0: return go<8, 4, 2, 4, true>(a, p, Tg, groups, slab, s);

@@ -570,8 +570,7 @@ class GatedMlp:
             gu = so.linear(x, self.w_gu, math=ctx.math)
             g = so.moe_glu(gu, self.F, self.limit, GLU_SLOPE, ctx.act_buffer(self.F))
             return so.linear(g, self.down, math=ctx.math)
-        u = so.linear(x, self.up, math=ctx.math)
-        g = so.linear(x, self.gate, act=self.act, mul=u, math=ctx.math, out=ctx.act_buffer(self.gate.shape[0]))   # act(gate h) * (up h)
+        g = so.linear_gated(x, self.gate, self.up, act=self.act, math=ctx.math, out=ctx.act_buffer(self.gate.shape[0]))   # act(gate h) * (up h)
         return so.linear(g, self.down, math=ctx.math)
 
 

@@ -65,6 +65,22 @@ def linear(x, w, bias=None, out=None, act=None, act_cols=None, mul=None, math=MA
     return y
 
 
+def linear_gated(x, gate, up, act=None, math=MATH_F32, out=None):
+    """y = act(x . gate^T) * (x . up^T): one launch where the kernels of bf16 operands have one for the sizes, else a product after the other"""
+    T, (N, K) = x.shape[0], gate.shape
+    assert up.shape == (N, K) and x.shape[1] == K and gate.is_contiguous() and up.is_contiguous()
+    y = out if out is not None else torch.empty(T, N, dtype=torch.float32, device=x.device)
+    assert y.shape == (T, N)
+    need = C.c_size_t(0)
+    if math == MATH_BF16 and x.dtype == gate.dtype == up.dtype == torch.bfloat16 and (x.data_ptr() | gate.data_ptr() | up.data_ptr()) % 16 == 0 and \
+            act != "softcap" and lib().dihip_linear_gated_query(T, N, K, _rows(x), C.byref(need)):
+        ws = torch.empty(need.value, dtype=torch.uint8, device=x.device) if need.value else None
+        check(lib().dihip_linear_gated(stream(), ptr(x), _rows(x), ptr(gate), ptr(up), ptr(y), dt(y), _rows(y), T, N, K, ACT[act], ptr(ws), need.value),
+              "dihip_linear_gated")
+        return y
+    return linear(x, gate, act=act, mul=linear(x, up, math=math), math=math, out=y)
+
+
 def embed_sum(ids, table, rows2=None, table2=None, out=None):
     T, K = ids.shape[0], table.shape[1]
     h = out if out is not None else torch.empty(T, K, dtype=torch.float32, device=table.device)

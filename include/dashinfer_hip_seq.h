@@ -54,6 +54,14 @@ int dihip_linear_ws(void* stream, const void* x, int x_dtype, long ldx, long x_g
                     const float* mul, long ldm, int mul_group, int T, int N, int K, int groups, int act, int act_lo, int act_hi,
                     float act_param, int math, void* ws, size_t ws_bytes);
 
+/* Gated feed-forward units, bf16 rows and weights (16-byte aligned): y = act(x . w_gate^T) * (x . w_up^T), both [N][K] row-major, y f32 or bf16 rows of
+ * stride ldy; act without a parameter.  One launch brings the rows of x once for both products and keeps their f32 sums on the chip; an element's sums
+ * are those of dihip_linear up to the number of K parts.  dihip_linear_gated_query: whether the sizes run this way (else 0: two calls of
+ * dihip_linear), and the workspace the call can use (0: none; with less, or NULL, K is not split). */
+int dihip_linear_gated_query(int T, int N, int K, long ldx, size_t* ws_bytes);
+int dihip_linear_gated(void* stream, const void* x, long ldx, const void* w_gate, const void* w_up, void* y, int y_dtype, long ldy, int T, int N, int K,
+                       int act, void* ws, size_t ws_bytes);
+
 /* The same product for rows that are grouped by owner (mixture of experts): group g owns the output rows seg[g] .. seg[g + 1]
  * (seg: [groups + 1] on the device, ascending, seg[groups] <= R), output row r reads the x row row_map[r] (NULL: r itself) and
  * the weight w[g] ([groups][N][K]); bias [groups][N] or NULL; `act` on every column.  seg_max_rows: a host-known bound on the
