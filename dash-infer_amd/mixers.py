@@ -398,10 +398,15 @@ class GatedLinearAttention:
         self.norm, self.o = w["norm"].contiguous(), w["o"].contiguous()
         assert w["q"].shape[0] == hd and w["v"].shape[0] == hv and self.a2.shape == (hd, w["a1"].shape[0]) and self.o.shape[1] == hv
         self.S = state.add_state(key + ".S", (heads, dim, vdim))
+        self.one = so.gla_gated_supported(self.a2, self.a2_b, self.norm, heads, dim, vdim)     # from input to output product in one kernel
 
     def __call__(self, ctx, h, h16=None):
         H, D, V = self.H, self.D, self.V
         a = so.linear(h16 if h16 is not None else h, self.w_in, act="silu", act_cols=(self.g_lo, self.a_lo), math=ctx.math)   # [q | k | v | silu g | a1 h]
+        if self.one and ctx.math == so.MATH_BF16:
+            on = so.gla_gated(a, self.k_lo, self.v_lo, self.g_lo, self.a_lo, self.a2, self.a2_b, self.norm, self.q_scale, self.tau, ctx.eps, self.S, ctx.ent_slot,
+                              ctx.ent_row0, ctx.ent_count, ctx.max_count, H, D, V, out=ctx.act_buffer(H * V))
+            return so.linear(on, self.o, math=ctx.math)
         z = so.linear(a[:, self.a_lo:], self.a2, self.a2_b, math=ctx.math)
         o = so.gla(a, a[:, self.k_lo:], a[:, self.v_lo:], z, self.q_scale, self.tau, self.S, ctx.ent_slot, ctx.ent_row0, ctx.ent_count,
                    ctx.max_count, H, D, V)

@@ -362,6 +362,25 @@ def gla(q, k, v, z, q_scale, tau, state, ent_slot, ent_row0, ent_count, max_coun
     return o
 
 
+def gla_gated_supported(a2, a2_b, norm, H, D, DV):
+    return a2.dtype == a2_b.dtype == norm.dtype == torch.bfloat16 and bool(lib().dihip_gla_gated_supported(H, D, DV, a2.shape[1]))
+
+
+def gla_gated(rows, k_lo, v_lo, g_lo, a_lo, a2, a2_b, norm, q_scale, tau, eps, state, ent_slot, ent_row0, ent_count, max_count, H, D, DV, out):
+    """rows: f32 [T, .] = [q | k | v | gate | a1 h], the parts starting at the columns 0, k_lo, ..  gla(q, k, v, a2 (a1 h) + a2_b), every head over its root mean square, times
+    norm, times gate -> out (f32 or bf16 rows)"""
+    T, E = rows.shape[0], ent_slot.shape[0]
+    assert rows.dtype == torch.float32 and rows.shape[1] >= a_lo + a2.shape[1] and state.shape[1:] == (H, D, DV) and state.is_contiguous() and out.shape == (T, H * DV)
+    assert a2.is_contiguous() and a2.shape[0] == H * D and a2_b.shape == (H * D,) and a2_b.is_contiguous() and norm.shape == (DV,) and norm.is_contiguous()
+    need = int(lib().dihip_gla_gated_workspace_bytes(E, int(max_count), H, D, DV))
+    ws = torch.empty(need, dtype=torch.uint8, device=rows.device) if need else None
+    col = lambda c: C.c_void_p(rows.data_ptr() + 4 * c)
+    check(lib().dihip_gla_gated(stream(), ptr(out), dt(out), _rows(out), col(0), col(k_lo), col(v_lo), col(g_lo), col(a_lo), _rows(rows), ptr(a2), ptr(a2_b), ptr(norm),
+                                a2.shape[1], float(q_scale), float(tau), float(eps), ptr(state), ptr(ent_slot), ptr(ent_row0), ptr(ent_count), T, E, int(max_count),
+                                H, D, DV, ptr(ws), need), "dihip_gla_gated")
+    return out
+
+
 def head_rmsnorm_mul(x, gamma, eps, H, DV, mul=None, out=None, div=None, out_scale=1.0):
     """per head: v = x * div[t, h]; v / rms(v) * gamma * mul * out_scale; gamma [DV] shared by the heads, [H * DV], or None"""
     T = x.shape[0]

@@ -216,6 +216,16 @@ int dihip_gla(void* stream, float* out, long ldo, const float* q, long ldq, cons
               const float* z, long ldz, float q_scale, float tau, float* state, const int32_t* ent_slot,
               const int32_t* ent_row0, const int32_t* ent_count, int T, int E, int max_count, int H, int D, int DV,
               int chunked, void* ws, size_t ws_bytes);
+/* The same from the rows of the input product to those of the output product, bf16 products:
+ *   z = bf16(a1[t]) . a2^T + a2_bias,   the recurrence above,   y[t, h, :] = out / sqrt(mean(out^2) + eps) * gamma * gate[t, h, :]
+ * q, k [H * D], v, gate [H * DV], a1 [rank]: columns of f32 rows of one stride ld;  a2 [H * D][rank], a2_bias [H * D], gamma [DV] bf16;  y of y_dtype.
+ * dihip_gla_gated_supported: the sizes it serves.  Portions of more than 16 rows run in chunks side by side and need the workspace. */
+int dihip_gla_gated_supported(int H, int D, int DV, int rank);
+size_t dihip_gla_gated_workspace_bytes(int E, int max_count, int H, int D, int DV);
+int dihip_gla_gated(void* stream, void* y, int y_dtype, long ldy, const float* q, const float* k, const float* v, const float* gate, const float* a1, long ld,
+                    const void* a2, const void* a2_bias, const void* gamma, int rank, float q_scale, float tau, float eps, float* state,
+                    const int32_t* ent_slot, const int32_t* ent_row0, const int32_t* ent_count, int T, int E, int max_count, int H, int D, int DV, void* ws,
+                    size_t ws_bytes);
 /* v = x[t, h, :] * div[t, h]  (div [T, H]; NULL: x itself);  y[t, h, :] = v / sqrt(mean(v^2) + eps) * gamma * mul[t, h, :] * out_scale
  * gamma: [DV] shared by the heads, [H * DV] with gamma_per_head, NULL: 1;  mul NULL: 1 */
 int dihip_head_rmsnorm_mul(void* stream, void* y, int y_dtype, long ldy, const float* x, long ldx, const void* gamma, int gamma_per_head,

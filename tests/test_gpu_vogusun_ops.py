@@ -248,6 +248,42 @@ def test_gla_sequences_side_by_side():
     assert rel_err(np.concatenate([a[1], b[0]]), want[1]) < 3e-5 and rel_err(a[2], want[2]) < 3e-5
 
 
+# portions below, at and past the 16 rows of a staged batch and the 16, 32 and 64 of a chunk (by the number of heads); channels that fill a wave's quarter or not, one and two columns per lane
+@pytest.mark.parametrize("H,D,DV,rank", [(3, 64, 128, 64), (2, 16, 4, 32), (1, 48, 100, 96), (2, 128, 128, 128), (4, 80, 64, 32), (32, 32, 8, 32), (128, 16, 4, 32)])
+@pytest.mark.parametrize("counts", [[1], [1, 1, 1], [16, 3], [17, 1, 16], [33, 64, 1, 2], [300, 1, 129, 128, 65]])
+def test_gla_in_one_kernel(H, D, DV, rank, counts):
+    """z, recurrence, norm and gate against 64 bits (the rank's rows rounded to bf16, as the product rounds them), and the states left in their slots: f32 sums"""
+    load_pkg()
+    from dash_infer_amd import seq_ops as so
+    rng = np.random.default_rng(D + DV + sum(counts))
+    T, E, tau, eps, sc = sum(counts), len(counts), 4.0, 1e-5, D ** -0.5
+    hd, hv = H * D, H * DV
+    rows = rng.normal(0, 1, (T, 2 * hd + 2 * hv + rank)).astype(np.float32)
+    a2, b2, norm = bf(rng.normal(0, rank ** -0.5, (hd, rank))), bf(rng.normal(1, 1, hd)), bf(1 + 0.2 * rng.normal(size=DV))
+    state = rng.normal(0, 1, (E + 2, H, D, DV)).astype(np.float32)
+    slots = rng.permutation(E + 2)[:E]
+    row0 = np.cumsum([0] + counts[:-1])
+    S_dev, y = dev(state), torch.full((T, hv + 4), 7.0, device="cuda")
+    wdev = lambda a: torch.tensor(a).cuda().to(torch.bfloat16)
+    assert so.gla_gated_supported(wdev(a2), wdev(b2), wdev(norm), H, D, DV)
+    lo = (hd, 2 * hd, 2 * hd + hv, 2 * hd + 2 * hv)
+    so.gla_gated(dev(rows), *lo, wdev(a2), wdev(b2), wdev(norm), sc, tau, eps, S_dev, i32(slots), i32(row0), i32(counts), max(counts), H, D, DV, out=y[:, :hv])
+    r = rows.astype(np.float64)
+    a1 = torch.tensor(rows[:, lo[3]:]).to(torch.bfloat16).double().numpy()
+    al = ((1 / (1 + np.exp(-(a1 @ a2.T.astype(np.float64) + b2)))) ** (1 / tau)).reshape(T, H, D)
+    q, k, v, g = (r[:, b:b + n].reshape(T, H, -1) for b, n in ((0, hd), (lo[0], hd), (lo[1], hv), (lo[2], hv)))
+    want, S_want = np.zeros((T, H, DV)), state.astype(np.float64)
+    for e in range(E):
+        S = S_want[slots[e]]
+        for t in range(row0[e], row0[e] + counts[e]):
+            S = al[t][:, :, None] * S + k[t][:, :, None] * v[t][:, None]
+            want[t] = (S * (q[t] * sc)[:, :, None]).sum(1)
+        S_want[slots[e]] = S
+    want = want / np.sqrt((want ** 2).mean(-1, keepdims=True) + eps) * norm * g
+    assert rel_err(y[:, :hv].cpu().numpy(), want.reshape(T, hv)) < 3e-5 and bool((y[:, hv:] == 7).all())
+    assert rel_err(S_dev.cpu().numpy(), S_want) < 3e-5
+
+
 # ---------------------------------------------------------------------------------------------------------------- feed-forward
 def test_gated_mlp():
     load_pkg()
