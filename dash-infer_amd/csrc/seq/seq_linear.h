@@ -13,7 +13,23 @@ struct LinArgs {
   int mul_group; float act_param;               // mul holds one number per group; the parameter of an activation that has one
   const int32_t* seg; const int32_t* row_map;   // segmented form: group g owns the output rows seg[g] .. seg[g + 1], row r reads x row row_map[r]
   const void* w2;                               // gated form: y = act(x . w^T) * (x . w2^T); w2 is shaped as w.  No groups, bias or mul
+  // residual form (res): y is the f32 residual stream, y += res_a + result, and, with norm_w, h16 = bf16(tanh(norm_alpha * y) * norm_w + norm_b), rows of N.  No groups
+  int res; const float* res_a; long res_lda; float norm_alpha; const void* norm_w; const void* norm_b; uint16_t* h16;   // (res_a NULL: the result alone; norm: bf16)
 };
+
+// the residual form's way out (the arithmetic of dihip_add_dyt, step by step)
+struct LinRes { float x, a, w, b; };
+__device__ __forceinline__ LinRes lin_res_load(const LinArgs& q, int t, int n) {
+  LinRes r{((const float*)q.y)[(size_t)t * q.ldy + n], 0.f, 0.f, 0.f};
+  if (q.res_a) r.a = q.res_a[(size_t)t * q.res_lda + n];
+  if (q.norm_w) { r.w = bf16_bits_to_f32(((const uint16_t*)q.norm_w)[n]); r.b = bf16_bits_to_f32(((const uint16_t*)q.norm_b)[n]); }
+  return r;
+}
+__device__ __forceinline__ void lin_res_store(const LinArgs& q, int t, int n, float v, const LinRes& r) {
+  const float x = r.x + (q.res_a ? r.a + v : v);
+  ((float*)q.y)[(size_t)t * q.ldy + n] = x;
+  if (q.norm_w) q.h16[(size_t)t * q.N + n] = (uint16_t)f32_to_bf16_bits(tanhf(q.norm_alpha * x) * r.w + r.b);
+}
 
 // the rows of group g: [lo, hi)
 __device__ __forceinline__ void lin_rows(const LinArgs& a, int g, int& lo, int& hi) {
@@ -28,6 +44,7 @@ __device__ __forceinline__ void lin_epilogue(const LinArgs& a, int g, int t, int
   if (col >= a.act_lo && col < a.act_hi) v = a.act == DIHIP_SEQ_ACT_SOFTCAP ? a.act_param * tanhf(v / a.act_param) : apply_act(v, a.act);
   const size_t o = (size_t)t * a.ldy + (size_t)g * a.yg + n;
   if (a.mul) v *= a.mul[(size_t)t * a.ldm + (a.mul_group ? (size_t)g : (size_t)g * a.yg + n)];
+  if (a.res) return lin_res_store(a, t, n, v, lin_res_load(a, t, n));
   st_any(a.y, o, a.ydt, v);
 }
 
@@ -36,7 +53,9 @@ __device__ __forceinline__ void lin_epilogue(const LinArgs& a, int g, int t, int
 inline bool lin_vec4(const LinArgs& a) {
   const bool mul = !a.mul || a.mul_group || ((reinterpret_cast<uintptr_t>(a.mul) & 15) == 0 && a.ldm % 4 == 0);
   return a.N % 4 == 0 && a.ldy % 4 == 0 && a.yg % 4 == 0 && (reinterpret_cast<uintptr_t>(a.y) & (a.ydt == DIHIP_F32 ? 15 : 7)) == 0 && mul &&
-         (!a.bias || (reinterpret_cast<uintptr_t>(a.bias) & 7) == 0);
+         (!a.bias || (reinterpret_cast<uintptr_t>(a.bias) & 7) == 0) &&
+         (!a.res || ((!a.res_a || ((reinterpret_cast<uintptr_t>(a.res_a) & 15) == 0 && a.res_lda % 4 == 0)) &&
+                     ((reinterpret_cast<uintptr_t>(a.norm_w) | reinterpret_cast<uintptr_t>(a.norm_b) | reinterpret_cast<uintptr_t>(a.h16)) & 7) == 0));
 }
 __device__ __forceinline__ f32x4_t lin_bias4(const LinArgs& a, int g, int n, bool vec4) {
   if (!vec4 || !a.bias || n >= a.N) return f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -63,6 +82,22 @@ __device__ __forceinline__ void lin_epilogue4(const LinArgs& a, int g, int t, in
     else v *= *reinterpret_cast<const f32x4_t*>(a.mul + (size_t)t * a.ldm + (size_t)g * a.yg + n);
   }
   const size_t o = (size_t)t * a.ldy + (size_t)g * a.yg + n;
+  if (a.res) {
+    f32x4_t* y = reinterpret_cast<f32x4_t*>((float*)a.y + o);
+    f32x4_t x = *y;
+    if (a.res_a) v = *reinterpret_cast<const f32x4_t*>(a.res_a + (size_t)t * a.res_lda + n) + v;
+    x += v;
+    *y = x;
+    if (a.norm_w) {
+      const u32x2_t w = *reinterpret_cast<const u32x2_t*>((const uint16_t*)a.norm_w + n), b2 = *reinterpret_cast<const u32x2_t*>((const uint16_t*)a.norm_b + n);
+      uint32_t h[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        h[r] = f32_to_bf16_bits(tanhf(a.norm_alpha * x[r]) * bf16_bits_to_f32((w[r >> 1] >> (r & 1) * 16) & 0xffffu) + bf16_bits_to_f32((b2[r >> 1] >> (r & 1) * 16) & 0xffffu));
+      *reinterpret_cast<u32x2_t*>(a.h16 + (size_t)t * a.N + n) = u32x2_t{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+    }
+    return;
+  }
   if (a.ydt == DIHIP_F32) *reinterpret_cast<f32x4_t*>((float*)a.y + o) = v;
   else *reinterpret_cast<u32x2_t*>((uint16_t*)a.y + o) = u32x2_t{f32_to_bf16_bits(v[0]) | (f32_to_bf16_bits(v[1]) << 16),
                                                                   f32_to_bf16_bits(v[2]) | (f32_to_bf16_bits(v[3]) << 16)};

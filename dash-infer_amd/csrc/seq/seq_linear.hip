@@ -561,6 +561,8 @@ __global__ __launch_bounds__(64 * ROW_WAVES, 2) void linear_row_kernel(LinArgs a
         if (r0 + r < rows) part[(r0 + r) * ROW_WAVES + wave] = v[r];
     }
   };
+  LinRes res{0.f, 0.f, 0.f, 0.f};
+  if (!GATED && a.res && tid < own) res = lin_res_load(a, 0, lo + tid);   // (a thread's first column: here long before it is used)
   for (int r0 = 0; r0 < rows; r0 += 2 * R) {
     load(wb, r0 + R);
     __builtin_amdgcn_sched_barrier(0);
@@ -578,6 +580,8 @@ __global__ __launch_bounds__(64 * ROW_WAVES, 2) void linear_row_kernel(LinArgs a
     if constexpr (GATED) {
       const f32x4_t u = *reinterpret_cast<const f32x4_t*>(part + (own + r) * ROW_WAVES);
       st_any(a.y, (size_t)(lo + r), a.ydt, apply_act(v, a.act) * ((u[0] + u[1]) + (u[2] + u[3])));
+    } else if (a.res && r == tid && !a.bias && !a.mul && a.act_hi <= a.act_lo) {
+      lin_res_store(a, 0, lo + r, v, res);
     } else {
       lin_epilogue(a, 0, 0, lo + r, v, DIHIP_BF16);
     }
@@ -788,7 +792,7 @@ using namespace dihip;
 static int linear_impl(void* stream, const void* x, int x_dtype, long ldx, long x_gstride, int x_groups, const void* w,
                        int w_dtype, const void* bias, void* y, int y_dtype, long ldy, long y_gstride, const float* mul,
                        long ldm, int mul_group, int T, int N, int K, int groups, int act, int act_lo, int act_hi, float act_param, int math,
-                       const int32_t* seg, const int32_t* row_map, int seg_max_rows, void* ws, size_t ws_bytes) {
+                       const int32_t* seg, const int32_t* row_map, int seg_max_rows, void* ws, size_t ws_bytes, const LinArgs* res = nullptr) {
   DIHIP_REQUIRE(T >= 0 && N > 0 && K > 0 && groups > 0 && x_groups > 0, DIHIP_PARAM_ERROR, "linear: bad shape T %d N %d K %d groups %d", T, N, K, groups);
   DIHIP_REQUIRE(seq_dtype_ok(x_dtype) && seq_dtype_ok(w_dtype) && seq_dtype_ok(y_dtype), DIHIP_PARAM_ERROR, "linear: f32 / bf16 only");
   DIHIP_REQUIRE(x && w && y, DIHIP_PARAM_ERROR, "linear: null pointer");
@@ -800,6 +804,10 @@ static int linear_impl(void* stream, const void* x, int x_dtype, long ldx, long 
   if (T == 0) return DIHIP_SUCCESS;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   LinArgs a{x, ldx, x_gstride, x_groups, w, bias, y, ldy, y_gstride, mul, ldm, T, N, K, act, act_lo, act_hi, y_dtype, 0, mul_group, act_param, seg, row_map};
+  if (res) {
+    a.res = 1; a.res_a = res->res_a; a.res_lda = res->res_lda;
+    a.norm_alpha = res->norm_alpha; a.norm_w = res->norm_w; a.norm_b = res->norm_b; a.h16 = res->h16;
+  }
   const int Tg = seg ? (seg_max_rows < T ? seg_max_rows : T) : T;   // the most rows one group can have
   const size_t xe = x_dtype == DIHIP_F32 ? 4 : 2;
   const bool vec = w_dtype == DIHIP_BF16 && K % 8 == 0 && aligned16(w) && aligned16(x) && (ldx * xe) % 16 == 0 &&
@@ -934,6 +942,16 @@ extern "C" int dihip_linear_ws(void* stream, const void* x, int x_dtype, long ld
   DIHIP_REQUIRE(!ws || aligned16(ws), DIHIP_PARAM_ERROR, "linear: a workspace starts on 16 bytes");
   return linear_impl(stream, x, x_dtype, ldx, x_gstride, x_groups, w, w_dtype, bias, y, y_dtype, ldy, y_gstride, mul, ldm, mul_group, T, N, K, groups,
                      act, act_lo, act_hi, act_param, math, nullptr, nullptr, 0, ws, ws_bytes);
+}
+
+extern "C" int dihip_linear_residual_dyt(void* stream, const void* x, long ldx, const void* w, float* stream_x, const float* a, long lda, float alpha, const void* norm_w,
+                                         const void* norm_b, void* h16, int T, int N, int K, void* ws, size_t ws_bytes) {
+  DIHIP_REQUIRE(!ws || aligned16(ws), DIHIP_PARAM_ERROR, "linear_residual_dyt: a workspace starts on 16 bytes");
+  DIHIP_REQUIRE((!a || lda >= N) && (!norm_w || (norm_b && h16)), DIHIP_PARAM_ERROR, "linear_residual_dyt: bad argument");
+  LinArgs r{};
+  r.res_a = a; r.res_lda = lda; r.norm_alpha = alpha; r.norm_w = norm_w; r.norm_b = norm_w ? norm_b : nullptr; r.h16 = norm_w ? (uint16_t*)h16 : nullptr;
+  return linear_impl(stream, x, DIHIP_BF16, ldx, K, 1, w, DIHIP_BF16, nullptr, stream_x, DIHIP_F32, N, N, nullptr, 0, 0, T, N, K, 1, 0, 0, 0, 0.f, DIHIP_MATH_BF16,
+                     nullptr, nullptr, 0, ws, ws_bytes, &r);
 }
 
 extern "C" int dihip_linear_segmented(void* stream, const void* x, int x_dtype, long ldx, const void* w, int w_dtype, const void* bias,

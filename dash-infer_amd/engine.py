@@ -138,6 +138,7 @@ class SeqEngine:
             g["graph"].replay()
             return g["logits"]
         ctx = self._context(g["meta"], cut, E, E, 1, bucket)
+        ctx.want_all = True
         logits = self.model.logits(ctx, self.model.forward(ctx), ctx.want_rows)
         if (E, bucket) in self._graphs:
             torch.cuda.synchronize()

@@ -50,6 +50,8 @@ class StepContext:
         self.ids, self.rows2, self.tok_slot, self.tok_pos, self.tok_off = ids, rows2, tok_slot, tok_pos, tok_off
         self.ent_slot, self.ent_row0, self.ent_count, self.want_rows = ent_slot, ent_row0, ent_count, want_rows
         self.math, self.eps = math, eps
+        self.final16 = None                     # the last norm's rows, where the last product of the step has made them
+        self.want_all = False                   # want_rows names every row in order (a host's knowledge)
         self.max_count, self.max_pos = T, 0     # host numbers: the largest portion and the last position of the step
         self.taps = None    # layer index -> [T, .] intermediate (diagnostics; None: off)
         self.shared = {}    # what a layer leaves for later layers of the SAME step (values to be mixed in)
@@ -569,14 +571,19 @@ class GatedMlp:
         else:
             self.gate, self.up = gate.contiguous(), up.contiguous()
 
-    def __call__(self, ctx, h, h16=None):
+    def _hidden(self, ctx, h, h16):
         x = h16 if h16 is not None else h
         if self.limit is not None:
             gu = so.linear(x, self.w_gu, math=ctx.math)
-            g = so.moe_glu(gu, self.F, self.limit, GLU_SLOPE, ctx.act_buffer(self.F))
-            return so.linear(g, self.down, math=ctx.math)
-        g = so.linear_gated(x, self.gate, self.up, act=self.act, math=ctx.math, out=ctx.act_buffer(self.gate.shape[0]))   # act(gate h) * (up h)
-        return so.linear(g, self.down, math=ctx.math)
+            return so.moe_glu(gu, self.F, self.limit, GLU_SLOPE, ctx.act_buffer(self.F))
+        return so.linear_gated(x, self.gate, self.up, act=self.act, math=ctx.math, out=ctx.act_buffer(self.gate.shape[0]))   # act(gate h) * (up h)
+
+    def __call__(self, ctx, h, h16=None):
+        return so.linear(self._hidden(ctx, h, h16), self.down, math=ctx.math)
+
+    def into(self, ctx, h16, x, other, norm):
+        """bf16 products: x += other + the block's rows, in place, as the way out of the last product -> the next norm's rows (norm None: None)"""
+        return so.linear_residual_dyt(self._hidden(ctx, None, h16), self.down, x, other, norm)
 
 
 class ExpertMlp:

@@ -85,6 +85,8 @@ class Vogusun:
                 else:
                     raise ValueError(f"layer {i}: unknown feed-forward kind {fc['kind']!r}")
             self.layers.append((_norm(w, "norm1"), mixer, ff))
+        norms = [self.final_norm] + [layer[0] for layer in self.layers]
+        self.dtypes = {self.embed.dtype} | {t.dtype for n in norms for t in n[1:]} | {ff.down.dtype for _, _, ff in self.layers if isinstance(ff, mixers.GatedMlp)}
 
     @classmethod
     def from_config(cls, config, tensors, state, dtype):
@@ -96,18 +98,34 @@ class Vogusun:
     def forward(self, ctx):
         """-> the residual stream after the last layer, [T, width] f32"""
         bf = self.math == so.MATH_BF16        # bf16 products read a bf16 copy of the norm's output: the same bits at half the traffic
-        x = so.embed_sum(ctx.ids, self.embed)
-        h, h16 = so.add_dyt(x, norm=self.layers[0][0], want16=bf) if self.layers else (None, None)
+        if not self.layers:
+            return so.embed_sum(ctx.ids, self.embed)
+        # bf16 checkpoints: the first norm is the embedding's way out, a dense block's last product ends in the residual step and the next norm
+        fused = bf and self.dtypes == {torch.bfloat16} and self.embed.is_contiguous()
+        if fused:
+            h = None
+            x, h16 = so.embed_dyt(ctx.ids, self.embed, self.layers[0][0])
+        else:
+            x = so.embed_sum(ctx.ids, self.embed)
+            h, h16 = so.add_dyt(x, norm=self.layers[0][0], want16=bf)
         for i, (_, mixer, ff) in enumerate(self.layers):
             mo = mixer(ctx, h, h16)
-            fo = ff(ctx, h, h16) if ff is not None else None
             nxt = self.layers[i + 1][0] if i + 1 < len(self.layers) else None
-            h, h16 = so.add_dyt(x, mo, fo, norm=nxt, x_out=x, want16=bf)
+            if fused and isinstance(ff, mixers.GatedMlp):
+                if nxt is None and ctx.want_all:
+                    ctx.final16 = ff.into(ctx, h16, x, mo, self.final_norm)
+                else:
+                    h16 = ff.into(ctx, h16, x, mo, nxt)
+            else:
+                fo = ff(ctx, h, h16) if ff is not None else None
+                h, h16 = so.add_dyt(x, mo, fo, norm=nxt, x_out=x, want16=bf)
             if ctx.taps is not None:
                 ctx.taps[i] = x.clone()
         return x
 
     def logits(self, ctx, x, rows):
         """rows: int32 device tensor of the row indices whose logits are wanted -> f32 [len(rows), vocab]"""
+        if rows is ctx.want_rows and ctx.final16 is not None:
+            return so.linear(ctx.final16, self.head, math=ctx.math)
         h, h16 = so.add_dyt(x, norm=self.final_norm, row_idx=rows, want16=self.math == so.MATH_BF16)
         return so.linear(h16 if h16 is not None else h, self.head, math=ctx.math)

@@ -81,6 +81,37 @@ def linear_gated(x, gate, up, act=None, math=MATH_F32, out=None):
     return linear(x, gate, act=act, mul=linear(x, up, math=math), math=math, out=y)
 
 
+def linear_residual_dyt(x, w, stream_x, a=None, norm=None):
+    """stream_x += a + x . w^T in place;  -> tanh(alpha * stream_x) * w + bias in bf16 for norm = (alpha, w, bias), else None.  bf16 rows, weights and norm: the way out of
+    the last product of a layer is the residual step and the next norm (linear, then add_dyt, to the bit)"""
+    (T, K), N = x.shape, w.shape[0]
+    assert w.shape == (N, K) and w.is_contiguous() and x.dtype == w.dtype == torch.bfloat16
+    assert stream_x.shape == (T, N) and stream_x.is_contiguous() and stream_x.dtype == torch.float32
+    assert a is None or (a.shape == (T, N) and a.dtype == torch.float32)
+    alpha, nw, nb, h16 = 0.0, None, None, None
+    if norm is not None:
+        alpha, nw, nb = norm
+        assert nw.dtype == nb.dtype == torch.bfloat16 and nw.shape == nb.shape == (N,)
+        h16 = torch.empty(T, N, dtype=torch.bfloat16, device=x.device)
+    ws, need = None, 0
+    if T > LINEAR_FEW_ROWS:
+        need = int(lib().dihip_linear_workspace_bytes(T, N, K, 1, _rows(x)))
+        ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+    check(lib().dihip_linear_residual_dyt(stream(), ptr(x), _rows(x), ptr(w), ptr(stream_x), ptr(a), _rows(a) if a is not None else 0, float(alpha), ptr(nw), ptr(nb), ptr(h16),
+                                          T, N, K, ptr(ws), need), "dihip_linear_residual_dyt")
+    return h16
+
+
+def embed_dyt(ids, table, norm):
+    """x = table[ids] in f32 and its norm in bf16 (add_dyt); table and norm bf16"""
+    T, K = ids.shape[0], table.shape[1]
+    alpha, w, bias = norm
+    assert table.dtype == w.dtype == bias.dtype == torch.bfloat16 and table.is_contiguous() and w.shape == bias.shape == (K,)
+    x, h16 = torch.empty(T, K, dtype=torch.float32, device=table.device), torch.empty(T, K, dtype=torch.bfloat16, device=table.device)
+    check(lib().dihip_embed_dyt(stream(), ptr(x), ptr(h16), ptr(ids), ptr(table), float(alpha), ptr(w), ptr(bias), T, K), "dihip_embed_dyt")
+    return x, h16
+
+
 def embed_sum(ids, table, rows2=None, table2=None, out=None):
     T, K = ids.shape[0], table.shape[1]
     h = out if out is not None else torch.empty(T, K, dtype=torch.float32, device=table.device)

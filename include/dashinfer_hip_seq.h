@@ -78,6 +78,16 @@ int dihip_add_dyt(void* stream, float* x_out, const float* x_in, const float* a,
                   const int32_t* row_idx, float alpha, const void* w, const void* bias, int w_dtype, float* h, void* h16,
                   int M, int K);
 
+/* The same step as the way out of a product (bf16 rows and weights, f32 sums): x . w^T is the second sublayer's result and is never written,
+ *   stream_x[t] += a[t] + x[t] . w^T   (a NULL: the product alone),   h16[t] = bf16(tanh(alpha * stream_x[t]) * norm_w + norm_b)   (norm_w NULL: no norm)
+ * stream_x f32 and h16 bf16: contiguous [T, N]; a: f32 rows of stride lda; norm_w, norm_b: bf16.  The arithmetic is that of dihip_linear and dihip_add_dyt one after the
+ * other, to the bit; ws as dihip_linear_ws takes it. */
+int dihip_linear_residual_dyt(void* stream, const void* x, long ldx, const void* w, float* stream_x, const float* a, long lda, float alpha, const void* norm_w,
+                              const void* norm_b, void* h16, int T, int N, int K, void* ws, size_t ws_bytes);
+
+/* x[t] = float(table[ids[t]]) and its norm, h16[t] = bf16(tanh(alpha * x[t]) * w + bias); table, w, bias bf16 */
+int dihip_embed_dyt(void* stream, float* x, void* h16, const int32_t* ids, const void* table, float alpha, const void* w, const void* bias, int T, int K);
+
 /* Layers that run their sublayers side by side on a layer-normed stream: the residual step and the NEXT input norm in one launch,
  *   x_out[r] = x_in[r] + mult * (a[r] + b[r] + sum_k wts[r, k] * rows[dst[r * top + k]])
  *              (each part may be absent: a NULL, b NULL (b goes with a), dst NULL; the sum is dihip_seq_moe_combine's; none: x_in itself),

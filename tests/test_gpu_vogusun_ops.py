@@ -51,6 +51,35 @@ def test_add_dyt_residual_norm_and_row_index(so):
     assert rel_err(only.cpu().numpy(), ov.dyt_norm(x.astype(np.float64) + a, alpha, w, bias)) < 2e-6
 
 
+# one row (whole and part pieces of K, more columns than a workgroup has threads for, the short-row kernel), rows streamed through LDS and past it, tiles whole and in K parts;
+# columns that do not come in fours
+@pytest.mark.parametrize("T,N,K", [(1, 4096, 14336), (1, 700, 2056), (1, 140000, 2048), (1, 40, 512), (3, 33, 200), (2, 130, 1024), (24, 2048, 8192), (33, 2050, 1088), (64, 100, 72), (65, 2048, 8192),
+                                   (300, 514, 192), (513, 1001, 1024), (70, 40, 72)])
+@pytest.mark.parametrize("left,normed", [(True, True), (False, True), (True, False)])
+def test_product_that_ends_in_the_residual_step_and_the_norm(so, T, N, K, left, normed):
+    """the same bits as the product, then add_dyt"""
+    g = torch.Generator("cuda").manual_seed(T + N + K)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    x, w = rand(T, K + 8).bfloat16()[:, 8:], (rand(N, K) * K ** -0.5).bfloat16()
+    stream, a = rand(T, N), rand(T, N + 4)[:, 4:] if left else None
+    norm = (0.75, rand(N).bfloat16(), rand(N).bfloat16()) if normed else None
+    want, got = stream.clone(), stream.clone()
+    y = so.linear(x, w, math=so.MATH_BF16)
+    _, h16 = so.add_dyt(want, a if left else y, y if left else None, norm=norm, x_out=want, want16=True)
+    out = so.linear_residual_dyt(x, w, got, a, norm)
+    assert torch.equal(got, want)
+    assert torch.equal(out, h16) if normed else out is None
+
+
+def test_embedding_and_its_norm(so):
+    g = torch.Generator("cuda").manual_seed(5)
+    table, w, b = (torch.randn(*s, generator=g, device="cuda").bfloat16() for s in ((50, 1100), (1100,), (1100,)))
+    ids = i32([3, 49, 0, 3, 17])
+    x, h16 = so.embed_dyt(ids, table, (0.7, w, b))
+    want = so.embed_sum(ids, table)
+    assert torch.equal(x, want) and torch.equal(h16, so.add_dyt(want, norm=(0.7, w, b), want16=True)[1])
+
+
 # ---------------------------------------------------------------------------------------------------------------- attention
 def attention_weights(rng, kind, width, H, G, D, V):
     r = lambda *s, sd=None: bf(rng.normal(0, sd if sd is not None else 1.0 / math.sqrt(s[-1]), s))
