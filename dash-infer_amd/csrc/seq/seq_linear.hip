@@ -289,7 +289,8 @@ constexpr int STREAM_LDS_WAVES = 4;
 // GATED (linear_gated): the first half of the workgroup's weight rows are w's, the second the same ones of w2.
 template <int ROWS, int TF, int WV, int D, bool SEG, bool GATED>
 __global__ __launch_bounds__(64 * WV, 2) void linear_stream_lds_kernel(LinArgs a, bool vec4) {
-  constexpr int RF = ROWS / 16, PER = 2 * (RF + TF), SLOT = PER * 1024, COLS = GATED ? ROWS / 2 : ROWS;   // (of y)
+  constexpr int RF = (ROWS + 15) / 16, WP = ROWS / 8, PER = WP + 2 * TF, SLOT = PER * 1024, COLS = GATED ? ROWS / 2 : ROWS;   // (WP: pieces of weights; COLS: of y)
+  static_assert(ROWS >= 16 || !GATED, "both halves are whole pieces");
   static_assert((D - 1) * PER < 64, "what is in flight is counted");
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -306,12 +307,12 @@ __global__ __launch_bounds__(64 * WV, 2) void linear_stream_lds_kernel(LinArgs a
   const char* xaddr[2 * TF];   // (SEG: of the next block)
 #pragma unroll
   for (int p = 0; p < PER; ++p) {
-    const int r = (p < 2 * RF ? p : p - 2 * RF) * 8 + prow;
-    if (p < 2 * RF) {
+    const int r = (p < WP ? p : p - WP) * 8 + prow;
+    if (p < WP) {
       off[p] = (uint32_t)min(r % COLS, a.N - 1 - n0) * (uint32_t)a.K * 2 + pchunk * 16;
     } else {
       const size_t from = lin_xrow(a, lo + min(r, count - 1)) * a.ldx * 2 + pchunk * 16;
-      if constexpr (SEG) xaddr[p - 2 * RF] = xbase + from + wave * 128;
+      if constexpr (SEG) xaddr[p - WP] = xbase + from + wave * 128;
       else off[p] = (uint32_t)from;
     }
   }
@@ -325,8 +326,9 @@ __global__ __launch_bounds__(64 * WV, 2) void linear_stream_lds_kernel(LinArgs a
 #pragma unroll
     for (int t = 0; t < TF; ++t) acc[r][t] = z4;
   const int f0 = (lane & 15) * 128 + (((lane >> 4) ^ (lane & 7)) * 16);
+  const int fw = ROWS == 8 ? f0 & ~1024 : f0;   // (8 weight rows: twice in their operand)
   auto ring = [&](auto used) {   // with the first TN row operands
-    constexpr int TN = decltype(used)::value, USED = 2 * (RF + TN);
+    constexpr int TN = decltype(used)::value, USED = WP + 2 * TN;
     auto fetch = [&](int i, int slot) {   // (called for i = 0, 1, 2, ..)
       const char* wk = wbase + (size_t)(wave + i * WV) * 128;
       const char* w2k = GATED ? w2base + (size_t)(wave + i * WV) * 128 : wk;
@@ -334,13 +336,13 @@ __global__ __launch_bounds__(64 * WV, 2) void linear_stream_lds_kernel(LinArgs a
 #pragma unroll
       for (int p = 0; p < USED; ++p) {
         const uint32_t to = lds0 + slot * SLOT + p * 1024;
-        if (SEG && p >= 2 * RF) {
-          const char* const from = xaddr[p - 2 * RF];
+        if (SEG && p >= WP) {
+          const char* const from = xaddr[p - WP];
           asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(to), "v"(from) : "memory");
-          xaddr[p - 2 * RF] += WV * 128;
+          xaddr[p - WP] += WV * 128;
         } else {
           const uint32_t o = off[p];
-          asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(o), "s"(p < (GATED ? RF : 2 * RF) ? wk : p < 2 * RF ? w2k : xk) : "memory");
+          asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(o), "s"(p < (GATED ? WP / 2 : WP) ? wk : p < WP ? w2k : xk) : "memory");
         }
       }
     };
@@ -350,9 +352,9 @@ __global__ __launch_bounds__(64 * WV, 2) void linear_stream_lds_kernel(LinArgs a
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
 #pragma unroll
-        for (int r = 0; r < RF; ++r) w[h][r] = *reinterpret_cast<const u32x4_t*>(b + r * 2048 + (h ? f0 ^ 64 : f0));
+        for (int r = 0; r < RF; ++r) w[h][r] = *reinterpret_cast<const u32x4_t*>(b + r * 2048 + (h ? fw ^ 64 : fw));
 #pragma unroll
-        for (int t = 0; t < TN; ++t) x[h][t] = *reinterpret_cast<const u32x4_t*>(b + (RF + t) * 2048 + (h ? f0 ^ 64 : f0));
+        for (int t = 0; t < TN; ++t) x[h][t] = *reinterpret_cast<const u32x4_t*>(b + WP * 1024 + t * 2048 + (h ? f0 ^ 64 : f0));
       }
 #pragma unroll
       for (int h = 0; h < 2; ++h)
@@ -401,7 +403,7 @@ __global__ __launch_bounds__(64 * WV, 2) void linear_stream_lds_kernel(LinArgs a
       else { f2 = f + RF / 2 * TF; l2 = l; }
     }
     const int t = (f % TF) * 16 + (l & 15), n = n0 + (f / TF) * 16 + (l >> 4) * 4;
-    if (t >= count) continue;
+    if (t >= count || (ROWS == 8 && l >= 32)) continue;
     auto sum = [&](int ff, int ll) {
       f32x4_t v = red[ff * 64 + ll];
 #pragma unroll
@@ -415,9 +417,9 @@ __global__ __launch_bounds__(64 * WV, 2) void linear_stream_lds_kernel(LinArgs a
 template <int ROWS, int TF, bool SEG, bool GATED>
 int launch_stream_lds_tf(const LinArgs& a, int groups, hipStream_t s) {
   // two workgroups per CU where two blocks per wave fit half of its LDS, else one
-  constexpr int WV = STREAM_LDS_WAVES, PER = 2 * (ROWS / 16 + TF), LDS_KB = ROWS < 64 && WV * 2 * PER <= 80 ? 80 : 160;
+  constexpr int WV = STREAM_LDS_WAVES, PER = ROWS / 8 + 2 * TF, LDS_KB = ROWS < 64 && WV * 2 * PER <= 80 ? 80 : 160;
   constexpr int BY_LDS = LDS_KB / (WV * PER), BY_COUNT = 63 / PER + 1, D = BY_LDS < BY_COUNT ? BY_LDS : BY_COUNT, LDS = WV * D * PER * 1024;
-  static_assert(D >= 2 && LDS >= WV * (ROWS / 16) * TF * 1024, "two blocks, and room for the sums");
+  static_assert(D >= 2 && LDS >= WV * ((ROWS + 15) / 16) * TF * 1024, "two blocks, and room for the sums");
   auto kern = linear_stream_lds_kernel<ROWS, TF, WV, D, SEG, GATED>;
   if (LDS > 64 * 1024)
     DIHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS), DIHIP_RUNTIME_ERROR);
@@ -432,15 +434,19 @@ int launch_stream_lds(const LinArgs& a, int Tg, int groups, hipStream_t s) {
 }
 // weight rows per workgroup: more of them bring the activations less often, but the workgroups have to fill 256 CUs.  16 / 32 / 64, us: 24 rows 4096 -> 4096
 // 11.1 / 13.6 / 17.1, 2048 -> 8192 11.4 / 10.6 / 13.0, 4096 -> 14336 30.5 / 29.3 / 25.7, 4096 -> 32000 61 / 58 / 58 (64 rows of x: 88 / 74 / 63); 2 rows, whose
-// activations are cheap, 9.1 / 9.8 / 11.0, 23.7 / 27.4 / 24.8 and 47 / 56 / 55.  Four waves in each form: an element's sum is the same in all of them.
+// activations are cheap, 9.1 / 9.8 / 11.0, 23.7 / 27.4 / 24.8 and 47 / 56 / 55.  Up to 2048 columns, of which 16 a workgroup leave half of the CUs without one, 8 (in an operand
+// that holds them twice): 8 / 16, us, weights from memory: 8192 -> 2048 2 rows 9.1 / 11.1, 24 rows 12.7 / 15.0, 64 rows 20.5 / 22.4; 2048 -> 2048 5.7 / 6.1 at 24 rows; 4096 -> 1024
+// 7.6 / 8.6; but 2048 -> 3072 8.0 / 6.5.  9 .. 16 rows of 4096 and more: 16 / 32 / 64 at 13 rows 4096 -> 8192 16.1 / 17.3 / 17.7, 4096 -> 32000 51.0 / 55.9 / 55.9, but 2048 -> 6208
+// 8.7 / 8.2 / 10.0.  24 rows 4096 -> 12352 29.1 / 27.9 / 24.7, 2048 -> 32000 33.1 / 31.1 / 32.5.  Four waves in each form: an element's sum is the same in all of them.
 // Segments hold few rows each, whatever the bound: 16 / 32 / 64 at 2048 -> 2816 of 64 experts, 6 per token, 4 tokens 49.3 / 50.9 / 56.0, 48 tokens 135.8 / 135.6 /
 // 143.4; 2048 -> 4096 of 32, 4 per token, 4 tokens 45.7 / 43.1 / 41.4; 4096 -> 4096 of 32, 3 tokens 65.9 / 79.4 / 73.8, 48 tokens 183 / 205 / 210; 64 tokens through 2048 -> 2816
 // 138.6 / 154.9 / 149.9 (four row operands leave the 32 form one workgroup per CU).
 inline int launch_stream_lds_rows(const LinArgs& a, int Tg, int groups, hipStream_t s) {
   const long n = (long)a.N * groups;
   if (a.seg) return a.K < 4096 && Tg <= 48 ? launch_stream_lds<32, true>(a, Tg, groups, s) : launch_stream_lds<16, true>(a, Tg, groups, s);
-  if (n < 6144 || Tg <= 8) return launch_stream_lds<16, false>(a, Tg, groups, s);
-  return n < 13312 ? launch_stream_lds<32, false>(a, Tg, groups, s) : launch_stream_lds<64, false>(a, Tg, groups, s);
+  if (n <= 2048) return launch_stream_lds<8, false>(a, Tg, groups, s);
+  if (n < 6144 || Tg <= (a.K >= 4096 ? 16 : 8)) return launch_stream_lds<16, false>(a, Tg, groups, s);
+  return n < 12288 || (a.K <= 2048 && Tg <= 48) ? launch_stream_lds<32, false>(a, Tg, groups, s) : launch_stream_lds<64, false>(a, Tg, groups, s);
 }
 
 // The gated form has twice the weight rows of one product, so its lines lie elsewhere.  Two products / 16 / 32 / 64, us (weights from memory): 2048 -> 1408 24 rows 10.7 / 5.7 /
