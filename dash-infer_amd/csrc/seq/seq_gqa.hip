@@ -100,6 +100,104 @@ __global__ __launch_bounds__(256) void qkv_prep_append_kernel(PrepArgs a) {
   }
 }
 
+// The same for head sizes of 64 and 128 in rows of whole 16-byte pieces and bf16 pages: a lane holds four neighbouring elements of a head, 16 or 32 lanes a head, every operand is
+// read once and the heads of a wave are in flight together; no barrier after the token's table.  The kernel above, an element per lane and two barriers per four heads,
+// waited for every group's loads.  Bound by the rows' bytes: 2048 rows of 32 + 8 heads of 128 40 -> 24 us (3.5 TB/s), 513 rows of 16 + 4 11.4 -> 7.7; decoding, one group of heads
+// per wave, 4.9 and 5.0 (24 rows), 4.8 and 4.6 (one).
+// PREP_HEADS: the groups of heads a wave has in flight
+template <int D, int PREP_HEADS>
+__global__ __launch_bounds__(256) void qkv_prep_append_vec_kernel(PrepArgs a) {
+  constexpr int LPH = D / 4, HPW = 64 / LPH;   // lanes per head, heads per wave
+  __shared__ float cs_t[64], sn_t[64];
+  const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = lane % LPH, d0 = sub * 4;
+  const int pos = a.tok_pos[t], nh = a.H + a.G, half = a.rot_dims >> 1;
+  const size_t sp = (size_t)a.tok_slot[t] * a.span_stride + pos / a.span_len, in_span = (size_t)(pos % a.span_len);
+  float* row = a.qkv + (size_t)t * a.ld;
+  uint16_t* const kdst = (uint16_t*)a.kspans[sp];
+  uint16_t* const vdst = (uint16_t*)a.vspans[sp];
+  const int first = (blockIdx.y * 4 + wave) * HPW + lane / LPH, step = 4 * HPW * gridDim.y;
+  auto column = [&](int h) { return h < a.H ? a.q_off + h * D : a.k_off + (h - a.H) * D; };
+  f32x4_t v[PREP_HEADS];
+  auto load = [&](int h0) {
+#pragma unroll
+    for (int i = 0; i < PREP_HEADS; ++i) {
+      const int h = h0 + i * step;
+      v[i] = *reinterpret_cast<const f32x4_t*>(row + column(min(h, nh - 1)) + d0);   // (past the heads: the last one's, not used)
+    }
+  };
+  load(first);
+  f32x4_t gq = {1.f, 1.f, 1.f, 1.f}, gk = gq;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (a.qnorm) gq[r] = ld_any(a.qnorm, d0 + r, a.wdt);
+    if (a.knorm) gk[r] = ld_any(a.knorm, d0 + r, a.wdt);
+  }
+  if (threadIdx.x < half) {
+    float sn, cs;
+    rope_sincos((uint32_t)pos, a.freq[threadIdx.x], &sn, &cs);
+    cs_t[threadIdx.x] = cs * a.mag;
+    sn_t[threadIdx.x] = sn * a.mag;
+  }
+  __syncthreads();
+  const bool turned = d0 < a.rot_dims, low = d0 < half;   // (rot_dims is a multiple of 8: a lane's four turn together)
+  f32x4_t cs = {1.f, 1.f, 1.f, 1.f}, sn = {0.f, 0.f, 0.f, 0.f};
+  if (turned) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int pair = a.layout == 0 ? (d0 + r) >> 1 : low ? d0 + r : d0 + r - half;
+      cs[r] = cs_t[pair];
+      sn[r] = (a.layout == 0 ? (r & 1) == 0 : low) ? -sn_t[pair] : sn_t[pair];   // y = v cs +- other sn
+    }
+  }
+  const int other = a.layout == 0 || !turned ? lane : low ? lane + half / 4 : lane - half / 4;
+  const bool kwide = (reinterpret_cast<uintptr_t>(kdst) & 7) == 0, vwide = (reinterpret_cast<uintptr_t>(vdst) & 7) == 0;   // (uniform)
+  auto store = [&](uint16_t* to, const f32x4_t& x, bool wide) {
+    const uint32_t e[4] = {f32_to_bf16_bits(x[0]), f32_to_bf16_bits(x[1]), f32_to_bf16_bits(x[2]), f32_to_bf16_bits(x[3])};
+    if (wide) *reinterpret_cast<u32x2_t*>(to) = u32x2_t{e[0] | (e[1] << 16), e[2] | (e[3] << 16)};
+    else
+#pragma unroll
+      for (int r = 0; r < 4; ++r) to[r] = (uint16_t)e[r];
+  };
+  for (int h0 = first, base = (int)blockIdx.y * 4 * HPW; base < nh; h0 += PREP_HEADS * step, base += PREP_HEADS * step) {   // (uniform)
+    if (h0 != first) load(h0);
+#pragma unroll
+    for (int i = 0; i < PREP_HEADS; ++i) {
+      const int h = h0 + i * step;
+      const bool is_q = h < a.H;
+      f32x4_t x = v[i];
+      float ss = __builtin_fmaf(x[3], x[3], __builtin_fmaf(x[2], x[2], __builtin_fmaf(x[1], x[1], x[0] * x[0])));
+#pragma unroll
+      for (int m = 1; m < LPH; m *= 2) ss += __shfl_xor(ss, m, 64);
+      if (is_q ? a.qnorm != nullptr : a.knorm != nullptr) {
+        const float inv = 1.f / sqrtf(ss / (float)D + a.eps);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] = x[r] * inv * (is_q ? gq[r] : gk[r]);
+      }
+      f32x4_t o;
+      if (a.layout == 0) {
+        o = f32x4_t{x[1], x[0], x[3], x[2]};
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = __shfl(x[r], other, 64);
+      }
+      if (turned) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] = x[r] * cs[r] + o[r] * sn[r];
+      }
+      if (h >= nh) continue;
+      if (is_q) *reinterpret_cast<f32x4_t*>(row + column(h) + d0) = x;
+      else store(kdst + (in_span * a.G + (size_t)(h - a.H)) * D + d0, x, kwide);
+    }
+  }
+  const int nv = a.GV * a.DV;
+  for (int e = (blockIdx.y * 256 + threadIdx.x) * 4; e < nv; e += 1024 * gridDim.y) {
+    f32x4_t x = *reinterpret_cast<const f32x4_t*>(row + a.v_off + e);
+    if (a.vfirst_in) x = (1.f - a.lam) * x + a.lam * *reinterpret_cast<const f32x4_t*>(a.vfirst_in + (size_t)t * a.ldvf + e);
+    if (a.vfirst_out) *reinterpret_cast<f32x4_t*>(a.vfirst_out + (size_t)t * a.ldvf + e) = x;
+    store(vdst + in_span * nv + e, x, vwide);
+  }
+}
+
 // ------------------------------------------------------------------------------------------------ convolution + prep + append
 // u[c] = sum_j w[j, c] x[t - (taps - 1) + j, c] for the channels [q | k | v] of the rows x (inputs of earlier steps: the slot's tail), then
 // the query row and the key row as a whole are divided by their root mean square and weighted, their heads rotated; queries go to q_out,
@@ -931,6 +1029,16 @@ int dihip_qkv_prep_append(void* stream, float* qkv, long ld, int q_off, int k_of
   if (T == 0) return DIHIP_SUCCESS;
   PrepArgs a{qkv, ld, q_off, k_off, v_off, H, G, D, DV, GV, qnorm, knorm, w_dtype, eps, freq, rot_dims, layout, mag, lam, vfirst_in, vfirst_out,
              ldvf, kspans, vspans, span_stride, span_len, cache_dtype, tok_slot, tok_pos};
+  const auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+  if ((D == 64 || D == 128) && rot_dims % 8 == 0 && cache_dtype == DIHIP_BF16 && (GV * DV) % 4 == 0 && al16(qkv) && ((ld | q_off | k_off | v_off) & 3) == 0 &&
+      al16(vfirst_in) && al16(vfirst_out) && ((!vfirst_in && !vfirst_out) || ldvf % 4 == 0)) {
+    // few rows (decoding): a token's heads one to a lane group; many rows: a workgroup per token
+    const int per = 4 * 64 / (D / 4), gy = T >= 256 ? 1 : (H + G + per - 1) / per;
+    const auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(T, gy), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), a); };
+    if (D == 64) gy > 1 || per >= H + G ? go(qkv_prep_append_vec_kernel<64, 1>) : go(qkv_prep_append_vec_kernel<64, 4>);
+    else gy > 1 || per >= H + G ? go(qkv_prep_append_vec_kernel<128, 1>) : go(qkv_prep_append_vec_kernel<128, 4>);
+    return launch_status();
+  }
   // few rows (decoding): the heads of a token are spread over workgroups of four; many rows: a workgroup per token
   hipLaunchKernelGGL(qkv_prep_append_kernel, dim3(T, T >= 256 ? 1 : (H + G + 3) / 4), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), a);
   return launch_status();

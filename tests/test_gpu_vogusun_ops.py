@@ -80,6 +80,39 @@ def test_embedding_and_its_norm(so):
     assert torch.equal(x, want) and torch.equal(h16, so.add_dyt(want, norm=(0.7, w, b), want16=True)[1])
 
 
+# heads that do not fill a wave or the workgroups, one batch of heads per wave and several, each rotary layout over none, a part and all of the head, two maps, mixed values
+@pytest.mark.parametrize("D,V,H,G,maps", [(128, 128, 16, 4, 1), (64, 64, 4, 4, 1), (128, 36, 6, 2, 2), (64, 100, 70, 35, 1), (128, 128, 64, 8, 1)])
+@pytest.mark.parametrize("T", [1, 5, 300])
+@pytest.mark.parametrize("layout,part", [(0, 1.0), (0, 0.25), (1, 1.0), (1, 0.625), (0, 0.0)])
+def test_prep_in_whole_pieces(so, D, V, H, G, maps, T, layout, part):
+    """the kernel of rows in 16-byte pieces against the one of any rows (columns off by two): sums of squares in another order, everything else the same"""
+    from dash_infer_amd.seq_state import SequenceStateManager
+    rot = int(D * part)
+    freq = torch.rand(max(rot // 2, 1), device="cuda") if rot else None
+    nq, nk, nv = H * maps * D, G * maps * D, G * V
+    g = torch.Generator("cuda").manual_seed(D + T + H)
+    src = torch.randn(T, nq + nk + nv, generator=g, device="cuda")
+    norms = [torch.randn(D, generator=g, device="cuda").bfloat16() if T != 5 else None for _ in range(2)]
+    first = torch.randn(T, nv, generator=g, device="cuda") if T != 1 else None
+    outs = []
+    for off in (0, 2):
+        st = SequenceStateManager(512, 2, 64, "cuda")
+        kt, vt = st.add_span_cache("k", G * maps * D, torch.bfloat16), st.add_span_cache("v", nv, torch.bfloat16)
+        st.admit("a")
+        st.reserve("a", T)
+        st.upload()
+        rows = torch.zeros(T, nq + nk + nv + 4, device="cuda")
+        rows[:, off:off + src.shape[1]] = src
+        keep = torch.zeros(T, nv, device="cuda") if T == 1 else None
+        so.qkv_prep_append(rows, off, off + nq, off + nq + nk, H, G, D, V, norms[0], norms[1], 1e-5, freq, rot, layout, 1.1, 0.3 if T != 1 else 0.0, first, keep, kt, vt,
+                           i32([st.live["a"].index] * T), i32(list(range(T))), maps=maps)
+        outs.append((rows[:, off:off + src.shape[1]].clone(), kt.pool.pool.view(torch.bfloat16).float().clone(), vt.pool.pool.view(torch.bfloat16).float().clone(), keep))
+    (r0, k0, v0, f0), (r1, k1, v1, f1) = outs
+    assert rel_err(r0.cpu().numpy(), r1.cpu().numpy()) < 2e-6
+    assert rel_err(k0.cpu().numpy(), k1.cpu().numpy()) < 2.0 ** -8 and float(k0.abs().max()) > 0      # a rounding to bf16 that goes the other way
+    assert torch.equal(v0, v1) and (f0 is None or torch.equal(f0, f1))
+
+
 # ---------------------------------------------------------------------------------------------------------------- attention
 def attention_weights(rng, kind, width, H, G, D, V):
     r = lambda *s, sd=None: bf(rng.normal(0, sd if sd is not None else 1.0 / math.sqrt(s[-1]), s))
