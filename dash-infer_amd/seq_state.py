@@ -23,10 +23,11 @@ class SpanTable:
         self.pool = ops.SpanPool(num_spans, 1, span_len, row_elems, "none", dtype, device, nbytes=span_len * row_elems * esz)
         self.span_len, self.row_elems, self.dtype, self.max_spans = span_len, row_elems, dtype, max_spans
         self.host = torch.zeros(slots, max_spans, dtype=torch.int64, pin_memory=torch.cuda.is_available())
+        self.entries = self.host.numpy()     # the same memory: an entry is written in a tenth of the time
         self.ptrs = torch.zeros(slots, max_spans, dtype=torch.int64, device=device)
 
     def bind(self, slot, k, page):
-        self.host[slot, k] = self.pool.span_ptr(page)
+        self.entries[slot, k] = self.pool.span_ptr(page)
 
     def upload(self):
         self.ptrs.copy_(self.host, non_blocking=True)
@@ -58,6 +59,7 @@ class SequenceStateManager:
         self.tables = {}    # key -> SpanTable
         self.states = {}    # key -> f32 tensor [slots, ...]
         self._dirty = False
+        self._uploaded = None    # event behind the last upload: until then its copies may still read the host tables
 
     # -- what the layers register at load ---------------------------------------------------------------------------
     def add_span_cache(self, key, row_elems, dtype):
@@ -92,6 +94,9 @@ class SequenceStateManager:
         need = self.pages_for(new_length)
         if need - len(s.pages) > len(self.free_pages):
             raise RuntimeError(f"the cache pool is exhausted ({self.num_pages} pages of {self.span_len} positions)")
+        if len(s.pages) < need and self._uploaded is not None:
+            self._uploaded.synchronize()     # a host that runs ahead of the device must not change what an earlier step is still to read
+            self._uploaded = None
         while len(s.pages) < need:
             p = self.free_pages.popleft()
             for t in self.tables.values():
@@ -105,6 +110,9 @@ class SequenceStateManager:
             for t in self.tables.values():
                 t.upload()
             self._dirty = False
+            if torch.cuda.is_available():
+                self._uploaded = torch.cuda.Event()
+                self._uploaded.record()
 
     def release(self, rid):
         s = self.live.pop(rid)
