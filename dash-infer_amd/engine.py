@@ -89,12 +89,10 @@ class SeqEngine:
         if not rows2:
             rows2 = [0] * T
         flat = ids + rows2 + tslot + tpos + toff + eslot + erow0 + ecnt + want
-        host = torch.tensor(flat, dtype=torch.int32)
         cut = [T, T, T, T, T, E, E, E, len(want)]
         if self.use_graphs and taps is None and T == E and want == list(range(E)):
-            return self._decode_step(host, cut, T, max(tpos))
-        if torch.cuda.is_available():
-            host = host.pin_memory()
+            return self._decode_step(torch.tensor(flat, dtype=torch.int32), cut, T, max(tpos))
+        host = torch.tensor(flat, dtype=torch.int32, pin_memory=torch.cuda.is_available())
         # the split of the attention's key walk follows the length bucket, as in the captured decode steps: the same step gives the
         # same bits whether it is launched or replayed
         ctx = self._context(host.to(self.device, non_blocking=True), cut, T, E, max(ecnt), self._bucket(max(tpos)))

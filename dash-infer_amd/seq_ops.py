@@ -8,7 +8,7 @@ import ctypes as C
 
 import torch
 
-from . import seq_capi
+from . import ops, seq_capi
 from .seq_capi import ACT, MATH_BF16, MATH_F32, MATH_F32_STREAM, check, lib
 
 _DT = {torch.float32: seq_capi.F32, torch.bfloat16: seq_capi.BF16}
@@ -20,7 +20,7 @@ def dt(t):
 
 
 def stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ops.cur_stream()
 
 
 def ptr(t):
