@@ -667,6 +667,11 @@ class DecodeSession:
     # -- state ---------------------------------------------------------------------------
     def set_state(self, ids, lens):
         """ids: next input token per request; lens: tokens already in the cache."""
+        if all(isinstance(t, torch.Tensor) and t.device == self.ids.device and t.dtype == dt and t.shape == (self.B,) and t.is_contiguous()
+               for t, dt in ((ids, torch.int64), (lens, torch.int32))):
+            check(lib().dihip_decode_state(ops.cur_stream(), ops.ptr(self.ids), ops.ptr(self.old_lens), ops.ptr(self.new_lens), ops.ptr(ids), ops.ptr(lens), self.B),
+                  "dihip_decode_state")
+            return
         self.ids.copy_(torch.as_tensor(ids, dtype=torch.int64))
         lens = torch.as_tensor(lens, dtype=torch.int32)
         self.old_lens.copy_(lens)

@@ -594,6 +594,8 @@ int dihip_embedding(void* stream, float* h, const int64_t* ids, const void* tabl
  * valid row instead of faulting */
 int dihip_embedding_v(void* stream, float* h, const int64_t* ids, const void* table, int M, int K, int vocab,
                       int dtype);
+/* the state of a decoding step from device tensors: ids[b] = ids_in[b], old_lens[b] = lens_in[b], new_lens[b] = lens_in[b] + 1 */
+int dihip_decode_state(void* stream, int64_t* ids, uint32_t* old_lens, uint32_t* new_lens, const int64_t* ids_in, const int32_t* lens_in, int B);
 /* seq_lens[b] += 1 (device-side step counter for graph replay) */
 int dihip_increment_u32(void* stream, uint32_t* v, int count);
 /* Read-only prefetch of up to 8 buffers into the on-die Infinity Cache (no reference counterpart):

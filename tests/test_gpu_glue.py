@@ -79,3 +79,33 @@ def test_nan_logits_and_wild_ids_stay_in_range(ops):
     h = ops.embedding(wild, table)
     torch.cuda.synchronize()
     assert torch.equal(h[0], table[3].float()) and torch.equal(h[1], table[9].float()) and torch.equal(h[2], table[0].float())
+
+
+# row lengths that come in fours and not, fewer columns than threads, one batch of loads per thread and more; ties go to the first column
+@pytest.mark.parametrize("M,N", [(1, 4), (3, 1003), (2, 65536), (5, 65540), (33, 152064), (2, 300004), (2, 300001)])
+def test_argmax_at_the_edges_of_its_loads(M, N):
+    from dash_infer_amd import ops
+    g = torch.Generator("cuda").manual_seed(N)
+    logits = torch.randn(M, N, generator=g, device="cuda")
+    at = [0, N - 1, N // 2, 65535 % N, (N // 3) | 3]
+    for m in range(M):
+        logits[m, min(at[m % 5], N - 1)] = 9.0
+    assert torch.equal(ops.argmax(logits), torch.argmax(logits, -1))
+    logits[:, N - 1] = logits[:, N // 2] = 12.0
+    assert ops.argmax(logits).tolist() == [N // 2] * M
+    logits[0] = float("-inf")
+    assert int(ops.argmax(logits)[0]) == 0
+
+
+@pytest.mark.parametrize("B", [1, 64, 65])
+def test_decode_state_from_device_tensors(B):
+    """set_state of a session: the same state from device tensors (one launch) as from host values"""
+    from types import SimpleNamespace
+    from dash_infer_amd import decoder
+    ids, lens = torch.randint(0, 1 << 40, (B,), device="cuda"), torch.randint(0, 1 << 20, (B,), device="cuda", dtype=torch.int32)
+    got = []
+    for a, b in ((ids, lens), (ids.cpu(), lens.tolist())):
+        s = SimpleNamespace(B=B, ids=torch.zeros(B, dtype=torch.int64, device="cuda"), **{k: torch.zeros(B, dtype=torch.int32, device="cuda") for k in ("old_lens", "new_lens")})
+        decoder.DecodeSession.set_state(s, a, b)
+        got.append((s.ids.tolist(), s.old_lens.tolist(), s.new_lens.tolist()))
+    assert got[0] == got[1] == (ids.tolist(), lens.tolist(), (lens + 1).tolist())
