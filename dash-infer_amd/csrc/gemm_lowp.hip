@@ -502,14 +502,16 @@ static PanelPlan make_panel_plan(int wbits, int M, int N, int K, int group_size,
 // DIHIP_PREFILL_TAIL_SPLIT=0: off.
 struct PrefillTail {
   int col_blocks, mblocks, tail_cb, ksplit, kunit;
+  int bm;   // rows of a workgroup
   size_t slab_bytes;
 };
-static PrefillTail prefill_tail_plan(int wbits, int M, int N, int K, int group_size, bool dual) {
+static PrefillTail prefill_tail_plan_rows(int wbits, int M, int N, int K, int group_size, bool dual, int bm) {
   PrefillTail t{};
+  t.bm = bm;
   const LowpDims d = lowp_dims(wbits, N, K, group_size);
   const int tpb = dual ? PF_WN * PF_CW / 2 : PF_WN * PF_CW;
   t.col_blocks = (d.NTILES + tpb - 1) / tpb;
-  t.mblocks = (M + PF_BM - 1) / PF_BM;
+  t.mblocks = (M + bm - 1) / bm;
   t.tail_cb = t.col_blocks;
   t.ksplit = 1;
   t.kunit = d.group ? std::max(d.group / d.KTILE, 1) : 1;  // K parts hold whole groups (per-channel: whole k-tiles)
@@ -534,8 +536,39 @@ static PrefillTail prefill_tail_plan(int wbits, int M, int N, int K, int group_s
   }
   t.tail_cb = t.col_blocks - tcb;
   t.ksplit = best;
-  t.slab_bytes = (size_t)tiles * best * PF_BM * 256 * sizeof(float);
+  t.slab_bytes = (size_t)tiles * best * bm * 256 * sizeof(float);
   return t;
+}
+// How many row tiles of 16 a workgroup takes, 5 .. 8: a k-tile costs the tiles' products and about 2.5 tiles' worth beside them (expansions, loads; 8 bits: 10, the expansions
+// of two k-steps), so rows past M are worth avoiding and a round more is not; a split costs its launch and the slab's way.  A fit to 224 products (64 .. 1024 rows, int4 and int8,
+// 1536 .. 37888 columns) with 5, 6, 7 and 8 tiles each: on average 0.2 % behind the best of the four, at worst 8 %, and 0.916 of the time of 8 (int4 3584 -> 18944 twice, us, 8 / chosen:
+// 64 rows 63 / 45, 150 rows 85 / 65, 326 rows 126 / 111, 513 rows 203 / 182; int8 326 rows 138 / 131).  An element's sum does not depend on it but through the K parts.
+static PrefillTail prefill_tail_plan(int wbits, int M, int N, int K, int group_size, bool dual) {
+  PrefillTail best = prefill_tail_plan_rows(wbits, M, N, K, group_size, dual, PF_BM);
+  if (M < 64 || M > 1024 || (wbits != 4 && wbits != 8)) return best;   // (past 1024 rows, where the fit ends, the last row tile is a small part)
+  int ncu = cached_num_cus();
+  if (ncu <= 0) ncu = 256;
+  const int KT = lowp_dims(wbits, N, K, group_size).KT;
+  const double tile_us = wbits == 4 ? 0.144 : 0.047, beside = wbits == 4 ? 2.5 : 10;   // of a k-tile and row tile; row tiles' worth beside the products
+  const auto cost = [&](const PrefillTail& t) {
+    int ktiles = (t.tail_cb * t.mblocks + ncu - 1) / ncu * KT;
+    double split_us = 0;
+    if (t.ksplit > 1) {
+      ktiles += (KT / t.kunit + t.ksplit - 1) / t.ksplit * t.kunit;
+      split_us = 4 + (double)(t.col_blocks - t.tail_cb) * t.ksplit * M * 256 * sizeof(float) / 4e6;
+    }
+    return ktiles * tile_us * (t.bm / 16 + beside) + split_us;
+  };
+  double least = cost(best);
+  for (int tr = PF_TR - 1; tr >= PF_TR_LEAST; --tr) {
+    const PrefillTail t = prefill_tail_plan_rows(wbits, M, N, K, group_size, dual, tr * 16);
+    const double c = cost(t);
+    if (c < least) {
+      best = t;
+      least = c;
+    }
+  }
+  return best;
 }
 
 // ---- batched decode, FRAG32 activations, register-resident K-slices (gemm_kslice_kernel.hpp) ---------------------
@@ -937,8 +970,9 @@ static int run_gemm(hipStream_t stream, const GemmCall& c) {
     g.col_blocks = (d.NTILES + tiles_per_block - 1) / tiles_per_block;
     g.tail_cb = g.col_blocks;
     g.ksplit = g.kunit = 1;
-    int blocks = g.col_blocks * ((c.M + PF_BM - 1) / PF_BM);
     const PrefillTail pt = prefill_tail_plan(c.wbits, c.M, c.N, c.K, c.group_size, dual);
+    g.bm = pt.bm;
+    int blocks = g.col_blocks * pt.mblocks;
     const bool far = pf_row * PF_BM > pf_reach;  // rows of 16 MiB and more: as many of them at a time as are within reach
     if (!far && pt.ksplit > 1 && c.ws && c.ws_bytes >= pt.slab_bytes && reinterpret_cast<uintptr_t>(c.ws) % 16 == 0) {
       g.tail_cb = pt.tail_cb;
@@ -951,7 +985,10 @@ static int run_gemm(hipStream_t stream, const GemmCall& c) {
     g.wide_out = c.N % 4 == 0 && (c.epi == EPI_ADDTO ? aligned(c.h_res, 16) && aligned(c.h_out, 16) : aligned(c.y, 8) && aligned(c.residual, 8));
     const bool gpt = g.ktpg == 1;
     const int rows = far ? (int)(pf_reach / pf_row) : c.M;
-    if (far) blocks = g.col_blocks;
+    if (far) {
+      blocks = g.col_blocks;
+      g.bm = PF_BM;
+    }
     hipError_t e = hipErrorInvalidValue;
     for (int m = 0; m < c.M; m += rows) {
       if (m > 0) {

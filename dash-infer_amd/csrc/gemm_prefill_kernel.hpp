@@ -6,11 +6,11 @@
 // the reference's dequantise + cuBLAS fall-back and its 16816 tensor-core kernels (gemm_a16w8_kernel.h:239-331,
 // hgemm_a16w4_subc_32x256x32, gemm_a16w4_subc_kernel.cu:466-815):
 //
-//   * workgroup tile 128 rows x 256 columns (8 waves side by side in N, each 128 x 32 = 8 row tiles x 2 column tiles of
+//   * workgroup tile 128 rows (or 112, 96, 80: TR) x 256 columns (8 waves side by side in N, each 128 x 32 = 8 row tiles x 2 column tiles of
 //     v_mfma_f32_16x16x32: 16 accumulators), K walked in packed k-tiles (W4: 128 k, W8: 64 k);
 //   * A (activations, FT row-major) goes straight from memory into LDS (global_load_lds: no registers, no instructions for staging),
 //     double-buffered: the loads of k-tile t + 1 are in flight while t is multiplied, ONE barrier per k-tile; every wave reads all
-//     8 row tiles;
+//     row tiles;
 //   * B (weights) never touches LDS: "dihip tile-major" packing makes a lane's 16-byte load the B fragment of its own column
 //     tile (x KSTEPS), and no two waves share a column tile;
 //   * the same exact-integer arithmetic as the decode kernels: q expands to 128 + q in FT with the magic-number trick, the MFMA
@@ -43,13 +43,13 @@ namespace dihip {
 
 constexpr int PF_WAVES = 8;
 constexpr int PF_THREADS = PF_WAVES * 64;
-constexpr int PF_BM = 128;           // rows per workgroup (8 row tiles)
+constexpr int PF_BM = 128;           // rows per workgroup at most (8 row tiles; PrefillArgs::bm, the kernel's TR: how many it takes)
 constexpr int PF_WM = 1;             // waves along M
 constexpr int PF_WN = PF_WAVES / PF_WM;
-constexpr int PF_TR = PF_BM / 16;    // row tiles of the workgroup (= waves: wave w stages row tile w)
-constexpr int PF_RT = PF_TR / PF_WM; // row tiles per wave
+constexpr int PF_TR = PF_BM / 16;    // row tiles of the workgroup at most (= waves: wave w stages row tile w)
+constexpr int PF_TR_LEAST = 5;       // ... and at least
 constexpr int PF_CW = 2 * PF_WM;     // column tiles per wave (the workgroup covers 256 columns either way)
-static_assert(PF_TR == PF_WAVES, "one staged row tile per wave");
+static_assert(PF_TR == PF_WAVES && PF_WM == 1, "one staged row tile per wave, every wave all of them");
 static_assert(PF_CW == 2, "the two column tiles of a wave are named one by one where the sums change hands");
 
 struct PrefillArgs {
@@ -73,6 +73,7 @@ struct PrefillArgs {
   int Gp;      // (scale, zero) groups stored per tile
   int ktpg;    // k-tiles per quantisation group (per-channel: >= KT)
   int col_blocks;
+  int bm;      // rows per workgroup: 16 * TR of the kernel
   // Split in K: column blocks [tail_cb, col_blocks) -- the workgroups that would otherwise run as a last, mostly empty
   // round on the chip (qkv of Qwen2-7B at 2048 rows: 288 tiles on 256 CUs), or all of them where the whole grid fills at most half
   // of it (short prompts) -- are walked by `ksplit` workgroups each, one K range apiece (whole quantisation groups; the ranges
@@ -82,17 +83,18 @@ struct PrefillArgs {
   int ksplit;
   int kunit;    // k-tiles that a K range must not cut (grouped weights: a group; per-channel: 1)
   int wide_out; // four neighbouring columns of an output (and residual) row make one aligned access
-  float* slab;  // [tail tile][ksplit][PF_BM][256] f32
+  float* slab;  // [tail tile][ksplit][bm][256] f32
 };
 
-template <int WBITS>
+template <int WBITS, int TR>
 constexpr size_t prefill_lds_bytes() {
-  // 2 x A tile (128 rows x KSTEPS x 64 bytes) + 2 x 128 row sums
-  return (size_t)2 * PF_TR * WTraits<WBITS>::KSTEPS * 1024 + 2 * PF_BM * sizeof(float);
+  // 2 x A tile (16 TR rows x KSTEPS x 64 bytes) + 2 x 128 row sums
+  return (size_t)2 * TR * WTraits<WBITS>::KSTEPS * 1024 + 2 * PF_BM * sizeof(float);
 }
 
 // (GPT -- one k-tile per quantisation group -- is a compile-time copy of the same code: the group test folds away)
-template <int WBITS, int FT, int EPI, int GPT>
+// TR: row tiles of a workgroup, 5 .. 8 (gemm_lowp.hip: prefill_tail_plan).  Rows past M cost what the others do: 326 rows are three tiles of 112 as well as three of 128
+template <int WBITS, int FT, int EPI, int GPT, int TR>
 __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const PrefillArgs a) {
   using WT = WTraits<WBITS>;
   using EX = ExpandV<WBITS, FT>;
@@ -100,7 +102,8 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
   constexpr int KTILE = WT::KTILE;
   constexpr bool DUAL = EPI == EPI_SWIGLU;
   constexpr bool LACE = GPT && WBITS == 4;  // fix-up under the first k-step's products (8 bits: two k-steps, no registers left for it)
-  constexpr size_t ABYTES = (size_t)PF_TR * KSTEPS * 1024;  // one A tile
+  constexpr int PF_RT = TR, BM = 16 * TR;
+  constexpr size_t ABYTES = (size_t)TR * KSTEPS * 1024;  // one A tile
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   float* xsum = reinterpret_cast<float*>(smem + 2 * ABYTES);  // [2][PF_BM]
 
@@ -109,7 +112,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
   const int ni = lane & 15, kb = lane >> 4;
   const int wm = wave / PF_WN, wn = wave - wm * PF_WN;  // this wave's place in the PF_WM x PF_WN grid
   // consecutive workgroups share a column block (its weights stay hot in the L2s) and walk the rows
-  const int mblocks = (a.M + PF_BM - 1) / PF_BM;
+  const int mblocks = (a.M + BM - 1) / BM;
   int cb = blockIdx.x / mblocks, mb = blockIdx.x - cb * mblocks;
   int kt0 = 0, kt1 = a.KT, split_part = -1, split_tile = 0;  // this workgroup's k-tiles; tail split: its part and tile
   if (cb >= a.tail_cb) {  // (uniform) mb fastest, then the K part, then the column block: the 16 row blocks of a part share its weights
@@ -124,7 +127,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
     kt1 = split_part + 1 == a.ksplit ? a.KT : (split_part + 1) * units / a.ksplit * ku;
     split_tile = cbt * mblocks + mb;
   }
-  const int m0 = mb * PF_BM;
+  const int m0 = mb * BM;
 
   // ---- this wave's column tiles -------------------------------------------------------------------
   // STD / ADDTO: PF_CW consecutive tiles of the one matrix;  SwiGLU: PF_CW / 2 tiles of gate (c < PF_CW / 2) and the same of up
@@ -146,7 +149,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
   // ---- A: wave w brings row tile w straight into LDS (global_load_lds: no registers, no instructions for staging), pieces of 8 rows x 128
   // bytes; the 16-byte chunks of a row change places on the memory side (chunk ^ row % 8): 8 consecutive lanes of an operand read then
   // touch every bank once.  Rows past M re-read the last row (masked on store)
-  constexpr int HALVES = KTILE / 64;                       // 64 k of 128 rows: 16 KiB
+  constexpr int HALVES = KTILE / 64;                       // 64 k of all rows: TR * 2 KiB
   const int prow = lane >> 3, pchunk = (lane & 7) ^ prow;
   const char* abase = reinterpret_cast<const char*>(a.x) + (size_t)m0 * a.ldx * 2;
   uint32_t aoff[2];
@@ -154,12 +157,13 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
   for (int p = 0; p < 2; ++p) aoff[p] = (uint32_t)((size_t)min(wave * 16 + p * 8 + prow, a.M - 1 - m0) * a.ldx * 2 + pchunk * 16);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem + wave * 2048;
   auto load_a = [&](int kt, int buf) {
+    if (TR < PF_TR && wave >= TR) return;   // (uniform)
     const char* src = abase + (size_t)kt * KTILE * 2;
 #pragma unroll
     for (int hh = 0; hh < HALVES; ++hh)
 #pragma unroll
       for (int p = 0; p < 2; ++p)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds0 + (uint32_t)(buf * ABYTES) + hh * 16384 + p * 1024),
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds0 + (uint32_t)(buf * ABYTES) + hh * (TR * 2048) + p * 1024),
                      "v"(aoff[p]), "s"(src + hh * 128) : "memory");
   };
   u32x4_t wreg[PF_CW];
@@ -169,9 +173,10 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
     for (int c = 0; c < PF_CW; ++c) wreg[c] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(wp[c], lane * 16, kt * 1024, 2));   // (2: nontemporal)
   };
   // operand (row ni of a row tile, 16 bytes kb of k-step ks)
+  const int mine = TR < PF_TR ? min(wave, TR - 1) : wave;   // the row tile whose sums this wave takes (the last one's more than once)
   const int f0 = ni * 128 + ((kb ^ (ni & 7)) * 16), f1 = f0 ^ 64;
   auto aread = [&](const unsigned char* tile, int rt, int ks) {
-    return *reinterpret_cast<const u32x4_t*>(tile + (ks >> 1) * 16384 + rt * 2048 + ((ks & 1) ? f1 : f0));
+    return *reinterpret_cast<const u32x4_t*>(tile + (ks >> 1) * (TR * 2048) + rt * 2048 + ((ks & 1) ? f1 : f0));
   };
 
   // acc: exact integer products of the running quantisation group (MFMA); tot: the scaled result.  The weights are the first operand: lane
@@ -255,7 +260,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
     if constexpr (LACE) xv = xs[0];
 #pragma unroll
     for (int rt = 0; rt < PF_RT; ++rt) af[rt] = aread(tile, wm * PF_RT + rt, 0);
-    own = aread(tile, wave, 0);
+    own = aread(tile, mine, 0);
 #pragma unroll
     for (int c = 0; c < PF_CW; ++c) bf[c] = EX::frag(wcur[c], 0, ex_mask, ex_magic);
     f32x4_t sx = zero4;
@@ -277,7 +282,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
         if (ks + 1 < KSTEPS) af[rt] = aread(tile, wm * PF_RT + rt, ks + 1);
         if (rt == 2) {
           sx = mfma16<FT>(ones, own, sx);
-          if (ks + 1 < KSTEPS) own = aread(tile, wave, ks + 1);
+          if (ks + 1 < KSTEPS) own = aread(tile, mine, ks + 1);
         }
         if (ks + 1 < KSTEPS && rt >= PF_RT - 1 - PF_CW && rt < PF_RT - 1) bn[rt - (PF_RT - 1 - PF_CW)] = EX::frag(wcur[rt - (PF_RT - 1 - PF_CW)], ks + 1, ex_mask, ex_magic);
         __builtin_amdgcn_sched_barrier(0);
@@ -290,7 +295,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
     kstep(0, std::integral_constant<bool, LACE>{});
 #pragma unroll
     for (int ks = 1; ks < KSTEPS; ++ks) kstep(ks, std::false_type{});
-    if (kb == 0) {   // the lane with kb == 0 of a row's lanes owns its entry: no race
+    if (kb == 0 && (TR == PF_TR || wave < TR)) {   // the lane with kb == 0 of a row's lanes owns its entry: no race
       float* p = xsum + (grp & 1) * PF_BM + wave * 16 + ni;
       *p = GPT || gl == 0 ? sx[0] : *p + sx[0];
     }
@@ -313,7 +318,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
 
   // ---- split in K: this part's f32 tile to the slab (rows / columns of the workgroup tile; SwiGLU: gate columns, then up) ----
   if (split_part >= 0) {  // (uniform)
-    float* st = a.slab + ((size_t)split_tile * a.ksplit + split_part) * (PF_BM * 256) + (size_t)(wm * PF_RT * 16 + ni) * 256;
+    float* st = a.slab + ((size_t)split_tile * a.ksplit + split_part) * (BM * 256) + (size_t)(wm * PF_RT * 16 + ni) * 256;
 #pragma unroll
     for (int rt = 0; rt < PF_RT; ++rt) {
       if (m0 + (wm * PF_RT + rt) * 16 >= a.M) break;  // (uniform) rows past M are never read
@@ -328,7 +333,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
   // ---- epilogue: lane (kb, ni) holds row rt * 16 + ni, columns kb * 4 .. + 3 of column tile c.  Through buffer accesses whose bounds drop what
   // lies past M and N: no branch per element, the exponentials and divisions of neighbours overlap (with a branch around every
   // element they ran one after the other: the epilogue was 15 % of the gate / up pair's time) ----
-  const int rows = min(PF_BM, a.M - m0);
+  const int rows = min(BM, a.M - m0);
   const bool wide = a.wide_out != 0;   // (uniform) four columns of a row are one aligned access
   constexpr int OB = EPI == EPI_ADDTO ? 4 : 2;
   const int ldo = EPI == EPI_ADDTO ? a.N : a.ldy;
@@ -417,20 +422,20 @@ template <int FT, int EPI>
 __global__ __launch_bounds__(256) void gemm_prefill_tail_reduce_kernel(const PrefillArgs a) {
   constexpr bool DUAL = EPI == EPI_SWIGLU;
   constexpr int NC = DUAL ? 128 : 256;  // output columns of a workgroup tile
-  constexpr int PITCH = PF_BM * 256;
-  const int mblocks = (a.M + PF_BM - 1) / PF_BM;
+  const int pitch = a.bm * 256;
+  const int mblocks = (a.M + a.bm - 1) / a.bm;
   const size_t total = (size_t)(a.col_blocks - a.tail_cb) * a.M * (NC / 4);
   for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < total; e += (size_t)gridDim.x * 256) {
     const int col = (int)(e % (NC / 4)) * 4;
     const size_t q = e / (NC / 4);
-    const int cbt = (int)(q / a.M), m = (int)(q - (size_t)cbt * a.M), mb = m / PF_BM, row = m - mb * PF_BM;
+    const int cbt = (int)(q / a.M), m = (int)(q - (size_t)cbt * a.M), mb = m / a.bm, row = m - mb * a.bm;
     const int n0 = (a.tail_cb + cbt) * NC + col;
     if (n0 >= a.N) continue;
-    const float* st = a.slab + (size_t)(cbt * mblocks + mb) * a.ksplit * PITCH + (size_t)row * 256 + col;
+    const float* st = a.slab + (size_t)(cbt * mblocks + mb) * a.ksplit * pitch + (size_t)row * 256 + col;
     f32x4_t v4 = {0.f, 0.f, 0.f, 0.f}, u4 = v4;
     for (int s = 0; s < a.ksplit; ++s) {
-      v4 += *reinterpret_cast<const f32x4_t*>(st + (size_t)s * PITCH);
-      if constexpr (DUAL) u4 += *reinterpret_cast<const f32x4_t*>(st + (size_t)s * PITCH + 128);
+      v4 += *reinterpret_cast<const f32x4_t*>(st + (size_t)s * pitch);
+      if constexpr (DUAL) u4 += *reinterpret_cast<const f32x4_t*>(st + (size_t)s * pitch + 128);
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -456,30 +461,39 @@ __global__ __launch_bounds__(256) void gemm_prefill_tail_reduce_kernel(const Pre
 template <int WBITS, int FT, int EPI, int GPT>
 hipError_t launch_gemm_prefill(const PrefillArgs& a, int blocks, hipStream_t stream);
 
-#define DIHIP_DEFINE_PREFILL_LAUNCH(WBITS, FT, EPI, GPT)                                                           \
-  template <>                                                                                                      \
-  hipError_t launch_gemm_prefill<WBITS, FT, EPI, GPT>(const PrefillArgs& a, int blocks, hipStream_t s) {           \
-    auto kern = gemm_prefill_kernel<WBITS, FT, EPI, GPT>;                                                          \
-    constexpr size_t lds = prefill_lds_bytes<WBITS>();                                                             \
-    if (lds > 64 * 1024) {  /* the grant is per DEVICE: once per device of this process */           \
-      static std::atomic<unsigned> granted_mask[4];  /* 128 device ids */                                          \
-      int dev = 0;                                                                                                 \
-      if (hipGetDevice(&dev) != hipSuccess) return hipGetLastError();                                              \
-      const unsigned bit = 1u << (dev & 31);                                                                       \
-      std::atomic<unsigned>* word = dev >= 0 && dev < 128 ? &granted_mask[dev >> 5] : nullptr;                     \
-      if (!word || !(word->load(std::memory_order_acquire) & bit)) {                                               \
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                              \
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);           \
-        if (e != hipSuccess) return e;                                                                             \
-        if (word) word->fetch_or(bit, std::memory_order_release);                                                  \
-      }                                                                                                            \
-    }                                                                                                              \
-    hipLaunchKernelGGL(kern, dim3(blocks), dim3(PF_THREADS), lds, s, a);                                           \
-    if (a.tail_cb < a.col_blocks) {                                                                                \
-      const size_t quads = (size_t)(a.col_blocks - a.tail_cb) * a.M * (EPI == EPI_SWIGLU ? 32 : 64);               \
-      hipLaunchKernelGGL((gemm_prefill_tail_reduce_kernel<FT, EPI>), dim3((unsigned)std::min<size_t>((quads + 255) / 256, 4096)), dim3(256), 0, s, a); \
-    }                                                                                                              \
-    return hipGetLastError();                                                                                      \
+template <int WBITS, int FT, int EPI, int GPT, int TR>
+hipError_t launch_gemm_prefill_rows(const PrefillArgs& a, int blocks, hipStream_t s) {
+  auto kern = gemm_prefill_kernel<WBITS, FT, EPI, GPT, TR>;
+  constexpr size_t lds = prefill_lds_bytes<WBITS, TR>();
+  if (lds > 64 * 1024) {  // the grant is per device: once per device of this process
+    static std::atomic<unsigned> granted_mask[4];  // 128 device ids
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return hipGetLastError();
+    const unsigned bit = 1u << (dev & 31);
+    std::atomic<unsigned>* word = dev >= 0 && dev < 128 ? &granted_mask[dev >> 5] : nullptr;
+    if (!word || !(word->load(std::memory_order_acquire) & bit)) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (e != hipSuccess) return e;
+      if (word) word->fetch_or(bit, std::memory_order_release);
+    }
+  }
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(PF_THREADS), lds, s, a);
+  if (a.tail_cb < a.col_blocks) {
+    const size_t quads = (size_t)(a.col_blocks - a.tail_cb) * a.M * (EPI == EPI_SWIGLU ? 32 : 64);
+    hipLaunchKernelGGL((gemm_prefill_tail_reduce_kernel<FT, EPI>), dim3((unsigned)std::min<size_t>((quads + 255) / 256, 4096)), dim3(256), 0, s, a);
+  }
+  return hipGetLastError();
+}
+
+#define DIHIP_DEFINE_PREFILL_LAUNCH(WBITS, FT, EPI, GPT)                                                                \
+  template <>                                                                                                           \
+  hipError_t launch_gemm_prefill<WBITS, FT, EPI, GPT>(const PrefillArgs& a, int blocks, hipStream_t s) {                \
+    switch (a.bm / 16) {                                                                                                \
+      case 5: return launch_gemm_prefill_rows<WBITS, FT, EPI, GPT, 5>(a, blocks, s);                                    \
+      case 6: return launch_gemm_prefill_rows<WBITS, FT, EPI, GPT, 6>(a, blocks, s);                                    \
+      case 7: return launch_gemm_prefill_rows<WBITS, FT, EPI, GPT, 7>(a, blocks, s);                                    \
+      default: return launch_gemm_prefill_rows<WBITS, FT, EPI, GPT, 8>(a, blocks, s);                                   \
+    }                                                                                                                   \
   }
 
 #define DIHIP_DEFINE_PREFILL_LAUNCH_SET(WBITS, FT)          \

@@ -668,6 +668,14 @@ def test_prefill_gemm_all_epilogues(ops, M, N, K, wbits, G):
     assert_close(act.float().cpu().numpy(), bf16_round(((g / (1 + np.exp(-g))) * u).astype(np.float32)), "bf16", what="prefill SwiGLU")
 
 
+# Workgroups of 5, 6, 7 and 8 row tiles (the plan's choice for so many columns on 256 CUs): rows that fill the last tile and one more.
+@pytest.mark.gpu
+@pytest.mark.parametrize("wbits,G", [(4, 128), (4, -1), (8, -1), (8, 64)])
+@pytest.mark.parametrize("M", [65, 80, 81, 96, 97, 112, 113])
+def test_prefill_gemm_row_tiles(ops, M, wbits, G):
+    test_prefill_gemm_all_epilogues(ops, M, 20008, 256, wbits, G)
+
+
 # ------------------------------------------------------------------------------------------------------------------
 # Context-phase GEMM, tail split (gemm_prefill_kernel.hpp, PrefillArgs::tail_cb): shapes whose grid of 128 x 256 tiles ends in a
 # round that fills at most half of the chip -- the column blocks of that round are split in K and added by a reduction launch.
