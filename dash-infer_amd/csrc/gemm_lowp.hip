@@ -514,7 +514,7 @@ static PrefillTail prefill_tail_plan_rows(int wbits, int M, int N, int K, int gr
   t.mblocks = (M + bm - 1) / bm;
   t.tail_cb = t.col_blocks;
   t.ksplit = 1;
-  t.kunit = d.group ? std::max(d.group / d.KTILE, 1) : 1;  // K parts hold whole groups (per-channel: whole k-tiles)
+  t.kunit = d.group ? std::max(d.group / d.KTILE, 1) : wbits == 8 ? 2 : 1;  // K parts hold whole groups (per-channel: what the kernel walks between two barriers)
   static const bool on = !env_off("DIHIP_PREFILL_TAIL_SPLIT");
   int ncu = cached_num_cus();
   if (ncu <= 0) ncu = 256;
@@ -539,17 +539,17 @@ static PrefillTail prefill_tail_plan_rows(int wbits, int M, int N, int K, int gr
   t.slab_bytes = (size_t)tiles * best * bm * 256 * sizeof(float);
   return t;
 }
-// How many row tiles of 16 a workgroup takes, 5 .. 8: a k-tile costs the tiles' products and about 2.5 tiles' worth beside them (expansions, loads; 8 bits: 10, the expansions
-// of two k-steps), so rows past M are worth avoiding and a round more is not; a split costs its launch and the slab's way.  A fit to 224 products (64 .. 1024 rows, int4 and int8,
+// How many row tiles of 16 a workgroup takes, 5 .. 8: a k-tile costs the tiles' products and about 2.5 tiles' worth beside them (expansions, loads, waits; 8 bits,
+// half as long a k-tile: 8), so rows past M are worth avoiding and a round more is not; a split costs its launch and the slab's way.  A fit to 224 products (64 .. 1024 rows, int4 and int8,
 // 1536 .. 37888 columns) with 5, 6, 7 and 8 tiles each: on average 0.2 % behind the best of the four, at worst 8 %, and 0.916 of the time of 8 (int4 3584 -> 18944 twice, us, 8 / chosen:
-// 64 rows 63 / 45, 150 rows 85 / 65, 326 rows 126 / 111, 513 rows 203 / 182; int8 326 rows 138 / 131).  An element's sum does not depend on it but through the K parts.
+// 64 rows 63 / 45, 150 rows 85 / 65, 326 rows 126 / 111, 513 rows 203 / 182; int8 64 rows 66 / 52, 326 rows 133 / 121).  An element's sum does not depend on it but through the K parts.
 static PrefillTail prefill_tail_plan(int wbits, int M, int N, int K, int group_size, bool dual) {
   PrefillTail best = prefill_tail_plan_rows(wbits, M, N, K, group_size, dual, PF_BM);
   if (M < 64 || M > 1024 || (wbits != 4 && wbits != 8)) return best;   // (past 1024 rows, where the fit ends, the last row tile is a small part)
   int ncu = cached_num_cus();
   if (ncu <= 0) ncu = 256;
   const int KT = lowp_dims(wbits, N, K, group_size).KT;
-  const double tile_us = wbits == 4 ? 0.144 : 0.047, beside = wbits == 4 ? 2.5 : 10;   // of a k-tile and row tile; row tiles' worth beside the products
+  const double tile_us = wbits == 4 ? 0.144 : 0.05, beside = wbits == 4 ? 2.5 : 8;   // of a k-tile and row tile; row tiles' worth beside the products
   const auto cost = [&](const PrefillTail& t) {
     int ktiles = (t.tail_cb * t.mblocks + ncu - 1) / ncu * KT;
     double split_us = 0;

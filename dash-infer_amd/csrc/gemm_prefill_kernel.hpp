@@ -7,7 +7,8 @@
 // hgemm_a16w4_subc_32x256x32, gemm_a16w4_subc_kernel.cu:466-815):
 //
 //   * workgroup tile 128 rows (or 112, 96, 80: TR) x 256 columns (8 waves side by side in N, each 128 x 32 = 8 row tiles x 2 column tiles of
-//     v_mfma_f32_16x16x32: 16 accumulators), K walked in packed k-tiles (W4: 128 k, W8: 64 k);
+//     v_mfma_f32_16x16x32: 16 accumulators), K walked in packed k-tiles (W4: 128 k, W8: 64 k, two of them where no group
+//     ends in between);
 //   * A (activations, FT row-major) goes straight from memory into LDS (global_load_lds: no registers, no instructions for staging),
 //     double-buffered: the loads of k-tile t + 1 are in flight while t is multiplied, ONE barrier per k-tile; every wave reads all
 //     row tiles;
@@ -86,24 +87,27 @@ struct PrefillArgs {
   float* slab;  // [tail tile][ksplit][bm][256] f32
 };
 
-template <int WBITS, int TR>
+template <int WBITS, int TR, int UK>
 constexpr size_t prefill_lds_bytes() {
-  // 2 x A tile (16 TR rows x KSTEPS x 64 bytes) + 2 x 128 row sums
-  return (size_t)2 * TR * WTraits<WBITS>::KSTEPS * 1024 + 2 * PF_BM * sizeof(float);
+  // 2 x A tile (16 TR rows x UK KSTEPS x 64 bytes) + 2 x 128 row sums
+  return (size_t)2 * TR * UK * WTraits<WBITS>::KSTEPS * 1024 + 2 * PF_BM * sizeof(float);
 }
 
 // (GPT -- one k-tile per quantisation group -- is a compile-time copy of the same code: the group test folds away)
 // TR: row tiles of a workgroup, 5 .. 8 (gemm_lowp.hip: prefill_tail_plan).  Rows past M cost what the others do: 326 rows are three tiles of 112 as well as three of 128
-template <int WBITS, int FT, int EPI, int GPT, int TR>
+// UK: k-tiles between two barriers.  8 bits: two where no group ends between them; of one with its two k-steps the wait, the first operand reads and the expansions before the first
+// product were more than half of the time.  int8 per channel, 326 rows 3584 -> 18944 twice 131.7 -> 121.2 us, 18944 -> 3584 74.3 -> 66.7, 64 rows 59.4 -> 51.0 and 37.5 -> 35.1
+template <int WBITS, int FT, int EPI, int GPT, int TR, int UK>
 __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const PrefillArgs a) {
   using WT = WTraits<WBITS>;
   using EX = ExpandV<WBITS, FT>;
   constexpr int KSTEPS = WT::KSTEPS;
-  constexpr int KTILE = WT::KTILE;
+  constexpr int KTILE = WT::KTILE, NKS = UK * KSTEPS;   // (NKS: k-steps of an iteration)
+  static_assert(UK == 1 || !GPT, "a group of one k-tile ends in every one");
   constexpr bool DUAL = EPI == EPI_SWIGLU;
   constexpr bool LACE = GPT && WBITS == 4;  // fix-up under the first k-step's products (8 bits: two k-steps, no registers left for it)
   constexpr int PF_RT = TR, BM = 16 * TR;
-  constexpr size_t ABYTES = (size_t)TR * KSTEPS * 1024;  // one A tile
+  constexpr size_t ABYTES = (size_t)TR * NKS * 1024;  // one A tile
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   float* xsum = reinterpret_cast<float*>(smem + 2 * ABYTES);  // [2][PF_BM]
 
@@ -149,7 +153,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
   // ---- A: wave w brings row tile w straight into LDS (global_load_lds: no registers, no instructions for staging), pieces of 8 rows x 128
   // bytes; the 16-byte chunks of a row change places on the memory side (chunk ^ row % 8): 8 consecutive lanes of an operand read then
   // touch every bank once.  Rows past M re-read the last row (masked on store)
-  constexpr int HALVES = KTILE / 64;                       // 64 k of all rows: TR * 2 KiB
+  constexpr int HALVES = UK * KTILE / 64;                       // 64 k of all rows: TR * 2 KiB
   const int prow = lane >> 3, pchunk = (lane & 7) ^ prow;
   const char* abase = reinterpret_cast<const char*>(a.x) + (size_t)m0 * a.ldx * 2;
   uint32_t aoff[2];
@@ -158,19 +162,24 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem + wave * 2048;
   auto load_a = [&](int kt, int buf) {
     if (TR < PF_TR && wave >= TR) return;   // (uniform)
-    const char* src = abase + (size_t)kt * KTILE * 2;
 #pragma unroll
-    for (int hh = 0; hh < HALVES; ++hh)
+    for (int hh = 0; hh < HALVES; ++hh) {
+      const char* src = abase + (UK > 1 ? (size_t)min(kt + hh, a.KT - 1) * KTILE * 2 : (size_t)kt * KTILE * 2 + hh * 128);   // (past K: the last once more, times nothing)
 #pragma unroll
       for (int p = 0; p < 2; ++p)
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds0 + (uint32_t)(buf * ABYTES) + hh * (TR * 2048) + p * 1024),
-                     "v"(aoff[p]), "s"(src + hh * 128) : "memory");
+                     "v"(aoff[p]), "s"(src) : "memory");
+    }
   };
-  u32x4_t wreg[PF_CW];
+  static_assert(UK == 1 || KTILE == 64, "a half per k-tile");
+  u32x4_t wreg[UK][PF_CW];
   u32x4_t szreg[PF_CW] = {};   // the running group's, of this lane's four columns of each tile
   auto load_b = [&](int kt) {
 #pragma unroll
-    for (int c = 0; c < PF_CW; ++c) wreg[c] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(wp[c], lane * 16, kt * 1024, 2));   // (2: nontemporal)
+    for (int u = 0; u < UK; ++u)
+#pragma unroll
+      for (int c = 0; c < PF_CW; ++c)
+        wreg[u][c] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(wp[c], lane * 16, (UK > 1 ? min(kt + u, a.KT - 1) : kt) * 1024, 2));   // (2: nontemporal)
   };
   // operand (row ni of a row tile, 16 bytes kb of k-step ks)
   const int mine = TR < PF_TR ? min(wave, TR - 1) : wave;   // the row tile whose sums this wave takes (the last one's more than once)
@@ -225,17 +234,30 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
     if (tid < 2 * PF_BM) xsum[tid] = 0.f;
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): scalar loads still in flight would make every wait for an LDS read this one
-  for (int kt = kt0; kt < kt1; ++kt) {
-    const int buf = (kt - kt0) & 1;
+  for (int kt = kt0, it = 0; kt < kt1; kt += UK, ++it) {
+    const int buf = it & 1;
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    u32x4_t wcur[PF_CW];
+    u32x4_t wcur[UK][PF_CW];
 #pragma unroll
     for (int c = 0; c < PF_CW; ++c) {
-      asm volatile("" : "+v"(wreg[c]), "+v"(szreg[c]));   // here they are: nothing further down waits for loads again
-      wcur[c] = wreg[c];
+      asm volatile("" : "+v"(szreg[c]));   // here they are: nothing further down waits for loads again
+#pragma unroll
+      for (int u = 0; u < UK; ++u) {
+        asm volatile("" : "+v"(wreg[u][c]));
+        wcur[u][c] = wreg[u][c];
+      }
     }
+    const uint32_t second = UK == 1 || kt + 1 < kt1 ? ~0u : 0u;   // (uniform) an odd range's last k-tile has no neighbour
+    const auto frag = [&](int c, int ks) {
+      u32x4_t f = EX::frag(wcur[ks / KSTEPS][c], ks % KSTEPS, ex_mask, ex_magic);
+      if (UK > 1 && ks >= KSTEPS) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) f[r] &= second;
+      }
+      return f;
+    };
     if constexpr (LACE) {
       open_fix(grp - 1);
     } else if (kt > kt0 && (GPT || gl == 0)) {                         // (uniform) the tile before closed its group
@@ -250,7 +272,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
         }
       }
     }
-    const int nkt = min(kt + 1, kt1 - 1);                       // past the end: once more the last, read by nobody
+    const int nkt = min(kt + UK, kt1 - 1);                      // past the end: once more the last, read by nobody
     load_a(nkt, buf ^ 1);
     load_b(nkt);
     load_sz(grp);
@@ -262,7 +284,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
     for (int rt = 0; rt < PF_RT; ++rt) af[rt] = aread(tile, wm * PF_RT + rt, 0);
     own = aread(tile, mine, 0);
 #pragma unroll
-    for (int c = 0; c < PF_CW; ++c) bf[c] = EX::frag(wcur[c], 0, ex_mask, ex_magic);
+    for (int c = 0; c < PF_CW; ++c) bf[c] = frag(c, 0);
     f32x4_t sx = zero4;
     __builtin_amdgcn_sched_barrier(0);
     auto kstep = [&](int ks, auto first) {
@@ -279,28 +301,33 @@ __global__ __launch_bounds__(PF_THREADS, 2) void gemm_prefill_kernel(const Prefi
         }
 #pragma unroll
         for (int c = 0; c < PF_CW; ++c) acc[rt][c] = mfma16<FT>(bf[c], af[rt], FIRST ? zero4 : acc[rt][c]);
-        if (ks + 1 < KSTEPS) af[rt] = aread(tile, wm * PF_RT + rt, ks + 1);
+        if (ks + 1 < NKS) af[rt] = aread(tile, wm * PF_RT + rt, ks + 1);
         if (rt == 2) {
-          sx = mfma16<FT>(ones, own, sx);
-          if (ks + 1 < KSTEPS) own = aread(tile, mine, ks + 1);
+          u32x4_t one = ones;
+          if (UK > 1 && ks >= KSTEPS) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) one[r] &= second;
+          }
+          sx = mfma16<FT>(one, own, sx);
+          if (ks + 1 < NKS) own = aread(tile, mine, ks + 1);
         }
-        if (ks + 1 < KSTEPS && rt >= PF_RT - 1 - PF_CW && rt < PF_RT - 1) bn[rt - (PF_RT - 1 - PF_CW)] = EX::frag(wcur[rt - (PF_RT - 1 - PF_CW)], ks + 1, ex_mask, ex_magic);
+        if (ks + 1 < NKS && rt >= PF_RT - 1 - PF_CW && rt < PF_RT - 1) bn[rt - (PF_RT - 1 - PF_CW)] = frag(rt - (PF_RT - 1 - PF_CW), ks + 1);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (ks + 1 < KSTEPS) {
+      if (ks + 1 < NKS) {
 #pragma unroll
         for (int c = 0; c < PF_CW; ++c) bf[c] = bn[c];
       }
     };
     kstep(0, std::integral_constant<bool, LACE>{});
 #pragma unroll
-    for (int ks = 1; ks < KSTEPS; ++ks) kstep(ks, std::false_type{});
+    for (int ks = 1; ks < NKS; ++ks) kstep(ks, std::false_type{});
     if (kb == 0 && (TR == PF_TR || wave < TR)) {   // the lane with kb == 0 of a row's lanes owns its entry: no race
       float* p = xsum + (grp & 1) * PF_BM + wave * 16 + ni;
       *p = GPT || gl == 0 ? sx[0] : *p + sx[0];
     }
-    ++gl;
-    if (GPT || gl == a.ktpg || kt + 1 == kt1) {
+    gl += UK;
+    if (GPT || gl == a.ktpg || kt + UK >= kt1) {
       gl = 0;
       ++grp;
     }
@@ -461,10 +488,10 @@ __global__ __launch_bounds__(256) void gemm_prefill_tail_reduce_kernel(const Pre
 template <int WBITS, int FT, int EPI, int GPT>
 hipError_t launch_gemm_prefill(const PrefillArgs& a, int blocks, hipStream_t stream);
 
-template <int WBITS, int FT, int EPI, int GPT, int TR>
-hipError_t launch_gemm_prefill_rows(const PrefillArgs& a, int blocks, hipStream_t s) {
-  auto kern = gemm_prefill_kernel<WBITS, FT, EPI, GPT, TR>;
-  constexpr size_t lds = prefill_lds_bytes<WBITS, TR>();
+template <int WBITS, int FT, int EPI, int GPT, int TR, int UK>
+hipError_t launch_gemm_prefill_unit(const PrefillArgs& a, int blocks, hipStream_t s) {
+  auto kern = gemm_prefill_kernel<WBITS, FT, EPI, GPT, TR, UK>;
+  constexpr size_t lds = prefill_lds_bytes<WBITS, TR, UK>();
   if (lds > 64 * 1024) {  // the grant is per device: once per device of this process
     static std::atomic<unsigned> granted_mask[4];  // 128 device ids
     int dev = 0;
@@ -483,6 +510,15 @@ hipError_t launch_gemm_prefill_rows(const PrefillArgs& a, int blocks, hipStream_
     hipLaunchKernelGGL((gemm_prefill_tail_reduce_kernel<FT, EPI>), dim3((unsigned)std::min<size_t>((quads + 255) / 256, 4096)), dim3(256), 0, s, a);
   }
   return hipGetLastError();
+}
+
+// (a group of an odd number of k-tiles ends between two of them)
+template <int WBITS, int FT, int EPI, int GPT, int TR>
+hipError_t launch_gemm_prefill_rows(const PrefillArgs& a, int blocks, hipStream_t s) {
+  if constexpr (WBITS == 8 && !GPT) {
+    if (a.ktpg % 2 == 0) return launch_gemm_prefill_unit<WBITS, FT, EPI, GPT, TR, 2>(a, blocks, s);
+  }
+  return launch_gemm_prefill_unit<WBITS, FT, EPI, GPT, TR, 1>(a, blocks, s);
 }
 
 #define DIHIP_DEFINE_PREFILL_LAUNCH(WBITS, FT, EPI, GPT)                                                                \
