@@ -3,19 +3,22 @@
 //
 // Bound by the weights' bytes (152064 x 3584: 1.09 GB).  The general kernel re-reads the rows for every few column tiles and keeps its loads
 // short; here one workgroup per CU lives for the whole launch:
-//   * it owns up to 40 neighbouring column tiles, 8 waves take them in turn and keep ALL their accumulators (5 tiles x 8 registers at 32 rows);
+//   * it owns up to 40 neighbouring column tiles; each of its 8 waves walks an eighth of them, counted in batches of 16 steps of K -- 37 tiles are not 8 waves' equal shares,
+//     and a wave is bound by its own loads' way: with whole tiles (five or four a wave) the last fifth of the time ran on five waves.  It keeps all its accumulators (6 tiles x 8
+//     registers at 32 rows); the sums of a tile that two waves share meet in LDS at the end;
 //   * the rows' operands lie in LDS -- all of K where they fit (16 rows x 3584), else one range of K after the other, each for all tiles --: they
 //     are read from the L2 once per CU, and the walk itself issues nothing but weight loads;
 //   * a wave asks for the next 8 KiB (the next batch of its tile, of its next tile, of the next range) before it multiplies the present ones: the
 //     stream does not stop at the ends of tiles.
-// 32 / 16 / 7 rows of 152064 x 3584: 210 / 198 / 196 us (the general kernel) -> 182 / 182 / 177 (6.0 - 6.2 TB/s).  What is left: 37 tiles are not 8 waves'
-// equal shares (the last fifth of the time runs on five waves), and the rows' way into LDS before the stream.
+// 32 / 16 / 7 rows of 152064 x 3584: 210 / 198 / 196 us (the general kernel) -> 182 / 182 / 177 (whole tiles) -> 176 / 174 / 173 (even shares: 6.2 TB/s).  What is left: the rows' way into LDS before the
+// stream (and between the ranges of K).
 #include "gemm_lowp_kernel.hpp"  // mfma16<FT>
 
 namespace dihip {
 namespace {
 
-constexpr int DS_WAVES = 8, DS_TILES = 5, DS_U = 8;   // column tiles per wave, K steps (of 32) per batch
+constexpr int DS_WAVES = 8, DS_TILES = 5, DS_SLOTS = DS_TILES + 1, DS_U = 8;   // column tiles per wave, tiles it may touch, K steps (of 32) per batch of loads
+constexpr int DS_UNIT = 2 * DS_U;   // K steps: what the waves' shares are counted in
 
 template <int FT, int MT>
 __global__ __launch_bounds__(64 * DS_WAVES, 2) void dense_stream_kernel(const u32x4_t* __restrict__ w, const u32x4_t* __restrict__ x, float* __restrict__ out,
@@ -23,11 +26,13 @@ __global__ __launch_bounds__(64 * DS_WAVES, 2) void dense_stream_kernel(const u3
   extern __shared__ __attribute__((aligned(16))) u32x4_t xs[];   // [K step of the range][MT][64]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lo = (int)((long)ntiles * blockIdx.x / gridDim.x), hi = (int)((long)ntiles * (blockIdx.x + 1) / gridDim.x);
-  const int mine = max(0, (hi - lo - wave + DS_WAVES - 1) / DS_WAVES);   // tiles lo + wave + 8 i
+  // wave w's share of T tiles begins T w / 8 tiles in: tiles first .. first + 5; in every range of K it is [T upt w / 8, T upt (w + 1) / 8) of the range's units (upt: units per
+  // tile), which lie in the same tiles whatever upt is
+  const int T = hi - lo, first = T * wave / DS_WAVES;
   const f32x4_t z4 = {0.f, 0.f, 0.f, 0.f};
-  f32x4_t acc[DS_TILES][MT];
+  f32x4_t acc[DS_SLOTS][MT];
 #pragma unroll
-  for (int i = 0; i < DS_TILES; ++i)
+  for (int i = 0; i < DS_SLOTS; ++i)
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[i][m] = z4;
   auto load = [&](u32x4_t (&d)[DS_U], const u32x4_t* p) {
@@ -40,25 +45,43 @@ __global__ __launch_bounds__(64 * DS_WAVES, 2) void dense_stream_kernel(const u3
 #pragma unroll
       for (int m = 0; m < MT; ++m) c[m] = mfma16<FT>(d[u], xs[((b + u) * MT + m) * 64 + lane], c[m]);
   };
-  auto tile = [&](int i) { return w + (size_t)(lo + wave + DS_WAVES * i) * KT * 64 + lane; };
+  auto tile = [&](int i) { return w + (size_t)(lo + first + i) * KT * 64 + lane; };
+  auto begin = [&](int wv, int upt) { return T * upt * wv / DS_WAVES; };
+  // the wave's first batch of the ranges from k0 on; it has none: its first tile's (loaded, not used)
+  auto start = [&](int k0) {
+    for (; k0 < KT; k0 += range) {
+      const int upt = min(range, KT - k0) / DS_UNIT, u = begin(wave, upt);
+      if (u < begin(wave + 1, upt)) return tile(0) + (size_t)(k0 + (u - first * upt) * DS_UNIT) * 64;
+    }
+    return w + (size_t)min(lo + first, ntiles - 1) * KT * 64 + lane;
+  };
   u32x4_t wa[DS_U], wb[DS_U];     // two batches in turn
-  if (mine > 0) load(wa, tile(0));
+  load(wa, start(0));
   for (int k0 = 0; k0 < KT; k0 += range) {
-    const int kn = min(range, KT - k0);
+    const int kn = min(range, KT - k0), upt = kn / DS_UNIT, u0 = begin(wave, upt), u1 = begin(wave + 1, upt);
     if (k0) __syncthreads();                    // the range before has been read
-    for (int e = tid; e < kn * MT * 64; e += 64 * DS_WAVES) xs[e] = x[(size_t)k0 * MT * 64 + e];
+    constexpr int AHEAD = 10;                   // (a thread's loads in flight: all of a range in two goes)
+    const u32x4_t* const from = x + (size_t)k0 * MT * 64;
+    for (int e = tid; e < kn * MT * 64; e += AHEAD * 64 * DS_WAVES) {
+      u32x4_t r[AHEAD];
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) r[j] = from[min(e + j * 64 * DS_WAVES, kn * MT * 64 - 1)];
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j)
+        if (e + j * 64 * DS_WAVES < kn * MT * 64) xs[e + j * 64 * DS_WAVES] = r[j];
+    }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < DS_TILES; ++i) {
-      if (i < mine) {                           // (uniform)
-        const u32x4_t* p = tile(i) + (size_t)k0 * 64;
-        // what follows the tile: the next one, the first one's next range, or (the walk's end) this batch once more
-        const u32x4_t* then = i + 1 < mine ? tile(i + 1) + (size_t)k0 * 64 : k0 + range < KT ? tile(0) + (size_t)(k0 + range) * 64 : p;
-        for (int b = 0; b < kn; b += 2 * DS_U) {
+    for (int i = 0; i < DS_SLOTS; ++i) {
+      const int at = (first + i) * upt, b0 = max(u0 - at, 0) * DS_UNIT, b1 = min(u1 - at, upt) * DS_UNIT;   // (uniform) this tile's part of the share
+      if (b0 < b1) {
+        const u32x4_t* p = tile(i) + (size_t)(k0 + b0) * 64;
+        const u32x4_t* then = u1 > at + upt ? tile(i + 1) + (size_t)k0 * 64 : start(k0 + range);   // what follows: the next tile, or the next range
+        for (int b = b0; b < b1; b += DS_UNIT) {
           load(wb, p + DS_U * 64);
           __builtin_amdgcn_sched_barrier(0);
           mul(wa, b, acc[i]);
-          p = b + 2 * DS_U < kn ? p + 2 * DS_U * 64 : then;
+          p = b + DS_UNIT < b1 ? p + DS_UNIT * 64 : then;
           load(wa, p);
           __builtin_amdgcn_sched_barrier(0);
           mul(wb, b + DS_U, acc[i]);
@@ -66,11 +89,24 @@ __global__ __launch_bounds__(64 * DS_WAVES, 2) void dense_stream_kernel(const u3
       }
     }
   }
+  // a share that begins inside a tile leaves its sums of it to the wave that has the tile's beginning, which adds them in the waves' order
+  __syncthreads();
+  f32x4_t* const part = reinterpret_cast<f32x4_t*>(xs);   // [wave][MT][64]
+  if (T * wave % DS_WAVES != 0) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) part[(wave * MT + m) * 64 + lane] = acc[0][m];
+  }
+  __syncthreads();
   // the weights were the A operand: a lane holds 4 neighbouring columns of row m * 16 + lane % 16
 #pragma unroll
-  for (int i = 0; i < DS_TILES; ++i) {
-    if (i < mine) {
-      const int n = (lo + wave + DS_WAVES * i) * 16 + (lane >> 4) * 4;
+  for (int i = 0; i < DS_SLOTS; ++i) {
+    const int t = first + i;
+    if (t < T && DS_WAVES * t < T * (wave + 1) && (i > 0 || T * wave % DS_WAVES == 0)) {   // (uniform) the tile's beginning is this wave's
+      for (int o = wave + 1; o < DS_WAVES && T * o / DS_WAVES == t && T * o % DS_WAVES != 0; ++o) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[i][m] += part[(o * MT + m) * 64 + lane];
+      }
+      const int n = (lo + t) * 16 + (lane >> 4) * 4;
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
         const int row = m * 16 + (lane & 15);
@@ -92,7 +128,7 @@ template <int FT, int MT>
 int go(hipStream_t s, const void* w, const void* x, float* out, int M, int N, int KT, int ntiles) {
   constexpr int LDS_STEPS = 152 / MT / (2 * DS_U) * (2 * DS_U);          // K steps of the rows' operands in 152 KiB, in whole pairs of batches
   const int ranges = (KT + LDS_STEPS - 1) / LDS_STEPS, range = ((KT + ranges - 1) / ranges + 2 * DS_U - 1) / (2 * DS_U) * (2 * DS_U);
-  const size_t lds = (size_t)std::min(range, KT) * MT * 1024;
+  const size_t lds = (size_t)std::max(std::min(range, KT), DS_WAVES) * MT * 1024;   // (the rows, at the end the shared tiles' sums)
   auto kern = dense_stream_kernel<FT, MT>;
   DIHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), DIHIP_RUNTIME_ERROR);
   int ncu = cached_num_cus();

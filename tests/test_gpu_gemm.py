@@ -328,6 +328,12 @@ def test_lm_head_of_a_batch_against_a_wide_matrix(ops, M, K, V, ft):
     assert np.abs(logits - ref).max() < (2 ** -9 if ft == "bf16" else 2 ** -12) * np.abs(ref).max()
 
 
+# Shares of 4, 4 and 5, 8, 9 and 40 column tiles per workgroup (a tile that two, three or no waves share), ranges of K of different lengths and one of a single batch
+@pytest.mark.parametrize("M,K,V,ft", [(32, 512, 16384, "bf16"), (32, 6656, 20480, "bf16"), (16, 1024, 32768, "bf16"), (20, 3584, 36864, "bf16"), (32, 1024, 163840, "f16"), (6, 512, 163841, "bf16")])
+def test_lm_head_of_a_batch_in_even_shares(ops, M, K, V, ft):
+    test_lm_head_of_a_batch_against_a_wide_matrix(ops, M, K, V, ft)
+
+
 @pytest.mark.parametrize("M,K,V", [(5, 512, 16400), (16, 3584, 20003), (32, 512, 30000)])
 def test_lm_head_refuses_a_workspace_below_the_general_kernel_s(ops, M, K, V):
     """Whatever kernel serves the rows: the least workspace is the general kernel's (its slab and the plain rows), and from there on the logits are there."""
