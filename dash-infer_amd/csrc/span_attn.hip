@@ -277,15 +277,16 @@ __global__ __launch_bounds__(ATTN_THREADS) void span_attn_decode_kernel(const At
 #ifndef DIHIP_U4_X
 #define DIHIP_U4_X 0
 #endif
-template <bool FUSED>
-__global__ __launch_bounds__(ATTN_THREADS) void span_attn_u4_mfma_kernel(const AttnArgs a) {
+// NW: waves of the workgroup.  A token range's cost is its own loads' way, its record's a merge's: 8 waves with half as many splits (attn_plan).  HC: heads a record area is laid
+// out for (the products always have 16 columns)
+template <bool FUSED, int NW, int HC>
+__global__ __launch_bounds__(64 * NW) void span_attn_u4_mfma_kernel(const AttnArgs a) {
   constexpr int H = 128;
-  constexpr int HC = MF_HC;
   constexpr int HB = H / 2;  // bytes per token-head row
-  constexpr int NEW_WAVE = ATTN_THREADS / 64 - 1;  // FUSED: the wave that handles this step's token
-  __shared__ __attribute__((aligned(16))) float lds[4 * HC * ATTN_PSTRIDE + 4];
+  constexpr int NEW_WAVE = NW - 1;  // FUSED: the wave that handles this step's token
+  __shared__ __attribute__((aligned(16))) float lds[NW * HC * ATTN_PSTRIDE + 4];
   __shared__ __attribute__((aligned(16))) unsigned char newrow[2][FUSED ? 80 : 16];  // FUSED: {64 B nibbles, zero, scale} of the new K / V head
-  unsigned* flag_lds = reinterpret_cast<unsigned*>(lds + 4 * HC * ATTN_PSTRIDE);
+  unsigned* flag_lds = reinterpret_cast<unsigned*>(lds + NW * HC * ATTN_PSTRIDE);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -293,8 +294,8 @@ __global__ __launch_bounds__(ATTN_THREADS) void span_attn_u4_mfma_kernel(const A
   const int split = blockIdx.x;
   const int grp = blockIdx.y / a.nchunks, hc = blockIdx.y % a.nchunks;
   const int b = blockIdx.z;
-  const int h0 = grp * a.hpg + hc * HC;
-  const int nh = min(HC, a.hpg - hc * HC);
+  const int h0 = grp * a.hpg + hc * MF_HC;
+  const int nh = min(HC, a.hpg - hc * MF_HC);
 
   const int len = (int)a.seq_lens[b] + a.len_bias;
   const int tps = ((len + a.nsplits - 1) / a.nsplits + 31) & ~31;
@@ -556,7 +557,7 @@ __global__ __launch_bounds__(ATTN_THREADS) void span_attn_u4_mfma_kernel(const A
 
   DIHIP_U4_STAMP(1);  // first loads issued, q fragments built
   if (active) {
-    constexpr int STEP = 4 * MF_TOK;  // the 4 waves interleave 32-token blocks
+    constexpr int STEP = NW * MF_TOK;  // the waves interleave 32-token blocks
     for (int tb = tb0; tb < t1; tb += 2 * STEP) {
       issue(bb, tb + STEP);  // unconditional (clamped inside): see the note in the VALU kernel
       process(ba, tb);
@@ -606,7 +607,7 @@ __global__ __launch_bounds__(ATTN_THREADS) void span_attn_u4_mfma_kernel(const A
       rec[H + 1] = l;
     }
   }
-  attn_block_epilogue<DIHIP_BF16, HC>(a, lds, flag_lds, b, h0, nh, split, trw);
+  attn_block_epilogue<DIHIP_BF16, HC, NW>(a, lds, flag_lds, b, h0, nh, split, trw);
   DIHIP_U4_STAMP(7);
 #undef DIHIP_U4_STAMP
 }
@@ -617,7 +618,7 @@ __global__ __launch_bounds__(ATTN_THREADS) void span_attn_u4_mfma_kernel(const A
 // ------------------------------------------------------------------------------------------
 struct AttnPlan {
   int HC, nchunks, nsplits;
-  int waves;  // live waves per workgroup: 4, or 8 for the wide form of the 16-bit MFMA kernel (batch 1)
+  int waves;  // live waves per workgroup: 4, or 8 for the wide forms (16-bit MFMA kernel at batch 1, uint4 kernel of up to 8 heads a group)
   bool mfma;
   size_t partial_bytes;
 };
@@ -629,20 +630,22 @@ static bool attn_use_mfma(int mode, int dtype) {
 }
 
 // the 16-bit cache's MFMA kernel has an 8-wave form (span_attn_ft_mfma_w8_kernel; the fused attention block runs the same body)
-static bool attn_wide_ok(int mode, int dtype) {
+enum { ATTN_WIDE_NO = 0, ATTN_WIDE_ONE = 1, ATTN_WIDE_U4 = 2 };
+static int attn_wide_ok(int mode, int dtype) {
+  if (mode == DIHIP_KV_U4 && dtype == DIHIP_BF16) return ATTN_WIDE_U4;
   // opt-in (DIHIP_ATTN_WIDE=1): measured at 2048 tokens, 28 / 4 heads -- 9 split records instead of 17, but the 8-wave workgroup's own merge
   // and its two waves per SIMD in the tile phase give the gain back: block 16.4 against 15.8 us per layer (profiles/r06_attn_block_polls.txt)
   static const bool enabled = [] { const char* e = getenv("DIHIP_ATTN_WIDE"); return e && e[0] == '1'; }();
-  return enabled && mode == DIHIP_KV_NONE && (dtype == DIHIP_BF16 || dtype == DIHIP_F16);
+  return enabled && mode == DIHIP_KV_NONE && (dtype == DIHIP_BF16 || dtype == DIHIP_F16) ? ATTN_WIDE_ONE : ATTN_WIDE_NO;
 }
 
 static AttnPlan attn_plan(int batch, int n_heads, int n_groups, int max_seq_len, int num_cus, bool mfma = false,
-                          int split_cap = 256, bool wide_ok = false) {
+                          int split_cap = 256, int wide = ATTN_WIDE_NO) {
   AttnPlan p;
   const int hpg = n_heads / n_groups;
   p.mfma = mfma;
   // batch 1, opt-in: one 8-wave workgroup per CU covers 256 tokens per pass -- half the split records of the 4-wave form
-  p.waves = mfma && wide_ok && batch == 1 ? 8 : 4;
+  p.waves = mfma && wide == ATTN_WIDE_ONE && batch == 1 ? 8 : 4;
   p.HC = mfma ? MF_HC : hpg <= 1 ? 1 : hpg <= 2 ? 2 : hpg <= 4 ? 4 : 8;
   p.nchunks = (hpg + p.HC - 1) / p.HC;
   if (num_cus <= 0) num_cus = cached_num_cus();
@@ -663,10 +666,26 @@ static AttnPlan attn_plan(int batch, int n_heads, int n_groups, int max_seq_len,
     const long one_per_cu = std::max<long>(1, (num_cus + base - 1) / base);
     p.nsplits = (int)std::max<long>(1, std::min<long>(p.nsplits, one_per_cu));
   }
+  // uint4 cache: half as many splits of 8 waves where a split is long and nearly every CU has one of them, or where there are many records to merge.  4 waves / 8, a step of four
+  // layers, us: 32 requests of 2048 tokens 532 / 522, 16 of 2048 475 / 468, 4 of 8000 452 / 447, one of 8000 396 / 382; but 20 of 1000 (240 of 256 CUs, 334 tokens a split)
+  // 511 / 543, 25 of 2000 (200 CUs) 544 / 555, 8 of 700 447 / 450
+  if (mfma && wide == ATTN_WIDE_U4 && hpg <= 8 && wgs_per_cu == 0) {
+    const long fit = std::max<long>(1, num_cus / base), most = std::max<long>(1, (max_seq_len + 255) / 256), ns = std::min<long>(std::min<long>(fit, most), split_cap);
+    if ((max_seq_len >= 448 * ns && 10 * ns * base >= 9 * num_cus && ns * base <= num_cus) || (p.nsplits > 32 && ns < p.nsplits)) {
+      p.waves = 8;
+      p.nsplits = (int)ns;
+    }
+  }
   static const int force_splits = env_int("DIHIP_ATTN_NSPLITS", 0);  // diagnostics
   if (force_splits > 0) p.nsplits = (int)std::min<long>(std::min<long>(force_splits, max_splits), split_cap);
   p.partial_bytes = p.nsplits > 1 ? (size_t)batch * n_heads * p.nsplits * ATTN_PSTRIDE * sizeof(float) : 0;
   return p;
+}
+
+template <bool FUSED>
+static void launch_u4(const AttnPlan& p, dim3 grid, hipStream_t s, const AttnArgs& a) {
+  if (p.waves == 8) hipLaunchKernelGGL((span_attn_u4_mfma_kernel<FUSED, 8, 8>), grid, dim3(512), 0, s, a);
+  else hipLaunchKernelGGL((span_attn_u4_mfma_kernel<FUSED, 4, MF_HC>), grid, dim3(256), 0, s, a);
 }
 
 template <int FT, int MODE>
@@ -767,7 +786,7 @@ static int run_decode(hipStream_t s, void* out, const void* q, const void* const
   a.trace = debug_trace_buffer((size_t)p.nsplits * g * p.nchunks * batch * 32 * sizeof(unsigned long long));
   bool ok = true;
   if (p.mfma && mode == DIHIP_KV_U4) {
-    hipLaunchKernelGGL(span_attn_u4_mfma_kernel<false>, grid, dim3(ATTN_THREADS), 0, s, a);
+    launch_u4<false>(p, grid, s, a);
   } else if (p.mfma && p.waves == 8) {
     if (!launch_w8(dtype, false, grid, s, a)) return DIHIP_SA_HIP_ERROR;
   } else if (p.mfma && dtype == DIHIP_BF16 && mode == DIHIP_KV_NONE) {
@@ -884,7 +903,7 @@ int span_attn_fused_mfma(void* stream, void* output, const void* qkv, void* cons
   const dim3 grid(p.nsplits, n_groups * p.nchunks, batch);
   a.trace = debug_trace_buffer((size_t)p.nsplits * n_groups * p.nchunks * batch * 32 * sizeof(unsigned long long));
   if (u4)
-    hipLaunchKernelGGL(span_attn_u4_mfma_kernel<true>, grid, dim3(ATTN_THREADS), 0, s, a);
+    launch_u4<true>(p, grid, s, a);
   else if (i8 && dtype == DIHIP_BF16)
     hipLaunchKernelGGL((span_attn_ft_mfma_kernel<DIHIP_BF16, DIHIP_KV_I8, true>), grid, dim3(ATTN_THREADS), 0, s, a);
   else if (i8)

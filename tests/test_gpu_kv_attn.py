@@ -464,6 +464,14 @@ def test_quantised_decode_step_matches_append_plus_attention(ops, n, g, S, lens,
                 assert torch.equal(pool.span_view(kv.k_idx[b][i]), pool2.span_view(kv2.k_idx[b][i])), f"K span {b}/{i} after step 2"
 
 
+# the uint4 kernel of 8 waves (the plan's choice on 256 CUs): two splits and one, 7 and 8 heads a group, ranges that end inside a wave's block, at a wave's, at a workgroup's pass; more
+# than 32 records of the 4-wave form for one request
+@pytest.mark.parametrize("n,g,S,lens", [(32, 4, 32, [1100, 0, 1, 31, 32, 33, 255, 256, 257, 511, 512, 513, 548, 549, 1023, 1024] * 2), (28, 4, 64, [700, 447, 449, 256, 0, 31, 289, 640] * 8),
+                                        (8, 1, 32, [4400]), (7, 1, 16, [9000])])
+def test_quantised_decode_step_of_eight_waves(ops, n, g, S, lens):
+    test_quantised_decode_step_matches_append_plus_attention(ops, n, g, S, lens, "u4")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("mode", ["none", "u4"])
 @pytest.mark.parametrize("B", [5, 24])
