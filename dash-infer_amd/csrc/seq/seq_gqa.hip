@@ -1002,6 +1002,366 @@ __global__ __launch_bounds__(256) void gqa_attn_merge_diff_kernel(void* __restri
   if (threadIdx.x < DV) st_any(y, (size_t)t * ldy + (size_t)h * DV + threadIdx.x, ydt, d * inv);
 }
 
+// One token of each request (decoding), from the rows of the input product to those of the output product: norm, rotation and append of prep, attention, and the merge of
+// the waves.  In three launches (prep, tile kernel in splits, merge) each waits for its own chain of slot, page and data, and of a tile kernel's four waves three had no row: a
+// workgroup owns a (request, key head), and its waves take 64-key tiles in turn, each with slots of LDS, a softmax and sums of its own, which meet in LDS at the end.
+//   * a wave asks for its next tile's keys behind the reads of this one's, for the values likewise: only the wave itself waits for its loads;
+//   * the token's own key and value are made by the wave whose tile holds their position, put over that tile's row in LDS (the page's is stale) and, behind the walk, into the page;
+//   * walks too long for a workgroup are split as the tile kernel's are (gqa_attn_merge_kernel adds them).
+// Bound by the chain of launch, slot, page pointer and tiles, and past that by one workgroup's LDS in flight (128 KB a unit): 32 heads over 8 of 128, one launch against three, in us
+// (keys: 100 / 700 / 1500 / 4000 / 12000): 1 request 8.0 / 11.0 / 12.5 / 13.1 / 18.1 (13.3 / 13.6 / 14.2 / 18.7 / 22.4), 4 requests 8.1 / 12.7 / 15.6 / 18.5 / 41.5 (13.5 / 16.3 / 18.3 /
+// 23.1 / 48.4), 32 requests 9.8 / 22.5 / 41.7 / 94.0 (17.5 / 31.2 / 52.0 / 110).
+template <int D, int DV, bool CAP>
+__global__ __launch_bounds__(256) void gqa_decode_step_kernel(PrepArgs p, GqaArgs a) {
+  constexpr int KS = D / 32, DT = DV / 16, NT = 4, WAVES = 4;
+  constexpr int KROW = D * 2, VROW = DV * 2, KBYTES = 64 * KROW, VBYTES = 64 * VROW, SLOT = KBYTES + VBYTES;
+  constexpr int KPP = 1024 / KROW, VPP = 1024 / VROW, KP = 64 / KPP, VP = 64 / VPP;   // keys per 1 KiB piece, pieces of a tile
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // [wave][keys | values]; at the end [wave][16 heads][DV + 4] f32
+  __shared__ float cs_t[64], sn_t[64];
+  const int H = a.H, G = a.G, hpg = H / G, e = blockIdx.x / G, g = blockIdx.x - e * G, split = blockIdx.y, nsplit = gridDim.y;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ni = lane & 15, kb = lane >> 4;
+  const int row0 = a.ent_row0[e];
+  void* const* gkp = a.kspans + (size_t)a.ent_slot[e] * a.span_stride;
+  void* const* gvp = a.vspans + (size_t)a.ent_slot[e] * a.span_stride;
+  const int first = split * WAVES + wave, stride = WAVES * nsplit;   // the wave's tiles: first + i * stride
+  const float* row = p.qkv + (size_t)row0 * p.ld;
+  // the wave's page pointers, 64 tiles at a time, one to a lane (a table row's entries past the request's pages are not followed)
+  const int tpp = a.span_len >> 6, room = a.span_stride * tpp;       // tiles per page, of a table row
+  uint64_t kptr = 0, vptr = 0;
+  auto pages = [&](int i0) {
+    const int t = first + stride * (i0 + lane);
+    if (t < room) {
+      kptr = (uint64_t)gload<void*>(gkp + t / tpp);
+      vptr = (uint64_t)gload<void*>(gvp + t / tpp);
+    }
+  };
+  auto tiles = [&](int i0) {         // .. from the page to the tile (apart: the loads are not waited for where they are asked for)
+    const int t = first + stride * (i0 + lane);
+    kptr += (size_t)(t % tpp) * 64 * G * KROW;
+    vptr += (size_t)(t % tpp) * 64 * G * VROW;
+  };
+  // where this lane's 16 bytes of pieces q, q + 4, .. come from (the chunks of a row change places as in the tile kernel)
+  const int kk = lane / (KROW / 16), kc = lane % (KROW / 16), vk = lane / (VROW / 16), vc = lane % (VROW / 16);
+  uint32_t koff[4], voff[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int key = q * KPP + kk, val = q * VPP + vk;
+    koff[q] = (uint32_t)(key * G + g) * KROW + (uint32_t)((kc ^ (D == 128 ? key & 15 : key & 7)) * 16);
+    voff[q] = (uint32_t)(val * G + g) * VROW + (uint32_t)((vc ^ (DV == 128 ? (val & 7) * 2 : ((val >> 1) & 3) * 2)) * 16);
+  }
+  unsigned char* const kbuf = smem + wave * SLOT;
+  unsigned char* const vbuf = kbuf + KBYTES;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem + wave * SLOT;
+  auto lane_ptr = [&](uint64_t ptr, int i) {
+    return (const char*)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)ptr, i) | (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(ptr >> 32), i) << 32);
+  };
+  auto fetch_k = [&](int i) {
+    const char* from = lane_ptr(kptr, i & 63);
+#pragma unroll
+    for (int j = 0; j < KP; ++j)
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds0 + j * 1024), "v"(koff[j & 3]), "s"(from + (size_t)(j >> 2) * 4 * KPP * G * KROW) : "memory");
+  };
+  auto fetch_v = [&](int i) {
+    const char* from = lane_ptr(vptr, i & 63);
+#pragma unroll
+    for (int j = 0; j < VP; ++j)
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds0 + KBYTES + j * 1024), "v"(voff[j & 3]), "s"(from + (size_t)(j >> 2) * 4 * VPP * G * VROW) : "memory");
+  };
+  // what the prologue reads, beside the page pointers and in front of the tiles (loads return in order: behind them it would wait for all of them): the query row of the
+  // lane's head, the token's key and value (D / 64, DV / 64 neighbours to a lane), the norms' weights
+  constexpr int KE = D / 64, VE = DV / 64;
+  const int h = g * hpg + min(ni, hpg - 1), half = p.rot_dims >> 1;
+  const float* qrow = row + p.q_off + (size_t)h * D + kb * 8;
+  pages(0);
+  f32x4_t qv[KS][2], qw[KS][2];
+  float kn[KE], kw[KE], vn[VE];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    qv[ks][0] = *reinterpret_cast<const f32x4_t*>(qrow + ks * 32);
+    qv[ks][1] = *reinterpret_cast<const f32x4_t*>(qrow + ks * 32 + 4);
+  }
+#pragma unroll
+  for (int i = 0; i < KE; ++i) kn[i] = row[p.k_off + (size_t)g * D + lane * KE + i];
+#pragma unroll
+  for (int i = 0; i < VE; ++i) vn[i] = row[p.v_off + (size_t)g * DV + lane * VE + i];
+  int pos = a.tok_pos[row0];
+  asm volatile("" : "+s"(pos));      // (asked for here, not where it is used)
+  const int last = pos >> 6, mine = last >= first ? (last - first) / stride + 1 : 0;
+  const bool owner = mine > 0 && (last - first) % stride == 0;       // (uniform) the wave's last tile holds the token
+  // (one branch on the weights' type around all of them, what is not there read from the row instead and not used: a branch for each would wait for each)
+  constexpr float LOG2E = 1.44269504088896341f;
+  const void* const qnp = p.qnorm ? p.qnorm : row;
+  const void* const knp = p.knorm ? p.knorm : row;
+  const bool w32 = p.wdt == DIHIP_F32;
+  uint32_t qb[KS * 8], kbits[KE];
+  if (w32) {
+#pragma unroll
+    for (int x = 0; x < KS * 8; ++x) qb[x] = ((const uint32_t*)qnp)[(x >> 3) * 32 + kb * 8 + (x & 7)];
+#pragma unroll
+    for (int i = 0; i < KE; ++i) kbits[i] = ((const uint32_t*)knp)[lane * KE + i];
+  } else {
+#pragma unroll
+    for (int x = 0; x < KS * 8; ++x) qb[x] = (uint32_t)((const uint16_t*)qnp)[(x >> 3) * 32 + kb * 8 + (x & 7)] << 16;
+#pragma unroll
+    for (int i = 0; i < KE; ++i) kbits[i] = (uint32_t)((const uint16_t*)knp)[lane * KE + i] << 16;
+  }
+  const bool with_sink = a.sink_mode != 0 && split == 0 && wave == 0;
+  float fr = tid < half ? p.freq[tid] : 0.f;
+  float m = with_sink ? (a.sink_mode == 1 ? ld_any(a.sink, h, a.wdt) * LOG2E : 0.f) : -1e30f, l = with_sink && kb == 0 ? 1.f : 0.f;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {   // all of it is here
+    asm volatile("" : "+v"(qv[ks][0]), "+v"(qv[ks][1]));
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+      qw[ks][x >> 2][x & 3] = p.qnorm ? __builtin_bit_cast(float, qb[ks * 8 + x]) : 1.f;
+    }
+    asm volatile("" : "+v"(qw[ks][0]), "+v"(qw[ks][1]));
+  }
+#pragma unroll
+  for (int i = 0; i < KE; ++i) {
+    kw[i] = p.knorm ? __builtin_bit_cast(float, kbits[i]) : 1.f;
+    asm volatile("" : "+v"(kn[i]), "+v"(kw[i]));
+  }
+#pragma unroll
+  for (int i = 0; i < VE; ++i) asm volatile("" : "+v"(vn[i]));
+  asm volatile("" : "+v"(m), "+v"(fr), "+v"(kptr), "+v"(vptr));
+  tiles(0);
+  if (mine > 0) {
+    fetch_k(0);
+    fetch_v(0);
+  }
+  if (tid < half) {
+    float sn, cs;
+    rope_sincos((uint32_t)pos, fr, &sn, &cs);
+    cs_t[tid] = cs * p.mag;
+    sn_t[tid] = sn * p.mag;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // (not __syncthreads: it would wait for the tiles)
+  u32x4_t qf[KS];
+  {
+    float ss = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ss = __builtin_fmaf(qv[ks][c][r], qv[ks][c][r], ss);
+    if (p.qnorm) {
+      const float inv = 1.f / sqrtf(rows_sum(ss) / (float)D + p.eps);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) qv[ks][c][r] = qv[ks][c][r] * inv * qw[ks][c][r];
+    }
+    if (half) {    // (rot_dims == D)
+      if (p.layout == 0) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; r += 2) {
+              const int pair = (ks * 32 + kb * 8 + c * 4 + r) >> 1;
+              const float x = qv[ks][c][r], y = qv[ks][c][r + 1], cs = cs_t[pair], sn = sn_t[pair];
+              qv[ks][c][r] = x * cs - y * sn;
+              qv[ks][c][r + 1] = y * cs + x * sn;
+            }
+      } else {
+#pragma unroll
+        for (int ks = 0; ks < KS / 2; ++ks)
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int pair = ks * 32 + kb * 8 + c * 4 + r;
+              const float x = qv[ks][c][r], y = qv[ks + KS / 2][c][r], cs = cs_t[pair], sn = sn_t[pair];
+              qv[ks][c][r] = x * cs - y * sn;
+              qv[ks + KS / 2][c][r] = y * cs + x * sn;
+            }
+      }
+    }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      qf[ks] = u32x4_t{pack_bf16x2(qv[ks][0][0], qv[ks][0][1]), pack_bf16x2(qv[ks][0][2], qv[ks][0][3]), pack_bf16x2(qv[ks][1][0], qv[ks][1][1]), pack_bf16x2(qv[ks][1][2], qv[ks][1][3])};
+  }
+  if (owner) {   // the token's key: norm, rotation
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < KE; ++i) ss = __builtin_fmaf(kn[i], kn[i], ss);
+    if (p.knorm) {
+      const float inv = 1.f / sqrtf(wave_sum(ss) / (float)D + p.eps);
+#pragma unroll
+      for (int i = 0; i < KE; ++i) kn[i] = kn[i] * inv * kw[i];
+    }
+    if (half) {
+      float other[KE];
+#pragma unroll
+      for (int i = 0; i < KE; ++i) other[i] = p.layout == 1 ? __shfl_xor(kn[i], 32, 64) : KE == 2 ? kn[KE - 1 - i] : __shfl_xor(kn[i], 1, 64);
+#pragma unroll
+      for (int i = 0; i < KE; ++i) {
+        const int d = lane * KE + i;
+        const bool low = p.layout == 1 ? d < half : (d & 1) == 0;
+        const int pair = p.layout == 1 ? (d < half ? d : d - half) : d >> 1;
+        kn[i] = low ? kn[i] * cs_t[pair] - other[i] * sn_t[pair] : kn[i] * cs_t[pair] + other[i] * sn_t[pair];
+      }
+    }
+  }
+  f32x4_t oacc[DT];
+#pragma unroll
+  for (int t = 0; t < DT; ++t) oacc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  int kfo[KS], vfo[DT];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) kfo[ks] = ni * KROW + (((ks * 4 + kb) ^ (D == 128 ? ni : ni & 7)) * 16);
+  {
+    const int vr = kb * 4 + (ni >> 2), f = DV == 128 ? (vr & 7) * 2 : ((vr >> 1) & 3) * 2;
+#pragma unroll
+    for (int t = 0; t < DT; ++t) vfo[t] = vr * VROW + (((2 * t) ^ f) + ((ni & 3) >> 1)) * 16 + (ni & 1) * 8;
+  }
+  const float sl2 = a.scale * LOG2E, cap = a.softcap, cap_in = CAP ? 2.f * a.scale * LOG2E / cap : 0.f, cap2 = cap * LOG2E;
+  for (int i = 0; i < mine; ++i) {
+    const int key0 = (first + stride * i) * 64;
+    const bool here = owner && i + 1 == mine;        // (uniform) the tile of the token, and of rows that no token has written
+    // keys: everything but the values' pieces behind them has landed
+    if (here) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(VP) : "memory");
+    const int r = pos & 63;
+    if (here) {
+      const int d = lane * KE;
+      unsigned char* to = kbuf + r * KROW + ((d >> 3) ^ (D == 128 ? r & 15 : r & 7)) * 16 + (d & 7) * 2;
+      if constexpr (KE == 2) *reinterpret_cast<uint32_t*>(to) = pack_bf16x2(kn[0], kn[1]);
+      else *reinterpret_cast<uint16_t*>(to) = (uint16_t)f32_to_bf16_bits(kn[0]);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    f32x4_t sacc[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) sacc[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      u32x4_t kf[NT];
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) kf[nt] = *reinterpret_cast<const u32x4_t*>(kbuf + kfo[ks] + nt * 16 * KROW);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) sacc[nt] = mfma_bf16g(kf[nt], qf[ks], sacc[nt]);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the keys have been read
+    const bool more = i + 1 < mine;
+    if (more) {
+      if (((i + 1) & 63) == 0) {
+        pages(i + 1);
+        tiles(i + 1);
+      }
+      fetch_k(i + 1);
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float x;
+        if constexpr (CAP) x = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(sacc[nt][q] * cap_in));   // cap * tanh(s / cap)
+        else x = sacc[nt][q] * sl2;
+        if (here && key0 + nt * 16 + kb * 4 + q > pos) x = -INFINITY;
+        sacc[nt][q] = x;
+        mx = fmaxf(mx, x);
+      }
+    mx = fmaxf(m, rows_max(mx));
+    const float corr = __builtin_amdgcn_exp2f(m - mx);
+    m = mx;
+    float ps = 0.f;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        sacc[nt][q] = __builtin_amdgcn_exp2f(sacc[nt][q] - mx);
+        ps += sacc[nt][q];
+      }
+    l = l * corr + ps;
+    u32x4_t pf[2];
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh)
+      pf[hh] = u32x4_t{pack_bf16x2(sacc[2 * hh][0], sacc[2 * hh][1]), pack_bf16x2(sacc[2 * hh][2], sacc[2 * hh][3]),
+                       pack_bf16x2(sacc[2 * hh + 1][0], sacc[2 * hh + 1][1]), pack_bf16x2(sacc[2 * hh + 1][2], sacc[2 * hh + 1][3])};
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) oacc[t][q] *= corr;
+    // values: this tile's have landed, the next one's keys may be on their way
+    if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(KP) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (here) {
+      const int d = lane * VE;
+      unsigned char* to = vbuf + r * VROW + ((d >> 3) ^ (DV == 128 ? (r & 7) * 2 : ((r >> 1) & 3) * 2)) * 16 + (d & 7) * 2;
+      if constexpr (VE == 2) *reinterpret_cast<uint32_t*>(to) = pack_bf16x2(vn[0], vn[1]);
+      else *reinterpret_cast<uint16_t*>(to) = (uint16_t)f32_to_bf16_bits(vn[0]);
+      for (int z = lane; z < (63 - r) * (VROW / 16); z += 64) *reinterpret_cast<u32x4_t*>(vbuf + (r + 1) * VROW + z * 16) = u32x4_t{0u, 0u, 0u, 0u};   // (an infinity there, times 0)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        const u32x2_t lo2 = lds_read_tr16(vbuf + vfo[t] + hh * 32 * VROW), hi2 = lds_read_tr16(vbuf + vfo[t] + hh * 32 * VROW + 16 * VROW);
+        const u32x4_t vf = {lo2[0], lo2[1], hi2[0], hi2[1]};
+        oacc[t] = mfma_bf16g(vf, pf[hh], oacc[t]);
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the values have been read
+    if (more) fetch_v(i + 1);
+  }
+  if (owner) {   // the token's key and value into their page, off the way of the tiles
+    const int i = (mine - 1) & 63, r = pos & 63;
+    uint16_t* kto = (uint16_t*)(lane_ptr(kptr, i) + (size_t)(r * G + g) * KROW) + lane * KE;
+    uint16_t* vto = (uint16_t*)(lane_ptr(vptr, i) + (size_t)(r * G + g) * VROW) + lane * VE;
+#pragma unroll
+    for (int x = 0; x < KE; ++x) kto[x] = (uint16_t)f32_to_bf16_bits(kn[x]);
+#pragma unroll
+    for (int x = 0; x < VE; ++x) vto[x] = (uint16_t)f32_to_bf16_bits(vn[x]);
+  }
+  l = rows_sum(l);
+  __syncthreads();     // every wave has read its last tile (and waited for its last load): the sums meet in their place
+  float* const rec = reinterpret_cast<float*>(smem);
+  if (ni < hpg) {
+    float* o = rec + (size_t)(wave * 16 + ni) * (DV + 4);
+#pragma unroll
+    for (int t = 0; t < DT; ++t) *reinterpret_cast<f32x4_t*>(o + t * 16 + kb * 4) = oacc[t];
+    if (kb == 0) {
+      o[DV] = m;
+      o[DV + 1] = l;
+    }
+  }
+  __syncthreads();
+  for (int x = tid; x < hpg * (DV / 4); x += 256) {
+    const int hh = x / (DV / 4), d = (x - hh * (DV / 4)) * 4;
+    float mw[WAVES], M = -1e30f, den = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      mw[w] = rec[(w * 16 + hh) * (DV + 4) + DV];
+      M = fmaxf(M, mw[w]);
+    }
+    f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float c = __builtin_amdgcn_exp2f(mw[w] - M);
+      const float* from = rec + (w * 16 + hh) * (DV + 4);
+      den = __builtin_fmaf(c, from[DV + 1], den);
+      o += c * *reinterpret_cast<const f32x4_t*>(from + d);
+    }
+    const int head = g * hpg + hh;
+    if (nsplit == 1) {
+      const float inv = (a.gate ? a.gate[(size_t)row0 * a.ldg + head] : 1.f) / den;
+      store4(a.out, (size_t)row0 * a.ldo + (size_t)head * DV + d, a.odt, o * inv);
+    } else {   // [split][row, query head][DV sums, maximum, denominator, ..]
+      float* to = a.ws + ((size_t)split * a.rows_total + (size_t)row0 * H + head) * (DV + 4);
+      *reinterpret_cast<f32x4_t*>(to + d) = o;
+      if (d == 0) {
+        to[DV] = M * 0.69314718055994531f;
+        to[DV + 1] = den;
+      }
+    }
+  }
+}
+
 }  // namespace
 }  // namespace dihip
 
@@ -1204,6 +1564,53 @@ int dihip_gqa_attn_mc(void* stream, void* out, int out_dtype, long ldo, const fl
   else if (diff_out)
     hipLaunchKernelGGL(maps_diff_norm_kernel, dim3((unsigned)(((long)T * H + 3) / 4)), dim3(256), 0, s, diff_out, diff_dtype, ldd, (const float*)out, ldo, lam, out_scale,
                        eps, T * H, H, DV);
+  return launch_status();
+}
+
+int dihip_gqa_decode_step_supported(int H, int G, int D, int DV, int span_len, int cache_dtype, int rot_dims) {
+  return cache_dtype == DIHIP_BF16 && G > 0 && H % G == 0 && H / G <= 16 && (D == 64 || D == 128) && (DV == 64 || DV == 128) && span_len % 64 == 0 && (rot_dims == 0 || rot_dims == D);
+}
+
+int dihip_gqa_decode_step(void* stream, void* out, int out_dtype, long ldo, const float* qkv, long ld, int q_off, int k_off, int v_off, const void* qnorm, const void* knorm,
+                          int norm_dtype, float eps, const float* freq, int rot_dims, int layout, float mag, void* const* kspans, void* const* vspans, int span_stride,
+                          int span_len, const void* sink, int w_dtype, int sink_mode, float softcap, const float* gate, long ldg, const int32_t* tok_pos,
+                          const int32_t* ent_slot, const int32_t* ent_row0, int E, int T, int H, int G, int D, int DV, float scale, int nsplit, void* ws, size_t ws_bytes) {
+  if (int rc = gqa_check("gqa_decode_step", out, out_dtype, ldo, qkv, ld, kspans, vspans, span_stride, span_len, sink, w_dtype, sink_mode, gate, ldg, H, G, D, DV, 1, 0)) return rc;
+  DIHIP_REQUIRE(dihip_gqa_decode_step_supported(H, G, D, DV, span_len, DIHIP_BF16, rot_dims), DIHIP_PARAM_ERROR, "gqa_decode_step: %d heads over %d of %d / %d, rotation %d, span_len %d not served",
+                H, G, D, DV, rot_dims, span_len);
+  DIHIP_REQUIRE(E >= 0 && T >= E && tok_pos && ent_slot && ent_row0 && seq_dtype_ok(norm_dtype) && (rot_dims == 0 || freq) && (layout == 0 || layout == 1), DIHIP_PARAM_ERROR,
+                "gqa_decode_step: bad argument");
+  DIHIP_REQUIRE(q_off >= 0 && k_off >= 0 && v_off >= 0 && ld >= (long)q_off + (long)H * D && ld >= (long)k_off + (long)G * D && ld >= (long)v_off + (long)G * DV, DIHIP_PARAM_ERROR,
+                "gqa_decode_step: columns outside the rows");
+  DIHIP_REQUIRE(((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(qkv)) & 15u) == 0 && ldo % 4 == 0 && ld % 4 == 0 && q_off % 4 == 0, DIHIP_PARAM_ERROR,
+                "gqa_decode_step: query and output rows in 16-byte pieces");
+  DIHIP_REQUIRE(nsplit >= 1 && nsplit <= 1024 && (long)E * G <= INT32_MAX, DIHIP_PARAM_ERROR, "gqa_decode_step: bad split / request count");
+  DIHIP_REQUIRE(ws_bytes >= dihip_gqa_attn_mc_workspace_bytes(T, H, DV, nsplit) && (nsplit == 1 || ws), DIHIP_PARAM_ERROR, "gqa_decode_step: workspace too small");
+  if (E == 0) return DIHIP_SUCCESS;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  PrepArgs p{const_cast<float*>(qkv), ld, q_off, k_off, v_off, H, G, D, DV, G, qnorm, knorm, norm_dtype, eps, freq, rot_dims, layout, mag};
+  GqaArgs a{out, out_dtype, ldo, nullptr, 0, kspans, vspans, span_stride, span_len, sink, w_dtype, sink_mode, softcap, gate, ldg, nullptr, tok_pos,
+            ent_slot, ent_row0, nullptr, H, G, D, DV, scale, (float*)ws, T * H, 1, 0, 0};
+  int rc = DIHIP_SUCCESS;
+  auto go = [&](auto d, auto v) {
+    constexpr int D_ = decltype(d)::value, V_ = decltype(v)::value;
+    const size_t tiles = (size_t)4 * 64 * (D_ + V_) * 2, recs = (size_t)4 * 16 * (V_ + 4) * 4, bytes = tiles > recs ? tiles : recs;
+    auto kern = softcap > 0.f ? gqa_decode_step_kernel<D_, V_, true> : gqa_decode_step_kernel<D_, V_, false>;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) {
+      rc = DIHIP_RUNTIME_ERROR;
+      return;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)(E * G), nsplit), dim3(256), bytes, s, p, a);
+  };
+  constexpr std::integral_constant<int, 64> c64{};
+  constexpr std::integral_constant<int, 128> c128{};
+  if (D == 64 && DV == 64) go(c64, c64);
+  else if (D == 64) go(c64, c128);
+  else if (DV == 64) go(c128, c64);
+  else go(c128, c128);
+  DIHIP_REQUIRE(rc == DIHIP_SUCCESS, DIHIP_RUNTIME_ERROR, "gqa_decode_step: LDS refused");
+  if (nsplit > 1)
+    hipLaunchKernelGGL(gqa_attn_merge_kernel, dim3(T * H), dim3(256), 0, s, out, out_dtype, ldo, (const float*)ws, nsplit, T * H, H, 1, DV, DV, gate, ldg);
   return launch_status();
 }
 

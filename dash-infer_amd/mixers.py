@@ -320,6 +320,8 @@ class GroupedQueryAttention:
         self.vtables = [state.add_span_cache(n + ".v", self.G * vdim, cache_dtype) for n in names]
         self.ktable, self.vtable = self.ktables[0], self.vtables[0]
         self.mc = so.gqa_attn_mc_supported(dim, vdim, self.ktable) and self.n_in % 4 == 0 and (heads * dim) % 4 == 0
+        self.step = (self.mc and self.maps == 1 and not self.taps and not self.window and value_mix is None and talk is None and not elem_gate
+                     and so.gqa_decode_step_supported(self.H, self.G, dim, vdim, self.ktable, self.rot_dims))
         self.talk32, self.talk_mc = None, False
         if self.talk is not None:
             self.talk32 = self.talk.float().contiguous()
@@ -342,6 +344,10 @@ class GroupedQueryAttention:
         q, gate = a, a[:, self.g_lo:] if self.head_gate else None
         if self.out_gain is not None:
             gate = self.out_gain.expand(ctx.T, H)
+        if self.step and ctx.math == so.MATH_BF16 and ctx.max_count == 1:
+            return so.gqa_decode_step(a, 0, self.k_lo, self.v_lo, H, G, D, V, self.q_norm, self.k_norm, ctx.eps, self.freq, self.rot_dims, self.layout, self.mag, ktable, vtable,
+                                      ctx.tok_pos, ctx.ent_slot, ctx.ent_row0, ctx.max_pos, self.scale, self.sink, self.sink_mode, self.softcap, gate,
+                                      out=out if out is not None else ctx.act_buffer(H * V))
         if self.taps:
             one_row = ctx.max_count == 1
             q = so.qkv_conv_prep_append(a, self.conv, self.tails[run], one_row, H, G, D, V, self.q_norm, self.k_norm, ctx.eps, self.freq, self.rot_dims,

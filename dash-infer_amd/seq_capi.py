@@ -24,6 +24,9 @@ _SIGS = {
     "dihip_linear_workspace_bytes": (sz, [i32, i32, i32, i32, lng]),
     "dihip_linear_ws": (i32, [vp, vp, i32, lng, lng, i32, vp, i32, vp, vp, i32, lng, lng, vp, lng, i32, i32, i32, i32, i32, i32, i32, i32, f32, i32, vp,
                               sz]),
+    "dihip_gqa_decode_step_supported": (i32, [i32, i32, i32, i32, i32, i32, i32]),
+    "dihip_gqa_decode_step": (i32, [vp, vp, i32, lng, vp, lng, i32, i32, i32, vp, vp, i32, f32, vp, i32, i32, f32, vp, vp, i32, i32, vp, i32, i32, f32, vp, lng, vp, vp, vp,
+                                    i32, i32, i32, i32, i32, i32, f32, i32, vp, sz]),
     "dihip_linear_residual_dyt": (i32, [vp, vp, lng, vp, vp, vp, lng, f32, vp, vp, vp, i32, i32, i32, vp, sz]),
     "dihip_embed_dyt": (i32, [vp, vp, vp, vp, vp, f32, vp, vp, i32, i32]),
     "dihip_linear_gated_query": (i32, [i32, i32, i32, lng, vp]),

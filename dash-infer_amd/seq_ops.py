@@ -366,6 +366,31 @@ def gqa_attn_mc(q, ktable, vtable, tok_pos, ent_slot, ent_row0, ent_count, max_c
     return diff[3] if diff else o
 
 
+def gqa_decode_step_supported(H, G, D, DV, table, rot_dims):
+    return bool(lib().dihip_gqa_decode_step_supported(H, G, D, DV, table.span_len, _DT[table.dtype], int(rot_dims)))
+
+
+def gqa_decode_step(a, q_off, k_off, v_off, H, G, D, DV, qnorm, knorm, eps, freq, rot_dims, layout, mag, ktable, vtable, tok_pos, ent_slot, ent_row0, max_pos, scale,
+                    sink=None, sink_mode=SINK_NONE, softcap=0.0, gate=None, out=None, nsplit=None):
+    """one token of each request: qkv_prep_append and gqa_attn_mc in one launch (the rows a are left as they are); max_pos: the largest position (a host number)"""
+    T, E = a.shape[0], ent_slot.shape[0]
+    assert a.dtype == torch.float32 and ktable.row_elems == G * D and vtable.row_elems == G * DV and ktable.dtype == vtable.dtype
+    o = out if out is not None else torch.empty(T, H * DV, dtype=torch.float32, device=a.device)
+    if nsplit is None:       # up to 16 tiles a launch more costs what a split gives (8 key heads, 12 tiles: 11.0 us, in two splits 12.4; 24 tiles: 15.5, in six 12.5); past that
+        # one workgroup a unit (more take turns), of a tile or more to each wave
+        tiles = (max_pos + 64) // 64
+        nsplit = 1 if tiles <= 16 else max(1, min(256 // max(1, E * G), tiles // 4))
+    need = int(lib().dihip_gqa_attn_mc_workspace_bytes(T, H, DV, nsplit)) if nsplit > 1 else 0
+    ws = torch.empty(need, dtype=torch.uint8, device=a.device) if need else None
+    wn = qnorm if qnorm is not None else knorm
+    check(lib().dihip_gqa_decode_step(stream(), ptr(o), dt(o), _rows(o), ptr(a), _rows(a), q_off, k_off, v_off, ptr(qnorm), ptr(knorm), dt(wn) if wn is not None else F32_CODE,
+                                      float(eps), ptr(freq), int(rot_dims), int(layout), float(mag), ptr(ktable.ptrs), ptr(vtable.ptrs), ktable.max_spans, ktable.span_len,
+                                      ptr(sink), dt(sink) if sink is not None else F32_CODE, int(sink_mode), float(softcap or 0.0), ptr(gate),
+                                      _rows(gate) if gate is not None else 0, ptr(tok_pos), ptr(ent_slot), ptr(ent_row0), E, T, H, G, D, DV, float(scale), int(nsplit), ptr(ws),
+                                      need), "dihip_gqa_decode_step")
+    return o
+
+
 def maps_diff_norm(x, lam, out_scale, eps, H, DV, out=None):
     """x: f32 [T, H * 2 * DV] (two maps per head side by side) -> (first - lam * second) / its root mean square * out_scale, [T, H * DV]"""
     T = x.shape[0]

@@ -478,3 +478,62 @@ def test_attention_in_64_key_tiles(so, H, G, D, V, maps, span, kw, nsplit):
     for r in range(len(past)):       # weights rounded to bf16 (2^-9 each, independent) against sums of as many
         g, w = got[row0[r]:row0[r] + counts[r]].cpu().numpy(), want[r].cpu().numpy()
         assert rel_err(g, w) < 2.0 ** -8, (r, nsplit)
+
+
+@pytest.mark.parametrize("H,G,D,V,span,kw", [
+    (8, 2, 128, 128, 64, dict(norm=True, layout=1, rot=True)),
+    (16, 1, 128, 64, 128, dict(sink=True, gate=True, layout=0, rot=True)),
+    (6, 6, 64, 64, 64, dict(softcap=8.0, norm=True, layout=0, rot=True)),
+    (9, 3, 64, 128, 256, dict(layout=1, rot=True, sink_zero=True)),
+    (64, 8, 128, 128, 64, dict(norm=True, softcap=30.0, gate=True)),
+    (1, 1, 64, 64, 64, dict(norm=True, layout=1, rot=True, far=True)),       # (more than 64 tiles to a wave)
+])
+@pytest.mark.parametrize("nsplit", [1, 3, 40])
+def test_decoding_step_of_attention_in_one_launch(so, H, G, D, V, span, kw, nsplit):
+    """Preparation, append and attention of one token per request against the launches one by one: the first row, both sides of the borders of tiles and of pages, a wave
+    without a tile, splits without one; what other requests left in the pages are infinities."""
+    from dash_infer_amd.seq_state import SequenceStateManager
+    torch.manual_seed(H * 1000 + D + V + span)
+    pos = [0, 1, 63, 64, 255, 256, 300, 1087] + ([17000] if kw.get("far") else [])
+    E = len(pos)
+    st = SequenceStateManager(sum(pos) + 256 * E, E, span, "cuda")
+    kt, vt = st.add_span_cache("k", G * D, torch.bfloat16), st.add_span_cache("v", G * V, torch.bfloat16)
+    for t in (kt, vt):
+        t.pool.pool.view(torch.bfloat16).fill_(float("inf"))
+    nq, nk = H * D, G * D
+    rot = D if kw.get("rot") else 0
+    freq = torch.tensor([10000.0 ** (-2.0 * i / D) for i in range(D // 2)], dtype=torch.float32, device="cuda") if rot else None
+    qn, kn = (torch.rand(D, device="cuda") + 0.5, torch.rand(D, device="cuda") + 0.5) if kw.get("norm") else (None, None)
+    args = (H, G, D, V, qn, kn, 1e-5, freq, rot, kw.get("layout", 0), 1.25)
+    slots = []
+    for r, p in enumerate(pos):
+        st.admit(r)
+        st.reserve(r, p + 1)
+        st.upload()
+        slots.append(st.live[r].index)
+        if p:
+            old = torch.randn(p, nq + nk + G * V, device="cuda")
+            so.qkv_prep_append(old, 0, nq, nq + nk, *args, 0.0, None, None, kt, vt, i32([slots[r]] * p), i32(list(range(p))))
+    order = list(reversed(range(E)))                 # (entries in another order than their rows)
+    rows = torch.randn(E, nq + nk + G * V, device="cuda")
+    rows[:, :nq] *= 2.0
+    sink = torch.randn(H, device="cuda") if kw.get("sink") else None
+    mode = so.SINK_PER_HEAD if sink is not None else so.SINK_ZERO if kw.get("sink_zero") else so.SINK_NONE
+    gate = torch.rand(E, H, device="cuda") if kw.get("gate") else None
+    before = rows.clone()
+    pools = [t.pool.pool.clone() for t in (kt, vt)]
+    entry = (i32(pos), i32([slots[r] for r in order]), i32(order))
+    got = so.gqa_decode_step(rows, 0, nq, nq + nk, *args, kt, vt, *entry, max(pos), D ** -0.5, sink, mode, kw.get("softcap", 0.0), gate, nsplit=nsplit)
+    assert torch.equal(rows, before)
+    new = [t.pool.pool.clone() for t in (kt, vt)]
+    for t, p in zip((kt, vt), pools):
+        t.pool.pool.copy_(p)
+    so.qkv_prep_append(rows, 0, nq, nq + nk, *args, 0.0, None, None, kt, vt, i32(slots), i32(pos))
+    want = so.gqa_attn_mc(rows, kt, vt, *entry, i32([1] * E), 1, max(pos), H, G, D, V, D ** -0.5, sink, mode, kw.get("softcap", 0.0), gate, nsplit=1)
+    assert torch.equal(new[1], vt.pool.pool)
+    a, b = new[0].view(torch.bfloat16).float(), kt.pool.pool.view(torch.bfloat16).float()
+    assert torch.equal(a.isinf(), b.isinf())
+    a, b = a[~a.isinf()], b[~b.isinf()]
+    assert bool(((a - b).abs() <= 2.0 ** -7 * b.abs() + 2.0 ** -20).all())       # (the sum under a norm's root in another order: at most the neighbouring bf16, and rotation's cancelled last bits)
+    for r in range(E):               # weights rounded to bf16 (2^-9 each, independent) on both sides
+        assert rel_err(got[r].cpu().numpy(), want[r].cpu().numpy()) < 2.0 ** -7, (r, nsplit)
