@@ -944,6 +944,11 @@ __global__ __launch_bounds__(256, 2) void gqa_attn_tile_kernel(GqaArgs a, int gx
 // The splits' (maximum, denominator, sums) records of one (row, query vector) -> column threadIdx.x of its softmax-weighted sum
 // (0 for threads past DV; DV <= 256).  wgt / red: LDS scratch of the workgroup; the call synchronises it.
 __device__ __forceinline__ float merge_splits(const float* __restrict__ base, size_t stride, int nsplit, int Vp, int DV, float* wgt, float* red) {
+  const int r = min((int)threadIdx.x, DV - 1);
+  // the sums of eight splits on their way beside the records' maxima (a loop behind those waits a second time, and for each of the splits past a multiple of its step: six splits of 32 heads 1.3 us more)
+  float part[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) part[i] = base[min(i, nsplit - 1) * stride + r];
   float mloc[4], lloc[4], mx = -INFINITY;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -967,12 +972,15 @@ __device__ __forceinline__ float merge_splits(const float* __restrict__ base, si
   }
   den = block256_sum(den, red);      // (its barriers publish wgt)
   float acc = 0.f;
-  const int r = threadIdx.x;
-  if (r < DV) {
-#pragma unroll 8
-    for (int s = 0; s < nsplit; ++s) acc = __builtin_fmaf(wgt[s], base[s * stride + r], acc);
+  for (int s0 = 0; s0 < nsplit; s0 += 8) {
+    if (s0)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) part[i] = base[min(s0 + i, nsplit - 1) * stride + r];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (s0 + i < nsplit) acc = __builtin_fmaf(wgt[s0 + i], part[i], acc);
   }
-  return acc / den;
+  return threadIdx.x < DV ? acc / den : 0.f;
 }
 
 // one workgroup per (row, query vector)
@@ -1009,7 +1017,7 @@ __global__ __launch_bounds__(256) void gqa_attn_merge_diff_kernel(void* __restri
 //   * the token's own key and value are made by the wave whose tile holds their position, put over that tile's row in LDS (the page's is stale) and, behind the walk, into the page;
 //   * walks too long for a workgroup are split as the tile kernel's are (gqa_attn_merge_kernel adds them).
 // Bound by the chain of launch, slot, page pointer and tiles, and past that by one workgroup's LDS in flight (128 KB a unit): 32 heads over 8 of 128, one launch against three, in us
-// (keys: 100 / 700 / 1500 / 4000 / 12000): 1 request 8.0 / 11.0 / 12.5 / 13.1 / 18.1 (13.3 / 13.6 / 14.2 / 18.7 / 22.4), 4 requests 8.1 / 12.7 / 15.6 / 18.5 / 41.5 (13.5 / 16.3 / 18.3 /
+// (keys: 100 / 700 / 1500 / 4000 / 12000): 1 request 8.0 / 11.0 / 11.1 / 13.1 / 18.1 (13.3 / 13.6 / 14.2 / 18.7 / 22.4), 4 requests 8.1 / 12.7 / 14.3 / 18.5 / 41.5 (13.5 / 16.3 / 18.3 /
 // 23.1 / 48.4), 32 requests 9.8 / 22.5 / 41.7 / 94.0 (17.5 / 31.2 / 52.0 / 110).
 template <int D, int DV, bool CAP>
 __global__ __launch_bounds__(256) void gqa_decode_step_kernel(PrepArgs p, GqaArgs a) {

@@ -376,10 +376,10 @@ def gqa_decode_step(a, q_off, k_off, v_off, H, G, D, DV, qnorm, knorm, eps, freq
     T, E = a.shape[0], ent_slot.shape[0]
     assert a.dtype == torch.float32 and ktable.row_elems == G * D and vtable.row_elems == G * DV and ktable.dtype == vtable.dtype
     o = out if out is not None else torch.empty(T, H * DV, dtype=torch.float32, device=a.device)
-    if nsplit is None:       # up to 16 tiles a launch more costs what a split gives (8 key heads, 12 tiles: 11.0 us, in two splits 12.4; 24 tiles: 15.5, in six 12.5); past that
-        # one workgroup a unit (more take turns), of a tile or more to each wave
+    if nsplit is None:       # up to 16 tiles a launch more costs what a split gives (8 key heads, 12 tiles: 11.0 us, in two splits 12.4; 24 tiles: 15.5, in five 12.4, in six
+        # 11.1); past that a tile to each wave, while every workgroup finds a unit of its own
         tiles = (max_pos + 64) // 64
-        nsplit = 1 if tiles <= 16 else max(1, min(256 // max(1, E * G), tiles // 4))
+        nsplit = 1 if tiles <= 16 else max(1, min(256 // max(1, E * G), (tiles + 3) // 4))
     need = int(lib().dihip_gqa_attn_mc_workspace_bytes(T, H, DV, nsplit)) if nsplit > 1 else 0
     ws = torch.empty(need, dtype=torch.uint8, device=a.device) if need else None
     wn = qnorm if qnorm is not None else knorm
