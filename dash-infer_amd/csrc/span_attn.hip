@@ -1152,7 +1152,8 @@ int dihip_debug_attn_plan(int batch, int n_heads, int n_groups, int max_seq_len,
                           int* mfma) {
   if (batch <= 0 || n_heads <= 0 || n_groups <= 0 || n_heads % n_groups || max_seq_len <= 0) return DIHIP_SA_PARAM_ERROR;
   const bool m = attn_use_mfma(kv_mode, dtype);
-  const AttnPlan p = attn_plan(batch, n_heads, n_groups, max_seq_len, num_cus, m, 256, attn_wide_ok(kv_mode, dtype));
+  const int wide = attn_wide_ok(kv_mode, dtype);   // (in splits of four waves, also where the uint4 launch then takes fewer of eight)
+  const AttnPlan p = attn_plan(batch, n_heads, n_groups, max_seq_len, num_cus, m, 256, wide == ATTN_WIDE_U4 ? ATTN_WIDE_NO : wide);
   if (nsplits) *nsplits = p.nsplits;
   if (mfma) *mfma = m ? 1 : 0;
   return DIHIP_SUCCESS;
