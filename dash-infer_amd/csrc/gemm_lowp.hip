@@ -514,7 +514,7 @@ static PrefillTail prefill_tail_plan_rows(int wbits, int M, int N, int K, int gr
   t.mblocks = (M + bm - 1) / bm;
   t.tail_cb = t.col_blocks;
   t.ksplit = 1;
-  t.kunit = d.group ? std::max(d.group / d.KTILE, 1) : wbits == 8 ? 2 : 1;  // K parts hold whole groups (per-channel: what the kernel walks between two barriers)
+  t.kunit = d.group ? std::max(d.group / d.KTILE, 1) : 1;  // K parts hold whole groups
   static const bool on = !env_off("DIHIP_PREFILL_TAIL_SPLIT");
   int ncu = cached_num_cus();
   if (ncu <= 0) ncu = 256;
@@ -523,6 +523,7 @@ static PrefillTail prefill_tail_plan_rows(int wbits, int M, int N, int K, int gr
   const int tcb = (rem + t.mblocks - 1) / t.mblocks, tiles = tcb * t.mblocks;
   if (tiles > ncu / 2 || tcb > t.col_blocks) return t;
   const bool all = tcb == t.col_blocks;
+  if (all && wbits == 8 && !d.group) t.kunit = 2;   // (and, where every tile is split, what the kernel walks between two barriers)
   const int units = d.KT / t.kunit, at_least = all ? std::max(1, 512 / (d.KTILE * t.kunit)) : 1;
   int best = 1;
   for (int ks = 2; ks <= (all ? 16 : 8) && tiles * ks <= ncu && units / ks >= at_least; ++ks)

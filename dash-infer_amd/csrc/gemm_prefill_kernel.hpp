@@ -82,7 +82,7 @@ struct PrefillArgs {
   // applies the epilogue.  tail_cb == col_blocks: no split.
   int tail_cb;
   int ksplit;
-  int kunit;    // k-tiles that a K range must not cut (grouped weights: a group; per-channel: 1)
+  int kunit;    // k-tiles that a K range must not cut (grouped weights: a group; per-channel: 1, 8 bits where every tile is split: 2)
   int wide_out; // four neighbouring columns of an output (and residual) row make one aligned access
   float* slab;  // [tail tile][ksplit][bm][256] f32
 };
