@@ -684,7 +684,7 @@ def test_prefill_gemm_row_tiles(ops, M, wbits, G):
 
 # Two k-tiles of 64 between two barriers: K of one k-tile, of odd numbers of them whole and in parts, groups of an odd number of k-tiles (one at a time) and of two.
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,G", [(64, 264, 64, -1), (100, 512, 192, -1), (97, 20008, 320, -1), (130, 300, 4160, -1), (64, 512, 576, 192), (217, 520, 1152, 384), (150, 264, 2688, 128)])
+@pytest.mark.parametrize("M,N,K,G", [(64, 264, 64, -1), (100, 512, 192, -1), (97, 20008, 320, -1), (130, 300, 4160, -1), (64, 512, 576, 192), (217, 520, 1152, 384), (150, 264, 2688, 128), (2048, 4608, 704, -1)])
 def test_prefill_gemm_pairs_of_k_tiles(ops, M, N, K, G):
     test_prefill_gemm_all_epilogues(ops, M, N, K, 8, G)
 
