@@ -32,7 +32,8 @@
 // expansions, - 10 % without the LDS reads of all but the first k-step, - 44 % without all of them (1 600 TFLOP/s).  The parts add up:
 // what is left is instruction issue and power, not one wait.
 // Measured: 2048 rows of four W4 layers 5.29 ms with A through registers and the fix-up between the tiles, 5.05 as above, 4.86 with four
-// neighbouring columns per lane and an epilogue without branches; 326 rows of four W8 layers 1.76 -> 1.63 ms.
+// neighbouring columns per lane and an epilogue without branches; 326 rows of four W8 layers 1.76 -> 1.63 ms, 1.33 on tiles of
+// 112 rows with two k-tiles between two barriers.
 // A 2 x 4 grid of waves with 64 x 64 tiles (half the LDS reads, twice the expansions and twice the weight loads) made those four layers 6 % slower.
 #pragma once
 #include <atomic>

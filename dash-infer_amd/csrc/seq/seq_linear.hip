@@ -1,7 +1,7 @@
 // seq_linear.hip -- dihip_linear: y = epilogue(x . W^T + bias) for row-major [N, K] weights as checkpoints store them,
 // grouped (block-diagonal / per-head) forms included.  The kernels:
 //   linear_tile_kernel   every product and sum in f32, k ascending (DIHIP_MATH_F32; also any operand type / odd shape)
-//   linear_pipe_kernel   bf16 operands on the matrix cores, pipelined tiles of 256 x 256, 192 x 256 or 128 x 128, K split where tiles are few (seq_linear_tile.hip)
+//   linear_pipe_kernel   bf16 operands on the matrix cores, pipelined tiles of eleven sizes, K split where tiles are few (seq_linear_tile.hip)
 //   linear_mfma_kernel   the same for f32 rows (rounded to bf16), K % 64 != 0 or unaligned operands: 128 x 128 x 32 tiles through registers (segments of a few
 //                        tokens too where that is faster: seg_in_tiles)
 //   linear_stream_lds_kernel  bf16 operands, 2 .. 64 rows, K % 64 == 0 and 1024 or more (segments: 512): both streamed through LDS, K split over a workgroup's waves
