@@ -133,7 +133,9 @@ struct LinTilePlan {
   int parts;
   size_t slab;
 };
-LinTilePlan plan_linear_tile(int Tg, int N, int K, int groups, long ldx, bool split);   // (gated form: N is the columns of both matrices)
+// the slab of one K part: [row][group][column], every row of a group padded to whole 4 columns (the gated form: its two matrices as two groups)
+inline size_t lin_slab_part_bytes(int T, int N, int groups) { return (size_t)T * groups * (((size_t)N + 3) & ~(size_t)3) * sizeof(float); }
+LinTilePlan plan_linear_tile(int Tg, int N, int K, int groups, long ldx, bool split, bool gated = false);   // (gated: N columns of each matrix, groups 1)
 int launch_linear_tile(const LinArgs& a, const LinTilePlan& p, int Tg, int groups, float* slab, hipStream_t s);
 
 }  // namespace dihip

@@ -905,12 +905,12 @@ static bool gated_as_one(int T, int N, int K, long ldx) {
   if (T < 1 || N < 1 || K < 1 || K % 8 != 0 || ldx < K || ldx % 8 != 0) return false;
   if (T == 1) return !no_skinny && row_kernel(2 * N, K);
   if (T <= STREAM_MAX_ROWS) return K % 64 == 0 && K >= 1024 && (size_t)64 * K * 2 < (1ull << 31) && (size_t)T * ldx * 2 < (1ull << 31);
-  return plan_linear_tile(T, 2 * N, K, 1, ldx, false).ok;
+  return plan_linear_tile(T, N, K, 1, ldx, false, true).ok;
 }
 
 extern "C" int dihip_linear_gated_query(int T, int N, int K, long ldx, size_t* ws_bytes) {
   if (N > INT32_MAX / 2 || !gated_as_one(T, N, K, ldx)) return 0;
-  *ws_bytes = T > STREAM_MAX_ROWS ? plan_linear_tile(T, 2 * N, K, 1, ldx, true).slab : 0;
+  *ws_bytes = T > STREAM_MAX_ROWS ? plan_linear_tile(T, N, K, 1, ldx, true, true).slab : 0;
   return 1;
 }
 
@@ -931,8 +931,8 @@ extern "C" int dihip_linear_gated(void* stream, const void* x, long ldx, const v
     return launch_status();
   }
   if (T <= STREAM_MAX_ROWS) return launch_stream_lds_gated(a, s);
-  LinTilePlan p = plan_linear_tile(T, 2 * N, K, 1, ldx, ws != nullptr);
-  if (p.slab > ws_bytes) p = plan_linear_tile(T, 2 * N, K, 1, ldx, false);
+  LinTilePlan p = plan_linear_tile(T, N, K, 1, ldx, ws != nullptr, true);
+  if (p.slab > ws_bytes) p = plan_linear_tile(T, N, K, 1, ldx, false, true);
   return launch_linear_tile(a, p, T, 1, (float*)ws, s);
 }
 

@@ -312,21 +312,23 @@ struct TileShape {
 };
 constexpr TileShape SHAPES[] = {{256, 256, 1.33}, {224, 256, 1.23}, {192, 256, 1.09}, {160, 256, .95}, {128, 256, .82}, {256, 128, .78},
                                 {192, 128, .62}, {160, 128, .57}, {128, 128, .485}, {96, 128, .413}, {64, 128, .331}};
-LinTilePlan plan_linear_tile(int Tg, int N, int K, int groups, long ldx, bool split) {
+LinTilePlan plan_linear_tile(int Tg, int N, int K, int groups, long ldx, bool split, bool gated) {
   LinTilePlan best{};
+  const int cols = gated ? 2 * N : N;
+  const size_t slab_part = lin_slab_part_bytes(Tg, N, gated ? 2 : groups);
   // (a tile's rows of w, and of x where no map names them, are addressed with 32-bit offsets)
   if (K % LT_BK || K <= 0 || (size_t)256 * (size_t)K * 2 >= (1ull << 31) || (size_t)256 * (size_t)ldx * 2 >= (1ull << 31)) return best;
   constexpr size_t MOST = (size_t)192 << 20;   // of slab
   constexpr double LAUNCH_US = 2.5, TILE_US = 3.9, PARTS_US = 4.0, PART_US = 0.6, SLAB_BYTES_PER_US = 5.5e6, HBM_BYTES_PER_US = 4.6e6;
   constexpr int ncu = 256;
   const int all = K / LT_BK;
-  const double hbm_us = 2.0 * K * (double)N * groups / HBM_BYTES_PER_US, hbm4 = hbm_us * hbm_us * hbm_us * hbm_us;
+  const double hbm_us = 2.0 * K * (double)cols * groups / HBM_BYTES_PER_US, hbm4 = hbm_us * hbm_us * hbm_us * hbm_us;
   double best_us = 0;
   for (int sh = 0; sh < (int)(sizeof(SHAPES) / sizeof(SHAPES[0])); ++sh) {
-    const long tiles = (long)((Tg + SHAPES[sh].bm - 1) / SHAPES[sh].bm) * ((N + SHAPES[sh].bn - 1) / SHAPES[sh].bn) * groups;
+    const long tiles = (long)((Tg + SHAPES[sh].bm - 1) / SHAPES[sh].bm) * ((cols + SHAPES[sh].bn - 1) / SHAPES[sh].bn) * groups;
     for (int p = 1; p <= (split ? 16 : 1); ++p) {
       if (p > 1 && (all / p < 4 || tiles * p > 2 * ncu)) break;
-      const size_t slab = p > 1 ? (size_t)p * Tg * groups * ((N + 3) & ~3) * sizeof(float) : 0;
+      const size_t slab = p > 1 ? p * slab_part : 0;
       if (slab > MOST) break;
       const double body = (SHAPES[sh].step_us * ((all + p - 1) / p) + TILE_US) * ((tiles * p + ncu - 1) / ncu);
       const double us = LAUNCH_US + std::sqrt(std::sqrt(body * body * body * body + hbm4)) + (p > 1 ? PARTS_US + PART_US * p + 2.0 * slab / SLAB_BYTES_PER_US : 0);

@@ -58,3 +58,13 @@ def test_prompts_that_share_products(lens, rows, top_k, want):
     """Neighbours of 64 rows and more, up to the row limit; with experts up to the 2048 slots of the grouped launches."""
     decoder = importlib.import_module("dash-infer_amd.decoder")
     assert decoder.prompt_groups(lens, rows, top_k) == want
+
+
+@pytest.mark.parametrize("T,N,K", [(129, 3050, 5760), (193, 2050, 4096), (65, 1001, 2048), (65, 1003, 2048), (65, 1000, 2048), (129, 3051, 5760), (70, 66, 4096), (513, 2045, 8192)])
+def test_gated_products_workspace_holds_both_halves_of_every_part(T, N, K):
+    """A K part's slab is [row][two matrices][columns padded to whole four] f32: the workspace is a whole number (two and more) of them, whatever N % 4 is."""
+    seq_capi = importlib.import_module("dash-infer_amd.seq_capi")
+    need = C.c_size_t(0)
+    assert seq_capi.lib().dihip_linear_gated_query(T, N, K, K, C.byref(need)) == 1
+    part = T * 2 * (N + 3 & ~3) * 4
+    assert need.value % part == 0 and need.value // part >= 2, (need.value, part)
