@@ -740,6 +740,7 @@ def tp_ab_runs(args, torch, decoder, model, comm, batch, max_len, kv_mode, ids, 
                 run_n(max(2, args.warmup))
                 med, times = timed_blocks(run_n, args.steps, blocks, world, dev,
                                           before_block=lambda sv=sv: sv.set_state(ids, [SEQ_LEN + args.warmup] * batch))
+                sv.check_handoffs()
                 row.update(tokens_per_s=round(batch * args.steps / med, 2), ms_per_step=round(med / args.steps * 1e3, 4), hipGraph=graph_on,
                            blocks=blocks_summary(times, args.steps), backend_label=c.backend)
                 if not overlap:
@@ -1197,7 +1198,7 @@ def main():
         for _ in range(2):
             sess.step()
         torch.cuda.synchronize()
-        ok, summary = comm.finish_verification(torch.device("cuda", local_rank))
+        ok, summary = comm.finish_verification(torch.device("cuda", local_rank))   # (a row that did not come is NaN: not within the bound)
         if ok:
             comm.backend = f"{comm.backend} (verified against rccl: {summary})"
         else:
@@ -1237,6 +1238,8 @@ def main():
     elapsed, block_times = timed_blocks(run_n, args.steps, blocks, world, torch.device("cuda", local_rank),
                                         before_block=lambda: sess.set_state(ids, [SEQ_LEN + args.warmup] * batch))
     last_ids = sess.ids.tolist()
+    if world > 1:
+        sess.check_handoffs()   # (a peer's row that did not come: no number)
     python_runner = {"tokens_per_s": round(batch * args.steps / elapsed, 2), "ms_per_step": round(elapsed / args.steps * 1e3, 4)}
     host_runner = None
     if host_leg:

@@ -26,8 +26,9 @@
 // epoch e - 2 whatever scope the load names.  An allocation that cannot be made that way is an error, never a
 // silent coarse-grained substitute.
 //
-// Bounded: messages up to P2P_MAX_BYTES; a poll that sees no progress for tens of seconds traps (a lost peer must not hang the
-// GPU silently).  Developed on a one-GPU box: ranks as host threads / processes on one GPU exercise the protocol
+// Bounded: messages up to P2P_MAX_BYTES; a poll that sees no progress for tens of seconds gives up (a lost peer must not hang the
+// GPU): the communicator's error word is set, the workgroup's piece of the result is NaN, and later launches do not wait any more.  The
+// kernel ends normally -- a trap would end the GPU for every process on it --; whoever reads results reads the word with them.  Developed on a one-GPU box: ranks as host threads / processes on one GPU exercise the protocol
 // (tests/test_gpu_tp_loopback.py, test_gpu_p2p_processes.py); it has NOT run across xGMI yet -- bench.py therefore verifies
 // every all-reduce of its warm-up steps against RCCL before it times this path (decoder.P2PComm.verify).
 #include <algorithm>
@@ -52,7 +53,7 @@ constexpr size_t P2P_BUFFER_BYTES = P2P_DATA_BYTES + P2P_FLAGS_BYTES;
 struct P2PState {  // device-resident, private to the rank
   unsigned epoch;  // completed calls
   unsigned done;   // workgroups of the running call that have finished
-  unsigned error;  // a wait gave up (probe mode: dihip_p2p_ar_set_timeout(.., trap = 0)); the communicator is unusable afterwards
+  unsigned error;  // a wait gave up; the communicator is unusable afterwards
 };
 
 struct P2PComm {
@@ -60,7 +61,7 @@ struct P2PComm {
   unsigned char* bufs[P2P_MAX_RANKS];
   P2PState* state;
   unsigned long long max_spins = 1ull << 24;  // tens of seconds
-  int trap = 1;
+  int trap = 0;
 };
 
 struct P2PArgs {
@@ -85,9 +86,12 @@ template <int FT>
 __global__ __launch_bounds__(P2P_THREADS) void p2p_allreduce_kernel(const P2PArgs a) {
   constexpr int ES = FT == DIHIP_F32 ? 4 : 2;
   constexpr int EPW = 8 / ES;  // elements per 8-byte word
-  __shared__ unsigned s_epoch;
+  __shared__ unsigned s_epoch, s_lost;   // s_lost: a peer's row did not come, in this launch or an earlier one
   const int tid = threadIdx.x, wg = blockIdx.x, nwg = gridDim.x;
-  if (tid == 0) s_epoch = __hip_atomic_load(&a.state->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+  if (tid == 0) {
+    s_epoch = __hip_atomic_load(&a.state->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+    s_lost = __hip_atomic_load(&a.state->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
   __syncthreads();
   const unsigned epoch = s_epoch, parity = epoch & 1u;
   // this workgroup's piece, in 8-byte words (the message is padded to whole words by the host contract: count % EPW == 0)
@@ -114,13 +118,15 @@ __global__ __launch_bounds__(P2P_THREADS) void p2p_allreduce_kernel(const P2PArg
   // ---- wait: the flags addressed to me for this piece
   if (tid < a.nranks) {
     const unsigned* f = flag_ptr(a.bufs[a.rank], parity, tid, wg);
+    const bool lost_before = s_lost != 0u;
     unsigned long long spins = 0;
     // signed distance: flags only move forward, a flag "ahead" of this epoch cannot occur for this parity
     while ((int)(__hip_atomic_load(f, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_SYSTEM) - epoch) < 0) {
       __builtin_amdgcn_s_sleep(2);
-      if (++spins > a.max_spins) {  // without the peer's row for that long: fail loudly, never hang the box
+      if (lost_before || ++spins > a.max_spins) {  // without the peer's row for that long: say so and leave
         if (a.trap) __builtin_trap();
-        __hip_atomic_store(&a.state->error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // probe mode: report and leave
+        __hip_atomic_store(&a.state->error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_lost = 1u;   // (several lanes may: the same value)
         break;
       }
     }
@@ -128,6 +134,7 @@ __global__ __launch_bounds__(P2P_THREADS) void p2p_allreduce_kernel(const P2PArg
   __syncthreads();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "");
   // ---- sum in rank order (f32), write the result
+  const bool lost = s_lost != 0u;
   unsigned long long* dst = reinterpret_cast<unsigned long long*>(a.out);
   for (unsigned i = w0 + tid; i < w1; i += P2P_THREADS) {
     float acc[EPW];
@@ -143,6 +150,10 @@ __global__ __launch_bounds__(P2P_THREADS) void p2p_allreduce_kernel(const P2PArg
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[e] += ft_bits_to_f32<FT>((unsigned)(v >> (16 * e)) & 0xFFFFu);
       }
+    }
+    if (lost) {
+#pragma unroll
+      for (int e = 0; e < EPW; ++e) acc[e] = __builtin_nanf("");
     }
     unsigned long long o = 0;
     if constexpr (FT == DIHIP_F32) {
@@ -295,6 +306,13 @@ int dihip_p2p_ar_set_timeout(void* comm, unsigned long long max_spins, int trap)
   P2PComm* c = reinterpret_cast<P2PComm*>(comm);
   c->max_spins = max_spins;
   c->trap = trap ? 1 : 0;
+  return DIHIP_SUCCESS;
+}
+
+int dihip_p2p_ar_error_async(void* comm, void* stream, unsigned* error_host) {
+  DIHIP_REQUIRE(comm && error_host, DIHIP_PARAM_ERROR, "p2p_ar_error_async: bad argument");
+  const hipError_t rc = hipMemcpyAsync(error_host, &reinterpret_cast<P2PComm*>(comm)->state->error, sizeof(unsigned), hipMemcpyDeviceToHost, reinterpret_cast<hipStream_t>(stream));
+  DIHIP_REQUIRE(rc == hipSuccess, DIHIP_RUNTIME_ERROR, "p2p_ar_error_async: hipMemcpyAsync: %s", hipGetErrorString(rc));
   return DIHIP_SUCCESS;
 }
 

@@ -353,9 +353,10 @@ class P2PComm:
     The (rare, tiny) all-gather of the arg-max pairs and messages beyond the slot size go through `rccl`.
 
     guarded=True (make_comm backend "auto"): every local stage is followed by an agreement between the ranks, and the first
-    exchanges run in the kernel's probe mode (a wait that gives up sets an error word instead of trapping), so that a node
-    on which the IPC / peer path does not work ends in P2PUnavailable on all ranks -- not in a hang, a trap or a rank that
-    sits alone in a collective."""
+    exchanges wait for about a second only, so that a node on which the IPC / peer path does not work ends in P2PUnavailable
+    on all ranks -- not in a hang or a rank that sits alone in a collective.
+
+    A wait that gives up sets an error word and leaves NaN: check_arrivals() where the host reads results."""
     backend = "p2p-oneshot"
 
     def __init__(self, rank, nranks, device, rccl, guarded=False):
@@ -400,19 +401,16 @@ class P2PComm:
         dist.barrier()  # every rank has opened every buffer before the first push
         if guarded:
             def probe():
-                check(l.dihip_p2p_ar_set_timeout(self.handle, 1 << 19, 0), "dihip_p2p_ar_set_timeout")  # ~ a second, no trap
+                check(l.dihip_p2p_ar_set_timeout(self.handle, 1 << 19, 0), "dihip_p2p_ar_set_timeout")  # ~ a second
                 want = nranks * (nranks + 1) / 2
                 for dt, n in ((torch.float32, 8), (torch.bfloat16, 3584)):
                     for _ in range(4):
                         t = torch.full((n,), float(rank + 1), dtype=dt, device=device)
                         self.allreduce_(t)
-                        e = C.c_int(0)
-                        check(l.dihip_p2p_ar_error(self.handle, C.byref(e)), "dihip_p2p_ar_error")
-                        if e.value:
-                            raise RuntimeError("a peer's row did not arrive (probe timeout)")
+                        self.check_arrivals()
                         if abs(float(t[0]) - want) > 1e-3 or abs(float(t[-1]) - want) > 1e-3:
                             raise RuntimeError(f"wrong sum {float(t[0])} (expected {want})")
-                check(l.dihip_p2p_ar_set_timeout(self.handle, 1 << 24, 1), "dihip_p2p_ar_set_timeout")
+                check(l.dihip_p2p_ar_set_timeout(self.handle, 1 << 24, 0), "dihip_p2p_ar_set_timeout")
             stage("probe exchange", probe)
 
     verify = False   # set by bench.py around its eager verification steps: every peer-to-peer sum is checked against RCCL
@@ -434,6 +432,13 @@ class P2PComm:
             ulp = 2.0 ** -7 if t.dtype in (torch.bfloat16,) else (2.0 ** -10 if t.dtype == torch.float16 else 2.0 ** -20)
             self.verify_log.append((diff, scale, diff <= 4 * ulp * max(scale, 1e-6) * max(1, self.nranks // 2)))
         return t
+
+    def check_arrivals(self):
+        """synchronises; RuntimeError if a peer's row did not come (the communicator cannot be used any more)"""
+        e = C.c_int(0)
+        check(lib().dihip_p2p_ar_error(self.handle, C.byref(e)), "dihip_p2p_ar_error")
+        if e.value:
+            raise RuntimeError("peer-to-peer all-reduce: a peer's row did not arrive; results since the last check are invalid")
 
     def _device_sum(self, t):
         check(lib().dihip_p2p_allreduce_sum(self.handle, ops.cur_stream(), ops.ptr(t), ops.ptr(t), t.numel(), ops.dt_code(t)),
@@ -1009,7 +1014,10 @@ class DecodeSession:
         """At a synchronisation point of the caller: the fused attention block's error word (word 1 of its sync buffer, set when a bounded
         hand-off wait of a launch gave up).  Non-zero -> the steps since the last check are invalid: the buffer's invariants are restored,
         the session keeps the three-launch chain from here (captured graphs are dropped: capture again) and RuntimeError is raised --
-        never silently wrong tokens (ADVICE r5).  The C++ runner does the same in HipModelRunner::Sync."""
+        never silently wrong tokens.  The same for the peer-to-peer communicator's error word, after which the communicator cannot be used
+        any more.  The C++ runner does both in HipModelRunner::Sync."""
+        if hasattr(self.comm, "check_arrivals"):
+            self.comm.check_arrivals()
         if not getattr(self, "attn_block", False):
             return
         torch.cuda.synchronize()

@@ -291,14 +291,31 @@ AsStatus HipModelRunner::Sync(std::vector<int64_t>* ids) {
     *blk_err = 0u;
     if (dihip_decode_attn_block_status_async(s, blk->second->GetDataPtr(), blk_err) != 0) return Fail(AsStatus::ALLSPARK_RUNTIME_ERROR, "block status readback");
   }
+  // ... and so does the peer-to-peer communicator's
+  unsigned* ar_err = block_err_pinned_ ? block_err_pinned_ + 1 : nullptr;
+  const bool ar_live = ctx_->GetP2PComm() && ar_err;
+  if (ar_live) {
+    *ar_err = 0u;
+    if (dihip_p2p_ar_error_async(ctx_->GetP2PComm(), s, ar_err) != 0) return Fail(AsStatus::ALLSPARK_RUNTIME_ERROR, "all-reduce status readback");
+  }
   if (hipStreamSynchronize(s) != hipSuccess) return Fail(AsStatus::ALLSPARK_RUNTIME_ERROR, "stream synchronise");
-  if (blk_live && *blk_err != 0u) {
-    const unsigned code = *blk_err;
-    // the step(s) since the last synchronise are invalid; the ids on the device are garbage: keep the host's last good ones, switch the
-    // layers back to their three launches (Reshape re-decides, the captured step is dropped) and restore the buffer's invariants
+  // the step(s) since the last synchronise are invalid; the ids on the device are garbage: keep the host's last good ones
+  const auto roll_back = [&] {
     for (auto& gc : running_) gc->step -= std::min(gc->step, steps_since_sync_);  // back to the state of the last good synchronise
     steps_since_sync_ = 0;
     handoff_failed_ = true;
+  };
+  if (ar_live && *ar_err != 0u) {
+    roll_back();
+    dirty_ = true;
+    DropGraph();
+    return Fail(AsStatus::ALLSPARK_RUNTIME_ERROR,
+                "all-reduce: a peer's row did not come: the decode steps since the last synchronise are invalid and the communicator cannot be used any more");
+  }
+  if (blk_live && *blk_err != 0u) {
+    const unsigned code = *blk_err;
+    // the layers go back to their three launches (Reshape re-decides, the captured step is dropped), the buffer's invariants are restored
+    roll_back();
     ctx_->DisableAttnBlock();
     (void)dihip_decode_attn_block_reset(s, blk->second->GetDataPtr(), blk->second->GetSizeInByte());
     (void)hipStreamSynchronize(s);

@@ -44,7 +44,7 @@ class HipModelRunner {
   // stream synchronise + the ids generated by the last step, one per running request
   AsStatus Sync(std::vector<int64_t>* ids);
   const std::string& last_error() const { return err_; }
-  // the last Sync failed on the fused attention block's error word: the running requests' gen_ctx->step are back at the last good
+  // the last Sync failed on the fused attention block's error word, or the peer-to-peer communicator's: the running requests' gen_ctx->step are back at the last good
   // synchronise and next ids are that synchronise's; the OWNER of the virtual caches rewinds them to gen_ctx->step (or fails the requests)
   bool handoff_failed() const { return handoff_failed_; }
 
@@ -68,7 +68,7 @@ class HipModelRunner {
   std::unique_ptr<AsTensor> prompt_dev_;
   int64_t* ids_pinned_ = nullptr;   // [max_batch] staging up, [max_batch] staging down
   int32_t* lens_pinned_ = nullptr;  // [2 * max_batch]
-  bool handoff_failed_ = false;            // the last Sync failed on the attention block's error word: requests rolled back (gen_ctx->step), caches are the owner's to rewind
+  bool handoff_failed_ = false;            // the last Sync failed on the attention block's or the all-reduce's error word: requests rolled back (gen_ctx->step), caches are the owner's to rewind
   int steps_since_sync_ = 0;               // decode steps enqueued since the last successful Sync (rolled back when the block's error word is set)
   unsigned* block_err_pinned_ = nullptr;  // the fused attention block's error word, read back with the ids (Sync)
   int64_t* prompt_pinned_ = nullptr;

@@ -1,6 +1,8 @@
 """GPU parity of the glue ops (RMSNorm, RoPE, Binary ADD, SiLU*MUL, embedding, step counter)
 against oracle/glue.py (which restates csrc/core/kernel/cpu/layernorm.cpp:110-157 and
 rotary.cpp:22-106)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -109,3 +111,28 @@ def test_decode_state_from_device_tensors(B):
         decoder.DecodeSession.set_state(s, a, b)
         got.append((s.ids.tolist(), s.old_lens.tolist(), s.new_lens.tolist()))
     assert got[0] == got[1] == (ids.tolist(), lens.tolist(), (lens + 1).tolist())
+
+
+@pytest.mark.parametrize("dtype,n", [(torch.float32, 3584), (torch.bfloat16, 4), (torch.float16, 32 * 3584)])
+def test_p2p_allreduce_gives_up_without_its_peer(pkg, dtype, n):
+    """The bounded wait of a rank whose peer never calls (a short limit from the host): the kernel ends, the error word is set, the sums are NaN -- also of
+    the next call, which does not wait.  A rank alone is not affected."""
+    from dash_infer_amd import ops
+    from dash_infer_amd.capi import check, lib
+    bufs = [torch.zeros(int(lib().dihip_p2p_ar_buffer_bytes()), dtype=torch.uint8, device="cuda") for _ in range(2)]
+    for ranks in (1, 2):
+        comm = C.c_void_p()
+        check(lib().dihip_p2p_ar_create(C.byref(comm), 0, ranks, (C.c_void_p * ranks)(*[b.data_ptr() for b in bufs[:ranks]])), "create")
+        check(lib().dihip_p2p_ar_set_timeout(comm, 64, 0), "limit")
+        word = torch.full((1,), 7, dtype=torch.int32).pin_memory()
+        for _ in range(2):
+            x = torch.randn(n, device="cuda").to(dtype)
+            y = torch.zeros_like(x)
+            check(lib().dihip_p2p_allreduce_sum(comm, ops.cur_stream(), ops.ptr(x), ops.ptr(y), n, ops.dt_code(x)), "sum")
+            check(lib().dihip_p2p_ar_error_async(comm, ops.cur_stream(), word.data_ptr()), "word")
+            torch.cuda.synchronize()
+            e = C.c_int(9)
+            check(lib().dihip_p2p_ar_error(comm, C.byref(e)), "error")
+            assert int(word[0]) == e.value == ranks - 1
+            assert torch.equal(y, x) if ranks == 1 else bool(torch.isnan(y).all())
+        lib().dihip_p2p_ar_destroy(comm)

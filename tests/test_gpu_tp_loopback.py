@@ -30,7 +30,7 @@ def run_worker(*args, timeout=600, env_extra=None):
 # ranks of the C++ operator layer as threads on ONE GPU: [8-none-16-4-128-True] ended in the trap of the all-reduce's bounded wait three times.  Between the barrier
 # and the first launch every rank thread still reshapes its operators, which frees and allocates device memory; hipFree waits for everything on the device, a peer's
 # waiting all-reduce among it
-CPP_LAYER_RANK_THREADS = pytest.mark.skip(reason="rank threads of the C++ operator layer on one GPU: an all-reduce wait that gives up traps and ends the GPU for everyone")
+CPP_LAYER_RANK_THREADS = pytest.mark.skip(reason="rank threads of the C++ operator layer on one GPU: a rank that still frees memory waits for its peers' all-reduces, which wait for it")
 
 
 @pytest.mark.parametrize("nranks", [2, 4, 8])
