@@ -606,6 +606,12 @@ int dihost_request_stop(dihost_model_t m, int index) {
   if (st != AsStatus::ALLSPARK_SUCCESS) g_err = m->runner->last_error();
   return (int)st;
 }
+int dihost_decode_prepare(dihost_model_t m, int use_graph) {
+  if (!m->runner) return (int)AsStatus::ALLSPARK_INVALID_CALL_ERROR;
+  const AsStatus st = m->runner->PrepareDecode(use_graph != 0);
+  if (st != AsStatus::ALLSPARK_SUCCESS) g_err = m->runner->last_error();
+  return (int)st;
+}
 int dihost_decode_steps(dihost_model_t m, int n, int use_graph) {
   if (!m->runner) return (int)AsStatus::ALLSPARK_INVALID_CALL_ERROR;
   const AsStatus st = m->runner->DecodeSteps(n, use_graph != 0);

@@ -36,6 +36,10 @@ class HipModelRunner {
   int batch() const { return (int)running_.size(); }
   const std::vector<std::shared_ptr<GenerateContext>>& running() const { return running_; }
 
+  // What the next decoder step of the running batch needs before it can be launched, if it is not there yet: operators reshaped for the batch (tensors grow: hipMalloc, and
+  // hipFree, which waits for all work on the device), the step captured and instantiated.  DecodeSteps does it by itself; ranks that share one GPU and wait for one another in
+  // their all-reduces all go through this first, then launch -- a rank that still frees memory would wait for a peer's all-reduce, which waits for this rank.
+  AsStatus PrepareDecode(bool use_graph);
   // n decoder steps of the running batch.  use_graph: capture the step once, replay it (fused list only)
   AsStatus DecodeSteps(int n, bool use_graph);
   // Benchmarks: every running request back to `cached_len` tokens (the caller rewinds the requests' caches; the span tables and

@@ -39,6 +39,7 @@ _SIGS = {
     "dihost_request_adopt": (i32, [vp, i32, C.c_int64, i32, i32, C.POINTER(vp), C.POINTER(vp)]),
     "dihost_request_stop": (i32, [vp, i32]),
     "dihost_decode_steps": (i32, [vp, i32, i32]),
+    "dihost_decode_prepare": (i32, [vp, i32]),
     "dihost_sync_ids": (i32, [vp, C.POINTER(C.c_int64), i32]),
     "dihost_request_attach": (i32, [vp, i32, C.POINTER(C.c_int64), i32, i32, i32, i32, C.POINTER(C.c_int64), i32, i32, i32]),
     "dihost_request_put_token": (i32, [vp, i32, i32, C.c_int64]),
@@ -216,6 +217,10 @@ class Model:
 
     def request_stop(self, index):
         _ck(lib().dihost_request_stop(self.h, index), "request_stop")
+
+    def decode_prepare(self, graph=False):
+        """what the next step allocates, frees or waits for, without launching it: ranks that share one GPU all call it before any of them runs a step"""
+        _ck(lib().dihost_decode_prepare(self.h, int(graph)), "decode_prepare")
 
     def decode_steps(self, n=1, graph=False):
         _ck(lib().dihost_decode_steps(self.h, n, int(graph)), "decode_steps")

@@ -99,6 +99,9 @@ int dihost_request_stop(dihost_model_t m, int index);
  * rounded up to DIHIP_PLAN_BUCKET tokens (default 512; 0: for max_len), never for more than max_len: when the bucket moves the runner
  * synchronises, reshapes the operators and captures the step again (host/model_runner.cpp; HIPContext::PlanLength). */
 int dihost_decode_steps(dihost_model_t m, int n, int use_graph);
+/* everything of the next step that allocates, frees or waits for the device, without launching it (host/model_runner.h PrepareDecode): ranks that share one GPU call it,
+ * meet, and then run their steps; a running batch that has not changed needs it once per DIHIP_PLAN_BUCKET tokens */
+int dihost_decode_prepare(dihost_model_t m, int use_graph);
 /* synchronises the stream; ids generated by the last step, one per running request -> count (negative AsStatus on error) */
 int dihost_sync_ids(dihost_model_t m, int64_t* ids_host, int capacity);
 /* the Request slice behind the id-processing operators (PreProcessId / UpdateId / PostProcessId, host/id_ops_hip.cpp):

@@ -27,12 +27,6 @@ def run_worker(*args, timeout=600, env_extra=None):
     assert r.returncode == 0 and "P2P_WORKER_OK" in r.stdout, (r.stdout[-2000:], r.stderr[-3000:])
 
 
-# ranks of the C++ operator layer as threads on ONE GPU: [8-none-16-4-128-True] ended in the trap of the all-reduce's bounded wait three times.  Between the barrier
-# and the first launch every rank thread still reshapes its operators, which frees and allocates device memory; hipFree waits for everything on the device, a peer's
-# waiting all-reduce among it
-CPP_LAYER_RANK_THREADS = pytest.mark.skip(reason="rank threads of the C++ operator layer on one GPU: a rank that still frees memory waits for its peers' all-reduces, which wait for it")
-
-
 @pytest.mark.parametrize("nranks", [2, 4, 8])
 def test_p2p_allreduce_between_rank_threads(pkg, nranks):
     """dihip_p2p_allreduce_sum: sums of bf16 / f16 / f32 rows of decode sizes (one 7 KB row ... the slot limit), in place,
@@ -66,7 +60,6 @@ def test_tp_decode_matches_single_rank(pkg, monkeypatch, nranks, kv_mode, batch,
                                   lm_head_split="k" if comm_kind.endswith("-ksplit") else None)
 
 
-@CPP_LAYER_RANK_THREADS
 @pytest.mark.parametrize("nranks,kv_mode,batch,wbits,group,graph", [
     (2, "none", 1, 4, 128, False), (4, "none", 2, 4, 128, False), (8, "none", 1, 4, 128, False), (2, "i8", 3, 8, -1, False),
     # round 6: the step state is device-resident under TP too (DihipGreedy behind the K-split tail) -> every rank thread captures its step,
@@ -83,7 +76,6 @@ def test_tp_decode_through_the_cpp_operator_layer(pkg, nranks, kv_mode, batch, w
     run_worker("hostdecode", nranks, kv_mode, batch, wbits, group, "graph" if graph else "eager")
 
 
-@CPP_LAYER_RANK_THREADS
 @pytest.mark.parametrize("nranks,kv_mode,batch,wbits,group,n_kv", [(2, "none", 1, 4, 128, 2), (4, "none", 2, 4, 128, 4), (2, "i8", 3, 8, -1, 2)])
 def test_tp_ranks_split_one_serialized_export_at_load(pkg, tmp_path, nranks, kv_mode, batch, wbits, group, n_kv):
     """a whole-model .asparam written by the reference's writer (the converter's SplitModes + group_lists) ->
@@ -103,7 +95,6 @@ def test_tp_ranks_split_one_serialized_export_at_load(pkg, tmp_path, nranks, kv_
         assert np.array_equal(out["bound"][k], out["file"][k]), f"{k}: split-at-load differs from the tensor-bound slices"
 
 
-@CPP_LAYER_RANK_THREADS
 @pytest.mark.parametrize("nranks,batch,graph", [(2, 1, False), (2, 1, True), (4, 16, True)])
 def test_allreduce_beside_the_next_weights_in_the_cpp_layer(pkg, nranks, batch, graph):
     """North star: "RCCL all-reduce ... overlapped with the next GEMM on a side HIP stream" -- in the C++ operator layer:

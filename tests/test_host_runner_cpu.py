@@ -28,3 +28,20 @@ def test_a_row_that_did_not_come_fails_the_synchronise(stand_in, graph):
     """The peer-to-peer communicator's error word behind a step: RUNTIME_ERROR with the reason, the requests back at the last good synchronise."""
     out = stand_in("lost", 0, 2, 3, 4, graph)
     assert "a peer's row did not come" in out["err"] and out["word"] == 1 and out["after"] == 3
+
+
+# what may wait for work of other streams, or take and give back device memory
+MEMORY = {"hipMalloc", "hipFree", "hipExtMallocWithFlags", "hipHostMalloc", "hipHostFree", "hipMemcpy", "hipMemset", "hipGraphInstantiate", "hipGraphExecDestroy", "hipGraphDestroy",
+          "hipStreamBeginCapture", "hipStreamSynchronize"}
+
+
+@pytest.mark.parametrize("rank,nranks,batch,wbits,graph", [(0, 8, 16, 4, 1), (1, 8, 16, 4, 1), (3, 8, 1, 4, 0), (0, 2, 16, 8, 1), (1, 4, 16, 4, 0), (0, 1, 3, 4, 1)])
+def test_a_prepared_step_only_launches(stand_in, rank, nranks, batch, wbits, graph):
+    """Ranks that share a GPU wait for one another in their all-reduces: behind decode_prepare a step neither frees memory (hipFree waits for everything on the device) nor
+    allocates, captures or synchronises, before its first launch or behind it.  Without it a step does, a batch of 16 as late as its last operators."""
+    out = stand_in("prepare", rank, nranks, batch, wbits, graph)
+    assert ("hipGraphLaunch" if graph else "launch") in out["first"]
+    assert not MEMORY & set(out["first"]), [c for c in out["first"] if c in MEMORY]
+    assert not out["again"] and out["ids"] == batch
+    plain = stand_in("unprepared", rank, nranks, batch, wbits, graph)["first"]
+    assert "hipFree" in plain

@@ -354,6 +354,13 @@ def run_tp_decode_host(nranks, kv_mode, batch, wbits, group, weight_file=None, n
                         m.request_adopt(0, ids0[b], ks, vs)
                     torch.cuda.synchronize()
                 shared.bar.wait()
+                # operators reshaped and the step captured BEFORE any rank launches one: growing a tensor frees the old one, and hipFree waits for everything on
+                # the device, so also for the all-reduce of a peer that is waiting for this rank.  One rank at a time, when no other synchronises the device: a
+                # capture in progress does not survive that
+                with SETUP_LOCK:
+                    m.decode_prepare(graph=graph)
+                    st.synchronize()
+                shared.bar.wait()
                 out = []
                 for _ in range(steps):
                     m.decode_steps(1, graph=graph)   # graph: every rank thread captures its step once (its all-reduce launches inside) and replays it
