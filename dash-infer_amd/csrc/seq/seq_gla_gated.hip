@@ -30,8 +30,8 @@ struct GlaGatedArgs {
   float q_scale, inv_tau, eps;
   float* state;
   const int32_t* ent_slot; const int32_t* ent_row0; const int32_t* ent_count;
-  int E, H, D, DV, chunk, max_chunks;
-  float* ws;   // [E][max_chunks][H] records: D * DV (state) + D (product of the decays) floats
+  int E, H, D, DV, chunk, chunks;   // (chunks: records there are)
+  float* ws;   // [chunk in gg_chunk's order][H] records: D * DV (state) + D (product of the decays) floats
 };
 
 // log(1 + x), 0 <= x <= 1: 2 atanh(x / (2 + x)), whose argument is at most a third: eight terms of the series leave 1.4e-8 of it.  (log1pf keeps a sum in two floats: 75 instructions,
@@ -74,6 +74,16 @@ __device__ __forceinline__ bool gg_chunk(const int32_t* __restrict__ count, int 
   return false;
 }
 
+// the number of portion e's first chunk in that order (every lane of the wave)
+__device__ __forceinline__ int gg_first(const int32_t* __restrict__ count, int e, int chunk) {
+  const int lane = threadIdx.x & 63;
+  int n = 0;
+  for (int i = lane; i < e; i += 64) n += (max(count[i], 0) + chunk - 1) / chunk;
+#pragma unroll
+  for (int d = 32; d > 0; d /= 2) n += __shfl_xor(n, d, 64);
+  return n;
+}
+
 // PASS 0: whole portions from the slot's state.  PASS 1: every chunk but the last from S = 0 -> its record.  PASS 3: every chunk from the state that the carry left in its record
 // (portions of one chunk: from the slot's).  RS: 32-element steps of the rank.
 template <int DPT, int RS, int PASS>
@@ -93,7 +103,7 @@ __global__ __launch_bounds__(256, 2) void gla_gated_kernel(GlaGatedArgs a) {
   if (lo >= cnt || (PASS == 1 && lo + a.chunk >= cnt)) return;
   const int n = PASS == 0 ? cnt : min(a.chunk, cnt - lo);
   const size_t row0 = (size_t)first_row + lo;
-  float* wrec = PASS == 0 ? nullptr : a.ws + (((size_t)e * a.max_chunks + ch) * a.H + h) * ((size_t)D * DV + D);
+  float* wrec = PASS == 0 ? nullptr : a.ws + ((size_t)blockIdx.x * a.H + h) * ((size_t)D * DV + D);
   float* sp = a.state + ((size_t)slot * a.H + h) * D * DV;
   // columns past the head and rows past the end are loaded from the last one: loads under a condition each would be a branch each
   const bool col[2] = {lane < DV, lane + 64 < DV};
@@ -281,9 +291,11 @@ __global__ __launch_bounds__(256, 2) void gla_gated_kernel(GlaGatedArgs a) {
 __global__ __launch_bounds__(256) void gla_gated_carry_kernel(GlaGatedArgs a) {
   const int e = blockIdx.z, h = blockIdx.y, idx = (blockIdx.x * 256 + threadIdx.x) * 4;
   const int chunks = (a.ent_count[e] + a.chunk - 1) / a.chunk;
-  if (chunks < 2 || idx >= a.D * a.DV) return;
+  if (chunks < 2) return;   // (uniform)
+  const int first = gg_first(a.ent_count, e, a.chunk);
+  if (idx >= a.D * a.DV || first + chunks > a.chunks) return;
   const size_t size = (size_t)a.D * a.DV + a.D, step = (size_t)a.H * size;
-  float* w0 = a.ws + ((size_t)e * a.max_chunks * a.H + h) * size;
+  float* w0 = a.ws + ((size_t)first * a.H + h) * size;
   const int i = idx / a.DV;   // (DV % 4 == 0: one channel)
   f32x4_t S = *reinterpret_cast<const f32x4_t*>(a.state + ((size_t)a.ent_slot[e] * a.H + h) * a.D * a.DV + idx);
   constexpr int U8 = 8;       // eight chunks' records in flight
@@ -317,6 +329,10 @@ int gla_gated_chunk(int max_count, int H) {
   return max_count > 128 ? 32 : 16;
 }
 
+// no more chunks than these, however the T rows are cut into E portions of at most max_count: a record each (numbered portion by portion.  With room for max_count rows in
+// every portion, 700 rows beside 24 of one and 32 heads took 581 MB for the 46 chunks that there are; 47 records are 50 MB)
+long gla_gated_chunks(int T, int E, int max_count, int rows) { return std::min<long>((long)E * ((max_count + rows - 1) / rows), T / rows + (long)E); }
+
 }  // namespace
 }  // namespace dihip
 
@@ -326,10 +342,10 @@ extern "C" {
 
 int dihip_gla_gated_supported(int H, int D, int DV, int rank) { return gla_gated_fits(H, D, DV, rank) ? 1 : 0; }
 
-size_t dihip_gla_gated_workspace_bytes(int E, int max_count, int H, int D, int DV) {
-  if (E <= 0 || H <= 0 || D <= 0 || DV <= 0 || max_count <= 16) return 0;
+size_t dihip_gla_gated_workspace_bytes(int T, int E, int max_count, int H, int D, int DV) {
+  if (T <= 0 || E <= 0 || H <= 0 || D <= 0 || DV <= 0 || max_count <= 16) return 0;
   const int rows = gla_gated_chunk(max_count, H);
-  return (size_t)E * ((max_count + rows - 1) / rows) * H * ((size_t)D * DV + D) * sizeof(float);
+  return (size_t)gla_gated_chunks(T, E, max_count, rows) * H * ((size_t)D * DV + D) * sizeof(float);
 }
 
 int dihip_gla_gated(void* stream, void* y, int y_dtype, long ldy, const float* q, const float* k, const float* v, const float* gate, const float* a1, long ld,
@@ -344,12 +360,11 @@ int dihip_gla_gated(void* stream, void* y, int y_dtype, long ldy, const float* q
                 DIHIP_PARAM_ERROR, "gla_gated: queries, keys, a1, a2, state and workspace start on 16 bytes, and so does every row");
   if (T == 0 || E == 0 || max_count == 0) return DIHIP_SUCCESS;
   const bool chunked = max_count > 16;
-  DIHIP_REQUIRE(!chunked || (ws && ws_bytes >= dihip_gla_gated_workspace_bytes(E, max_count, H, D, DV)), DIHIP_PARAM_ERROR, "gla_gated: workspace too small");
+  DIHIP_REQUIRE(!chunked || (ws && ws_bytes >= dihip_gla_gated_workspace_bytes(T, E, max_count, H, D, DV)), DIHIP_PARAM_ERROR, "gla_gated: workspace too small");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int rows = chunked ? gla_gated_chunk(max_count, H) : max_count, chunks = (max_count + rows - 1) / rows;
+  const int rows = chunked ? gla_gated_chunk(max_count, H) : max_count, all = (int)gla_gated_chunks(T, E, max_count, rows);
   const GlaGatedArgs a{y, y_dtype, ldy, q, k, v, gate, a1, ld, (const uint16_t*)a2, (const uint16_t*)a2_bias, (const uint16_t*)gamma, q_scale, 1.f / tau, eps, state,
-                       ent_slot, ent_row0, ent_count, E, H, D, DV, rows, chunks, (float*)ws};
-  const int all = (int)std::min<long>((long)E * chunks, T / rows + E);   // no more chunks than these
+                       ent_slot, ent_row0, ent_count, E, H, D, DV, rows, all, (float*)ws};
   auto go = [&](auto dpt, auto rs) {
     constexpr int DPT = decltype(dpt)::value, RS = decltype(rs)::value, REC = 2 * GG_RB * gg_row(DPT) * 4, PART = GG_SUB * 4 * 128 * 4;
     static_assert(REC + PART <= 65536, "what a launch may ask for without a grant");

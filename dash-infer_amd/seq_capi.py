@@ -32,7 +32,7 @@ _SIGS = {
     "dihip_linear_gated_query": (i32, [i32, i32, i32, lng, vp]),
     "dihip_linear_gated": (i32, [vp, vp, lng, vp, vp, vp, i32, lng, i32, i32, i32, i32, vp, sz]),
     "dihip_gla_gated_supported": (i32, [i32, i32, i32, i32]),
-    "dihip_gla_gated_workspace_bytes": (sz, [i32, i32, i32, i32, i32]),
+    "dihip_gla_gated_workspace_bytes": (sz, [i32, i32, i32, i32, i32, i32]),
     "dihip_gla_gated": (i32, [vp, vp, i32, lng, vp, vp, vp, vp, vp, lng, vp, vp, vp, i32, f32, f32, f32, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp, sz]),
     "dihip_embed_sum": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32]),
     "dihip_embed_rows": (i32, [vp, vp, i32, lng, vp, vp, i32, lng, lng, f32, i32, i32]),

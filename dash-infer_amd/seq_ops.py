@@ -428,7 +428,7 @@ def gla_gated(rows, k_lo, v_lo, g_lo, a_lo, a2, a2_b, norm, q_scale, tau, eps, s
     T, E = rows.shape[0], ent_slot.shape[0]
     assert rows.dtype == torch.float32 and rows.shape[1] >= a_lo + a2.shape[1] and state.shape[1:] == (H, D, DV) and state.is_contiguous() and out.shape == (T, H * DV)
     assert a2.is_contiguous() and a2.shape[0] == H * D and a2_b.shape == (H * D,) and a2_b.is_contiguous() and norm.shape == (DV,) and norm.is_contiguous()
-    need = int(lib().dihip_gla_gated_workspace_bytes(E, int(max_count), H, D, DV))
+    need = int(lib().dihip_gla_gated_workspace_bytes(T, E, int(max_count), H, D, DV))
     ws = torch.empty(need, dtype=torch.uint8, device=rows.device) if need else None
     col = lambda c: C.c_void_p(rows.data_ptr() + 4 * c)
     check(lib().dihip_gla_gated(stream(), ptr(out), dt(out), _rows(out), col(0), col(k_lo), col(v_lo), col(g_lo), col(a_lo), _rows(rows), ptr(a2), ptr(a2_b), ptr(norm),

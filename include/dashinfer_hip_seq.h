@@ -238,9 +238,10 @@ int dihip_gla(void* stream, float* out, long ldo, const float* q, long ldq, cons
 /* The same from the rows of the input product to those of the output product, bf16 products:
  *   z = bf16(a1[t]) . a2^T + a2_bias,   the recurrence above,   y[t, h, :] = out / sqrt(mean(out^2) + eps) * gamma * gate[t, h, :]
  * q, k [H * D], v, gate [H * DV], a1 [rank]: columns of f32 rows of one stride ld;  a2 [H * D][rank], a2_bias [H * D], gamma [DV] bf16;  y of y_dtype.
- * dihip_gla_gated_supported: the sizes it serves.  Portions of more than 16 rows run in chunks side by side and need the workspace. */
+ * dihip_gla_gated_supported: the sizes it serves.  Portions of more than 16 rows run in chunks side by side and need the workspace (a record
+ * for every chunk that E portions of T rows in all, max_count of them at most in one, can make). */
 int dihip_gla_gated_supported(int H, int D, int DV, int rank);
-size_t dihip_gla_gated_workspace_bytes(int E, int max_count, int H, int D, int DV);
+size_t dihip_gla_gated_workspace_bytes(int T, int E, int max_count, int H, int D, int DV);
 int dihip_gla_gated(void* stream, void* y, int y_dtype, long ldy, const float* q, const float* k, const float* v, const float* gate, const float* a1, long ld,
                     const void* a2, const void* a2_bias, const void* gamma, int rank, float q_scale, float tau, float eps, float* state,
                     const int32_t* ent_slot, const int32_t* ent_row0, const int32_t* ent_count, int T, int E, int max_count, int H, int D, int DV, void* ws,

@@ -1,6 +1,7 @@
 """The mechanisms of the Vogusun design, each alone, against the float64 restatement in oracle/vogusun.py: the norm without
 statistics and the parallel residual step, grouped-query attention in both of its forms (norm, rotation layouts, sink, cap, gate,
 value mixing, pages), gated linear attention (state, portions, chunks), the gated and the routed feed-forward."""
+import ctypes as C
 import math
 
 import numpy as np
@@ -344,6 +345,32 @@ def test_gla_in_one_kernel(H, D, DV, rank, counts):
     want = want / np.sqrt((want ** 2).mean(-1, keepdims=True) + eps) * norm * g
     assert rel_err(y[:, :hv].cpu().numpy(), want.reshape(T, hv)) < 3e-5 and bool((y[:, hv:] == 7).all())
     assert rel_err(S_dev.cpu().numpy(), S_want) < 3e-5
+
+
+@pytest.mark.parametrize("H,counts", [(32, [200] + [1] * 24), (2, [17, 300, 1, 16, 33]), (3, [130] * 5)])
+def test_gla_in_one_kernel_stays_in_its_workspace(H, counts):
+    """long and short portions in any order with a workspace of exactly the queried size: the bytes behind it are left alone, and every portion comes out as it does by itself"""
+    load_pkg()
+    from dash_infer_amd import seq_ops as so
+    D, DV, rank, T, E = 64, 128, 64, sum(counts), len(counts)
+    g = torch.Generator("cuda").manual_seed(T)
+    hd, hv = H * D, H * DV
+    rows = torch.randn(T, 2 * hd + 2 * hv + rank, generator=g, device="cuda")
+    a2, b2, gamma = ((torch.randn(*s, generator=g, device="cuda") * 0.125).to(torch.bfloat16) for s in ((hd, rank), (hd,), (DV,)))
+    state, row0 = torch.randn(E, H, D, DV, generator=g, device="cuda"), np.cumsum([0] + counts[:-1])
+    need = int(so.lib().dihip_gla_gated_workspace_bytes(T, E, max(counts), H, D, DV))
+    ws = torch.full((need + (1 << 20),), 0x5A, dtype=torch.uint8, device="cuda")
+    col = lambda c: C.c_void_p(rows.data_ptr() + 4 * c)
+    S, y, slots, first, count = state.clone(), torch.empty(T, hv, device="cuda"), i32(list(range(E))), i32(row0), i32(counts)
+    so.check(so.lib().dihip_gla_gated(so.stream(), so.ptr(y), so.dt(y), hv, col(0), col(hd), col(2 * hd), col(2 * hd + hv), col(2 * hd + 2 * hv), rows.shape[1], so.ptr(a2), so.ptr(b2),
+                                      so.ptr(gamma), rank, 0.125, 4.0, 1e-5, so.ptr(S), so.ptr(slots), so.ptr(first), so.ptr(count), T, E, max(counts), H, D, DV,
+                                      so.ptr(ws), need), "gla_gated")
+    assert bool((ws[need:] == 0x5A).all())
+    for e, n in enumerate(counts):
+        S1, y1 = state[e:e + 1].clone(), torch.empty(n, hv, device="cuda")
+        part = rows[row0[e]:row0[e] + n].contiguous()
+        so.gla_gated(part, hd, 2 * hd, 2 * hd + hv, 2 * hd + 2 * hv, a2, b2, gamma, 0.125, 4.0, 1e-5, S1, i32([0]), i32([0]), i32([n]), n, H, D, DV, out=y1)
+        assert rel_err(y[row0[e]:row0[e] + n].cpu().numpy(), y1.cpu().numpy()) < 3e-5 and rel_err(S[e:e + 1].cpu().numpy(), S1.cpu().numpy()) < 3e-5
 
 
 # ---------------------------------------------------------------------------------------------------------------- feed-forward

@@ -68,3 +68,16 @@ def test_gated_products_workspace_holds_both_halves_of_every_part(T, N, K):
     assert seq_capi.lib().dihip_linear_gated_query(T, N, K, K, C.byref(need)) == 1
     part = T * 2 * (N + 3 & ~3) * 4
     assert need.value % part == 0 and need.value // part >= 2, (need.value, part)
+
+
+@pytest.mark.parametrize("H,counts", [(32, [700] + [1] * 24), (32, [2048]), (16, [500] + [1] * 13), (8, [300, 1, 129, 128, 65]), (2, [17] * 40), (128, [40, 17])])
+def test_gated_linear_attention_workspace_counts_the_chunks_there_are(H, counts):
+    """One record (64 x 128 state and 64 decays, f32) and head for every chunk that the portions can make, whatever their chunks' length, and at most one a portion more."""
+    seq_capi = importlib.import_module("dash-infer_amd.seq_capi")
+    T, E, size = sum(counts), len(counts), H * (64 * 128 + 64) * 4
+    need = seq_capi.lib().dihip_gla_gated_workspace_bytes(T, E, max(counts), H, 64, 128)
+    assert need % size == 0
+    fits = [rows for rows in (16, 32, 64) if sum(-(-c // rows) for c in counts) <= need // size <= T // rows + E]
+    assert fits, (need // size, counts)
+    if counts == [700] + [1] * 24:
+        assert need < 60e6
