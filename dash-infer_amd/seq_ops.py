@@ -419,7 +419,9 @@ def gla(q, k, v, z, q_scale, tau, state, ent_slot, ent_row0, ent_count, max_coun
 
 
 def gla_gated_supported(a2, a2_b, norm, H, D, DV):
-    return a2.dtype == a2_b.dtype == norm.dtype == torch.bfloat16 and bool(lib().dihip_gla_gated_supported(H, D, DV, a2.shape[1]))
+    """types, sizes, and weights that start where the kernel's loads need it (a view into a larger buffer may not)"""
+    return a2.dtype == a2_b.dtype == norm.dtype == torch.bfloat16 and a2.data_ptr() % 16 == 0 and a2_b.data_ptr() % 8 == 0 and \
+        bool(lib().dihip_gla_gated_supported(H, D, DV, a2.shape[1]))
 
 
 def gla_gated(rows, k_lo, v_lo, g_lo, a_lo, a2, a2_b, norm, q_scale, tau, eps, state, ent_slot, ent_row0, ent_count, max_count, H, D, DV, out):

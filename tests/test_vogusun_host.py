@@ -69,3 +69,18 @@ def test_oracle_sink_takes_its_share():
     assert np.allclose(ov.causal_attention_rows(q, k, v, 1.0, sink_one=False), 1.0)
     big = ov.causal_attention_rows(np.full((1, 1, 2), 10.0), np.full((1, 1, 2), 10.0), v, 1.0, softcap=2.0)
     assert np.allclose(big, 1.0) and math.isclose(2.0 * math.tanh(200.0 / 2.0), 2.0)
+
+
+def test_decay_weights_that_start_off_their_boundary_take_the_general_kernels():
+    """Parameters may be views into a larger buffer: the one-kernel form is for those whose 16-byte (bias: 8-byte) loads are aligned, the others keep the chain of launches."""
+    import torch
+    load_pkg()
+    from dash_infer_amd import seq_ops as so
+    H, D, V, rank = 2, 64, 128, 64
+    buf = torch.zeros(H * D * rank + 16, dtype=torch.bfloat16)
+    at = (-buf.data_ptr() % 16) // 2
+    a2 = lambda o: buf[at + o: at + o + H * D * rank].view(H * D, rank)
+    b2 = lambda o: buf[at + o: at + o + H * D]
+    norm = torch.ones(V + 1, dtype=torch.bfloat16)
+    assert so.gla_gated_supported(a2(0), b2(0), norm[1:], H, D, V) and so.gla_gated_supported(a2(8), b2(4), norm[:V], H, D, V)
+    assert not so.gla_gated_supported(a2(4), b2(0), norm[:V], H, D, V) and not so.gla_gated_supported(a2(0), b2(2), norm[:V], H, D, V)
