@@ -983,14 +983,15 @@ __device__ __forceinline__ float merge_splits(const float* __restrict__ base, si
   return threadIdx.x < DV ? acc / den : 0.f;
 }
 
-// one workgroup per (row, query vector)
+// one workgroup per (row, query vector); row0: the rows' numbers (NULL: 0, 1, ..)
 __global__ __launch_bounds__(256) void gqa_attn_merge_kernel(void* __restrict__ out, int odt, long ldo, const float* __restrict__ ws, int nsplit,
-                                                             int rows_total, int H, int maps, int DV, int Vp, const float* __restrict__ gate, long ldg) {
+                                                             int rows_total, int H, int maps, int DV, int Vp, const float* __restrict__ gate, long ldg,
+                                                             const int32_t* __restrict__ row0) {
   __shared__ float wgt[1024];
   __shared__ float red[4];
-  const int gi = blockIdx.x, HQ = H * maps, t = gi / HQ, hq = gi - t * HQ, h = hq / maps;
+  const int HQ = H * maps, u = blockIdx.x / HQ, hq = blockIdx.x - u * HQ, h = hq / maps, t = row0 ? row0[u] : u;
   const size_t rec = (size_t)Vp + 4;
-  const float v = merge_splits(ws + (size_t)gi * rec, (size_t)rows_total * rec, nsplit, Vp, DV, wgt, red);
+  const float v = merge_splits(ws + ((size_t)t * HQ + hq) * rec, (size_t)rows_total * rec, nsplit, Vp, DV, wgt, red);
   if (threadIdx.x < DV) st_any(out, (size_t)t * ldo + (size_t)hq * DV + threadIdx.x, odt, v * (gate ? gate[(size_t)t * ldg + h] : 1.f));
 }
 
@@ -1568,7 +1569,8 @@ int dihip_gqa_attn_mc(void* stream, void* out, int out_dtype, long ldo, const fl
     hipLaunchKernelGGL(gqa_attn_merge_diff_kernel, dim3(T * H), dim3(256), 0, s, diff_out, diff_dtype, ldd, (const float*)ws, nsplit, T * H * maps, H, DV,
                        Vp, gate, ldg, lam, out_scale, eps);
   else if (nsplit > 1)
-    hipLaunchKernelGGL(gqa_attn_merge_kernel, dim3(T * H * maps), dim3(256), 0, s, out, out_dtype, ldo, (const float*)ws, nsplit, T * H * maps, H, maps, DV, Vp, gate, ldg);
+    hipLaunchKernelGGL(gqa_attn_merge_kernel, dim3(T * H * maps), dim3(256), 0, s, out, out_dtype, ldo, (const float*)ws, nsplit, T * H * maps, H, maps, DV, Vp, gate, ldg,
+                       (const int32_t*)nullptr);
   else if (diff_out)
     hipLaunchKernelGGL(maps_diff_norm_kernel, dim3((unsigned)(((long)T * H + 3) / 4)), dim3(256), 0, s, diff_out, diff_dtype, ldd, (const float*)out, ldo, lam, out_scale,
                        eps, T * H, H, DV);
@@ -1618,7 +1620,7 @@ int dihip_gqa_decode_step(void* stream, void* out, int out_dtype, long ldo, cons
   else go(c128, c128);
   DIHIP_REQUIRE(rc == DIHIP_SUCCESS, DIHIP_RUNTIME_ERROR, "gqa_decode_step: LDS refused");
   if (nsplit > 1)
-    hipLaunchKernelGGL(gqa_attn_merge_kernel, dim3(T * H), dim3(256), 0, s, out, out_dtype, ldo, (const float*)ws, nsplit, T * H, H, 1, DV, DV, gate, ldg);
+    hipLaunchKernelGGL(gqa_attn_merge_kernel, dim3(E * H), dim3(256), 0, s, out, out_dtype, ldo, (const float*)ws, nsplit, T * H, H, 1, DV, DV, gate, ldg, ent_row0);
   return launch_status();
 }
 

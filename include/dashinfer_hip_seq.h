@@ -199,7 +199,7 @@ int dihip_gqa_attn(void* stream, void* out, int out_dtype, long ldo, const float
                    int span_stride, int span_len, int cache_dtype, const void* sink, int w_dtype, int sink_mode, float softcap,
                    const float* gate, long ldg, const int32_t* tok_slot, const int32_t* tok_pos, int T, int H, int G, int D,
                    int DV, float scale, int maps, int window, int keep_first);
-/* One token of each of E requests (decoding; row ent_row0[e], T rows in all) in one launch: dihip_qkv_prep_append's norm, rotation and append, and dihip_gqa_attn_mc's attention
+/* One token of each of E requests (decoding; row ent_row0[e], T rows in all, of which the others are left alone) in one launch: dihip_qkv_prep_append's norm, rotation and append, and dihip_gqa_attn_mc's attention
  * over keys 0 .. its position, from the rows qkv of the input product (not changed) to out.  Up to 16 heads a group, head sizes 64 / 128, bf16 pages of whole 64-key tiles,
  * the whole head rotated or none of it.  nsplit, ws: as dihip_gqa_attn_mc (1: no workspace, no merge launch). */
 int dihip_gqa_decode_step_supported(int H, int G, int D, int DV, int span_len, int cache_dtype, int rot_dims);

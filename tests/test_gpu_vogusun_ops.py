@@ -564,3 +564,28 @@ def test_decoding_step_of_attention_in_one_launch(so, H, G, D, V, span, kw, nspl
     assert bool(((a - b).abs() <= 2.0 ** -7 * b.abs() + 2.0 ** -20).all())       # (the sum under a norm's root in another order: at most the neighbouring bf16, and rotation's cancelled last bits)
     for r in range(E):               # weights rounded to bf16 (2^-9 each, independent) on both sides
         assert rel_err(got[r].cpu().numpy(), want[r].cpu().numpy()) < 2.0 ** -7, (r, nsplit)
+
+
+@pytest.mark.parametrize("nsplit", [1, 3])
+def test_decoding_step_of_attention_leaves_other_rows_alone(so, nsplit):
+    """fewer requests than rows, in any order: the rows that no request names keep what they held, the others are those of a call with their rows alone"""
+    from dash_infer_amd.seq_state import SequenceStateManager
+    H, G, D, T, order = 8, 2, 128, 6, [4, 0, 3]
+    st = SequenceStateManager(64 * 12, T, 64, "cuda")
+    kt, vt = st.add_span_cache("k", G * D, torch.bfloat16), st.add_span_cache("v", G * D, torch.bfloat16)
+    for r in range(T):
+        st.admit(r)
+        st.reserve(r, 90)
+    st.upload()
+    for t in (kt, vt):
+        t.pool.pool.view(torch.bfloat16).normal_()
+    slot = [st.live[r].index for r in range(T)]
+    rows, pos = torch.randn(T, (H + 2 * G) * D, device="cuda"), [70 + r for r in range(T)]
+    pools = [t.pool.pool.clone() for t in (kt, vt)]
+    call = lambda x, p, s, r0, out: so.gqa_decode_step(x, 0, H * D, (H + G) * D, H, G, D, D, None, None, 1e-5, None, 0, 0, 1.0, kt, vt, i32(p), i32(s), i32(r0), max(pos), D ** -0.5,
+                                                       out=out, nsplit=nsplit)
+    out = call(rows, pos, [slot[r] for r in order], order, torch.full((T, H * D), 7.0, device="cuda"))
+    for t, p in zip((kt, vt), pools):
+        t.pool.pool.copy_(p)
+    alone = call(rows[order].contiguous(), [pos[r] for r in order], [slot[r] for r in order], [0, 1, 2], torch.empty(3, H * D, device="cuda"))
+    assert torch.equal(out[order], alone) and bool((out[[r for r in range(T) if r not in order]] == 7.0).all())
