@@ -671,7 +671,8 @@ static AttnPlan attn_plan(int batch, int n_heads, int n_groups, int max_seq_len,
   // 511 / 543, 25 of 2000 (200 CUs) 544 / 555, 8 of 700 447 / 450
   if (mfma && wide == ATTN_WIDE_U4 && hpg <= 8 && wgs_per_cu == 0) {
     const long fit = std::max<long>(1, num_cus / base), most = std::max<long>(1, (max_seq_len + 255) / 256), ns = std::min<long>(std::min<long>(fit, most), split_cap);
-    if ((max_seq_len >= 448 * ns && 10 * ns * base >= 9 * num_cus && ns * base <= num_cus) || (p.nsplits > 32 && ns < p.nsplits)) {
+    // (never more splits than the four-wave plan's, which the workspace queries answer for: with DIHIP_ATTN_SPLIT_TOKENS above 256 that has fewer)
+    if ((ns <= p.nsplits && max_seq_len >= 448 * ns && 10 * ns * base >= 9 * num_cus && ns * base <= num_cus) || (p.nsplits > 32 && ns < p.nsplits)) {
       p.waves = 8;
       p.nsplits = (int)ns;
     }
@@ -1148,15 +1149,21 @@ int dihip_span_attn_run(void* output, const void* query, const void* const* k_sp
                     handle->num_cus, DIHIP_ACT_ROWMAJOR, 0, handle->counter_bytes);
 }
 
-int dihip_debug_attn_plan(int batch, int n_heads, int n_groups, int max_seq_len, int kv_mode, int dtype, int num_cus, int* nsplits,
-                          int* mfma) {
+int dihip_debug_attn_launch_plan(int batch, int n_heads, int n_groups, int max_seq_len, int kv_mode, int dtype, int num_cus, int* nsplits, int* mfma, int* waves,
+                                 size_t* partial_bytes) {
   if (batch <= 0 || n_heads <= 0 || n_groups <= 0 || n_heads % n_groups || max_seq_len <= 0) return DIHIP_SA_PARAM_ERROR;
   const bool m = attn_use_mfma(kv_mode, dtype);
-  const int wide = attn_wide_ok(kv_mode, dtype);   // (in splits of four waves, also where the uint4 launch then takes fewer of eight)
-  const AttnPlan p = attn_plan(batch, n_heads, n_groups, max_seq_len, num_cus, m, 256, wide == ATTN_WIDE_U4 ? ATTN_WIDE_NO : wide);
+  const AttnPlan p = attn_plan(batch, n_heads, n_groups, max_seq_len, num_cus, m, 256, attn_wide_ok(kv_mode, dtype));
   if (nsplits) *nsplits = p.nsplits;
   if (mfma) *mfma = m ? 1 : 0;
+  if (waves) *waves = p.waves;
+  if (partial_bytes) *partial_bytes = p.partial_bytes;
   return DIHIP_SUCCESS;
+}
+
+int dihip_debug_attn_plan(int batch, int n_heads, int n_groups, int max_seq_len, int kv_mode, int dtype, int num_cus, int* nsplits,
+                          int* mfma) {
+  return dihip_debug_attn_launch_plan(batch, n_heads, n_groups, max_seq_len, kv_mode, dtype, num_cus, nsplits, mfma, nullptr, nullptr);
 }
 
 }  // extern "C"

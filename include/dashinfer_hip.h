@@ -664,10 +664,12 @@ int dihip_debug_set_trace(void* buf, size_t bytes);
 /* launch plan of the decode GEMV for a shape (DIHIP_PARAM_ERROR when the general kernel is used) */
 int dihip_debug_gemv_plan(int wbits, int M, int N, int K, int group_size, int dual, int* blocks,
                           int* upb, int* wk, int* wn, size_t* lds_bytes);
-/* split plan of the decode attention for a shape on `num_cus` CUs (0: this device's count, 256 without a device), in splits of four waves:
- * where walks are long the uint4 launch takes fewer splits of eight in their place */
+/* split plan of the decode attention for a shape on `num_cus` CUs (0: this device's count, 256 without a device), as it is launched */
 int dihip_debug_attn_plan(int batch, int n_heads, int n_groups, int max_seq_len, int kv_mode, int dtype, int num_cus,
                           int* nsplits, int* mfma);
+/* the same with the waves of a split's workgroup and the bytes of the splits' records */
+int dihip_debug_attn_launch_plan(int batch, int n_heads, int n_groups, int max_seq_len, int kv_mode, int dtype, int num_cus, int* nsplits, int* mfma, int* waves,
+                                 size_t* partial_bytes);
 
 #ifdef __cplusplus
 }

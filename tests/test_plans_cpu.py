@@ -1,10 +1,13 @@
 """Launch-plan heuristics that need no GPU (host code of libdashinfer_hip.so): the split plan of the decode attention.
 
-The numbers are the ones the round-3 measurements settled on (profiles/r03_attn_timeline.txt, r03ab_*): 17 splits at batch 1,
-4 at BASELINE configs[2] (batch 32, uint4 cache), 16 -- not 32 -- for one TP = 8 rank of Qwen2-72B, 4 -- not 8 -- for the 57B MoE
+The numbers are measured ones (profiles/r03_attn_timeline.txt, r03ab_*; the uint4 rule's stand at attn_plan): 17 splits at batch 1,
+2 of eight waves for batch 32 of 2048 tokens on the uint4 cache, 16 -- not 32 -- for one TP = 8 rank of Qwen2-72B, 4 -- not 8 -- for the 57B MoE
 step; and the invariants behind them."""
 import ctypes as C
 import importlib
+import os
+import subprocess
+import sys
 
 import pytest
 
@@ -22,9 +25,9 @@ def plan(batch, n_heads, n_groups, max_len, kv="none", dtype=None, cus=256):
 
 @pytest.mark.parametrize("shape,expect", [
     ((1, 28, 4, 2049, "none"), 17),      # headline: 17 x 4 workgroups of 128 tokens
-    ((32, 28, 4, 2049, "u4"), 4),        # configs[2]: two workgroups per CU, 512 tokens per split
-    ((16, 8, 1, 4097, "none"), 16),      # configs[3] rank: one workgroup per CU (32 splits of 128 tokens measured 3 us slower)
-    ((16, 28, 4, 1025, "none"), 4),      # configs[4] step
+    ((32, 28, 4, 2049, "u4"), 2),        # one workgroup of eight waves per CU, 1024 tokens per split
+    ((16, 8, 1, 4097, "none"), 16),      # one workgroup per CU (32 splits of 128 tokens measured 3 us slower)
+    ((16, 28, 4, 1025, "none"), 4),
 ])
 def test_measured_shapes_keep_their_split_counts(shape, expect):
     b, n, g, L, kv = shape
@@ -42,6 +45,57 @@ def test_split_plan_invariants(batch, n, g, L):
     assert ns <= max(1, (L + 127) // 128)                # >= 128 tokens per split before rounding
     if batch * g * ns > 256 + batch * g:                 # clearly more than one workgroup per CU (past the rounding of the split
         assert ns == 1 or (L + ns - 1) // ns >= 256      # count) only while a split keeps >= 256 tokens
+
+
+def launch_plan(batch, n_heads, n_groups, max_len, kv="u4"):
+    ns, mf, waves, part = C.c_int(), C.c_int(), C.c_int(), C.c_size_t()
+    assert capi.lib().dihip_debug_attn_launch_plan(batch, n_heads, n_groups, max_len, capi.KV[kv], capi.BF16, 0, C.byref(ns), C.byref(mf), C.byref(waves), C.byref(part)) == 0
+    return ns.value, waves.value, part.value
+
+
+# uint4 cache, 256 CUs: eight waves where nine tenths of the CUs and more get one long split (448 tokens and more), or where four waves would leave more than 32 records
+@pytest.mark.parametrize("shape,expect", [
+    ((32, 28, 4, 2049), (2, 8)), ((32, 28, 4, 896), (2, 8)), ((32, 28, 4, 895), (2, 4)),       # 448 tokens a split, one less
+    ((16, 28, 4, 2048), (4, 8)), ((20, 28, 4, 1400), (3, 8)), ((29, 28, 4, 3000), (2, 8)),     # 256, 240 and 232 of 256 CUs have a split
+    ((20, 28, 4, 1000), (4, 4)),                                                               # 240, but 334 tokens a split
+    ((25, 28, 4, 2000), (6, 4)), ((28, 28, 4, 2000), (5, 4)), ((40, 28, 4, 2000), (4, 4)),     # 200, 224, 160
+    ((4, 28, 4, 8000), (16, 8)), ((4, 28, 4, 4096), (16, 4)), ((1, 28, 4, 4096), (32, 4)), ((1, 28, 4, 4097), (17, 8)), ((1, 28, 4, 8000), (32, 8)),
+    ((64, 28, 4, 8000), (1, 8)), ((65, 28, 4, 8000), (2, 4)),                                  # 256 CUs with one split each; more requests than that
+    ((32, 64, 4, 2049), (4, 4)),                                                               # 16 heads a group: four waves only
+])
+def test_uint4_splits_of_four_and_eight_waves(shape, expect):
+    assert launch_plan(*shape)[:2] == expect
+
+
+CHECK_PARTS = """
+import ctypes as C, importlib
+capi = importlib.import_module("dash-infer_amd.capi")
+l, seen = capi.lib(), set()
+for batch in (1, 2, 3, 5, 8, 16, 20, 25, 32, 33, 64, 65, 200):
+    for n, g in ((28, 4), (8, 1), (8, 2), (64, 8), (32, 32), (7, 7), (64, 4), (4, 1)):
+        for L in (1, 100, 257, 447, 448, 600, 895, 897, 1000, 1793, 2049, 4097, 8000, 8193, 32768):
+            for kv in ("none", "i8", "u4"):
+                ns, mf, waves, part = C.c_int(), C.c_int(), C.c_int(), C.c_size_t()
+                assert l.dihip_debug_attn_launch_plan(batch, n, g, L, capi.KV[kv], capi.BF16, 0, C.byref(ns), C.byref(mf), C.byref(waves), C.byref(part)) == 0
+                seen.add((kv, waves.value))
+                room = min(l.dihip_span_attn_decode_workspace_bytes(batch, n, 128, L, 0), l.dihip_span_attn_fused_workspace_bytes(batch, n, g, 128, L))
+                assert part.value <= room, (batch, n, g, L, kv, ns.value, waves.value, part.value, room)
+                # (buffers are sized for the longest length a request may have, plans made for shorter ones)
+                assert part.value <= l.dihip_span_attn_decode_workspace_bytes(batch, n, 128, 32768, 0)
+print("uint4, eight waves:", ("u4", 8) in seen)
+"""
+
+
+@pytest.mark.parametrize("tokens", [None, 32, 256, 512, 2000])
+def test_launched_splits_fit_the_workspace_queries(tokens):
+    """The records of the plan that is launched never need more than the queries answer, whatever DIHIP_ATTN_SPLIT_TOKENS is (read once: a process each)."""
+    env = dict(os.environ)
+    env.pop("DIHIP_ATTN_SPLIT_TOKENS", None)
+    if tokens:
+        env["DIHIP_ATTN_SPLIT_TOKENS"] = str(tokens)
+    r = subprocess.run([sys.executable, "-c", CHECK_PARTS], env=env, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-1500:]
+    assert "True" in r.stdout
 
 
 def test_plan_rejects_bad_shapes():
