@@ -464,6 +464,30 @@ def test_prompts_that_share_products_equal_prompts_alone(pkg, wbits, group, kv_m
             assert float((both.logits[b] - one.logits[0]).abs().max()) <= 2 * tol
 
 
+def test_next_token_of_a_prompt_whose_logits_hold_a_nan(pkg, monkeypatch):
+    """torch.argmax's answer: the NaN's column, in one of two rows"""
+    from dash_infer_amd import decoder, ops
+    cfg = decoder.ModelConfig("nan-test", **SMALL)
+    s = decoder.DecodeSession(decoder.build_random_model(cfg, decoder.QuantSpec(4, 128), seed=80), 2, max_len=64, span_len=16)
+    head = ops.lm_head
+
+    def with_nan(h, *a, out, **kw):
+        head(h, *a, out=out, **kw)
+        if out.data_ptr() == rows[0]:
+            out[0, 77] = float("nan")
+    real, rows = torch.empty, []
+
+    def empty(*size, **kw):                     # (the first row of the logits that prefill makes)
+        t = real(*size, **kw)
+        if size[:2] == (2, cfg.vocab):
+            rows.append(t.data_ptr())
+        return t
+    monkeypatch.setattr(ops, "lm_head", with_nan)
+    monkeypatch.setattr(torch, "empty", empty)
+    logits = s.prefill([[1, 2, 3], [4, 5]])
+    assert len(rows) == 1 and s.ids.tolist() == [77, int(logits[1].argmax())]
+
+
 @pytest.mark.parametrize("lens,rows", [([64] * 40, 4096),                     # one group of 40 prompts: more last rows than a streaming kernel takes
                                        ([100, 64, 92, 65, 191, 64, 300, 70], 256)])   # groups that end at, before and beyond the row limit; one prompt above it
 def test_groups_of_prompts_at_the_row_limit(pkg, monkeypatch, lens, rows):
