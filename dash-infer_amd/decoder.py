@@ -527,6 +527,13 @@ def prompt_groups(lens, max_rows, top_k=0):
     return groups
 
 
+def _behind_prefill(session):
+    """The current stream waits for the session's last context phase where that ran on another one (prefill itself does not wait for the device)"""
+    filled = getattr(session, "_filled", None)
+    if filled is not None and filled[0] != ops.cur_stream().value and not torch.cuda.is_current_stream_capturing():   # (a capture begins behind everything)
+        torch.cuda.current_stream().wait_event(filled[1])
+
+
 class DecodeSession:
     """Buffers + KV spans for a fixed batch; `step()` enqueues one decode step."""
 
@@ -672,6 +679,7 @@ class DecodeSession:
     # -- state ---------------------------------------------------------------------------
     def set_state(self, ids, lens):
         """ids: next input token per request; lens: tokens already in the cache."""
+        _behind_prefill(self)
         if all(isinstance(t, torch.Tensor) and t.device == self.ids.device and t.dtype == dt and t.shape == (self.B,) and t.is_contiguous()
                for t, dt in ((ids, torch.int64), (lens, torch.int32))):
             check(lib().dihip_decode_state(ops.cur_stream(), ops.ptr(self.ids), ops.ptr(self.old_lens), ops.ptr(self.new_lens), ops.ptr(ids), ops.ptr(lens), self.B),
@@ -708,8 +716,10 @@ class DecodeSession:
         RMSNorm + qkv GEMM(+bias) -> Rotary on the fused rows -> ContextSpanCopy of K, V into the request's spans ->
         causal prefill attention -> o GEMM + residual -> RMSNorm + gate/up GEMM + SwiGLU -> down GEMM + residual;
         final norm + lm_head on the last row.  Leaves the session ready to decode: lens = len(seq), ids = greedy next
-        token.  seqs: one token-id list per request (single rank).  Everything is enqueued on the current stream; nothing waits for the device."""
+        token.  seqs: one token-id list per request (single rank).  Everything is enqueued on the current stream; nothing waits for the device.
+        The session's own steps on another stream wait for it; whoever reads the logits, ids or spans there orders that, as with any tensor."""
         m, cfg = self.model, self.model.cfg
+        _behind_prefill(self)
         assert m.nranks == 1 and len(seqs) == self.B
         n, g, H, dev = self.n_loc, self.g_loc, self.H, self.h.device
         lens = [len(s) for s in seqs]
@@ -760,6 +770,9 @@ class DecodeSession:
                 ops.lm_head(last, m.final_norm, cfg.eps, m.lm_head, sc, out=logits[grp[0]:grp[-1] + 1])
         # (torch's: a row with a NaN gives the NaN's column, as it always has here; ops.argmax, which decoding uses, passes over them)
         self.set_state(torch.argmax(logits, dim=-1) if return_logits else torch.zeros(self.B, dtype=torch.int64, device=dev), lens_dev)
+        event = torch.cuda.Event()
+        event.record()
+        self._filled = (ops.cur_stream().value, event)
         return logits
 
     def _moe_rows(self, h, lw, sc):
@@ -786,6 +799,7 @@ class DecodeSession:
     # -- one decode step -------------------------------------------------------------------
     def step(self):
         m = self.model
+        _behind_prefill(self)
         ops.embedding(self.ids, m.embed, out=self.h)
         L = len(m.layers)
         for li in range(L):
@@ -1032,11 +1046,13 @@ class DecodeSession:
                                "invalid, the launch chain serves from here")
 
     def replay(self):
+        _behind_prefill(self)
         self.graph.replay()
 
     def replay_steps(self, n):
         """n decode steps: whole multi-step graphs first, single-step graphs for the remainder."""
         k = self.steps_per_graph
+        _behind_prefill(self)
         while self.graph_multi is not None and n >= k:
             self.graph_multi.replay()
             n -= k

@@ -464,6 +464,41 @@ def test_prompts_that_share_products_equal_prompts_alone(pkg, wbits, group, kv_m
             assert float((both.logits[b] - one.logits[0]).abs().max()) <= 2 * tol
 
 
+@pytest.mark.parametrize("how", ["step", "replay", "replay_steps", "set_state", "prefill"])
+def test_steps_on_another_stream_wait_for_the_prompt(pkg, how):
+    """prefill returns before the device has run it; what the session does next on another stream comes behind it all the same"""
+    from dash_infer_amd import decoder
+    cfg = decoder.ModelConfig("streams-test", **SMALL)
+    model = decoder.build_random_model(cfg, decoder.QuantSpec(4, 128), seed=81)
+    prompt, other = [5, 6, 7, 8] * 10, [9, 3] * 20
+
+    def run(busy):
+        s = decoder.DecodeSession(model, 1, max_len=64, span_len=16)
+        if how.startswith("replay"):
+            s.set_state([0], [0])
+            s.capture()
+        s.prefill([other])
+        torch.cuda.synchronize()
+        side = torch.cuda.Stream()
+        with torch.cuda.stream(side):
+            if busy:
+                torch.cuda._sleep(200_000_000)      # (the prompt's launches stand behind this)
+            s.prefill([prompt])
+        if not busy:
+            torch.cuda.synchronize()
+        if how == "prefill":
+            s.prefill([other[:30]])
+        elif how == "set_state":
+            s.set_state(torch.tensor([3], device="cuda"), torch.tensor([17], dtype=torch.int32, device="cuda"))
+            s.step()
+        else:
+            {"step": s.step, "replay": s.replay, "replay_steps": lambda: s.replay_steps(1)}[how]()
+        torch.cuda.synchronize()
+        return s.ids.tolist(), s.old_lens.tolist(), s.pool.pool.clone()
+    want, got = run(False), run(True)
+    assert got[:2] == want[:2] and torch.equal(got[2], want[2])
+
+
 def test_next_token_of_a_prompt_whose_logits_hold_a_nan(pkg, monkeypatch):
     """torch.argmax's answer: the NaN's column, in one of two rows"""
     from dash_infer_amd import decoder, ops
