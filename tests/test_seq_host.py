@@ -139,3 +139,17 @@ def test_seq_library_exports_every_header_symbol():
     assert lib.dihip_latent_window_attn_mc_supported(48, 64, seq_capi.BF16) == 0 and lib.dihip_latent_window_attn_mc_supported(64, 64, seq_capi.F32) == 0
     assert lib.dihip_latent_window_attn_mc_workspace_bytes(4, 32, 512, 16) == 16 * 4 * 32 * 516 * 4
     assert lib.dihip_gated_recurrence_chunked_workspace_bytes(2, 130, 100) == 2 * 3 * 2 * 100 * 4
+
+
+@pytest.mark.parametrize("gone", ["_RAW_STREAM", "_DEVICE"])
+def test_the_stream_handle_without_torchs_private_calls(monkeypatch, gone):
+    """Operators ask for the current stream's handle; a torch without the private calls is asked for the Stream object."""
+    from types import SimpleNamespace
+
+    from dash_infer_amd import ops
+    monkeypatch.setattr(ops, "_RAW_STREAM", lambda device: 0x1000 + device)
+    monkeypatch.setattr(ops, "_DEVICE", lambda: 3)
+    assert ops.cur_stream().value == 0x1003
+    monkeypatch.setattr(ops, gone, None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: SimpleNamespace(cuda_stream=0x2000))
+    assert ops.cur_stream().value == 0x2000
