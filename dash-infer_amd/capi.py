@@ -110,6 +110,7 @@ _SIGS = {
     "dihip_gemm_a16w16": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, f32, vp, sz, vp, i32]),
     "dihip_lm_head": (i32, [vp, vp, vp, vp, f32, vp, i32, i32, i32, vp, sz, vp, i32]),
     "dihip_argmax": (i32, [vp, vp, vp, i32, i32, vp, sz]),
+    "dihip_argmax_nan_first": (i32, [vp, vp, vp, i32, i32, vp, sz]),
     "dihip_argmax_advance": (i32, [vp, vp, vp, i32, i32, vp, sz, vp, vp]),
     "dihip_sample": (i32, [vp, vp, vp, i32, i32, vp, vp, vp, vp, vp, vp, vp, vp, vp]),
     "dihip_sample_rows": (i32, [vp, vp, vp, i32, i32, vp, vp, vp, vp, vp, vp, vp, i32]),

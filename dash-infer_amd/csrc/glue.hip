@@ -106,19 +106,27 @@ struct ArgPair {
   float v;
   int i;
 };
+// NAN_FIRST: a NaN before any number, as torch.argmax has it (else it is passed over)
+template <bool NAN_FIRST = false>
 __device__ __forceinline__ ArgPair arg_better(ArgPair a, ArgPair b) {
+  if constexpr (NAN_FIRST) {
+    const bool an = a.v != a.v, bn = b.v != b.v;
+    if (an || bn) return bn && (!an || b.i < a.i) ? b : a;
+  }
   return (b.v > a.v || (b.v == a.v && b.i < a.i)) ? b : a;
 }
+template <bool NAN_FIRST = false>
 __device__ __forceinline__ ArgPair wave_argmax(ArgPair p) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     ArgPair q{__shfl_xor(p.v, o, 64), __shfl_xor(p.i, o, 64)};
-    p = arg_better(p, q);
+    p = arg_better<NAN_FIRST>(p, q);
   }
   return p;
 }
 // stage 1: grid (blocks, M) -> partial[m][block]; stage 2: one wave per row.  Bound by launch and latency: four neighbours per load and four loads in flight where rows come in
 // 16-byte pieces (152064 columns, one row: 5.6 -> 4.7 us, 32 rows 6.7 -> 5.8)
+template <bool NAN_FIRST>
 __global__ __launch_bounds__(256) void argmax_stage1(ArgPair* __restrict__ partial, const float* __restrict__ logits,
                                                      int N) {
   __shared__ ArgPair red[4];
@@ -134,26 +142,27 @@ __global__ __launch_bounds__(256) void argmax_stage1(ArgPair* __restrict__ parti
 #pragma unroll
       for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) best = arg_better(best, ArgPair{v[u][r], min(q + u * step, quads - 1) * 4 + r});
+        for (int r = 0; r < 4; ++r) best = arg_better<NAN_FIRST>(best, ArgPair{v[u][r], min(q + u * step, quads - 1) * 4 + r});
     }
   } else {
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < N; i += gridDim.x * 256) best = arg_better(best, ArgPair{row[i], i});
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < N; i += gridDim.x * 256) best = arg_better<NAN_FIRST>(best, ArgPair{row[i], i});
   }
-  best = wave_argmax(best);
+  best = wave_argmax<NAN_FIRST>(best);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = best;
   __syncthreads();
   if (threadIdx.x == 0) {
-    ArgPair r = arg_better(arg_better(red[0], red[1]), arg_better(red[2], red[3]));
+    ArgPair r = arg_better<NAN_FIRST>(arg_better<NAN_FIRST>(red[0], red[1]), arg_better<NAN_FIRST>(red[2], red[3]));
     partial[(size_t)m * gridDim.x + blockIdx.x] = r;
   }
 }
 // adv_a / adv_b (optional): per-request u32 counters (sequence lengths) advanced by one with the sampled id
+template <bool NAN_FIRST>
 __global__ __launch_bounds__(64) void argmax_stage2(int64_t* __restrict__ ids, const ArgPair* __restrict__ partial,
                                                     int nblocks, uint32_t* adv_a, uint32_t* adv_b) {
   const int m = blockIdx.x;
   ArgPair r{-INFINITY, 0x7fffffff};
-  for (int i = threadIdx.x; i < nblocks; i += 64) r = arg_better(r, partial[(size_t)m * nblocks + i]);
-  r = wave_argmax(r);
+  for (int i = threadIdx.x; i < nblocks; i += 64) r = arg_better<NAN_FIRST>(r, partial[(size_t)m * nblocks + i]);
+  r = wave_argmax<NAN_FIRST>(r);
   if (threadIdx.x == 0) {
     ids[m] = r.i == 0x7fffffff ? 0 : (int64_t)r.i;  // an all-NaN row never beats the sentinel: a valid id, not 2^31 - 1
     if (adv_a) adv_a[m] += 1u;
@@ -335,28 +344,31 @@ int dihip_cast_to_f32(void* stream, float* y, const void* x, size_t count, int d
   return launch_status();
 }
 
-int dihip_argmax(void* stream, int64_t* ids, const float* logits, int M, int N, void* ws, size_t ws_bytes) {
-  DIHIP_REQUIRE(M >= 0 && N > 0 && ids && logits, DIHIP_PARAM_ERROR, "argmax: bad argument");
+}  // extern "C"
+template <bool NAN_FIRST>
+static int argmax_launch(const char* what, void* stream, int64_t* ids, const float* logits, int M, int N, void* ws, size_t ws_bytes, uint32_t* counters_a, uint32_t* counters_b) {
+  DIHIP_REQUIRE(M >= 0 && N > 0 && ids && logits, DIHIP_PARAM_ERROR, "%s: bad argument", what);
   if (M == 0) return DIHIP_SUCCESS;
   DIHIP_REQUIRE(ws && ws_bytes >= (size_t)M * ARGMAX_BLOCKS * sizeof(ArgPair), DIHIP_MEMORY_ERROR,
-                "argmax: workspace needs %zu bytes", (size_t)M * ARGMAX_BLOCKS * sizeof(ArgPair));
+                "%s: workspace needs %zu bytes", what, (size_t)M * ARGMAX_BLOCKS * sizeof(ArgPair));
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(argmax_stage1, dim3(ARGMAX_BLOCKS, M), dim3(256), 0, s, (ArgPair*)ws, logits, N);
-  hipLaunchKernelGGL(argmax_stage2, dim3(M), dim3(64), 0, s, ids, (const ArgPair*)ws, ARGMAX_BLOCKS, (uint32_t*)nullptr,
-                     (uint32_t*)nullptr);
+  hipLaunchKernelGGL(argmax_stage1<NAN_FIRST>, dim3(ARGMAX_BLOCKS, M), dim3(256), 0, s, (ArgPair*)ws, logits, N);
+  hipLaunchKernelGGL(argmax_stage2<NAN_FIRST>, dim3(M), dim3(64), 0, s, ids, (const ArgPair*)ws, ARGMAX_BLOCKS, counters_a, counters_b);
   return launch_status();
+}
+extern "C" {
+
+int dihip_argmax(void* stream, int64_t* ids, const float* logits, int M, int N, void* ws, size_t ws_bytes) {
+  return argmax_launch<false>("argmax", stream, ids, logits, M, N, ws, ws_bytes, nullptr, nullptr);
+}
+
+int dihip_argmax_nan_first(void* stream, int64_t* ids, const float* logits, int M, int N, void* ws, size_t ws_bytes) {
+  return argmax_launch<true>("argmax_nan_first", stream, ids, logits, M, N, ws, ws_bytes, nullptr, nullptr);
 }
 
 int dihip_argmax_advance(void* stream, int64_t* ids, const float* logits, int M, int N, void* ws, size_t ws_bytes,
                          uint32_t* counters_a, uint32_t* counters_b) {
-  DIHIP_REQUIRE(M >= 0 && N > 0 && ids && logits, DIHIP_PARAM_ERROR, "argmax_advance: bad argument");
-  if (M == 0) return DIHIP_SUCCESS;
-  DIHIP_REQUIRE(ws && ws_bytes >= (size_t)M * ARGMAX_BLOCKS * sizeof(ArgPair), DIHIP_MEMORY_ERROR,
-                "argmax_advance: workspace needs %zu bytes", (size_t)M * ARGMAX_BLOCKS * sizeof(ArgPair));
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(argmax_stage1, dim3(ARGMAX_BLOCKS, M), dim3(256), 0, s, (ArgPair*)ws, logits, N);
-  hipLaunchKernelGGL(argmax_stage2, dim3(M), dim3(64), 0, s, ids, (const ArgPair*)ws, ARGMAX_BLOCKS, counters_a, counters_b);
-  return launch_status();
+  return argmax_launch<false>("argmax_advance", stream, ids, logits, M, N, ws, ws_bytes, counters_a, counters_b);
 }
 
 // TP vocabulary-parallel greedy sampling: each rank reduces its logits slice to one (value, global
@@ -368,7 +380,7 @@ int dihip_argmax_partial(void* stream, void* pairs_out, const float* logits, int
   DIHIP_REQUIRE(ws && ws_bytes >= (size_t)M * ARGMAX_BLOCKS * sizeof(ArgPair), DIHIP_MEMORY_ERROR,
                 "argmax_partial: workspace needs %zu bytes", (size_t)M * ARGMAX_BLOCKS * sizeof(ArgPair));
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(argmax_stage1, dim3(ARGMAX_BLOCKS, M), dim3(256), 0, s, (ArgPair*)ws, logits, N);
+  hipLaunchKernelGGL(argmax_stage1<false>, dim3(ARGMAX_BLOCKS, M), dim3(256), 0, s, (ArgPair*)ws, logits, N);
   hipLaunchKernelGGL(argmax_merge_kernel, dim3(M), dim3(64), 0, s, (int64_t*)nullptr, (ArgPair*)pairs_out,
                      (const ArgPair*)ws, ARGMAX_BLOCKS, ARGMAX_BLOCKS, 1, index_offset);
   return launch_status();

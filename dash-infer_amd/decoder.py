@@ -768,8 +768,8 @@ class DecodeSession:
             if return_logits:
                 last = h[-1:] if len(grp) == 1 else torch.stack([h[hi - 1] for hi in cut[1:]])
                 ops.lm_head(last, m.final_norm, cfg.eps, m.lm_head, sc, out=logits[grp[0]:grp[-1] + 1])
-        # (torch's: a row with a NaN gives the NaN's column, as it always has here; ops.argmax, which decoding uses, passes over them)
-        self.set_state(torch.argmax(logits, dim=-1) if return_logits else torch.zeros(self.B, dtype=torch.int64, device=dev), lens_dev)
+        # (as torch.argmax has it: a row with a NaN gives the NaN's column.  Decoding's argmax passes over them)
+        self.set_state(ops.argmax(logits, nan_first=True) if return_logits else torch.zeros(self.B, dtype=torch.int64, device=dev), lens_dev)
         event = torch.cuda.Event()
         event.record()
         self._filled = (ops.cur_stream().value, event)

@@ -599,8 +599,9 @@ def silu_mul(gate, up):
     return y
 
 
-def argmax(logits, ws=None, out=None, advance=()):
-    """Greedy sampling; `advance`: up to two per-request u32 counter tensors incremented in the same launch."""
+def argmax(logits, ws=None, out=None, advance=(), nan_first=False):
+    """Greedy sampling; `advance`: up to two per-request u32 counter tensors incremented in the same launch; nan_first: a NaN before any number (torch.argmax), else it is passed over."""
+    assert not (advance and nan_first)
     M, N = logits.shape
     ids = out if out is not None else torch.empty(M, dtype=torch.int64, device=logits.device)
     ws = ws if ws is not None else torch.empty(M * 64 * 8, dtype=torch.uint8, device=logits.device)
@@ -610,7 +611,8 @@ def argmax(logits, ws=None, out=None, advance=()):
         check(lib().dihip_argmax_advance(cur_stream(), ptr(ids), ptr(logits), M, N, ptr(ws), ws.numel(), ptr(a), ptr(b)),
               "dihip_argmax_advance")
     else:
-        check(lib().dihip_argmax(cur_stream(), ptr(ids), ptr(logits), M, N, ptr(ws), ws.numel()), "dihip_argmax")
+        fn = lib().dihip_argmax_nan_first if nan_first else lib().dihip_argmax
+        check(fn(cur_stream(), ptr(ids), ptr(logits), M, N, ptr(ws), ws.numel()), "dihip_argmax")
     return ids
 
 

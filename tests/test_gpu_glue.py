@@ -99,6 +99,27 @@ def test_argmax_at_the_edges_of_its_loads(M, N):
     assert int(ops.argmax(logits)[0]) == 0
 
 
+@pytest.mark.parametrize("M,N", [(1, 4), (3, 1003), (5, 65540), (33, 152064), (2, 300001)])
+def test_argmax_with_nan(M, N):
+    """NaN first is torch.argmax, whatever else the row holds (infinities, NaN of either sign, nothing but NaN, the first of several); without it a NaN is passed over"""
+    from dash_infer_amd import ops
+    g = torch.Generator("cuda").manual_seed(N)
+    logits = torch.randn(M, N, generator=g, device="cuda")
+    assert torch.equal(ops.argmax(logits, nan_first=True), torch.argmax(logits, -1))
+    logits[:, N // 2] = float("inf")
+    logits[:, 1] = float("-inf")
+    assert torch.equal(ops.argmax(logits, nan_first=True), torch.argmax(logits, -1))
+    for m in range(M):
+        logits[m, (m * 7919 + N - 1) % N] = float("nan") if m % 2 else -float("nan")
+        logits[m, N - 1] = float("nan")
+    want = torch.argmax(logits, -1)
+    assert torch.equal(ops.argmax(logits, nan_first=True), want) and bool(torch.isnan(logits[torch.arange(M), want]).all())
+    plain = ops.argmax(logits)
+    assert torch.equal(plain, torch.argmax(torch.where(torch.isnan(logits), float("-inf"), logits), -1))
+    logits[0] = float("nan")
+    assert ops.argmax(logits, nan_first=True)[0] == 0 and ops.argmax(logits)[0] == 0
+
+
 @pytest.mark.parametrize("B", [1, 64, 65])
 def test_decode_state_from_device_tensors(B):
     """set_state of a session: the same state from device tensors (one launch) as from host values"""
