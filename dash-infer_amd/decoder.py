@@ -531,7 +531,7 @@ def _behind_prefill(session):
     """The current stream waits for the session's last context phase where that ran on another one (prefill itself does not wait for the device)"""
     filled = getattr(session, "_filled", None)
     if filled is not None and filled[0] != ops.cur_stream().value and not torch.cuda.is_current_stream_capturing():   # (a capture begins behind everything)
-        torch.cuda.current_stream().wait_event(filled[1])
+        torch.cuda.current_stream().wait_event(filled[1] or torch.cuda.default_stream().record_event())
 
 
 class DecodeSession:
@@ -770,9 +770,9 @@ class DecodeSession:
                 ops.lm_head(last, m.final_norm, cfg.eps, m.lm_head, sc, out=logits[grp[0]:grp[-1] + 1])
         # (as torch.argmax has it: a row with a NaN gives the NaN's column.  Decoding's argmax passes over them)
         self.set_state(ops.argmax(logits, nan_first=True) if return_logits else torch.zeros(self.B, dtype=torch.int64, device=dev), lens_dev)
-        event = torch.cuda.Event()
-        event.record()
-        self._filled = (ops.cur_stream().value, event)
+        # for steps on another stream.  (The default stream outlives every session: its event can wait until one is needed -- 7 us of a pass)
+        here = ops.cur_stream().value
+        self._filled = (here, torch.cuda.current_stream().record_event() if here else None)
         return logits
 
     def _moe_rows(self, h, lw, sc):

@@ -464,8 +464,9 @@ def test_prompts_that_share_products_equal_prompts_alone(pkg, wbits, group, kv_m
             assert float((both.logits[b] - one.logits[0]).abs().max()) <= 2 * tol
 
 
+@pytest.mark.parametrize("first", ["side", "default"])
 @pytest.mark.parametrize("how", ["step", "replay", "replay_steps", "set_state", "prefill"])
-def test_steps_on_another_stream_wait_for_the_prompt(pkg, how):
+def test_steps_on_another_stream_wait_for_the_prompt(pkg, how, first):
     """prefill returns before the device has run it; what the session does next on another stream comes behind it all the same"""
     from dash_infer_amd import decoder
     cfg = decoder.ModelConfig("streams-test", **SMALL)
@@ -479,20 +480,24 @@ def test_steps_on_another_stream_wait_for_the_prompt(pkg, how):
             s.capture()
         s.prefill([other])
         torch.cuda.synchronize()
-        side = torch.cuda.Stream()
-        with torch.cuda.stream(side):
+        streams = [torch.cuda.Stream(), torch.cuda.default_stream()]
+        a, b = streams if first == "side" else streams[::-1]
+        ids, lens = torch.tensor([3], device="cuda"), torch.tensor([17], dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        with torch.cuda.stream(a):
             if busy:
                 torch.cuda._sleep(200_000_000)      # (the prompt's launches stand behind this)
             s.prefill([prompt])
         if not busy:
             torch.cuda.synchronize()
-        if how == "prefill":
-            s.prefill([other[:30]])
-        elif how == "set_state":
-            s.set_state(torch.tensor([3], device="cuda"), torch.tensor([17], dtype=torch.int32, device="cuda"))
-            s.step()
-        else:
-            {"step": s.step, "replay": s.replay, "replay_steps": lambda: s.replay_steps(1)}[how]()
+        with torch.cuda.stream(b):
+            if how == "prefill":
+                s.prefill([other[:30]])
+            elif how == "set_state":
+                s.set_state(ids, lens)
+                s.step()
+            else:
+                {"step": s.step, "replay": s.replay, "replay_steps": lambda: s.replay_steps(1)}[how]()
         torch.cuda.synchronize()
         return s.ids.tolist(), s.old_lens.tolist(), s.pool.pool.clone()
     want, got = run(False), run(True)
