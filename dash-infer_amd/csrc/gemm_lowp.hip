@@ -938,7 +938,7 @@ static int run_gemm(hipStream_t stream, const GemmCall& c) {
   DIHIP_REQUIRE(!want_frag, DIHIP_PARAM_ERROR,
                 "gemm_lowp: the FRAG32 activation layout needs the small-batch kernel (see dihip_gemm_lowp_prefers_frag)");
   DIHIP_REQUIRE(!c.rowsq, DIHIP_PARAM_ERROR, "gemm_lowp: this shape is not served by a kernel that takes deferred row norms");
-  // context phase (M >= 64 rows): 128 x 256 workgroup tiles, A through LDS, every weight byte read once per 128 rows
+  // context phase (M >= 64 rows): workgroup tiles of 80 .. 128 rows x 256 columns, A through LDS, every weight byte read once per row tile
   // (gemm_prefill_kernel.hpp).  DIHIP_GEMM_PREFILL=0 keeps the general kernel (A/B, diagnostics).
   static const bool prefill_on = !env_off("DIHIP_GEMM_PREFILL");
   // a workgroup's rows of x and of the output, and a column tile of the weights, are addressed with 31-bit byte offsets

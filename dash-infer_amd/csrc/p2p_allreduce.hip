@@ -23,7 +23,7 @@
 // The receive buffer (slots + flags) is FINE-GRAINED / uncached device memory (hipExtMallocWithFlags, as RCCL allocates its
 // own flag and LL buffers): peers write it over xGMI while the owner's kernel polls and reads it in the same launch, and
 // coarse-grained memory (plain hipMalloc) is only coherent at kernel boundaries -- the owner's L2 may keep a line of
-// epoch e - 2 whatever scope the load names (ADVICE r2).  An allocation that cannot be made that way is an error, never a
+// epoch e - 2 whatever scope the load names.  An allocation that cannot be made that way is an error, never a
 // silent coarse-grained substitute.
 //
 // Bounded: messages up to P2P_MAX_BYTES; a poll that sees no progress for tens of seconds gives up (a lost peer must not hang the

@@ -407,7 +407,7 @@ def run_tp_decode_host(nranks, kv_mode, batch, wbits, group, weight_file=None, n
 
 
 def run_tp_decode_host_from_file(nranks, kv_mode, batch, wbits, group, n_kv, which, out_path):
-    """VERDICT r5 missing #1 / next #7: ONE serialized export of the whole model (written by the reference's own writer with the
+    """ONE serialized export of the whole model (written by the reference's own writer with the
     converter's SplitModes and group_lists) feeds every rank of a TP group -- each rank's C++ model splits the records for itself at load
     (dihost_weights_load_file: host/weight_file.h SliceForRank = the reference's WeightSplitter rules).  The decode must be BIT-IDENTICAL
     to the same ranks bound to dash-infer_amd/tp.py's slices as tensors, logits row and tokens, every step, every rank.
