@@ -680,7 +680,8 @@ class DecodeSession:
     def set_state(self, ids, lens):
         """ids: next input token per request; lens: tokens already in the cache."""
         _behind_prefill(self)
-        if all(isinstance(t, torch.Tensor) and t.device == self.ids.device and t.dtype == dt and t.shape == (self.B,) and t.is_contiguous()
+        # (one launch for tensors of the session's device while that is the current one: the launch goes to the current device's stream)
+        if all(isinstance(t, torch.Tensor) and t.device == self.ids.device and t.device.index == torch.cuda.current_device() and t.dtype == dt and t.shape == (self.B,) and t.is_contiguous()
                for t, dt in ((ids, torch.int64), (lens, torch.int32))):
             check(lib().dihip_decode_state(ops.cur_stream(), ops.ptr(self.ids), ops.ptr(self.old_lens), ops.ptr(self.new_lens), ops.ptr(ids), ops.ptr(lens), self.B),
                   "dihip_decode_state")

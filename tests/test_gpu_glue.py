@@ -134,6 +134,18 @@ def test_decode_state_from_device_tensors(B):
     assert got[0] == got[1] == (ids.tolist(), lens.tolist(), (lens + 1).tolist())
 
 
+def test_decode_state_while_another_device_is_current(monkeypatch):
+    """no launch on another device's stream: the copies find the session's device by themselves"""
+    from types import SimpleNamespace
+    from dash_infer_amd import decoder
+    s = SimpleNamespace(B=2, ids=torch.zeros(2, dtype=torch.int64, device="cuda"), **{k: torch.zeros(2, dtype=torch.int32, device="cuda") for k in ("old_lens", "new_lens")})
+    ids, lens = torch.tensor([5, 9], device="cuda"), torch.tensor([3, 4], dtype=torch.int32, device="cuda")
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    monkeypatch.setattr(decoder, "lib", lambda: pytest.fail("launched on the current device's stream"))
+    decoder.DecodeSession.set_state(s, ids, lens)
+    assert (s.ids.tolist(), s.old_lens.tolist(), s.new_lens.tolist()) == ([5, 9], [3, 4], [4, 5])
+
+
 @pytest.mark.parametrize("dtype,n", [(torch.float32, 3584), (torch.bfloat16, 4), (torch.float16, 32 * 3584)])
 def test_p2p_allreduce_gives_up_without_its_peer(pkg, dtype, n):
     """The bounded wait of a rank whose peer never calls (a short limit from the host): the kernel ends, the error word is set, the sums are NaN -- also of
