@@ -546,7 +546,10 @@ static PrefillTail prefill_tail_plan_rows(int wbits, int M, int N, int K, int gr
 // 64 rows 63 / 45, 150 rows 85 / 65, 326 rows 126 / 111, 513 rows 203 / 182; int8 64 rows 66 / 52, 326 rows 133 / 121).  An element's sum does not depend on it but through the K parts.
 static PrefillTail prefill_tail_plan(int wbits, int M, int N, int K, int group_size, bool dual) {
   PrefillTail best = prefill_tail_plan_rows(wbits, M, N, K, group_size, dual, PF_BM);
-  if (M < 64 || M > 1024 || (wbits != 4 && wbits != 8)) return best;   // (past 1024 rows, where the fit ends, the last row tile is a small part)
+  if (M < 64 || M > 1024 || (wbits != 4 && wbits != 8)) return best;
+  // (Past 1024 rows the fit ends, and the rule with it.  That is no line of the kernels': with the rule there too, us, 128 rows / by the rule, 1200 rows int4 3584 -> 3584 77.9 / 50.5,
+  // 18944 -> 3584 289 / 216, 3584 -> 18944 twice 392 / 375, int8 80.2 / 60.0, 306 / 254, 431 / 421; 1500 rows 76.5 / 58.5, 289 / 248, 450 / 441; 2048 and 3000 rows within 3 % but for
+  // 1024 -> 1536 (27 / 19); slower at 1030 .. 1150 rows 3584 -> 3584 (48 / 52).)
   int ncu = cached_num_cus();
   if (ncu <= 0) ncu = 256;
   const int KT = lowp_dims(wbits, N, K, group_size).KT;
