@@ -38,13 +38,15 @@ __device__ __forceinline__ void lin_rows(const LinArgs& a, int g, int& lo, int& 
 }
 __device__ __forceinline__ size_t lin_xrow(const LinArgs& a, int r) { return (size_t)(a.row_map ? a.row_map[r] : r); }
 
+// RES_TOO: a.res may be set.  (The residual form's code in an unrolled epilogue of 16 pieces -- linear_mfma_kernel -- kept the compiler from unrolling it: the sums went through scratch memory)
+template <bool RES_TOO = true>
 __device__ __forceinline__ void lin_epilogue(const LinArgs& a, int g, int t, int n, float v, int wdt) {
   if (a.bias) v += ld_any(a.bias, (size_t)g * a.N + n, wdt);
   const int col = g * a.N + n;
   if (col >= a.act_lo && col < a.act_hi) v = a.act == DIHIP_SEQ_ACT_SOFTCAP ? a.act_param * tanhf(v / a.act_param) : apply_act(v, a.act);
   const size_t o = (size_t)t * a.ldy + (size_t)g * a.yg + n;
   if (a.mul) v *= a.mul[(size_t)t * a.ldm + (a.mul_group ? (size_t)g : (size_t)g * a.yg + n)];
-  if (a.res) return lin_res_store(a, t, n, v, lin_res_load(a, t, n));
+  if (RES_TOO && a.res) return lin_res_store(a, t, n, v, lin_res_load(a, t, n));
   st_any(a.y, o, a.ydt, v);
 }
 
@@ -62,11 +64,36 @@ __device__ __forceinline__ f32x4_t lin_bias4(const LinArgs& a, int g, int n, boo
   const u32x2_t u = *reinterpret_cast<const u32x2_t*>((const uint16_t*)a.bias + (size_t)g * a.N + n);
   return f32x4_t{bf16_bits_to_f32(u[0] & 0xffffu), bf16_bits_to_f32(u[0] >> 16), bf16_bits_to_f32(u[1] & 0xffffu), bf16_bits_to_f32(u[1] >> 16)};
 }
-__device__ __forceinline__ void lin_epilogue4(const LinArgs& a, int g, int t, int n, f32x4_t v, const f32x4_t& bias, bool vec4) {
+// the residual form's: columns n .. n + 3 of row t, the product's sums v and nothing else on them
+__device__ __forceinline__ void lin_res4(const LinArgs& a, int t, int n, f32x4_t v, bool vec4) {
   if (!vec4) {
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      if (n + r < a.N) lin_epilogue(a, g, t, n + r, v[r], DIHIP_BF16);
+      if (n + r < a.N) lin_res_store(a, t, n + r, v[r], lin_res_load(a, t, n + r));
+    return;
+  }
+  if (n >= a.N) return;
+  f32x4_t* y = reinterpret_cast<f32x4_t*>((float*)a.y + (size_t)t * a.ldy + n);
+  f32x4_t x = *y;
+  if (a.res_a) v = *reinterpret_cast<const f32x4_t*>(a.res_a + (size_t)t * a.res_lda + n) + v;
+  x += v;
+  *y = x;
+  if (a.norm_w) {
+    const u32x2_t w = *reinterpret_cast<const u32x2_t*>((const uint16_t*)a.norm_w + n), b2 = *reinterpret_cast<const u32x2_t*>((const uint16_t*)a.norm_b + n);
+    uint32_t h[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      h[r] = f32_to_bf16_bits(tanhf(a.norm_alpha * x[r]) * bf16_bits_to_f32((w[r >> 1] >> (r & 1) * 16) & 0xffffu) + bf16_bits_to_f32((b2[r >> 1] >> (r & 1) * 16) & 0xffffu));
+    *reinterpret_cast<u32x2_t*>(a.h16 + (size_t)t * a.N + n) = u32x2_t{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+  }
+}
+template <bool RES_TOO = true>
+__device__ __forceinline__ void lin_epilogue4(const LinArgs& a, int g, int t, int n, f32x4_t v, const f32x4_t& bias, bool vec4) {
+  if (RES_TOO && a.res) return lin_res4(a, t, n, v, vec4);   // (uniform; no bias, activation or factor beside it)
+  if (!vec4) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (n + r < a.N) lin_epilogue<false>(a, g, t, n + r, v[r], DIHIP_BF16);
     return;
   }
   if (n >= a.N) return;
@@ -82,22 +109,6 @@ __device__ __forceinline__ void lin_epilogue4(const LinArgs& a, int g, int t, in
     else v *= *reinterpret_cast<const f32x4_t*>(a.mul + (size_t)t * a.ldm + (size_t)g * a.yg + n);
   }
   const size_t o = (size_t)t * a.ldy + (size_t)g * a.yg + n;
-  if (a.res) {
-    f32x4_t* y = reinterpret_cast<f32x4_t*>((float*)a.y + o);
-    f32x4_t x = *y;
-    if (a.res_a) v = *reinterpret_cast<const f32x4_t*>(a.res_a + (size_t)t * a.res_lda + n) + v;
-    x += v;
-    *y = x;
-    if (a.norm_w) {
-      const u32x2_t w = *reinterpret_cast<const u32x2_t*>((const uint16_t*)a.norm_w + n), b2 = *reinterpret_cast<const u32x2_t*>((const uint16_t*)a.norm_b + n);
-      uint32_t h[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        h[r] = f32_to_bf16_bits(tanhf(a.norm_alpha * x[r]) * bf16_bits_to_f32((w[r >> 1] >> (r & 1) * 16) & 0xffffu) + bf16_bits_to_f32((b2[r >> 1] >> (r & 1) * 16) & 0xffffu));
-      *reinterpret_cast<u32x2_t*>(a.h16 + (size_t)t * a.N + n) = u32x2_t{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
-    }
-    return;
-  }
   if (a.ydt == DIHIP_F32) *reinterpret_cast<f32x4_t*>((float*)a.y + o) = v;
   else *reinterpret_cast<u32x2_t*>((uint16_t*)a.y + o) = u32x2_t{f32_to_bf16_bits(v[0]) | (f32_to_bf16_bits(v[1]) << 16),
                                                                   f32_to_bf16_bits(v[2]) | (f32_to_bf16_bits(v[3]) << 16)};

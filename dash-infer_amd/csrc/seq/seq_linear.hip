@@ -100,7 +100,9 @@ __device__ __forceinline__ u32x4_t load8_bf16(const void* p, size_t i, int kleft
   return r;
 }
 
-template <int XT, bool VEC>
+// RES: the residual form, a kernel of its own: its code beside the other epilogue's was too much to unroll, the sums were indexed in scratch memory (f32 rows, 2048 of 4096 ->
+// 4096 188 -> 687 us)
+template <int XT, bool VEC, bool RES>
 __global__ __launch_bounds__(256) void linear_mfma_kernel(LinArgs a, bool vec4) {
   constexpr int BK = 32, UPR = BK / 8, UN = 128 * UPR / 256;   // k per step (64 measured slower: fewer workgroups per CU), 16-byte units per tile row, units per thread
   constexpr int LD = BK + 8;  // bf16 elements per LDS row: 8 of padding (80 bytes: 16-byte aligned fragments)
@@ -168,7 +170,9 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(LinArgs a, bool vec4) 
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int t = m0 + wm * 64 + i * 16 + (lane & 15);
-      if (t < t_hi) lin_epilogue4(a, g, t, n, acc[i][j], b, vec4);
+      if (t >= t_hi) continue;
+      if constexpr (RES) lin_res4(a, t, n, acc[i][j], vec4);
+      else lin_epilogue4<false>(a, g, t, n, acc[i][j], b, vec4);
     }
   }
 }
@@ -873,11 +877,14 @@ static int linear_impl(void* stream, const void* x, int x_dtype, long ldx, long 
     DIHIP_REQUIRE(grid.y <= 65535, DIHIP_PARAM_ERROR, "linear: too many rows for one launch");
     const bool vec4 = lin_vec4(a);
     if (x_dtype == DIHIP_F32) {
-      if (vec) hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_F32, true>), grid, dim3(256), 0, s, a, vec4);
-      else hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_F32, false>), grid, dim3(256), 0, s, a, vec4);
+      if (vec) hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_F32, true, false>), grid, dim3(256), 0, s, a, vec4);
+      else hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_F32, false, false>), grid, dim3(256), 0, s, a, vec4);
+    } else if (a.res) {
+      if (vec) hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_BF16, true, true>), grid, dim3(256), 0, s, a, vec4);
+      else hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_BF16, false, true>), grid, dim3(256), 0, s, a, vec4);
     } else {
-      if (vec) hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_BF16, true>), grid, dim3(256), 0, s, a, vec4);
-      else hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_BF16, false>), grid, dim3(256), 0, s, a, vec4);
+      if (vec) hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_BF16, true, false>), grid, dim3(256), 0, s, a, vec4);
+      else hipLaunchKernelGGL((linear_mfma_kernel<DIHIP_BF16, false, false>), grid, dim3(256), 0, s, a, vec4);
     }
     return launch_status();
   }
