@@ -71,7 +71,7 @@ __global__ __launch_bounds__(256) void linear_tile_kernel(LinArgs a) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int n = n0 + tx * 4 + j;
-      if (n < a.N) lin_epilogue(a, g, t, n, acc[i][j], WT);
+      if (n < a.N) lin_epilogue<false>(a, g, t, n, acc[i][j], WT);
     }
   }
 }
@@ -415,7 +415,7 @@ __global__ __launch_bounds__(64 * WV, 2) void linear_stream_lds_kernel(LinArgs a
       return v;
     };
     if constexpr (GATED) lin_gated4(a, lo + t, n, sum(f, l), sum(f2, l2), vec4);
-    else lin_epilogue4(a, g, lo + t, n, sum(f, l), lin_bias4(a, g, n, vec4), vec4);
+    else lin_epilogue4<!SEG>(a, g, lo + t, n, sum(f, l), lin_bias4(a, g, n, vec4), vec4);
   }
 }
 template <int ROWS, int TF, bool SEG, bool GATED>
@@ -788,7 +788,7 @@ __global__ __launch_bounds__(256) void linear_fewcols_kernel(LinArgs a) {
       acc = __builtin_fmaf(__uint_as_float(wv[3] & 0xffff0000u), hi[3], acc);
     }
     acc = wave_sum(acc);
-    if (lane == 0) lin_epilogue(a, 0, t, n, acc, DIHIP_BF16);
+    if (lane == 0) lin_epilogue<false>(a, 0, t, n, acc, DIHIP_BF16);
   }
 }
 

@@ -238,7 +238,7 @@ __global__ __launch_bounds__(64 * WM * WN, (WM * WN) / 4) void linear_pipe_kerne
           *reinterpret_cast<f32x4_t*>(to + n4) = u;
         }
       } else if (parts == 1) {
-        lin_epilogue4(a, g, t, n, v, b, vec4);
+        lin_epilogue4<!MAP>(a, g, t, n, v, b, vec4);
       } else {
         *reinterpret_cast<f32x4_t*>(slab + (((size_t)part * a.T + t) * gridDim.y + g) * n4 + n) = v;
       }
