@@ -344,7 +344,7 @@ class GroupedQueryAttention:
         q, gate = a, a[:, self.g_lo:] if self.head_gate else None
         if self.out_gain is not None:
             gate = self.out_gain.expand(ctx.T, H)
-        if self.step and ctx.math == so.MATH_BF16 and ctx.max_count == 1:
+        if self.step and ctx.math == so.MATH_BF16 and ctx.max_count == 1 and so.gqa_decode_step_pays(ctx.E * G, D, V, ctx.max_pos):
             return so.gqa_decode_step(a, 0, self.k_lo, self.v_lo, H, G, D, V, self.q_norm, self.k_norm, ctx.eps, self.freq, self.rot_dims, self.layout, self.mag, ktable, vtable,
                                       ctx.tok_pos, ctx.ent_slot, ctx.ent_row0, ctx.max_pos, self.scale, self.sink, self.sink_mode, self.softcap, gate,
                                       out=out if out is not None else ctx.act_buffer(H * V))

@@ -370,16 +370,44 @@ def gqa_decode_step_supported(H, G, D, DV, table, rot_dims):
     return bool(lib().dihip_gqa_decode_step_supported(H, G, D, DV, table.span_len, _DT[table.dtype], int(rot_dims)))
 
 
+def gqa_decode_step_splits(units, D, DV, max_pos):
+    """over how many workgroups each of `units` (request, key head) pairs walks its keys"""
+    tiles = (max_pos + 64) // 64
+    if tiles <= 16:      # a launch more costs what a split gives (8 key heads, 12 tiles: 11.0 us, in two splits 12.4; 24 tiles: 15.5, in five 12.4, in six 11.1)
+        return 1
+    # past that a tile to each wave, while every workgroup finds a unit of its own; with heads of 64 / 64 two share one, which long walks need (12000 keys, 96 pairs: in 2 splits 64.1 us,
+    # in 5 57.8, the two launches 56.8; 160 pairs: in 1 117.9, in 3 102.1, 101.8; 192 pairs in 2, no third fits: 132, in 1 126)
+    slots = 512 if D + DV == 128 and tiles >= 96 and 64 < units <= 170 else 256
+    return max(1, min(slots // max(1, units), (tiles + 3) // 4))
+
+
+def gqa_decode_step_pays(units, D, DV, max_pos):
+    """whether gqa_decode_step is no slower than qkv_prep_append and gqa_attn_mc for `units` (request, key head) pairs.  A workgroup takes 512 bytes of LDS for each of D + DV, so a unit
+    holds one (256) or two (128), and the two launches' many more; us, one launch (two launches):
+      * up to 256 pairs it is faster: 32 heads over 8 of 128, 32 requests of 700 22.5 (31.2), of 4000 94.0 (110);
+      * not many more than the units are a last round that is nearly empty, and long walks show it: 32 heads of 128, 320 pairs of 900 keys faster, of 1500 48.6 (47.6), of 6000 205 (184),
+        of 12000 401 (353), 384 pairs of 6000 219 (206), 512 pairs of 6000 262 (265); heads of 64, 384 pairs of 2000 keys 35.1 (42.2), of 3000 60.6 (59.3; 320 pairs 47.0, 56.4), of 4000 89.1 (81.1),
+        of 12000 250 (220),
+        512 pairs of 12000 291 (272), 640 pairs 397 (396);
+      * in many rounds of few keys each round waits for its own chain of loads: 32 heads of 128, 2048 pairs of 10 / 100 / 400 keys 49.0 / 52.5 / 103 (32.5 / 40.8 / 98.6), 896 pairs 25.6 /
+        28.0 / 45.7 (17.9 / 23.9 / 44.4), 768 pairs 19.4 / 21.2 / 39.6 (16.7 / 22.3 / 44.6); heads of 64, 2048 pairs of 100 faster.
+        (From 257 pairs on the first keys of a 512-key bucket are up to 3 us slower, 32 heads of 128, 416 pairs of 10 / 100 / 500 keys 12.3 / 12.1 / 24.9 (11.6 / 13.0 / 26.2): a captured step
+        knows the bucket alone.)"""
+    if units <= 256 or units > 65535:        # (more than the two launches take)
+        return True
+    if units <= (512 if D + DV == 128 else 448):
+        return max_pos < (1024 if D + DV == 256 else 3584)
+    return D + DV < 256 or units < 896 or max_pos >= 512
+
+
 def gqa_decode_step(a, q_off, k_off, v_off, H, G, D, DV, qnorm, knorm, eps, freq, rot_dims, layout, mag, ktable, vtable, tok_pos, ent_slot, ent_row0, max_pos, scale,
                     sink=None, sink_mode=SINK_NONE, softcap=0.0, gate=None, out=None, nsplit=None):
     """one token of each request: qkv_prep_append and gqa_attn_mc in one launch (the rows a are left as they are); max_pos: the largest position (a host number)"""
     T, E = a.shape[0], ent_slot.shape[0]
     assert a.dtype == torch.float32 and ktable.row_elems == G * D and vtable.row_elems == G * DV and ktable.dtype == vtable.dtype
     o = out if out is not None else torch.empty(T, H * DV, dtype=torch.float32, device=a.device)
-    if nsplit is None:       # up to 16 tiles a launch more costs what a split gives (8 key heads, 12 tiles: 11.0 us, in two splits 12.4; 24 tiles: 15.5, in five 12.4, in six
-        # 11.1); past that a tile to each wave, while every workgroup finds a unit of its own
-        tiles = (max_pos + 64) // 64
-        nsplit = 1 if tiles <= 16 else max(1, min(256 // max(1, E * G), (tiles + 3) // 4))
+    if nsplit is None:
+        nsplit = gqa_decode_step_splits(E * G, D, DV, max_pos)
     need = int(lib().dihip_gqa_attn_mc_workspace_bytes(T, H, DV, nsplit)) if nsplit > 1 else 0
     ws = torch.empty(need, dtype=torch.uint8, device=a.device) if need else None
     wn = qnorm if qnorm is not None else knorm

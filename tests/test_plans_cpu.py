@@ -8,6 +8,7 @@ import importlib
 import os
 import subprocess
 import sys
+import types
 
 import pytest
 
@@ -135,3 +136,30 @@ def test_gated_linear_attention_workspace_counts_the_chunks_there_are(H, counts)
     assert fits, (need // size, counts)
     if counts == [700] + [1] * 24:
         assert need < 60e6
+
+
+@pytest.mark.parametrize("H,G,D,E,keys,one", [
+    (32, 8, 128, 32, 12000, True), (32, 32, 128, 8, 10, True), (32, 32, 128, 10, 900, True), (32, 32, 128, 10, 1500, False), (32, 8, 128, 48, 6000, False), (32, 32, 128, 16, 6000, True),
+    (16, 16, 64, 24, 3000, True), (16, 16, 64, 24, 4000, False), (16, 16, 64, 32, 12000, False), (32, 32, 64, 20, 12000, True), (32, 32, 64, 64, 100, True), (32, 32, 128, 24, 100, True),
+    (32, 32, 128, 28, 100, False), (32, 32, 128, 64, 400, False), (32, 32, 128, 64, 1000, True), (32, 32, 128, 2047, 100, False), (32, 32, 128, 2048, 100, True)])
+def test_decoding_step_of_attention_in_one_launch_only_where_it_is_no_slower(monkeypatch, H, G, D, E, keys, one):
+    """More (request, key head) pairs than units, with long walks or in many short rounds: the two launches, which these measured faster (and which take 65535 pairs)."""
+    mixers, so = importlib.import_module("dash-infer_amd.mixers"), importlib.import_module("dash-infer_amd.seq_ops")
+    taken = []
+    for name in ("gqa_decode_step", "gqa_attn_mc"):
+        monkeypatch.setattr(so, name, lambda *a, _n=name, **k: taken.append(_n))
+    m = mixers.GroupedQueryAttention.__new__(mixers.GroupedQueryAttention)
+    m.__dict__.update(H=H, G=G, D=D, V=D, k_lo=H * D, v_lo=(H + G) * D, ktables=[None], vtables=[None], head_gate=False, elem_gate=False, out_gain=None, step=True, mc=True, taps=0, talk=None,
+                      differential=None, value_mix=None, maps=1, window=0, keep_first=0, q_norm=None, k_norm=None, freq=None, rot_dims=0, layout=0, mag=1.0, scale=1.0, sink=None, sink_mode=0,
+                      softcap=0.0, _prep=lambda *a: taken.append("prep"))
+    ctx = types.SimpleNamespace(E=E, T=E, math=so.MATH_BF16, max_count=1, max_pos=(keys + 511) // 512 * 512 - 1, eps=1e-6, tok_pos=None, ent_slot=None, ent_row0=None, ent_count=None,
+                                act_buffer=lambda n: None)
+    m.mix(ctx, None)
+    assert taken == (["gqa_decode_step"] if one else ["prep", "gqa_attn_mc"])
+
+
+@pytest.mark.parametrize("units,D,DV,keys,want", [(96, 64, 64, 12000, 5), (160, 64, 64, 12000, 3), (192, 64, 64, 12000, 1), (96, 64, 128, 12000, 2), (96, 64, 64, 1000, 1), (8, 128, 128, 12000, 32),
+                                                  (48, 64, 64, 12000, 5), (1, 128, 128, 1025, 6), (300, 128, 128, 12000, 1)])
+def test_splits_of_the_decoding_steps_attention(units, D, DV, keys, want):
+    so = importlib.import_module("dash-infer_amd.seq_ops")
+    assert so.gqa_decode_step_splits(units, D, DV, (keys + 511) // 512 * 512 - 1) == want
