@@ -382,21 +382,20 @@ def gqa_decode_step_splits(units, D, DV, max_pos):
 
 
 def gqa_decode_step_pays(units, D, DV, max_pos):
-    """whether gqa_decode_step is no slower than qkv_prep_append and gqa_attn_mc for `units` (request, key head) pairs.  A workgroup takes 512 bytes of LDS for each of D + DV, so a unit
-    holds one (256) or two (128), and the two launches' many more; us, one launch (two launches):
-      * up to 256 pairs it is faster: 32 heads over 8 of 128, 32 requests of 700 22.5 (31.2), of 4000 94.0 (110);
-      * not many more than the units are a last round that is nearly empty, and long walks show it: 32 heads of 128, 320 pairs of 900 keys faster, of 1500 48.6 (47.6), of 6000 205 (184),
-        of 12000 401 (353), 384 pairs of 6000 219 (206), 512 pairs of 6000 262 (265); heads of 64, 384 pairs of 2000 keys 35.1 (42.2), of 3000 60.6 (59.3; 320 pairs 47.0, 56.4), of 4000 89.1 (81.1),
-        of 12000 250 (220),
-        512 pairs of 12000 291 (272), 640 pairs 397 (396);
-      * in many rounds of few keys each round waits for its own chain of loads: 32 heads of 128, 2048 pairs of 10 / 100 / 400 keys 49.0 / 52.5 / 103 (32.5 / 40.8 / 98.6), 896 pairs 25.6 /
-        28.0 / 45.7 (17.9 / 23.9 / 44.4), 768 pairs 19.4 / 21.2 / 39.6 (16.7 / 22.3 / 44.6); heads of 64, 2048 pairs of 100 faster.
-        (From 257 pairs on the first keys of a 512-key bucket are up to 3 us slower, 32 heads of 128, 416 pairs of 10 / 100 / 500 keys 12.3 / 12.1 / 24.9 (11.6 / 13.0 / 26.2): a captured step
-        knows the bucket alone.)"""
+    """whether gqa_decode_step is no slower than qkv_prep_append and gqa_attn_mc for `units` (request, key head) pairs.  A workgroup takes 512 bytes of LDS for each of D + DV, so a compute
+    unit holds one (256) or two (128) of them, and many more of the two launches'; one launch (two launches) in us, keys and values not in a cache:
+      * up to 256 pairs it is faster: 32 heads over 8 of 128, 32 requests of 700 keys 22.5 (31.2), of 4000 94.0 (110);
+      * not many more leave the last round nearly empty, which long walks show: 32 heads of 128, 320 pairs of 500 keys 27.5 (26.5), of 900 42.3 (39.5), of 6000 205 (184), 384 pairs of 900
+        44.3 (42.1), of 6000 219 (206), 416 pairs of 6000 226 (218), 448 pairs of 900 57.6 (60.7), of 1400 83.3 (87.8), 512 pairs of 6000 262 (265);
+        heads of 64 / 128, 384 pairs of 3000 113 (115), of 4000 116 (109); heads of 64, 320 pairs of 2000 54.5 (52.5), of 4000 107 (95.5), 448 pairs of 3000 97.4 (99.6), of 4000 127 (122), 512 pairs of 4000 107 (102), of 12000 291 (272), 640 of 12000 397 (396);
+      * in many rounds of few keys each round waits for its own chain of loads: 32 heads of 128, 2048 pairs of 10 / 100 / 400 keys 48.5 / 54.8 / 122 (33.9 / 43.0 / 122), 896 pairs 24.8 /
+        28.9 / 52.5 (21.2 / 27.1 / 50.3), 768 pairs 19.5 / 23.6 / 49.9 (19.4 / 25.1 / 56.8); heads of 64, 2048 pairs of 100 keys 25.2 (27.2)."""
     if units <= 256 or units > 65535:        # (more than the two launches take)
         return True
-    if units <= (512 if D + DV == 128 else 448):
-        return max_pos < (1024 if D + DV == 256 else 3584)
+    if units <= 400:
+        return max_pos < {256: 512, 192: 3584, 128: 2048}[D + DV]
+    if units <= 512:
+        return max_pos < 3584 or (units > 448 and D + DV > 128)
     return D + DV < 256 or units < 896 or max_pos >= 512
 
 

@@ -139,8 +139,8 @@ def test_gated_linear_attention_workspace_counts_the_chunks_there_are(H, counts)
 
 
 @pytest.mark.parametrize("H,G,D,E,keys,one", [
-    (32, 8, 128, 32, 12000, True), (32, 32, 128, 8, 10, True), (32, 32, 128, 10, 900, True), (32, 32, 128, 10, 1500, False), (32, 8, 128, 48, 6000, False), (32, 32, 128, 16, 6000, True),
-    (16, 16, 64, 24, 3000, True), (16, 16, 64, 24, 4000, False), (16, 16, 64, 32, 12000, False), (32, 32, 64, 20, 12000, True), (32, 32, 64, 64, 100, True), (32, 32, 128, 24, 100, True),
+    (32, 8, 128, 32, 12000, True), (32, 32, 128, 8, 10, True), (32, 32, 128, 10, 500, True), (32, 32, 128, 10, 900, False), (32, 32, 128, 13, 2000, True), (32, 32, 128, 13, 6000, False), (32, 8, 128, 48, 6000, False), (32, 32, 128, 16, 6000, True),
+    (16, 16, 64, 24, 2000, True), (16, 16, 64, 24, 2100, False), (16, 16, 64, 28, 3000, True), (16, 16, 64, 28, 4000, False), (16, 16, 64, 32, 12000, False), (32, 32, 64, 20, 12000, True), (32, 32, 64, 64, 100, True), (32, 32, 128, 24, 100, True),
     (32, 32, 128, 28, 100, False), (32, 32, 128, 64, 400, False), (32, 32, 128, 64, 1000, True), (32, 32, 128, 2047, 100, False), (32, 32, 128, 2048, 100, True)])
 def test_decoding_step_of_attention_in_one_launch_only_where_it_is_no_slower(monkeypatch, H, G, D, E, keys, one):
     """More (request, key head) pairs than units, with long walks or in many short rounds: the two launches, which these measured faster (and which take 65535 pairs)."""
