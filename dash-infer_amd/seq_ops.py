@@ -88,6 +88,13 @@ def linear_residual_dyt(x, w, stream_x, a=None, norm=None):
     assert w.shape == (N, K) and w.is_contiguous() and x.dtype == w.dtype == torch.bfloat16
     assert stream_x.shape == (T, N) and stream_x.is_contiguous() and stream_x.dtype == torch.float32
     assert a is None or (a.shape == (T, N) and a.dtype == torch.float32)
+    if T > LINEAR_FEW_ROWS and K % 64 and ((T + 127) // 128) * ((N + 127) // 128) <= 64:
+        # 128 x 128 tiles of a workgroup each, that leave most units idle while a few compute the tanh of all elements: 1000 -> 2048 65 rows 31.0 us (the two launches 28.4), 330 rows (48
+        # tiles) 33.4 (31.6), 700 rows (96) 35.5 (42.8); 1000 -> 4096 130 rows (64) 32.9 (30.8), 330 rows (96) 35.4 (39.6); 2056 -> 1024 330 rows (24) 50.1 (49.3), 1200 rows (80) 66.3 (66.6)
+        if norm is not None:
+            assert norm[1].dtype == norm[2].dtype == torch.bfloat16 and norm[1].shape == norm[2].shape == (N,)
+        y = linear(x, w, math=MATH_BF16)
+        return add_dyt(stream_x, y if a is None else a, None if a is None else y, norm, x_out=stream_x, want16=True)[1]
     alpha, nw, nb, h16 = 0.0, None, None, None
     if norm is not None:
         alpha, nw, nb = norm

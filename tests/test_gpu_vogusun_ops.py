@@ -72,6 +72,13 @@ def test_product_that_ends_in_the_residual_step_and_the_norm(so, T, N, K, left, 
     assert torch.equal(out, h16) if normed else out is None
 
 
+# K no whole number of 64: 56 and 64 tiles (the two launches), 72 (one)
+@pytest.mark.parametrize("T,N,K", [(1000, 896, 200), (1024, 897, 200), (1100, 1001, 76), (1100, 1004, 1000)])
+@pytest.mark.parametrize("left,normed", [(True, True), (False, True), (True, False)])
+def test_product_of_an_uneven_k_that_ends_in_the_residual_step(so, T, N, K, left, normed):
+    test_product_that_ends_in_the_residual_step_and_the_norm(so, T, N, K, left, normed)
+
+
 def test_embedding_and_its_norm(so):
     g = torch.Generator("cuda").manual_seed(5)
     table, w, b = (torch.randn(*s, generator=g, device="cuda").bfloat16() for s in ((50, 1100), (1100,), (1100,)))

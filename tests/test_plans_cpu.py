@@ -163,3 +163,23 @@ def test_decoding_step_of_attention_in_one_launch_only_where_it_is_no_slower(mon
 def test_splits_of_the_decoding_steps_attention(units, D, DV, keys, want):
     so = importlib.import_module("dash-infer_amd.seq_ops")
     assert so.gqa_decode_step_splits(units, D, DV, (keys + 511) // 512 * 512 - 1) == want
+
+
+@pytest.mark.parametrize("T,N,K,one", [(64, 2048, 1000, True), (65, 2048, 1000, False), (330, 2048, 1000, False), (700, 2048, 1000, True), (65, 2048, 1024, True), (1025, 1024, 200, True),
+                                       (1024, 1024, 200, False)])
+@pytest.mark.parametrize("left", [True, False])
+def test_products_with_the_residual_step_take_it_along_only_where_that_is_no_slower(monkeypatch, T, N, K, one, left):
+    """K no whole number of 64 and few tiles: the product, then the step (the sums in the same order)"""
+    so = importlib.import_module("dash-infer_amd.seq_ops")
+    torch = so.torch
+    taken = []
+    real, lib = so.lib(), types.SimpleNamespace(dihip_linear_residual_dyt=lambda *a: taken.append("one") or 0)
+    lib.dihip_linear_workspace_bytes = real.dihip_linear_workspace_bytes
+    monkeypatch.setattr(so, "lib", lambda: lib)
+    monkeypatch.setattr(so, "stream", lambda: 0)
+    monkeypatch.setattr(so, "linear", lambda *a, **k: taken.append("linear") or "y")
+    monkeypatch.setattr(so, "add_dyt", lambda x, a, b, norm, x_out, want16: taken.append((a is not None, b is not None, x is x_out, want16)) or (None, "h16"))
+    x, w, s, bf = torch.empty(T, K, dtype=torch.bfloat16), torch.empty(N, K, dtype=torch.bfloat16), torch.empty(T, N), torch.empty(N, dtype=torch.bfloat16)
+    h = so.linear_residual_dyt(x, w, s, torch.empty(T, N) if left else None, (0.5, bf, bf))
+    assert taken == (["one"] if one else ["linear", (True, left, True, True)])
+    assert h.shape == (T, N) if one else h == "h16"
